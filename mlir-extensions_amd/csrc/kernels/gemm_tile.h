@@ -134,6 +134,9 @@ struct StoreF32 {       // C = acc
   __device__ __forceinline__ void operator()(int64_t m, int64_t n, int64_t N, float acc) const {
     C[m * N + n] = acc; // ordinary store: C stays in the last-level cache for whoever reads it next
   }
+  __device__ __forceinline__ void vec4(int64_t m, int64_t n, int64_t N, f32x4 acc) const {
+    *reinterpret_cast<f32x4u *>(C + m * N + n) = acc;
+  }
 };
 // Epilogues that read C first also offer the two halves separately -- fetch() the old value, put() the new one
 // computed from it -- so that the tiled path can issue a whole batch of reads before the first dependent store
@@ -148,6 +151,10 @@ struct AccumulateF32 {  // C = C + acc   (the reference kernel loads C as its in
   }
   __device__ __forceinline__ void operator()(int64_t m, int64_t n, int64_t N, float acc) const {
     put(m, n, N, acc, fetch(m, n, N));
+  }
+  __device__ __forceinline__ void vec4(int64_t m, int64_t n, int64_t N, f32x4 acc) const {
+    f32x4u *p = reinterpret_cast<f32x4u *>(C + m * N + n);
+    *p = *p + acc;
   }
 };
 struct BiasAccumulateF32 { // C = bias[n] + (C + acc)  (bias.mlir:88-94,112-113)
@@ -680,6 +687,21 @@ __device__ __forceinline__ void gemm_tile_mainloop(f32x4 (&acc)[FI][FJ], const u
   wait_vmcnt<0>();
 }
 
+template <bool kValue> struct BoolConstant { static constexpr bool value = kValue; };
+
+// Columns n .. n + 3 of row m, those of them that exist.
+template <typename Epi>
+__device__ __forceinline__ void store_columns(const Epi &epi, int64_t m, int64_t n, int64_t N, f32x4 v) {
+  if (n + 4 <= N) {
+    epi.vec4(m, n, N, v);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (n + r < N)
+        epi(m, n + r, N, v[r]);
+  }
+}
+
 // The epilogue of a tile: what `epi` does with every element of acc that lies inside C.
 template <typename Epi, int kProbe = 0>
 __device__ __forceinline__ void gemm_tile_epilogue(f32x4 (&acc)[FI][FJ], int64_t M, int64_t N, Epi epi, int64_t m0,
@@ -743,16 +765,14 @@ __device__ __forceinline__ void gemm_tile_epilogue(f32x4 (&acc)[FI][FJ], int64_t
         for (int j = 0; j < FJ; ++j)
           epi.vec4(mBase + i * 16, nBase + j * 16, N, acc[i][j]);
     } else {
+      // An edge tile stores groups of four columns as well; only the group that N cuts goes element by element
+      // (one store and one bias load per element made a ragged MLP tile 20 us longer than an even one).
 #pragma unroll
       for (int i = 0; i < FI; ++i)
 #pragma unroll
         for (int j = 0; j < FJ; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int64_t m = mBase + i * 16, n = nBase + j * 16 + r;
-            if (m < M && n < N)
-              epi(m, n, N, acc[i][j][r]);
-          }
+          if (mBase + i * 16 < M && nBase + j * 16 < N)
+            store_columns(epi, mBase + i * 16, nBase + j * 16, N, acc[i][j]);
     }
   } else {
     // Blocks j and j+1 sit side by side in C.  Swapping the odd 16-lane rows of one with the
@@ -773,17 +793,28 @@ __device__ __forceinline__ void gemm_tile_epilogue(f32x4 (&acc)[FI][FJ], int64_t
                        : "+v"(acc[i][j][r]), "+v"(acc[i][j + 1][r])); // -> rows r, r+8 | rows r+4, r+12
         }
     if constexpr (ReadsC<Epi>::value) {
-      if (interior) {
-        // the old values of row block i + 1 are requested before row block i is combined and stored
+      // The old values of row block i + 1 are requested before row block i is combined and stored.  An edge tile
+      // does the same with the addresses of what lies outside C moved to C's last row and column, and stores what
+      // lies inside: loads under a condition would each be waited for before the next (33 us for a 920 x 2064
+      // problem whose arithmetic takes 5).
+      auto finish = [&](auto edge) {
+        constexpr bool kEdge = decltype(edge)::value;
         float old[2][FJ * 4];
+        auto at = [&](int i, int r) { return kEdge ? min(mBase + i * 16 + r, M - 1) : mBase + i * 16 + r; };
+        auto col = [&](int j) { return kEdge ? min(nBase + j * 16, N - 1) : nBase + j * 16; };
         auto fetch_block = [&](int i, float(&into)[FJ * 4]) {
 #pragma unroll
           for (int j = 0; j < FJ; j += 2)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              into[j * 4 + r] = epi.fetch(mBase + i * 16 + r, nBase + j * 16, N);
-              into[j * 4 + 4 + r] = epi.fetch(mBase + i * 16 + r + 4, nBase + j * 16, N);
+              into[j * 4 + r] = epi.fetch(at(i, r), col(j), N);
+              into[j * 4 + 4 + r] = epi.fetch(at(i, r + 4), col(j), N);
             }
+        };
+        auto put = [&](int i, int r, int j, float v, float o) {
+          const int64_t m = mBase + i * 16 + r, n = nBase + j * 16;
+          if (!kEdge || (m < M && n < N))
+            epi.put(m, n, N, v, o);
         };
         fetch_block(0, old[0]);
 #pragma unroll
@@ -794,12 +825,16 @@ __device__ __forceinline__ void gemm_tile_epilogue(f32x4 (&acc)[FI][FJ], int64_t
           for (int j = 0; j < FJ; j += 2)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              epi.put(mBase + i * 16 + r, nBase + j * 16, N, acc[i][j][r], old[i & 1][j * 4 + r]);
-              epi.put(mBase + i * 16 + r + 4, nBase + j * 16, N, acc[i][j + 1][r], old[i & 1][j * 4 + 4 + r]);
+              put(i, r, j, acc[i][j][r], old[i & 1][j * 4 + r]);
+              put(i, r + 4, j, acc[i][j + 1][r], old[i & 1][j * 4 + 4 + r]);
             }
         }
-        return;
-      }
+      };
+      if (interior)
+        finish(BoolConstant<false>{});
+      else
+        finish(BoolConstant<true>{});
+      return;
     }
     if (interior) {
 #pragma unroll
@@ -1024,21 +1059,25 @@ __device__ __forceinline__ bool streamk_applies(const void *A, const void *B, in
          (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && int(gridDim.x * gridDim.y) <= kStreamKMaxWorkgroups;
 }
 
+// What the MFMA paths take: 16-byte aligned rows in memory, i.e. K % 8 == 0 (rows of A [M,K], of B [N,K]), and
+// as a row of B [K,N] (of A [K,M]) is N (M) elements long, those multiples of 8 as well.  K need not fill the
+// last step: its copies fetch zeros beyond K.  M and N need not divide the tile: edge tiles multiply padding and
+// store what exists.  An operand whose rows are strided in memory is addressed with 32-bit byte offsets from one
+// buffer descriptor, so it has to stay below 2 GiB; a k-contiguous one below 4 Mi elements per row.
+template <bool kAT, bool kBT>
+__device__ __forceinline__ bool mfma_takes(const void *A, const void *B, int64_t M, int64_t N, int64_t K) {
+  constexpr int64_t kMaxBytes = int64_t(1) << 31, kMaxRow = int64_t(1) << 22;
+  const bool fitsA = kAT ? K * M * 2 < kMaxBytes : K < kMaxRow;
+  const bool fitsB = kBT ? K < kMaxRow : K * N * 2 < kMaxBytes;
+  return M > 0 && N > 0 && K > 0 && K % 8 == 0 && (kBT || N % 8 == 0) && (!kAT || M % 8 == 0) && fitsA && fitsB &&
+         ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
+}
+
 // kWideOk: take A as 64-k-wide slabs where the shape allows (A [M,K], K a multiple of 64)
 template <typename T, bool kAT, bool kBT, int kProbe = 0, bool kWideOk = true, typename Epi>
 __device__ __forceinline__ void gemm_dispatch(const uint16_t *A, const uint16_t *B, int64_t M, int64_t N, int64_t K,
                                               Epi epi, char *lds) {
-  // The MFMA path wants 16-byte aligned rows in memory: K % 8 == 0 (rows of A [M,K], of B [N,K]), and a
-  // row of B [K,N] (or of A [K,M] when transposed) is N (M) elements long, so those must be multiples
-  // of 8 as well.  K need not fill the last 32-wide step: its copies fetch zeros beyond K.  M and N need not divide the tile: edge tiles multiply padding and store what exists.
-  // An operand whose rows are strided in memory is addressed with 32-bit byte offsets from one
-  // buffer descriptor, so it has to stay below 2 GiB; a k-contiguous one below 4 Mi elements per row.
-  constexpr int64_t kMaxBytes = int64_t(1) << 31, kMaxRow = int64_t(1) << 22;
-  const bool fitsA = kAT ? K * M * 2 < kMaxBytes : K < kMaxRow;
-  const bool fitsB = kBT ? K < kMaxRow : K * N * 2 < kMaxBytes;
-  const bool tileable = M > 0 && N > 0 && K > 0 && K % 8 == 0 && (kBT || N % 8 == 0) && (!kAT || M % 8 == 0) &&
-                        fitsA && fitsB &&
-                        ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
+  const bool tileable = mfma_takes<kAT, kBT>(A, B, M, N, K);
   if (!kAT && kWideOk && tileable && K % (2 * RK) == 0)
     gemm_tiled<T, kAT, kBT, Epi, kProbe, false, !kAT && kWideOk>(A, B, M, N, K, epi, lds);
   else if (tileable && K % RK == 0)
