@@ -5,9 +5,10 @@
  *
  * libimex-hip-kernels.so embeds the code objects (what a `gpu.binary`
  * attribute would hold, cf. lib/Transforms/SerializeSPIRV.cpp:65-69) and
- * answers two questions host code has to settle before calling
+ * answers three questions host code has to settle before calling
  * gpuModuleLoad / gpuKernelGet / gpuLaunchKernel (imex_hip_runtime.h):
- * which blob holds a kernel, and with what grid and block it is launched.
+ * which form of an operator suits a problem's size, which blob holds that
+ * kernel, and with what grid and block it is launched.
  *
  * Kernel argument convention (lib/Conversion/GPUXToLLVM/GPUXToLLVMPass.cpp:571-584):
  * one raw aligned base pointer per memref, scalars by value; `index` is i64.
@@ -50,6 +51,33 @@
  *       WG/gemm_4kx4kx4k_transpose_a.mlir:31-55          dims = {M, N, K}
  *   imex_gemm_bf16_bias_silu_bf16  (A, B, bias, out, M:i64, N:i64, K:i64)
  *       WG/gemm_4kx4kx4k_f16_f16_f32_bias.mlir:88-113 + silu_gpu.mlir.in:3-19
+ *   imex_gemm_f16_f16_f32_t128, imex_gemm_f16_f16_f32_t128x64,
+ *   imex_gemm_f16_f16_f32_t64,
+ *   imex_gemm_f16_f16_f32_t32, imex_gemm_f16_f16_f32_t16
+ *   imex_gemm_f16_f16_f32_acc_t128, imex_gemm_f16_f16_f32_acc_t128x64,
+ *   imex_gemm_f16_f16_f32_acc_t64,
+ *   imex_gemm_f16_f16_f32_acc_t32, imex_gemm_f16_f16_f32_acc_t16
+ *   imex_gemm_bf16_bf16_f32_t128, imex_gemm_bf16_bf16_f32_t128x64,
+ *   imex_gemm_bf16_bf16_f32_t64,
+ *   imex_gemm_bf16_bf16_f32_t32, imex_gemm_bf16_bf16_f32_t16
+ *   imex_gemm_bf16_bf16_f32_acc_t128, imex_gemm_bf16_bf16_f32_acc_t128x64,
+ *   imex_gemm_bf16_bf16_f32_acc_t64,
+ *   imex_gemm_bf16_bf16_f32_acc_t32, imex_gemm_bf16_bf16_f32_acc_t16
+ *   imex_gemm_f16_f16_f16_t128, imex_gemm_f16_f16_f16_t128x64,
+ *   imex_gemm_f16_f16_f16_t64,
+ *   imex_gemm_f16_f16_f16_t32, imex_gemm_f16_f16_f16_t16
+ *   imex_gemm_f16_f16_f32_tb_t128, imex_gemm_f16_f16_f32_tb_t128x64,
+ *   imex_gemm_f16_f16_f32_tb_t64,
+ *   imex_gemm_f16_f16_f32_tb_t32, imex_gemm_f16_f16_f32_tb_t16
+ *   imex_gemm_f16_f16_f32_ta_t128, imex_gemm_f16_f16_f32_ta_t128x64,
+ *   imex_gemm_f16_f16_f32_ta_t64,
+ *   imex_gemm_f16_f16_f32_ta_t32, imex_gemm_f16_f16_f32_ta_t16
+ *   imex_gemm_bf16_bias_silu_bf16_t128, imex_gemm_bf16_bias_silu_bf16_t128x64,
+ *   imex_gemm_bf16_bias_silu_bf16_t64,
+ *   imex_gemm_bf16_bias_silu_bf16_t32, imex_gemm_bf16_bias_silu_bf16_t16
+ *       the operator without the suffix, same arguments, on tiles of 128 x 128, 128 x 64, 64 x 64, 32 x 64 and 16 x 64
+ *       outputs: what imexHipKernelVariant names for problems that would leave most of the chip idle
+ *                                                          dims = {M, N, K}
  *   imex_gemm_bf16_bias_silu_bf16_streamk  (A, B, bias, out, M:i64, N:i64, K:i64, workspace, epoch:i64, spin_limit:i64)
  *       the same operator with the last, partial round of tiles split along K over all workgroups (no
  *       counterpart in the reference); workspace: imexHipStreamKWorkspaceBytes(grid) bytes of device
@@ -83,6 +111,12 @@ const char *imexHipKernelSignature(int index);
  * gpuModuleLoad).  The pointer is stable for the life of the process, so the
  * runtime's by-pointer module cache hits.  NULL if the name is unknown. */
 const void *imexHipKernelModule(const char *kernel, size_t *size);
+
+/* The catalogue kernel to launch for the operator `kernel` on a problem of the given dims: one with the same
+ * arguments and results that is faster at that size, or `kernel` itself (also for dims the kernel does not take).
+ * Every such kernel is correct at every size, as `kernel` itself is; this is advice, not a requirement.  NULL if
+ * the name is unknown. */
+const char *imexHipKernelVariant(const char *kernel, const int64_t *dims, int ndims);
 
 /* Grid (in workgroups), block and dynamic shared memory for `kernel` on a
  * problem of the given dims (see the table above).  Returns 0 on success,

@@ -409,6 +409,7 @@ int runWorkload(const Workload &w, const Options &opt) {
   size_t grid[3] = {1, 1, 1}, block[3] = {static_cast<size_t>(w.probeBlock), 1, 1}, smem = 0;
   size_t blobSize = 0;
   const void *blob = nullptr;
+  const char *kernelName = w.kernel;
   if (w.probe) {
     grid[0] = w.probeGrid ? static_cast<size_t>(w.probeGrid)
                           : static_cast<size_t>((w.dims[0] + w.probeBlock - 1) / w.probeBlock);
@@ -420,18 +421,21 @@ int runWorkload(const Workload &w, const Options &opt) {
     blob = probeBlob.data();
     blobSize = probeBlob.size();
   } else {
-    if (imexHipKernelLaunchShape(w.kernel, w.dims.data(), static_cast<int>(w.dims.size()), grid, block, &smem) != 0) {
+    const int ndims = static_cast<int>(w.dims.size());
+    if (const char *variant = opt.grid > 0 ? nullptr : imexHipKernelVariant(w.kernel, w.dims.data(), ndims))
+      kernelName = variant;
+    if (imexHipKernelLaunchShape(kernelName, w.dims.data(), ndims, grid, block, &smem) != 0) {
       fprintf(stderr, "%s: no launch shape for %s\n", w.name, w.kernel);
       return 1;
     }
-    blob = imexHipKernelModule(w.kernel, &blobSize);
+    blob = imexHipKernelModule(kernelName, &blobSize);
   }
   if (opt.grid > 0) { // every kernel strides over its work, so any grid computes the same thing
     grid[0] = static_cast<size_t>(opt.grid);
     grid[1] = grid[2] = 1;
   }
   void *module = gpuModuleLoad(stream, blob, blobSize);
-  void *kernel = gpuKernelGet(stream, module, w.kernel);
+  void *kernel = gpuKernelGet(stream, module, kernelName);
 
   // Further copies of the tensors for --rotate: set s holds its own buffers, inputs copied from set 0.
   std::vector<std::vector<void *>> sets(1, dev);

@@ -1,0 +1,269 @@
+// Tile code of the MFMA GEMM for problems that leave most of the chip idle under the 256 x 256 tiles of
+// gemm_tile.h: C[M,N] = A[M,K] . B[K,N], A and B f16 or bf16 (also A stored [K,M], B stored [N,K]), f32 sums.
+// Entry points: gemm_small.hip.  The reference kernels these stand for are those of gemm_tile.h.
+//
+// What bounds such a problem is not arithmetic but a chain: a workgroup walks its K loop alone, and with few
+// workgroups the chip waits for that walk.  So: smaller tiles (more workgroups), and inside a workgroup the
+// eight wavefronts share the tile's k as well as its rows and columns -- KG key groups each multiply their own
+// 32-wide slices of every K step -- which makes the walk shorter without a workspace or a second launch.
+//
+//   workgroup   512 lanes = WMC x WNC x KG wavefronts on a TM x TN tile; a K step is BK = 32 KG k;
+//   operands    global -> LDS directly (16 bytes per lane), a ring of S stages, S - 1 of them in flight; the
+//               images and their swizzles follow the LDS service rules of gemm_tile.h: k-contiguous operands as
+//               64-k slabs of 128-byte rows, group c of row r at c ^ ((r >> 1) & 7); strided ones as k rows of TM
+//               (TN) elements whose 32-byte pairs trade places with the k row (pair_swizzle);
+//   registers   the fragments of step t + 1 are read while step t is multiplied (one barrier per step);
+//   result      the product is taken transposed (a lane holds four consecutive columns of a row); the KG partial
+//               tiles meet in LDS (pitch TN + 4 floats: no bank conflicts on either side), are added in group
+//               order and leave as four consecutive columns per lane, whole lines per row.
+//
+// Steps past the end of K are fetched through a descriptor of size zero (nothing moves, LDS gets zeros).
+// Operands whose rows are not 16-byte aligned take gemm_blocked, as in gemm_tile.h.
+
+#ifndef IMEX_HIP_GEMM_SMALL_H
+#define IMEX_HIP_GEMM_SMALL_H
+
+#include "gemm_tile.h"
+
+namespace imexhip_gemm {
+
+// Which 32-byte pair of a strided operand's k row `row` holds pair 0: a transpose read takes, for sixteen lanes,
+// four k rows (row & 3) and, for the next sixteen, the rows eight further; all eight must lie in different banks
+// (256 bytes apart repeats).  NP = pairs per row.
+template <int NP> __device__ __forceinline__ int pair_swizzle(int row) {
+  if constexpr (NP >= 8)
+    return (row & 3) | (((row >> 3) & 1) << 2);
+  else if constexpr (NP == 4) // 128-byte rows: odd and even rows are apart already
+    return ((row >> 1) & 1) | (((row >> 3) & 1) << 1);
+  else if constexpr (NP == 2)
+    return (row >> 3) & 1;
+  else
+    return 0;
+}
+
+// One operand's TR x BK (rows x k) slab per step.
+template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
+  static constexpr int kBytes = TR * BK * 2;
+  static constexpr int kCopies = kBytes / 1024 / kWaves; // 1 KiB copies per wavefront and step
+  static_assert(kBytes % (1024 * kWaves) == 0, "every wavefront makes the same number of whole copies");
+  const uint16_t *base;
+  int range;          // bytes the descriptor covers
+  int voff[kCopies];  // per-lane byte offsets at step 0
+  int voffT[kCopies]; // the same for the last step, pieces at k >= K sent out of range
+  int step;           // bytes per step in memory
+  int dst;            // this wavefront's copies inside the image
+  int rd;             // per-lane LDS address of fragment 0, slice 0 (strided: without the pair)
+  int swz;            // strided: pair swizzle of this lane's k rows
+
+  __device__ __forceinline__ void setup(const uint16_t *ptr, int64_t ld, int64_t first, int w0, int64_t extent,
+                                        int wave, int lane, int kRem) {
+    dst = wave * kCopies * 1024;
+    if constexpr (!kStrided) {
+      const int64_t rows = extent / ld - first;
+      const int last = rows < TR ? int(rows) - 1 : TR - 1;
+      base = ptr + first * ld;
+      range = int(int64_t(last + 1) * ld * 2);
+#pragma unroll
+      for (int q = 0; q < kCopies; ++q) {
+        const int id = wave * kCopies + q, slab = id / (TR / 8), row = (id % (TR / 8)) * 8 + (lane >> 3);
+        const int k = slab * 64 + (((lane & 7) ^ ((row >> 1) & 7)) << 3);
+        voff[q] = int((int64_t(min(row, last)) * ld + k) * 2);
+        voffT[q] = k < kRem ? voff[q] : kOutOfRange;
+      }
+      step = BK * 2;
+      const int r = lane & 15;
+      rd = (w0 + r) * 128 + (((lane >> 4) ^ ((r >> 1) & 7)) << 4);
+      swz = 0;
+    } else {
+      constexpr int kRow = TR * 2, kChunks = kRow / 16; // bytes and 16-byte chunks per k row
+      base = ptr + first;
+      const int64_t bytes = (extent - first) * 2;
+      range = bytes > 0x7fffffff ? 0x7fffffff : int(bytes);
+#pragma unroll
+      for (int q = 0; q < kCopies; ++q) {
+        const int row = (wave * kCopies + q) * (1024 / kRow) + lane / kChunks, chunk = lane % kChunks;
+        const int pair = (chunk >> 1) ^ pair_swizzle<TR / 16>(row);
+        const int64_t col = min(int64_t(pair * 16 + (chunk & 1) * 8), ld - 8 - first); // ld % 8 == 0
+        voff[q] = int((int64_t(row) * ld + col) * 2);
+        voffT[q] = row < kRem ? voff[q] : kOutOfRange;
+      }
+      step = int(BK * ld * 2);
+      const int t = lane & 15, row = (lane >> 4) * 8 + (t >> 2);
+      rd = row * kRow + (t & 3) * 8;
+      swz = pair_swizzle<TR / 16>(row) ^ (w0 / 16);
+    }
+  }
+  // step `kt` of `steps` into the image at `image`
+  __device__ __forceinline__ void dma(LdsChar *lds, int image, int kt, int steps) const {
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0, kt < steps ? range : 0, 0x00020000);
+    const bool tail = kt == steps - 1;
+#pragma unroll
+    for (int q = 0; q < kCopies; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds + image + dst + q * 1024, 16, tail ? voffT[q] : voff[q],
+                                               kt * step, 0, 0);
+  }
+  // fragment f (16 rows from w0 + 16 f), 32-wide slice s of the step
+  __device__ __forceinline__ typename T::Frag read(const char *lds, int image, int f, int s) const {
+    if constexpr (!kStrided) {
+      return *reinterpret_cast<const typename T::Frag *>(lds + image + (s >> 1) * (TR * 128) +
+                                                         ((rd ^ ((s & 1) * 64)) + f * 16 * 128));
+    } else {
+      const char *p = lds + image + s * (32 * TR * 2) + rd + ((f ^ swz) << 5);
+      const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p));
+      const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p + 4 * TR * 2));
+      return __builtin_bit_cast(typename T::Frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+  }
+};
+
+template <int TMv, int TNv, int WMCv, int WNCv, int KGv, int Sv> struct SmallShape {
+  static constexpr int TM = TMv, TN = TNv, WMC = WMCv, WNC = WNCv, KG = KGv, S = Sv;
+  static constexpr int BK = 32 * KG;
+  static constexpr int FI = TM / WMC / 16, FJ = TN / WNC / 16;
+  static constexpr int kStageBytes = (TM + TN) * BK * 2;
+  static constexpr int kPitch = TN + 4; // floats per row of a partial tile in LDS
+  static constexpr int kMergeBytes = KG * TM * kPitch * 4;
+  static constexpr int kLds = S * kStageBytes > kMergeBytes ? S * kStageBytes : kMergeBytes;
+  static constexpr int kWavesPerEu = kLds <= 80 * 1024 ? 4 : 2; // two workgroups on a CU where LDS has room for two
+  static_assert(WMC * WNC * KG == kWaves && BK % 64 == 0 && kLds <= 160 * 1024, "eight wavefronts, one CU's LDS");
+};
+
+template <typename T, bool kAT, bool kBT, typename P, typename Epi>
+__device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                                                int64_t M, int64_t N, int64_t K, Epi epi, char *lds, int64_t m0,
+                                                int64_t n0) {
+  constexpr int FI = P::FI, FJ = P::FJ, S = P::S;
+  LdsChar *ldsBase = (LdsChar *)lds;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave / (P::WMC * P::WNC), wmn = wave % (P::WMC * P::WNC);
+  const int wm = wmn / P::WNC, wn = wmn % P::WNC;
+  const int steps = int((K + P::BK - 1) / P::BK), kRem = int(K - int64_t(steps - 1) * P::BK);
+  SmallOperand<T, kAT, P::TM, P::BK> opA;
+  SmallOperand<T, !kBT, P::TN, P::BK> opB;
+  opA.setup(A, kAT ? M : K, m0, wm * (P::TM / P::WMC), M * K, wave, lane, kRem);
+  opB.setup(B, kBT ? K : N, n0, wn * (P::TN / P::WNC), K * N, wave, lane, kRem);
+  constexpr int kImageA = 0, kImageB = P::TM * P::BK * 2;
+  constexpr int kCopies = decltype(opA)::kCopies + decltype(opB)::kCopies;
+
+  f32x4 acc[FI][FJ];
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+#pragma unroll
+    for (int j = 0; j < FJ; ++j)
+      acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  typename T::Frag af[2][FI], bf[2][FJ];
+  auto dma = [&](int kt, int slot) {
+    opA.dma(ldsBase, slot * P::kStageBytes + kImageA, kt, steps);
+    opB.dma(ldsBase, slot * P::kStageBytes + kImageB, kt, steps);
+  };
+  auto read = [&](int p, int slot) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+      af[p][i] = opA.read(lds, slot * P::kStageBytes + kImageA, i, kg);
+#pragma unroll
+    for (int j = 0; j < FJ; ++j)
+      bf[p][j] = opB.read(lds, slot * P::kStageBytes + kImageB, j, kg);
+  };
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t)
+    dma(t, t);
+  wait_vmcnt<(S - 2) * kCopies>();
+  __builtin_amdgcn_s_barrier();
+  IMEX_FENCE();
+  read(0, 0);
+  // Step t: slab t + 1 has landed and everybody has step t's fragments in registers, so the slot they came from
+  // ... is free one step later (it is the one slab t + S - 1 went into at step t - 1's barrier).
+  int cur = 0; // slot of step t
+  auto step = [&](int p, int t) {
+    const int nxt = cur + 1 == S ? 0 : cur + 1, free = cur == 0 ? S - 1 : cur - 1;
+    dma(t + S - 1, free); // slot of step t - 1: its fragments were in registers before the barrier at the end of t - 1
+    wait_vmcnt<(S - 2) * kCopies>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    IMEX_FENCE();
+    read(p ^ 1, nxt);
+    IMEX_FENCE();
+#pragma unroll
+    for (int j = 0; j < FJ; ++j)
+#pragma unroll
+      for (int s = 0; s < FI; ++s) {
+        const int i = (j & 1) ? FI - 1 - s : s;
+        acc[i][j] = T::mfma(bf[p][j], af[p][i], acc[i][j]);
+      }
+    cur = nxt;
+  };
+  int t = 0;
+  for (; t + 1 < steps; t += 2) {
+    step(0, t);
+    step(1, t + 1);
+  }
+  if (t < steps)
+    step(0, t);
+  wait_vmcnt<0>();
+  __syncthreads(); // the ring is free
+
+  // partial tiles side by side in LDS: lane holds row lane % 16, columns (lane / 16) * 4 .. + 3 of a block
+  float *part = reinterpret_cast<float *>(lds);
+  {
+    float *mine = part + kg * (P::TM * P::kPitch) + (wm * (P::TM / P::WMC) + (lane & 15)) * P::kPitch +
+                  wn * (P::TN / P::WNC) + (lane >> 4) * 4;
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+      for (int j = 0; j < FJ; ++j)
+        *reinterpret_cast<f32x4 *>(mine + i * 16 * P::kPitch + j * 16) = acc[i][j];
+  }
+  __syncthreads();
+  constexpr int kVecs = P::TM * P::TN / 4;
+#pragma unroll
+  for (int u = 0; u < (kVecs + kThreads - 1) / kThreads; ++u) {
+    const int v = u * kThreads + tid;
+    if (kVecs % kThreads == 0 || v < kVecs) {
+      const int r = v / (P::TN / 4), c = (v % (P::TN / 4)) * 4;
+      f32x4 sum = *reinterpret_cast<const f32x4 *>(part + r * P::kPitch + c);
+#pragma unroll
+      for (int g = 1; g < P::KG; ++g)
+        sum += *reinterpret_cast<const f32x4 *>(part + g * (P::TM * P::kPitch) + r * P::kPitch + c);
+      if (m0 + r < M && n0 + c < N)
+        store_columns(epi, m0 + r, n0 + c, N, sum);
+    }
+  }
+}
+
+// Tile number -> tile, as tile_origin of gemm_tile.h: the workgroups of an XCD (ids congruent mod 8) take a compact
+// band of tiles, four tile rows high.
+template <typename P> __device__ __forceinline__ TileOrigin small_tile_origin(int id, int tilesM, int tilesN) {
+  const int tiles = tilesM * tilesN;
+  int pid = id;
+  const int whole = tiles / 8 * 8;
+  if (id < whole)
+    pid = (id % 8) * (whole / 8) + id / 8;
+  const int group = kGroupM * tilesN;
+  const int firstM = (pid / group) * kGroupM;
+  const int groupRows = min(tilesM - firstM, kGroupM);
+  return TileOrigin{int64_t(firstM + (pid % group) % groupRows) * P::TM, int64_t((pid % group) / groupRows) * P::TN};
+}
+
+template <typename T, bool kAT, bool kBT, typename P, typename Epi>
+__device__ __forceinline__ void gemm_small_entry(const uint16_t *A, const uint16_t *B, int64_t M, int64_t N, int64_t K,
+                                                 Epi epi) {
+  __shared__ __attribute__((aligned(16))) char lds[P::kLds];
+  if (!mfma_takes<kAT, kBT>(A, B, M, N, K)) {
+    gemm_blocked<T, kAT, kBT, Epi>(A, B, M, N, K, epi, lds);
+    return;
+  }
+  const int tilesM = int((M + P::TM - 1) / P::TM), tilesN = int((N + P::TN - 1) / P::TN);
+  const int tiles = tilesM * tilesN, workgroups = gridDim.x * gridDim.y;
+  for (int id = blockIdx.y * gridDim.x + blockIdx.x; id < tiles; id += workgroups) {
+    const TileOrigin o = small_tile_origin<P>(id, tilesM, tilesN);
+    gemm_small_tile<T, kAT, kBT, P, Epi>(A, B, M, N, K, epi, lds, o.m0, o.n0);
+    if (id + workgroups < tiles)
+      __syncthreads(); // the partial tiles are read before the ring is filled again
+  }
+}
+
+} // namespace imexhip_gemm
+
+#endif

@@ -94,6 +94,7 @@ _KERNEL_SYMBOLS = {
     "imexHipKernelModule": (C.c_void_p, [C.c_char_p, C.POINTER(C.c_size_t)]),
     "imexHipKernelLaunchShape": (C.c_int, [C.c_char_p, C.POINTER(C.c_int64), C.c_int, C.POINTER(C.c_size_t),
                                            C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]),
+    "imexHipKernelVariant": (C.c_char_p, [C.c_char_p, C.POINTER(C.c_int64), C.c_int]),
     "imexHipStreamKWorkspaceBytes": (C.c_size_t, [C.c_size_t]),
 }
 
@@ -185,6 +186,12 @@ def launch_shape(kernel, dims):
     if rc != 0:
         raise ValueError("imexHipKernelLaunchShape(%s, %s) -> %d" % (kernel, list(dims), rc))
     return tuple(grid), tuple(block), smem.value
+
+
+def variant(kernel, dims):
+    """The catalogue kernel to launch for operator `kernel` at `dims` (imexHipKernelVariant)."""
+    name = kernels().imexHipKernelVariant(kernel.encode(), (C.c_int64 * max(len(dims), 1))(*dims), len(dims))
+    return name.decode() if name else kernel
 
 
 _SIGNATURE_TYPES = {}
@@ -322,7 +329,10 @@ class Stream:
 
     def launch(self, name, dims, args, deps=None, grid=None, block=None):
         """gpuModuleLoad + gpuKernelGet + gpuLaunchKernel; returns the event (or
-        None when the launch shape is empty).  `grid` / `block` replace the catalogue's."""
+        None when the launch shape is empty).  `grid` / `block` replace the catalogue's, and with one of
+        them given it is `name` itself that is launched; otherwise the variant the catalogue advises."""
+        if grid is None and block is None:
+            name = variant(name, dims)
         cat_grid, cat_block, smem = launch_shape(name, dims)
         grid = tuple(grid) if grid is not None else cat_grid
         block = tuple(block) if block is not None else cat_block
@@ -342,6 +352,7 @@ class Stream:
         """Resolve the kernel, its launch shape and its ParamDesc list once and
         return a zero-argument callable that performs just the gpuLaunchKernel
         call (what JIT'd host code does inside a loop)."""
+        name = variant(name, dims)
         grid, block, smem = launch_shape(name, dims)
         if 0 in grid:
             return lambda: None
@@ -358,6 +369,7 @@ class Stream:
 
     def profile(self, name, dims, args, warmups=5, rounds=20, flush_bytes=0, mode=0):
         """Per-launch times in ms (mode 0) or [total ms] over `rounds` back-to-back launches (mode 1)."""
+        name = variant(name, dims)
         grid, block, smem = launch_shape(name, dims)
         fn = self.kernel(name)
         descs, keep = _pack_params(args, signature_types(name))

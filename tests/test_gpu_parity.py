@@ -901,6 +901,43 @@ def test_gemm_ragged_tiles(host, orc, stream, M, N, K):
     assert np.max(np.abs(orc.bfloat_to_float(fused)[rows] - ref)) <= 5e-3 * np.max(np.abs(ref)) + 2.0 ** -9
 
 
+@pytest.mark.parametrize("tile", ["", "_t128", "_t128x64", "_t64", "_t32", "_t16"])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (64, 64, 256), (127, 136, 72), (129, 264, 520), (520, 72, 1032)])
+def test_gemm_every_tile_integers_exact(host, orc, stream, tile, M, N, K):
+    """Each tile size (\"\": 256 x 256) on shapes below, at and beyond its edges in M, N and K, for every operand
+    layout and epilogue.  Integer operands give the exact f32 sum in any order; results rounded to a 16-bit type
+    are that sum's rounding (f16; |sum| < 2048 with K <= 1032 and |a b| <= 1) or within the bias + SiLU bar."""
+    say("gemm tile %s %dx%dx%d" % (tile or "_t256", M, N, K))
+    Mt = (M + 7) // 8 * 8
+    for which in ("plain", "acc", "ta", "tb", "f16", "mlp"):
+        m, dtype = (Mt if which == "ta" else M), "bf16" if which in ("mlp", "acc") else "f16"
+        a = orc.fill_int(m * K, dtype, 95, -1, 1).reshape(m, K)
+        b = orc.fill_int(K * N, dtype, 96, -1, 1).reshape(K, N)
+        want = orc.to_float(a, dtype).astype(np.int64) @ orc.to_float(b, dtype).astype(np.int64)
+        name = {"plain": "f16_f16_f32", "acc": "bf16_bf16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb",
+                "f16": "f16_f16_f16", "mlp": "bf16_bias_silu_bf16"}[which]
+        name = "imex_gemm_" + name + tile
+        bias = orc.fill_int(N, "f32", 97, -3, 3)
+        c0 = np.full((m + 256, N), 7, np.uint16 if which in ("f16", "mlp") else np.float32)
+        bufs = [stream.to_device(np.ascontiguousarray(a.T) if which == "ta" else a),
+                stream.to_device(np.ascontiguousarray(b.T) if which == "tb" else b)]
+        bufs += [stream.to_device(bias)] if which == "mlp" else []
+        bufs.append(stream.to_device(c0))
+        stream.launch(name, [m, N, K], bufs + [m, N, K], grid=host.launch_shape(name, [m, N, K])[0])
+        stream.wait()
+        got = stream.from_device(bufs[-1], c0.shape, c0.dtype)
+        for p in bufs:
+            stream.free(p)
+        assert np.array_equal(got[m:], c0[m:]), "%s wrote past row %d" % (name, m)
+        if which == "mlp":
+            ref = orc.bfloat_to_float(orc.bias_silu_bf16(want.astype(np.float32), bias))
+            assert np.max(np.abs(orc.bfloat_to_float(got[:m]) - ref)) <= 2.0 ** -7 * np.max(np.abs(ref)) + 1e-6
+        elif which == "f16":
+            assert np.array_equal(orc.half_to_float(got[:m]).astype(np.int64), want), name
+        else:
+            assert np.array_equal(got[:m].astype(np.int64), want + (7 if which == "acc" else 0)), name
+
+
 @pytest.mark.parametrize("which,M,N,K", [("ta", 248, 264, 64), ("ta", 8, 8, 32), ("tb", 100, 37, 64), ("tb", 300, 515, 96)])
 def test_gemm_ragged_tiles_transposed_operands(host, orc, stream, which, M, N, K):
     """Edge tiles with A stored [K,M] (M % 8 == 0) or B stored [N,K] (any N)."""

@@ -149,6 +149,29 @@ def test_launch_shapes(host):
         ls("nope", [1])
 
 
+def test_kernel_variants(host):
+    """What imexHipKernelVariant names is in the catalogue, takes the operator's arguments, and stays the operator
+    itself where that is the fastest form or the MFMA paths do not take the shape."""
+    v = host.variant
+    assert v("imex_gemm_f16_f16_f32", [4096, 4096, 4096]) == "imex_gemm_f16_f16_f32"
+    assert v("imex_gemm_bf16_bias_silu_bf16", [4096, 11008, 4096]) == "imex_gemm_bf16_bias_silu_bf16"
+    assert v("imex_gemm_f16_f16_f32_tb", [1000, 1000, 1000]) == "imex_gemm_f16_f16_f32_tb_t64"
+    assert v("imex_relu_f32", [1000]) == "imex_relu_f32"
+    assert host.kernels().imexHipKernelVariant(b"nope", None, 0) is None
+    seen = set()
+    for base in ("imex_gemm_f16_f16_f32", "imex_gemm_f16_f16_f32_acc", "imex_gemm_bf16_bf16_f32", "imex_gemm_f16_f16_f16",
+                 "imex_gemm_bf16_bf16_f32_acc", "imex_gemm_bf16_bias_silu_bf16", "imex_gemm_f16_f16_f32_ta",
+                 "imex_gemm_f16_f16_f32_tb"):
+        for m in (1, 16, 64, 300, 1000, 2048):
+            for n in (8, 64, 1000, 4096):
+                for k in (8, 256, 1000, 4096):
+                    name = v(base, [m, n, k])
+                    assert name.startswith(base) and host.signature_types(name) == host.signature_types(base)
+                    assert host.launch_shape(name, [m, n, k])[0][0] >= 1
+                    seen.add(name[len(base):])
+    assert {"_t128", "_t64", "_t32", "_t16"} <= seen
+
+
 def test_param_desc_packing(host):
     descs, keep = host._pack_params([host.Ptr(0x1000), 7, 2.5])
     assert C.sizeof(host.ParamDesc) == 16
