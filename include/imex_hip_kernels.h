@@ -30,6 +30,9 @@
  *       WG/reduction_4D_3D_mean_intra_sg_intra_lane.mlir:51-52   dims = {rows, cols}
  *   imex_reduce_outer_f32 / _f16 / _bf16  (in, out, outer:i64, inner:i64, init:f32)
  *       benchmarks/reduce/reduce_gpu.mlir.in:4-21        dims = {outer, inner}
+ *   imex_reduce_outer_f32_tall, imex_reduce_outer_f16_tall, imex_reduce_outer_bf16_tall
+ *   imex_reduce_outer_f32_deep, imex_reduce_outer_f16_deep, imex_reduce_outer_bf16_deep
+ *       the same for many slices of few (tall) or more (deep) outputs          dims = {outer, inner}
  *   imex_transpose2d_b16 / _b32    (in, out, rows:i64, cols:i64)
  *       benchmarks/transpose/transpose2d_gpu.mlir.in:4-11 dims = {rows, cols}
  *   imex_transpose3d_b16 / _b32    (in, out, d0:i64, d1:i64, d2:i64)

@@ -12,6 +12,8 @@
 //    owns groups of four adjacent outputs and adds the `outer` slices in order,
 //    which is the reference's summation order, so this one is bit-exact.
 //
+//    imex_reduce_outer_*_tall and _deep are the same sums for shapes that leave most of the chip idle in that form.
+//
 //  * imex_rowmean_f32: out[r] = (0 + sum_c in[r, c]) / cols, the same reduction with the
 //    division the reference applies afterwards
 //    (WG/reduction_4D_3D_mean_intra_sg_intra_lane.mlir:51-52, 1x24x1024x64 -> 1x24x1024x1).
@@ -245,4 +247,298 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16(co
                                                                              int64_t outer, int64_t inner,
                                                                              float init) {
   reduce_outer<io::Dt::BF16>(in, out, outer, inner, init);
+}
+
+// ---- outer-dimension sum, sixteen slices in flight ------------------------------------------------------
+// A lane owns one piece: a vector of four (eight) outputs, or one output where the slices are no whole 16-byte vectors
+// (kVec false).  For outputs that are too few to fill the chip with the wide spans above but enough for a lane each:
+// what bounds it is how many loads are in flight, so the ring is sixteen slices deep, the remaining slices' loads are in
+// flight together too, and it is a kernel of its own with few registers (eight wavefronts per SIMD, where the wide spans
+// leave room for one).  512 x 131072 f32: 73 -> 45 us (floor 42 for its bytes); slices of no whole vectors, one load
+// at a time before: f32 238 x 209827 350 -> 40 us, bf16 64 x 524291 210 -> 15.
+constexpr int kDeepRing = 16;
+template <bool kFirst, typename A, typename B> struct Select { using Type = A; };
+template <typename A, typename B> struct Select<false, A, B> { using Type = B; };
+template <io::Dt D, bool kVec>
+__device__ __forceinline__ void reduce_outer_deep(const void *__restrict__ in, void *__restrict__ out, int64_t outer,
+                                                  int64_t inner, float init) {
+  using E = io::Elem<D>;
+  constexpr int kPer = kVec ? E::kPerVec : 1; // outputs per piece
+  constexpr int kRing = kDeepRing;
+  using Raw = typename Select<kVec, u32x4, uint32_t>::Type; // as it comes from memory: widening an element here would wait for it
+  const int64_t pitch = inner * E::kBytes;
+  for (int64_t base = int64_t(blockIdx.x) * kThreads * kPer; base < inner; base += int64_t(gridDim.x) * kThreads * kPer) {
+    // Lanes past the end read the last piece instead (and store nothing): the loads are unconditional, so the wait for
+    // one slice leaves the loads of the next ones in flight.
+    const int64_t i = base + threadIdx.x * kPer;
+    const uint32_t at = static_cast<uint32_t>(min(i, inner - kPer) - base) * E::kBytes;
+    const char *slice = static_cast<const char *>(in) + base * E::kBytes; // of the slice that is fetched next
+    float acc[kPer];
+#pragma unroll
+    for (int e = 0; e < kPer; ++e)
+      acc[e] = init;
+    auto load = [&]() -> Raw {
+      if constexpr (kVec)
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(slice + at));
+      else if constexpr (D == io::Dt::F32)
+        return *reinterpret_cast<const uint32_t *>(slice + at);
+      else
+        return *reinterpret_cast<const uint16_t *>(slice + at);
+    };
+    auto add = [&](const Raw &raw) {
+      float f[kPer];
+      if constexpr (kVec)
+        E::unpack(raw, f);
+      else if constexpr (D == io::Dt::F32)
+        f[0] = u2f(raw);
+      else
+        f[0] = E::widen(raw);
+#pragma unroll
+      for (int e = 0; e < kPer; ++e)
+        acc[e] = acc[e] + f[e];
+    };
+    // Slice o is added, in slice order, and its register is at once reloaded with slice o + kRing.
+    if (outer > 0) {
+      Raw t[kRing];
+#pragma unroll
+      for (int u = 0; u < kRing; ++u) { // fewer slices than the ring holds: the last one again, not added
+        t[u] = load();
+        slice += u + 1 < outer ? pitch : 0;
+      }
+      int64_t o = 0;
+      for (; o + 2 * kRing <= outer; o += kRing) {
+#pragma unroll
+        for (int u = 0; u < kRing; ++u) {
+          add(t[u]);
+          t[u] = load();
+          slice += pitch;
+          __builtin_amdgcn_sched_barrier(0); // slice by slice: gathered up, the widened values cost 100 registers
+        }
+      }
+      const int left = int(outer - o) - kRing; // beyond those in registers; negative: not all of those exist
+      if (left > 0) { // the remaining slices' loads together, the last one's standing in for those past it
+#pragma unroll
+        for (int u = 0; u < kRing; ++u) {
+          add(t[u]);
+          t[u] = load();
+          slice += u + 1 < left ? pitch : 0;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      const int last = left > 0 ? left : left + kRing;
+#pragma unroll
+      for (int u = 0; u < kRing; ++u) {
+        if (u < last)
+          add(t[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (i < inner) {
+      if constexpr (kVec)
+        static_cast<u32x4 *>(out)[i / kPer] = E::pack(acc);
+      else
+        E::put(out, i, acc[0]);
+    }
+  }
+}
+
+template <io::Dt D>
+__device__ __forceinline__ void reduce_outer_deep_entry(const void *in, void *out, int64_t outer, int64_t inner, float init) {
+  using E = io::Elem<D>;
+  if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 && inner % E::kPerVec == 0)
+    reduce_outer_deep<D, true>(in, out, outer, inner, init);
+  else
+    reduce_outer_deep<D, false>(in, out, outer, inner, init);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_f32_deep(const float *in, float *out,
+                                                                                 int64_t outer, int64_t inner,
+                                                                                 float init) {
+  reduce_outer_deep_entry<io::Dt::F32>(in, out, outer, inner, init);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_f16_deep(const uint16_t *in, uint16_t *out,
+                                                                                 int64_t outer, int64_t inner,
+                                                                                 float init) {
+  reduce_outer_deep_entry<io::Dt::F16>(in, out, outer, inner, init);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16_deep(const uint16_t *in, uint16_t *out,
+                                                                                  int64_t outer, int64_t inner,
+                                                                                  float init) {
+  reduce_outer_deep_entry<io::Dt::BF16>(in, out, outer, inner, init);
+}
+
+// ---- outer-dimension sum, many slices of few outputs -------------------------------------------------
+// With 4 .. 32 KiB of every slice per workgroup, a tall matrix (column sums of [8192, 4096]: 4 workgroups of the
+// form above) leaves the chip idle and waits for one slice's latency per four slices.  What bounds it is the chain:
+// the additions of one output are ordered, so a column costs `outer` dependent additions (6 cycles each from a lone
+// wavefront) whatever is done -- the rest is keeping that chain fed and free of other instructions.  A workgroup
+// owns the columns of a 128-byte segment (32 f32, 64 16-bit ones) and walks all slices in chunks of 64: copier
+// wavefronts bring the chunks from global memory straight into a ring of LDS (1 KiB = eight slices per copy, seven
+// chunks = 56 KiB in flight), and ONE wavefront does nothing but add, a lane per column, sixteen slices' reads ahead
+// of the additions.  One barrier per chunk hands a chunk over and the oldest one back.
+// Slices that are not made of whole 16-byte vectors are copied element by element (one slice of 64 columns per
+// copy; the copy itself widens a 2-byte element to a word), by four copier wavefronts.
+// 8192 x 4096 f32: 980 us in the plain form, now 45 (floor 21 for its bytes; the chain alone is 8192 x 6.3 cycles = 22);
+// 700 x 3001 f32: 651 -> 7.3; bf16 4429 x 544: 505 -> 34.  A wavefront that copies for itself between its additions
+// took 76 us on the first: 22 cycles per slice where these take 12.
+typedef __attribute__((address_space(3))) char LdsChar;
+constexpr int kTallRing = 64 * 1024; // bytes of LDS
+constexpr int kTallRows = 64;        // slices per chunk
+constexpr int kTallVecThreads = 128, kTallElemThreads = 320;
+
+template <io::Dt D> __device__ __forceinline__ void add_slice(float &acc, uint32_t raw) {
+  if constexpr (D == io::Dt::F32)
+    acc = acc + u2f(raw);
+  else if constexpr (D == io::Dt::BF16)
+    acc = acc + u2f(raw << 16);
+  else // the f16 operand widens inside the instruction (exactly), times 1.0, plus acc: one rounding
+    asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(raw));
+}
+
+template <int N> __device__ __forceinline__ void chunk_landed() { // this wavefront's copies, all but the N youngest
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+}
+
+template <io::Dt D, bool kVec>
+__device__ __forceinline__ void reduce_outer_tall(const void *__restrict__ in, void *__restrict__ out, int64_t outer,
+                                                  int64_t inner, float init, char *lds) {
+  using E = io::Elem<D>;
+  constexpr int kCols = kVec ? 128 / E::kBytes : 64;
+  constexpr int kSlice = kVec ? 128 : 256;               // bytes of a slice's segment in LDS
+  constexpr int kElem = kVec ? E::kBytes : 4;            // bytes of an element in LDS
+  constexpr int kChunk = kTallRows * kSlice;             // 8 or 16 KiB
+  constexpr int kRing = kTallRing / kChunk;              // 8 or 4 chunks
+  constexpr int kCopiers = (kVec ? kTallVecThreads : kTallElemThreads) / kWave - 1;
+  constexpr int kCopies = kVec ? kTallRows / 8 : kTallRows / kCopiers; // per copier and chunk: 8 or 16
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int pitch = int(inner * E::kBytes);
+  const int chunks = int((outer + kTallRows - 1) / kTallRows), lastRows = int(outer - int64_t(chunks - 1) * kTallRows);
+  for (int64_t c0 = int64_t(blockIdx.x) * kCols; c0 < inner; c0 += int64_t(gridDim.x) * kCols) {
+    if (wave != 0) {
+      // Columns past the end re-read the last ones, slices past the end the last one (never added); chunks past the
+      // end go through a descriptor of size zero, so that every chunk is the same number of copies.
+      const int first = kVec ? lane >> 3 : (wave - 1) * kCopies; // slice of this lane's first copy within a chunk
+      const int col = kVec ? int(min((lane & 7) * 16 + c0 * E::kBytes, int64_t(pitch) - 16))
+                           : int(min(c0 + lane, inner - 1) * E::kBytes);
+      constexpr int kStep = kVec ? 8 : 1; // slices per copy
+      auto fetch = [&](int k) {
+        const char *base = static_cast<const char *>(in) + int64_t(k) * kTallRows * pitch;
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(base), 0, k < chunks ? 0x7ffffff0 : 0, 0x00020000);
+        LdsChar *dst = (LdsChar *)lds + (k & (kRing - 1)) * kChunk + (kVec ? 0 : first * kSlice);
+        if (k != chunks - 1) {
+          const int voff = kVec ? first * pitch + col : col;
+          int soff = kVec ? 0 : first * pitch;
+#pragma unroll
+          for (int u = 0; u < kCopies; ++u, soff += kStep * pitch)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst + u * kStep * kSlice, kVec ? 16 : E::kBytes, voff, soff, 0, 0);
+        } else {
+#pragma unroll
+          for (int u = 0; u < kCopies; ++u)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst + u * kStep * kSlice, kVec ? 16 : E::kBytes,
+                                                     min(first + u * kStep, lastRows - 1) * pitch + col, 0, 0, 0);
+        }
+      };
+      for (int k = 0; k < kRing - 1; ++k)
+        fetch(k);
+      for (int k = 0; k < chunks; ++k) {
+        chunk_landed<(kRing - 2) * kCopies>(); // chunk k is there; the adder has taken chunk k - 1, whose place ...
+        fetch(k + kRing - 1);                  // ... this one goes to
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else if (chunks > 0) {
+      const int at = (lane % kCols) * kElem;
+      uint32_t x[16], y[16];
+      auto read = [&](uint32_t(&v)[16], int k, int q) { // slices 16 q .. 16 q + 15 of chunk k
+        const char *p = lds + (k & (kRing - 1)) * kChunk + q * (16 * kSlice) + at;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          v[r] = kElem == 4 ? *reinterpret_cast<const uint32_t *>(p + r * kSlice)
+                            : *reinterpret_cast<const uint16_t *>(p + r * kSlice);
+      };
+      float acc = init;
+      auto add = [&](const uint32_t(&v)[16]) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          add_slice<D>(acc, v[r]);
+      };
+      auto next_chunk = [&] { // everything read so far is in registers
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      next_chunk();
+      read(x, 0, 0);
+      for (int k = 0; k + 1 < chunks; ++k) {
+        read(y, k, 1);
+        add(x);
+        read(x, k, 2);
+        add(y);
+        read(y, k, 3);
+        add(x);
+        next_chunk();
+        read(x, k + 1, 0);
+        add(y);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) { // the last chunk: 1 .. 64 slices
+        if (16 * q + 16 <= lastRows) {
+          add(x);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 15; ++r)
+            if (16 * q + r < lastRows)
+              add_slice<D>(acc, x[r]);
+        }
+        if (q < 3)
+          read(x, chunks - 1, q + 1);
+      }
+      if (lane < kCols && c0 + lane < inner)
+        E::put(out, c0 + lane, acc);
+    } else if (lane < kCols && c0 + lane < inner) {
+      E::put(out, c0 + lane, init);
+    }
+    __syncthreads(); // the ring is free for the next columns
+  }
+}
+
+// 128 lanes ask for the 16-byte form, 320 for the element form, which takes any slices.  Other launches, and slices of
+// 32 MiB and more (offsets inside a chunk are 31 bits), add slice by slice as the kernel without the suffix does.
+template <io::Dt D>
+__device__ __forceinline__ void reduce_outer_tall_entry(const void *in, void *out, int64_t outer, int64_t inner, float init) {
+  using E = io::Elem<D>;
+  __shared__ __attribute__((aligned(16))) char lds[kTallRing];
+  const bool fits = inner * E::kBytes < (int64_t(1) << 31) / kTallRows && outer < (int64_t(1) << 31);
+  if (fits && blockDim.x == kTallVecThreads && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && inner % E::kPerVec == 0)
+    reduce_outer_tall<D, true>(in, out, outer, inner, init, lds);
+  else if (fits && blockDim.x == kTallElemThreads)
+    reduce_outer_tall<D, false>(in, out, outer, inner, init, lds);
+  else
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < inner; i += int64_t(gridDim.x) * blockDim.x) {
+      float acc = init;
+      for (int64_t o = 0; o < outer; ++o)
+        acc = acc + E::get(in, o * inner + i);
+      E::put(out, i, acc);
+    }
+}
+
+extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_f32_tall(const float *in, float *out,
+                                                                                 int64_t outer, int64_t inner,
+                                                                                 float init) {
+  reduce_outer_tall_entry<io::Dt::F32>(in, out, outer, inner, init);
+}
+
+extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_f16_tall(const uint16_t *in, uint16_t *out,
+                                                                                 int64_t outer, int64_t inner,
+                                                                                 float init) {
+  reduce_outer_tall_entry<io::Dt::F16>(in, out, outer, inner, init);
+}
+
+extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_bf16_tall(const uint16_t *in, uint16_t *out,
+                                                                                  int64_t outer, int64_t inner,
+                                                                                  float init) {
+  reduce_outer_tall_entry<io::Dt::BF16>(in, out, outer, inner, init);
 }

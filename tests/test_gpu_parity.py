@@ -340,6 +340,32 @@ def test_reduce_outer_bit_exact(host, orc, stream, shape):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("form", ["_tall", "_deep"])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,inner", [(1, 8), (16, 1), (17, 65), (63, 40), (64, 130), (65, 1032), (129, 67), (520, 8),
+                                         (577, 2049), (0, 16)])
+def test_reduce_outer_forms_bit_exact(host, orc, stream, form, dtype, outer, inner):
+    """Both further forms of the outer-dimension sum around their rings (16 slices; chunks of 64, eight of them) and
+    segments (32 / 64 columns, 256 lanes), with and without whole 16-byte vectors: the slices are added in order, so
+    the result is the oracle's bit for bit; nothing behind it is written, and any grid computes it."""
+    x = orc.fill_uniform(max(outer * inner, 1), dtype, 91, -1.0, 1.0)[:outer * inner].reshape(outer, inner)
+    want = orc.reduce_outer_f32(orc.to_float(x, dtype) if dtype != "f32" else x, 0.25) if outer else None
+    want = np.full(inner, 0.25, np.float32) if want is None else want
+    want = want if dtype == "f32" else orc.from_float(want, dtype)
+    fill = np.full(inner + 256, 3, x.dtype)
+    name = "imex_reduce_outer_" + dtype + form
+    d_in, d_out = stream.to_device(x), stream.to_device(fill)
+    for grid in (None, (2, 1, 1)):
+        stream.copy(d_out, fill.ctypes.data, fill.nbytes)
+        stream.launch(name, [outer, inner], [d_in, d_out, outer, inner, 0.25], grid=grid)
+        stream.wait()
+        got = stream.from_device(d_out, fill.shape, fill.dtype)
+        assert np.array_equal(got[:inner], want), (name, outer, inner, grid)
+        assert np.array_equal(got[inner:], fill[inner:]), (name, outer, inner, grid)
+    stream.free(d_in)
+    stream.free(d_out)
+
+
 def test_reduce_outer_benchmark_shape_and_any_grid(host, orc, stream):
     """32x16x512x512 (the reference suite's reduce shape, README.md:335): integer-valued inputs
     make the sum exact; then the same kernel on a grid of 7 workgroups, which must stride."""
