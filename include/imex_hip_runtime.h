@@ -99,6 +99,13 @@ void *gpuLaunchKernel(void *queue, void *kernel, size_t gridX, size_t gridY, siz
                       size_t blockX, size_t blockY, size_t blockZ, size_t sharedMemBytes,
                       void *params, void *depEvents);
 
+/* gpuLaunchKernel for host code that keeps a launch's shape and its argument values in arrays (an interpreter's
+ * binding pays per argument of a call; this one has five).  No counterpart in the reference.  shape: grid x, y, z
+ * (workgroups), block x, y, z, bytes of dynamic shared memory; values: `count` arguments of 8 bytes each, a
+ * narrower one in its low bytes.  Everything is read before the call returns.  Same checks, profiling mode and
+ * returned event as gpuLaunchKernel. */
+void *imexHipLaunchValues(void *queue, void *kernel, const uint32_t shape[7], const void *values, size_t count);
+
 /* LevelZeroRuntimeWrappers.cpp:666-671 (SYCL twin: queue.wait(),
  * SyclRuntimeWrappers.cpp:498-505).  Blocks until the stream is idle. */
 void gpuWait(void *queue);

@@ -342,8 +342,9 @@ struct LaunchArgs {
   std::vector<void *> kernelParams;
 };
 
-LaunchArgs makeLaunch(void *kernel, size_t gx, size_t gy, size_t gz, size_t bx, size_t by, size_t bz,
-                      size_t sharedMemBytes, ImexParamDesc *params) {
+// Everything but the arguments.
+LaunchArgs launchShape(void *kernel, size_t gx, size_t gy, size_t gz, size_t bx, size_t by, size_t bz,
+                       size_t sharedMemBytes) {
   if (!kernel)
     throw std::runtime_error("gpuLaunchKernel: null kernel");
   LaunchArgs la;
@@ -364,6 +365,12 @@ LaunchArgs makeLaunch(void *kernel, size_t gx, size_t gy, size_t gz, size_t bx, 
     throw std::runtime_error("gpuLaunchKernel: more than 1024 threads per workgroup");
   // The call site passes an i32 (GPUXToLLVMPass.cpp:157); ignore the upper half.
   la.sharedMemBytes = static_cast<unsigned>(sharedMemBytes & 0xffffffffull);
+  return la;
+}
+
+LaunchArgs makeLaunch(void *kernel, size_t gx, size_t gy, size_t gz, size_t bx, size_t by, size_t bz,
+                      size_t sharedMemBytes, ImexParamDesc *params) {
+  LaunchArgs la = launchShape(kernel, gx, gy, gz, bx, by, bz, sharedMemBytes);
   size_t count = countUntil(params, [](const ImexParamDesc &p) { return p.data == nullptr && p.size == 0; });
   // LevelZeroRuntimeWrappers.cpp:462-475: the last entry stands for dynamic
   // shared memory; on HIP that is the launch's sharedMemBytes, not an argument.
@@ -487,6 +494,8 @@ hipEvent_t materialise(LaunchEvent *le) {
   return le->event;
 }
 
+LaunchEvent *submit(GpuHipQueue *queue, LaunchArgs &la);
+
 LaunchEvent *launchKernel(GpuHipQueue *queue, void *kernel, size_t gx, size_t gy, size_t gz, size_t bx,
                           size_t by, size_t bz, size_t sharedMemBytes, ImexParamDesc *params,
                           ImexEventDesc *depEvents) {
@@ -503,6 +512,11 @@ LaunchEvent *launchKernel(GpuHipQueue *queue, void *kernel, size_t gx, size_t gy
     CHECK_HIP(hipSetDevice(queue->device));
     CHECK_HIP(hipStreamWaitEvent(queue->stream, ev, 0));
   }
+  return submit(queue, la);
+}
+
+// The launch itself, after the reference's profiling loop if that is asked for.
+LaunchEvent *submit(GpuHipQueue *queue, LaunchArgs &la) {
   CHECK_HIP(hipSetDevice(queue->device));
 
   if (getenv("IMEX_ENABLE_PROFILING")) {
@@ -622,6 +636,21 @@ extern "C" void *gpuLaunchKernel(void *queue, void *kernel, size_t gridX, size_t
   return catchAll([&]() -> void * {
     return launchKernel(asQueue(queue), kernel, gridX, gridY, gridZ, blockX, blockY, blockZ, sharedMemBytes,
                         static_cast<ImexParamDesc *>(params), static_cast<ImexEventDesc *>(depEvents));
+  });
+}
+
+extern "C" void *imexHipLaunchValues(void *queue, void *kernel, const uint32_t shape[7], const void *values,
+                                     size_t count) {
+  return catchAll([&]() -> void * {
+    if (!queue)
+      throw std::runtime_error("imexHipLaunchValues: null stream");
+    if (!shape || (count && !values))
+      throw std::runtime_error("imexHipLaunchValues: null shape or values");
+    LaunchArgs la = launchShape(kernel, shape[0], shape[1], shape[2], shape[3], shape[4], shape[5], shape[6]);
+    la.kernelParams.reserve(count);
+    for (size_t i = 0; i < count; ++i)
+      la.kernelParams.push_back(const_cast<char *>(static_cast<const char *>(values)) + 8 * i);
+    return submit(asQueue(queue), la);
   });
 }
 

@@ -11,8 +11,10 @@ of the runtime raises, and every operator goes through the HIP kernels.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 import re
+import struct
 
 import numpy as np
 
@@ -52,6 +54,7 @@ _RUNTIME_SYMBOLS = {
     "gpuModuleLoad": (C.c_void_p, [C.c_void_p, C.c_void_p, C.c_size_t]),
     "gpuKernelGet": (C.c_void_p, [C.c_void_p, C.c_void_p, C.c_char_p]),
     "gpuLaunchKernel": (C.c_void_p, [C.c_void_p, C.c_void_p] + [C.c_size_t] * 7 + [C.c_void_p, C.c_void_p]),
+    "imexHipLaunchValues": (C.c_void_p, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_char_p, C.c_size_t]),
     "gpuWait": (None, [C.c_void_p]),
     "gpuModuleUnload": (None, [C.c_void_p, C.c_void_p]),
     "mgpuStreamCreate": (C.c_void_p, []),
@@ -248,6 +251,32 @@ def _pack_params(args, types=None):
     return descs, storage
 
 
+class _Plan:
+    """What a launch of one operator at one size needs besides its arguments: the resolved kernel of the
+    variant the catalogue advises, its launch shape, and how the arguments are packed (8 bytes each, an f32
+    in the low four)."""
+    __slots__ = ("kernel", "shape", "types", "packer", "pointers")
+
+    def __init__(self, stream, name, dims):
+        name = variant(name, dims)
+        grid, block, smem = launch_shape(name, dims)
+        self.types = signature_types(name)
+        self.kernel = None if 0 in grid else stream.kernel(name)
+        self.shape = (C.c_uint32 * 7)(*grid, *block, smem)
+        self.packer = struct.Struct("<" + "".join({"ptr": "Q", "i64": "q", "f32": "f4x"}[t] for t in self.types))
+        self.pointers = [i for i, t in enumerate(self.types) if t == "ptr"]
+
+    def pack(self, args):
+        """The arguments' values as imexHipLaunchValues takes them; _pack_params' errors for wrong ones."""
+        if len(args) == len(self.types) and all(isinstance(args[i], Ptr) for i in self.pointers):
+            try:
+                return self.packer.pack(*args)
+            except (struct.error, OverflowError):
+                pass  # a value that needs converting (an index given as 2.0), or one no conversion fits
+        descs, keep = _pack_params(args, self.types)
+        return b"".join(C.string_at(d.data, d.size).ljust(8, b"\0") for d in descs[:len(self.types)])
+
+
 class Stream:
     """gpux stream: the object every gpu* call takes first (GPUToGPUX.cpp:36-59)."""
 
@@ -256,7 +285,7 @@ class Stream:
         creating its own; the queue does not destroy it."""
         self.rt = runtime()
         self.handle = self.rt.gpuCreateStream(None, hip_stream)
-        self._events = []
+        self._plans = {}  # (operator, dims) -> _Plan
 
     def close(self):
         if self.handle:
@@ -331,6 +360,11 @@ class Stream:
         """gpuModuleLoad + gpuKernelGet + gpuLaunchKernel; returns the event (or
         None when the launch shape is empty).  `grid` / `block` replace the catalogue's, and with one of
         them given it is `name` itself that is launched; otherwise the variant the catalogue advises."""
+        if grid is None and block is None and not deps:
+            plan = self._plans.get((name, *dims)) or self._plan(name, dims)
+            if plan.kernel is None:
+                return None
+            return self.rt.imexHipLaunchValues(self.handle, plan.kernel, plan.shape, plan.pack(args), len(plan.types))
         if grid is None and block is None:
             name = variant(name, dims)
         cat_grid, cat_block, smem = launch_shape(name, dims)
@@ -348,24 +382,21 @@ class Stream:
         del keep
         return ev
 
-    def prepare(self, name, dims, args):
-        """Resolve the kernel, its launch shape and its ParamDesc list once and
-        return a zero-argument callable that performs just the gpuLaunchKernel
-        call (what JIT'd host code does inside a loop)."""
-        name = variant(name, dims)
-        grid, block, smem = launch_shape(name, dims)
-        if 0 in grid:
-            return lambda: None
-        fn = self.kernel(name)
-        descs, keep = _pack_params(args, signature_types(name))
-        params = C.cast(descs, C.c_void_p)
-        launch, handle = self.rt.gpuLaunchKernel, self.handle
-        gx, gy, gz = grid
-        bx, by, bz = block
+    def _plan(self, name, dims):
+        if len(self._plans) >= 4096:  # sizes that change without end: start over rather than grow
+            self._plans.clear()
+        plan = self._plans[(name, *dims)] = _Plan(self, name, dims)
+        return plan
 
-        def run(_keep=(descs, keep)):
-            return launch(handle, fn, gx, gy, gz, bx, by, bz, smem, params, None)
-        return run
+    def prepare(self, name, dims, args):
+        """Resolve the kernel, its launch shape and its argument values once and
+        return a zero-argument callable that performs just the launch
+        (what JIT'd host code does inside a loop)."""
+        plan = self._plan(name, dims)
+        if plan.kernel is None:
+            return lambda: None
+        return functools.partial(self.rt.imexHipLaunchValues, self.handle, plan.kernel, plan.shape, plan.pack(args),
+                                 len(plan.types))
 
     def profile(self, name, dims, args, warmups=5, rounds=20, flush_bytes=0, mode=0):
         """Per-launch times in ms (mode 0) or [total ms] over `rounds` back-to-back launches (mode 1)."""

@@ -182,6 +182,23 @@ def test_param_desc_packing(host):
     assert C.cast(descs[2].data, C.POINTER(C.c_float))[0] == 2.5
 
 
+def test_plan_packs_arguments_as_the_kernel_declares_them(host):
+    """Stream.launch's fast path: 8 bytes per argument, an f32 in the low four, with _pack_params' conversions and errors."""
+    class Resolver:
+        def kernel(self, name):
+            return 1
+    plan = host._Plan(Resolver(), "imex_rowsum_f32", [3, 5])
+    p, q = host.Ptr(0x1000), host.Ptr(0x2000)
+    want = np.array([0x1000, 0x2000, 3, 5], np.int64).tobytes() + np.array([2.5, 0], np.float32).tobytes()
+    assert plan.pack([p, q, 3, 5, 2.5]) == want
+    assert plan.pack([p, q, 3.0, np.int32(5), np.float64(2.5)]) == want
+    assert plan.pack([p, q, 3, 5, 1e300])[-8:-4] == np.array([np.inf], np.float32).tobytes()
+    assert list(plan.shape) == [1, 1, 1, 256, 1, 1, 0]
+    for bad in ([p, 0x2000, 3, 5, 2.5], [p, q, 3.5, 5, 2.5], [p, q, 3, 5]):
+        with pytest.raises(TypeError):
+            plan.pack(bad)
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
