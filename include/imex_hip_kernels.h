@@ -81,6 +81,17 @@
  *       the operator without the suffix, same arguments, on tiles of 128 x 128, 128 x 64, 64 x 64, 32 x 64 and 16 x 64
  *       outputs: what imexHipKernelVariant names for problems that would leave most of the chip idle
  *                                                          dims = {M, N, K}
+ *   imex_gemm_f16_f16_f32_u128, imex_gemm_f16_f16_f32_u64
+ *   imex_gemm_f16_f16_f32_acc_u128, imex_gemm_f16_f16_f32_acc_u64
+ *   imex_gemm_bf16_bf16_f32_u128, imex_gemm_bf16_bf16_f32_u64
+ *   imex_gemm_bf16_bf16_f32_acc_u128, imex_gemm_bf16_bf16_f32_acc_u64
+ *   imex_gemm_f16_f16_f16_u128, imex_gemm_f16_f16_f16_u64
+ *   imex_gemm_f16_f16_f32_tb_u128, imex_gemm_f16_f16_f32_tb_u64
+ *   imex_gemm_f16_f16_f32_ta_u128, imex_gemm_f16_f16_f32_ta_u64
+ *   imex_gemm_bf16_bias_silu_bf16_u128, imex_gemm_bf16_bias_silu_bf16_u64
+ *       the operator without the suffix, same arguments, on the matrix cores for operands whose rows are not 16-byte
+ *       aligned (tiles of 128 x 128, 64 x 64); f32 sums in another order than the operator's own sequential one
+ *                                                          dims = {M, N, K}
  *   imex_gemm_bf16_bias_silu_bf16_streamk  (A, B, bias, out, M:i64, N:i64, K:i64, workspace, epoch:i64, spin_limit:i64)
  *       the same operator with the last, partial round of tiles split along K over all workgroups (no
  *       counterpart in the reference); workspace: imexHipStreamKWorkspaceBytes(grid) bytes of device

@@ -29,7 +29,7 @@ INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-KERNEL_GROUPS = ["eltwise", "softmax", "reduce", "transpose", "gemm", "gemm_small", "fusion", "attention"]
+KERNEL_GROUPS = ["eltwise", "softmax", "reduce", "transpose", "gemm", "gemm_small", "gemm_unaligned", "fusion", "attention"]
 # Measurement kernels: a code object of their own (lib/imex_probe.hsaco) that bench.py and the
 # driver load from the file; the catalogue library holds operators only.
 BENCH_ONLY_GROUPS = ["probe"]

@@ -18,7 +18,7 @@
 //               order and leave as four consecutive columns per lane, whole lines per row.
 //
 // Steps past the end of K are fetched through a descriptor of size zero (nothing moves, LDS gets zeros).
-// Operands whose rows are not 16-byte aligned take gemm_blocked, as in gemm_tile.h.
+// Operands whose rows are not 16-byte aligned take gemm_blocked, as in gemm_tile.h, or the kernels of gemm_unaligned.h.
 
 #ifndef IMEX_HIP_GEMM_SMALL_H
 #define IMEX_HIP_GEMM_SMALL_H
@@ -55,9 +55,22 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
   int rd;             // per-lane LDS address of fragment 0, slice 0 (strided: without the pair)
   int swz;            // strided: pair swizzle of this lane's k rows
 
+  // where a wavefront whose fragments start at row w0 of the slab reads them
+  __device__ __forceinline__ void setup_read(int w0, int lane) {
+    if constexpr (!kStrided) {
+      const int r = lane & 15;
+      rd = (w0 + r) * 128 + (((lane >> 4) ^ ((r >> 1) & 7)) << 4);
+      swz = 0;
+    } else {
+      const int t = lane & 15, row = (lane >> 4) * 8 + (t >> 2);
+      rd = row * (TR * 2) + (t & 3) * 8;
+      swz = pair_swizzle<TR / 16>(row) ^ (w0 / 16);
+    }
+  }
   __device__ __forceinline__ void setup(const uint16_t *ptr, int64_t ld, int64_t first, int w0, int64_t extent,
                                         int wave, int lane, int kRem) {
     dst = wave * kCopies * 1024;
+    setup_read(w0, lane);
     if constexpr (!kStrided) {
       const int64_t rows = extent / ld - first;
       const int last = rows < TR ? int(rows) - 1 : TR - 1;
@@ -71,9 +84,6 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
         voffT[q] = k < kRem ? voff[q] : kOutOfRange;
       }
       step = BK * 2;
-      const int r = lane & 15;
-      rd = (w0 + r) * 128 + (((lane >> 4) ^ ((r >> 1) & 7)) << 4);
-      swz = 0;
     } else {
       constexpr int kRow = TR * 2, kChunks = kRow / 16; // bytes and 16-byte chunks per k row
       base = ptr + first;
@@ -88,9 +98,6 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
         voffT[q] = row < kRem ? voff[q] : kOutOfRange;
       }
       step = int(BK * ld * 2);
-      const int t = lane & 15, row = (lane >> 4) * 8 + (t >> 2);
-      rd = row * kRow + (t & 3) * 8;
-      swz = pair_swizzle<TR / 16>(row) ^ (w0 / 16);
     }
   }
   // step `kt` of `steps` into the image at `image`
@@ -128,6 +135,42 @@ template <int TMv, int TNv, int WMCv, int WNCv, int KGv, int Sv> struct SmallSha
   static constexpr int kWavesPerEu = kLds <= 80 * 1024 ? 4 : 2; // two workgroups on a CU where LDS has room for two
   static_assert(WMC * WNC * KG == kWaves && BK % 64 == 0 && kLds <= 160 * 1024, "eight wavefronts, one CU's LDS");
 };
+
+// The end of a tile: the KG partial tiles meet in LDS (which nobody reads or writes any more: a barrier has been
+// passed since), are added in group order, and what lies inside C goes through the epilogue.
+template <typename P, typename Epi>
+__device__ __forceinline__ void merge_and_store(const f32x4 (&acc)[P::FI][P::FJ], char *lds, int64_t M, int64_t N,
+                                                const Epi &epi, int64_t m0, int64_t n0, int kg, int wm, int wn,
+                                                int lane) {
+  constexpr int FI = P::FI, FJ = P::FJ;
+  const int tid = threadIdx.x;
+  // partial tiles side by side in LDS: lane holds row lane % 16, columns (lane / 16) * 4 .. + 3 of a block
+  float *part = reinterpret_cast<float *>(lds);
+  {
+    float *mine = part + kg * (P::TM * P::kPitch) + (wm * (P::TM / P::WMC) + (lane & 15)) * P::kPitch +
+                  wn * (P::TN / P::WNC) + (lane >> 4) * 4;
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+      for (int j = 0; j < FJ; ++j)
+        *reinterpret_cast<f32x4 *>(mine + i * 16 * P::kPitch + j * 16) = acc[i][j];
+  }
+  __syncthreads();
+  constexpr int kVecs = P::TM * P::TN / 4;
+#pragma unroll
+  for (int u = 0; u < (kVecs + kThreads - 1) / kThreads; ++u) {
+    const int v = u * kThreads + tid;
+    if (kVecs % kThreads == 0 || v < kVecs) {
+      const int r = v / (P::TN / 4), c = (v % (P::TN / 4)) * 4;
+      f32x4 sum = *reinterpret_cast<const f32x4 *>(part + r * P::kPitch + c);
+#pragma unroll
+      for (int g = 1; g < P::KG; ++g)
+        sum += *reinterpret_cast<const f32x4 *>(part + g * (P::TM * P::kPitch) + r * P::kPitch + c);
+      if (m0 + r < M && n0 + c < N)
+        store_columns(epi, m0 + r, n0 + c, N, sum);
+    }
+  }
+}
 
 template <typename T, bool kAT, bool kBT, typename P, typename Epi>
 __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
@@ -204,32 +247,7 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
   wait_vmcnt<0>();
   __syncthreads(); // the ring is free
 
-  // partial tiles side by side in LDS: lane holds row lane % 16, columns (lane / 16) * 4 .. + 3 of a block
-  float *part = reinterpret_cast<float *>(lds);
-  {
-    float *mine = part + kg * (P::TM * P::kPitch) + (wm * (P::TM / P::WMC) + (lane & 15)) * P::kPitch +
-                  wn * (P::TN / P::WNC) + (lane >> 4) * 4;
-#pragma unroll
-    for (int i = 0; i < FI; ++i)
-#pragma unroll
-      for (int j = 0; j < FJ; ++j)
-        *reinterpret_cast<f32x4 *>(mine + i * 16 * P::kPitch + j * 16) = acc[i][j];
-  }
-  __syncthreads();
-  constexpr int kVecs = P::TM * P::TN / 4;
-#pragma unroll
-  for (int u = 0; u < (kVecs + kThreads - 1) / kThreads; ++u) {
-    const int v = u * kThreads + tid;
-    if (kVecs % kThreads == 0 || v < kVecs) {
-      const int r = v / (P::TN / 4), c = (v % (P::TN / 4)) * 4;
-      f32x4 sum = *reinterpret_cast<const f32x4 *>(part + r * P::kPitch + c);
-#pragma unroll
-      for (int g = 1; g < P::KG; ++g)
-        sum += *reinterpret_cast<const f32x4 *>(part + g * (P::TM * P::kPitch) + r * P::kPitch + c);
-      if (m0 + r < M && n0 + c < N)
-        store_columns(epi, m0 + r, n0 + c, N, sum);
-    }
-  }
+  merge_and_store<P>(acc, lds, M, N, epi, m0, n0, kg, wm, wn, lane);
 }
 
 // Tile number -> tile, as tile_origin of gemm_tile.h: the workgroups of an XCD (ids congruent mod 8) take a compact

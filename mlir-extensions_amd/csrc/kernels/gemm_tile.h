@@ -236,7 +236,8 @@ struct StoreF16 {       // C(f16) = acc   (WG/gemm_4kx4kx4k_f16_f16_f16.mlir)
 };
 
 // ---- any-shape path: 128 x 128 tiles on the vector ALUs -----------------------------------
-// For operands the MFMA path cannot take (rows that are not 16-byte aligned in memory).  Every output is
+// For operands the MFMA path cannot take (rows that are not 16-byte aligned in memory), in problems too small or with
+// sums too short for gemm_unaligned.h (imexHipKernelVariant draws the line).  Every output is
 // the reference's CPU loop (lib/ExecutionEngine/ImexRunnerUtils.cpp:308-317): acc = 0, then for ascending
 // k a rounded multiply and a rounded add (this file is built with contraction off), so the result is the
 // oracle's bit for bit; the tiling only shares the operand loads.  512 lanes hold 8 x 4 outputs each; A

@@ -964,6 +964,63 @@ def test_gemm_every_tile_integers_exact(host, orc, stream, tile, M, N, K):
             assert np.array_equal(got[:m].astype(np.int64), want + (7 if which == "acc" else 0)), name
 
 
+@pytest.mark.parametrize("tile", ["_u128", "_u64"])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (9, 11, 13), (64, 64, 64), (63, 65, 71), (129, 67, 257), (130, 255, 65),
+                                   (201, 129, 579)])
+def test_gemm_unaligned_rows(host, orc, stream, tile, M, N, K):
+    """Rows that are not 16-byte aligned on the matrix cores: shapes below, at and beyond the tiles' edges in M, N and
+    K, every operand layout and epilogue.  Integer operands give the exact f32 sum in any order; an infinity in the
+    row (k row) that follows reaches nothing but its own results, as it would if a piece beyond K were multiplied by
+    something; nothing is stored outside C."""
+    say("gemm unaligned %s %dx%dx%d" % (tile, M, N, K))
+    for which in ("plain", "acc", "ta", "tb", "f16", "mlp"):
+        dtype = "bf16" if which in ("mlp", "acc") else "f16"
+        a = orc.fill_int(M * K, dtype, 95, -1, 1).reshape(M, K)
+        b = orc.fill_int(K * N, dtype, 96, -1, 1).reshape(K, N)
+        a[M - 1, 0] = b[0, N - 1] = 0x7f80 if dtype == "bf16" else 0x7c00
+        fa, fb = orc.to_float(a, dtype).astype(np.float64), orc.to_float(b, dtype).astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            want = fa[:-1, :] @ fb[:, :-1]
+        name = {"plain": "f16_f16_f32", "acc": "bf16_bf16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb",
+                "f16": "f16_f16_f16", "mlp": "bf16_bias_silu_bf16"}[which]
+        name = "imex_gemm_" + name + tile
+        bias = orc.fill_int(N, "f32", 97, -3, 3)
+        c0 = np.full((M + 256, N), 7, np.uint16 if which in ("f16", "mlp") else np.float32)
+        bufs = [stream.to_device(np.ascontiguousarray(a.T) if which == "ta" else a),
+                stream.to_device(np.ascontiguousarray(b.T) if which == "tb" else b)]
+        bufs += [stream.to_device(bias)] if which == "mlp" else []
+        bufs.append(stream.to_device(c0))
+        stream.launch(name, [M, N, K], bufs + [M, N, K])
+        stream.wait()
+        got = stream.from_device(bufs[-1], c0.shape, c0.dtype)
+        for p in bufs:
+            stream.free(p)
+        assert np.array_equal(got[M:], c0[M:]), "%s wrote past row %d" % (name, M)
+        got = got[:M - 1, :N - 1]
+        if which == "mlp":
+            ref = orc.bfloat_to_float(orc.bias_silu_bf16(np.ascontiguousarray(want, np.float32), bias[:-1]))
+            assert np.max(np.abs(orc.bfloat_to_float(got) - ref)) <= 2.0 ** -7 * np.max(np.abs(ref)) + 1e-6
+        elif which == "f16":
+            assert np.array_equal(orc.half_to_float(np.ascontiguousarray(got)), want), name
+        else:
+            assert np.array_equal(got, want + (7 if which == "acc" else 0)), name
+
+
+@pytest.mark.parametrize("which", ["", "_ta", "_tb"])
+def test_gemm_unaligned_rows_chosen(host, orc, stream, which):
+    """What the operator takes at an ordinary odd size, random operands: against 64 bits within the rounding of 32-bit
+    sums, (K + 1) half-ulps of the sum of magnitudes in any order."""
+    M, N, K = 301, 517, 259
+    name = "imex_gemm_f16_f16_f32" + which
+    assert host.variant(name, [M, N, K]) != name
+    a = orc.fill_uniform(M * K, "f16", 98, -1, 1).reshape(M, K)
+    b = orc.fill_uniform(K * N, "f16", 99, -1, 1).reshape(K, N)
+    fa, fb = orc.to_float(a, "f16").astype(np.float64), orc.to_float(b, "f16").astype(np.float64)
+    sa, sb = (np.ascontiguousarray(a.T) if which == "_ta" else a), (np.ascontiguousarray(b.T) if which == "_tb" else b)
+    got = _gemm_guarded(host, stream, name, sa, sb, M, N, K)
+    assert np.all(np.abs(got - fa @ fb) <= (K + 1) * 2.0 ** -24 * (np.abs(fa) @ np.abs(fb)))
+
+
 @pytest.mark.parametrize("which,M,N,K", [("ta", 248, 264, 64), ("ta", 8, 8, 32), ("tb", 100, 37, 64), ("tb", 300, 515, 96)])
 def test_gemm_ragged_tiles_transposed_operands(host, orc, stream, which, M, N, K):
     """Edge tiles with A stored [K,M] (M % 8 == 0) or B stored [N,K] (any N)."""

@@ -172,6 +172,22 @@ def test_kernel_variants(host):
     assert {"_t128", "_t64", "_t32", "_t16"} <= seen
 
 
+def test_kernel_variants_for_unaligned_rows(host):
+    """Rows that are not 16-byte aligned: the operator's own loop for small products of short sums, the matrix cores
+    beyond, and the operator again where a row holds no whole 16 bytes or an offset would not fit."""
+    v, shape = host.variant, host.launch_shape
+    for base in ("imex_gemm_f16_f16_f32", "imex_gemm_f16_f16_f32_ta", "imex_gemm_f16_f16_f32_tb",
+                 "imex_gemm_bf16_bias_silu_bf16"):
+        assert v(base, [129, 129, 17]) == base and v(base, [101, 101, 191]) == base
+        assert v(base, [101, 101, 193]) == base + "_u64" and v(base, [1001, 1003, 99]) == base + "_u64"
+        assert v(base, [4097, 4097, 4097]) == base + "_u128"
+        assert shape(base + "_u64", [130, 65, 9])[0][0] == 6 and shape(base + "_u128", [130, 65, 9])[0][0] == 2
+        assert v(base, [4097, 4097, 7]) == base and v(base, [4097, 4097, (1 << 22) + 1]) == base
+    assert v("imex_gemm_f16_f16_f32", [99999, 7, 4097]) == "imex_gemm_f16_f16_f32"
+    assert v("imex_gemm_f16_f16_f32_tb", [99999, 7, 4097]) != "imex_gemm_f16_f16_f32_tb"
+    assert v("imex_gemm_f16_f16_f32_ta", [7, 99999, 4097]) == "imex_gemm_f16_f16_f32_ta"
+
+
 def test_param_desc_packing(host):
     descs, keep = host._pack_params([host.Ptr(0x1000), 7, 2.5])
     assert C.sizeof(host.ParamDesc) == 16
