@@ -24,6 +24,8 @@
  *       test/Integration/Dialect/XeGPU/WG/arith_maximumf.mlir:51-66   dims = {n}
  *   imex_softmax_f32 / _f16 / _bf16 (in, out, rows:i64, cols:i64)
  *       benchmarks/softmax/softmax_gpu.mlir.in:4-44      dims = {rows, cols}
+ *   imex_softmax_f32_shared, imex_softmax_f16_shared, imex_softmax_bf16_shared
+ *       the same with a row's lanes chosen by its length                   dims = {rows, cols}
  *   imex_rowsum_f32                (in, out, rows:i64, cols:i64, init:f32)
  *       WG/reduction_2D_1D_cross_sg_cross_lane.mlir:31-37 dims = {rows, cols}
  *   imex_rowmean_f32               (in, out, rows:i64, cols:i64)   out[r] = (sum_c in[r,c]) / cols

@@ -6,18 +6,19 @@
 // test/Integration/Dialect/XeGPU/WG/softmax_intra_sg_cross_lane.mlir:118-205.
 //
 // Here: ONE kernel, input read once from HBM and output written once.
-//  * rows of up to 128 lanes x 16 B (1024 16-bit / 512 f32 elements): a
-//    wavefront owns a row and keeps it in registers; max and sum are wavefront-64
-//    reductions on the VALU's cross-lane paths (DPP), no LDS.
-//    f16: a wavefront walks rows w, w + W, ... with the next row's loads in
-//    flight while it computes the current one, and the arithmetic is written for
-//    the instruction count (packed f16 maximum, mixed-precision FMAs straight
-//    from and into the f16 halves, one reciprocal per row): about 6 vector
-//    instructions per element where the generic form below needs 14.
-//    f32 / bf16: the generic form, a wavefront owns one row (two from 16384 rows
-//    on, all loads issued before the first reduction), eight wavefronts per SIMD.
-//  * rows of up to 4096 elements: a workgroup owns a row and stages it in LDS
-//    as f32 (read once, three passes over LDS).
+//  * rows of up to 256 pieces of 16 bytes (2048 16-bit / 1024 f32 elements) belong to 4 .. 64 lanes of a wavefront,
+//    up to four pieces a lane, so a wavefront has up to sixteen rows at once; max and sum are reductions on the VALU's
+//    cross-lane paths (DPP), no LDS.  Longer rows, up to 4096 pieces, and more than 64 pieces where there are fewer
+//    than 2048 rows to give to wavefronts, belong to a workgroup.  Either way a row stays in registers from its one
+//    read to its one write, and neither its length nor its address need be multiples of anything.
+//    Bound by HBM on whole pieces (f32 16384 x 1024: 23.1 us, 5.8 TB/s; one and two rows per wavefront before: 24.4;
+//    bf16 8192 x 2000, staged in LDS before: 16.8 -> 13.2); odd rows cost a second transaction per request on both
+//    sides (bf16 6000 x 3001: 35.1 -> 17.2 us, 4.2 TB/s, with buffers that are not in the caches; one element at a
+//    time through LDS before), short ones are cut to size (bf16 65536 x 32: 20.5 -> 3.2; 200001 x 77: 119 -> 16.5).
+//  * f16 rows of 65 .. 128 whole pieces: a wavefront walks rows w, w + W, ... with the next row's loads in
+//    flight while it computes the current one, and the arithmetic is written for the instruction count (packed f16
+//    maximum, mixed-precision FMAs straight from and into the f16 halves, one reciprocal per row): about 6 vector
+//    instructions per element where the general form needs 10.
 //  * longer rows: workgroup per row, the streaming form -- a running (max, sum)
 //    pair rescaled as the maximum moves, then a second read of the row to
 //    normalise (WG/softmax_intra_sg_cross_lane.mlir:135-175): two reads, one write.
@@ -25,10 +26,10 @@
 // on the GPU: extend to f32, compute, truncate (docs/Transforms/BF16ToGpu.md:17-26).
 //
 // Arguments: (in, out, rows: i64, cols: i64).
-// Launch: block (256,1,1); any grid >= 1 is correct (workgroups stride over the
-// rows); the catalogue sizes it to one pass: ceil(rows/4) for register-resident
-// rows (ceil(rows/8) from 16384 rows on; f16: min(ceil(rows/4), 2048) -- one
-// wavefront per wavefront slot of the chip), else min(rows, 65535 * 16).
+// Launch: any grid >= 1 is correct (workgroups stride over the rows), with block (256,1,1); the _shared forms also
+// take (512,1,1) and (1024,1,1) for rows of a workgroup, and the catalogue's launch of these gives every group of lanes
+// one row and a workgroup's row the smallest block that holds it (bf16 6000 x 3001: 17.3 us with 256 lanes, 23.8 with
+// 512, 43.5 with 1024).
 
 #include "device_common.h"
 
@@ -38,15 +39,16 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kRegChunks = 2;          // 16-byte chunks per lane and row on the register path
-constexpr int64_t kTwoRowsFrom = 16384; // rows from which a wavefront takes two: every wavefront slot of the chip is then filled
-constexpr int kLdsCols = 4096;         // longest row staged in LDS
+constexpr int kRegChunks = 2;          // 16-byte chunks per lane and row of the f16 walk
+constexpr int kMaxWaves = 16;          // of a workgroup that has a long row
+constexpr int64_t kManyRows = 2048;    // wavefronts' worth of rows from which a lane takes up to four pieces of one
 
 enum class Dt { F32, F16, BF16 };
 
 template <Dt D> struct Elem;
 template <> struct Elem<Dt::F32> {
   static constexpr int kBytes = 4;
+  typedef uint32_t Unaligned __attribute__((ext_vector_type(4), aligned(4)));
   static constexpr int kPerVec = 4;
   static __device__ __forceinline__ void unpack(u32x4 v, float *f) {
     f[0] = u2f(v.x); f[1] = u2f(v.y); f[2] = u2f(v.z); f[3] = u2f(v.w);
@@ -59,6 +61,7 @@ template <> struct Elem<Dt::F32> {
 };
 template <> struct Elem<Dt::F16> {
   static constexpr int kBytes = 2;
+  typedef uint32_t Unaligned __attribute__((ext_vector_type(4), aligned(2)));
   static constexpr int kPerVec = 8;
   static __device__ __forceinline__ void unpack(u32x4 v, float *f) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -82,8 +85,14 @@ template <> struct Elem<Dt::F16> {
     static_cast<uint16_t *>(p)[i] = static_cast<uint16_t>(float_to_half_bits(v));
   }
 };
+// Two values rounded to bf16 (nearest even) by v_cvt_pk_bf16_f32.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
+}
 template <> struct Elem<Dt::BF16> {
   static constexpr int kBytes = 2;
+  typedef uint32_t Unaligned __attribute__((ext_vector_type(4), aligned(2)));
   static constexpr int kPerVec = 8;
   static __device__ __forceinline__ void unpack(u32x4 v, float *f) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -97,7 +106,7 @@ template <> struct Elem<Dt::BF16> {
     uint32_t w[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      w[i] = float_to_bf16_bits(f[2 * i]) | (float_to_bf16_bits(f[2 * i + 1]) << 16);
+      w[i] = pack_bf16(f[2 * i], f[2 * i + 1]);
     return u32x4{w[0], w[1], w[2], w[3]};
   }
   static __device__ __forceinline__ float load(const void *p, int64_t i) {
@@ -116,74 +125,179 @@ __device__ __forceinline__ float fast_exp(float x) { return __expf(x); }
 // (softmax_gpu.mlir.in:6).
 constexpr float kMaxInit = -3.40282347e+38f;
 
-// ---- register path: a wavefront owns kRowsPerWave rows ---------------------------
-template <Dt D, bool kStream, int kRowsPerWave>
-__device__ __forceinline__ void softmax_rows_in_regs(const void *in, void *out, int64_t rows, int64_t cols) {
+// ---- rows in registers, any length up to 4 vectors per lane, any alignment -----------------------------------
+// A row is cut into 16-byte pieces, piece v at element v * P; the last piece of a row that is no whole number of
+// pieces starts at cols - P instead, so it repeats elements of the piece before: harmless in the maximum, left out
+// of the sum, and stored twice with the same value.  Loads and stores take any address (an element's own alignment is
+// enough for them), and no lane's load leaves the row: lanes past the last piece load that one again.
+// kLanes lanes share a row -- several rows per wavefront where a row is short, a whole workgroup where it is long.
+template <Dt D, int kPieces, bool kStream> struct RowPieces {
   using E = Elem<D>;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int64_t vecsPerRow = cols / E::kPerVec;
-  const int64_t rowBytes = cols * E::kBytes;
-  const int64_t groups = (rows + kRowsPerWave - 1) / kRowsPerWave;
-  for (int64_t g = int64_t(blockIdx.x) * kWaves + wave; g < groups; g += int64_t(gridDim.x) * kWaves) {
-    float x[kRowsPerWave][kRegChunks][E::kPerVec];
-    u32x4 raw[kRowsPerWave][kRegChunks];
-    // all loads of both rows first
+  static constexpr int P = E::kPerVec;
+  typedef typename E::Unaligned Vec;
+  uint32_t start[kPieces]; // first element of the lane's pieces
+  int first;               // lane's number within the row, lanes per row, pieces per row
+  int lanes, pieces;
+  float x[kPieces][P];
+
+  __device__ __forceinline__ RowPieces(int l, int lanesPerRow, int cols) {
+    first = l;
+    lanes = lanesPerRow;
+    pieces = (cols + P - 1) / P;
 #pragma unroll
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const int64_t row = g * kRowsPerWave + r;
-      const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(in) + row * rowBytes);
+    for (int c = 0; c < kPieces; ++c)
+      start[c] = min((c * lanes + first) * P, cols - P);
+  }
+  __device__ __forceinline__ float load_and_max(const char *row) {
+    u32x4 raw[kPieces];
 #pragma unroll
-      for (int c = 0; c < kRegChunks; ++c) {
-        const int64_t v = int64_t(c) * kWave + lane;
-        if (row < rows && v < vecsPerRow)
-          raw[r][c] = load128<kStream>(src + v);
+    for (int c = 0; c < kPieces; ++c)
+      if constexpr (kStream)
+        raw[c] = __builtin_nontemporal_load(reinterpret_cast<const Vec *>(row + start[c] * E::kBytes));
+      else
+        raw[c] = *reinterpret_cast<const Vec *>(row + start[c] * E::kBytes);
+    float m = kMaxInit;
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      E::unpack(raw[c], x[c]);
+#pragma unroll
+      for (int i = 0; i < P; ++i)
+        m = fmaxf(m, x[c][i]);
+    }
+    return m;
+  }
+  __device__ __forceinline__ float exp_and_sum(float m, int cols) {
+    const int whole = cols / P; // pieces that repeat nothing
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+#pragma unroll
+      for (int i = 0; i < P; ++i)
+        x[c][i] = fast_exp(x[c][i] - m);
+      if ((c + 1) * lanes <= whole) {
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+          s += x[c][i];
+      } else {
+        int repeated = (c * lanes + first) * P - int(start[c]);
+        asm volatile("" : "+v"(repeated)); // (compared here, in every row: kept over the rows the masks spill)
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+          s += i >= repeated ? x[c][i] : 0.0f;
       }
     }
+    return s;
+  }
+  __device__ __forceinline__ void store(char *row, float inv) {
 #pragma unroll
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const int64_t row = g * kRowsPerWave + r;
-      if (row >= rows)
-        continue; // uniform across the wavefront
-      float m = kMaxInit;
+    for (int c = 0; c < kPieces; ++c) {
 #pragma unroll
-      for (int c = 0; c < kRegChunks; ++c) {
-        const bool live = int64_t(c) * kWave + lane < vecsPerRow;
-        if (live)
-          E::unpack(raw[r][c], x[r][c]);
-#pragma unroll
-        for (int i = 0; i < E::kPerVec; ++i) {
-          x[r][c][i] = live ? x[r][c][i] : kMaxInit;
-          m = fmaxf(m, x[r][c][i]);
-        }
-      }
-      m = wave_max(m);
-      float s = 0.0f;
-#pragma unroll
-      for (int c = 0; c < kRegChunks; ++c) {
-        const bool live = int64_t(c) * kWave + lane < vecsPerRow;
-#pragma unroll
-        for (int i = 0; i < E::kPerVec; ++i) {
-          x[r][c][i] = live ? fast_exp(x[r][c][i] - m) : 0.0f;
-          s += x[r][c][i];
-        }
-      }
-      s = wave_sum(s);
-      // one IEEE division per row, then multiplies (differs from z / s by at
-      // most an f32 rounding, far inside the 1e-3 bar)
-      const float inv = 1.0f / s;
-      u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + row * rowBytes);
-#pragma unroll
-      for (int c = 0; c < kRegChunks; ++c) {
-        const int64_t v = int64_t(c) * kWave + lane;
-        if (v < vecsPerRow) {
-#pragma unroll
-          for (int i = 0; i < E::kPerVec; ++i)
-            x[r][c][i] = x[r][c][i] * inv;
-          store128<kStream>(E::pack(x[r][c]), dst + v);
-        }
+      for (int i = 0; i < P; ++i)
+        x[c][i] *= inv;
+      if (c * lanes + first < pieces) {
+        Vec *to = reinterpret_cast<Vec *>(row + start[c] * E::kBytes);
+        if constexpr (kStream)
+          __builtin_nontemporal_store(Vec(E::pack(x[c])), to);
+        else
+          *to = E::pack(x[c]);
       }
     }
+  }
+};
+
+// Reductions over groups of 4 .. 64 neighbouring lanes, the result in every lane of the group.
+template <int kLanes> __device__ __forceinline__ float lanes_sum(float v) {
+  if constexpr (kLanes == kWave)
+    return wave_sum(v);
+  v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0xB1, 0xf, 0xf, true));  // lane ^ 1
+  v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x4E, 0xf, 0xf, true));  // lane ^ 2
+  if constexpr (kLanes > 4)
+    v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x141, 0xf, 0xf, true)); // mirrored within eight
+  if constexpr (kLanes > 8)
+    v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x140, 0xf, 0xf, true)); // mirrored within sixteen
+  if constexpr (kLanes > 16)
+    v += u2f(__builtin_amdgcn_ds_swizzle(f2u(v), 0x401f)); // lane ^ 16
+  return v;
+}
+template <int kLanes> __device__ __forceinline__ float lanes_max(float v) {
+  if constexpr (kLanes == kWave)
+    return wave_max(v);
+  v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0xB1, 0xf, 0xf, true)));
+  v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x4E, 0xf, 0xf, true)));
+  if constexpr (kLanes > 4)
+    v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x141, 0xf, 0xf, true)));
+  if constexpr (kLanes > 8)
+    v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x140, 0xf, 0xf, true)));
+  if constexpr (kLanes > 16)
+    v = fmaxf(v, u2f(__builtin_amdgcn_ds_swizzle(f2u(v), 0x401f)));
+  return v;
+}
+
+template <Dt D, int kLanes, int kPieces, bool kStream>
+__device__ __forceinline__ void softmax_rows_by_lanes(const void *in, void *out, int64_t rows, int64_t cols) {
+  const int64_t rowBytes = cols * Elem<D>::kBytes;
+  RowPieces<D, kPieces, kStream> r(threadIdx.x % kLanes, kLanes, int(cols));
+  for (int64_t row = int64_t(blockIdx.x) * (kThreads / kLanes) + threadIdx.x / kLanes; row < rows;
+       row += int64_t(gridDim.x) * (kThreads / kLanes)) {
+    const float m = lanes_max<kLanes>(r.load_and_max(static_cast<const char *>(in) + row * rowBytes));
+    const float s = lanes_sum<kLanes>(r.exp_and_sum(m, int(cols)));
+    // one IEEE division per row, then multiplies (differs from z / s by at
+    // most an f32 rounding, far inside the 1e-3 bar)
+    r.store(static_cast<char *>(out) + row * rowBytes, 1.0f / s);
+  }
+}
+
+template <Dt D, int kPieces>
+__device__ __forceinline__ void softmax_rows_by_workgroup(const void *in, void *out, int64_t rows, int64_t cols,
+                                                          f32x4 (&part)[2][kMaxWaves / 4]) {
+  const int64_t rowBytes = cols * Elem<D>::kBytes;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), quads = blockDim.x / kWave / 4;
+  RowPieces<D, kPieces, true> r(threadIdx.x, blockDim.x, int(cols));
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    float m = wave_max(r.load_and_max(static_cast<const char *>(in) + row * rowBytes));
+    if (lane == 0)
+      reinterpret_cast<float *>(part[0])[wave] = m;
+    __syncthreads(); // (also: the sums of the row before have been read)
+    for (int q = 0; q < quads; ++q) {
+      const f32x4 v = part[0][q];
+      m = fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));
+    }
+    const float t = wave_sum(r.exp_and_sum(m, int(cols)));
+    if (lane == 0)
+      reinterpret_cast<float *>(part[1])[wave] = t;
+    __syncthreads(); // (also: the maxima have been read)
+    float s = 0.0f;
+    for (int q = 0; q < quads; ++q) {
+      const f32x4 v = part[1][q];
+      s += (v.x + v.y) + (v.z + v.w);
+    }
+    r.store(static_cast<char *>(out) + row * rowBytes, 1.0f / s);
+  }
+}
+
+// A row shorter than one piece: a lane has it.
+template <Dt D>
+__device__ __forceinline__ void softmax_rows_of_a_lane(const void *in, void *out, int64_t rows, int64_t cols) {
+  using E = Elem<D>;
+  for (int64_t row = int64_t(blockIdx.x) * kThreads + threadIdx.x; row < rows; row += int64_t(gridDim.x) * kThreads) {
+    float x[E::kPerVec - 1], m = kMaxInit, s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < E::kPerVec - 1; ++i)
+      if (i < cols) {
+        x[i] = E::load(in, row * cols + i);
+        m = fmaxf(m, x[i]);
+      }
+#pragma unroll
+    for (int i = 0; i < E::kPerVec - 1; ++i)
+      if (i < cols) {
+        x[i] = fast_exp(x[i] - m);
+        s += x[i];
+      }
+    const float inv = 1.0f / s;
+#pragma unroll
+    for (int i = 0; i < E::kPerVec - 1; ++i)
+      if (i < cols)
+        E::store(out, row * cols + i, x[i] * inv);
   }
 }
 
@@ -358,72 +472,6 @@ __device__ __forceinline__ float block_reduce(float v, bool isMax, float *scratc
   return r;
 }
 
-// ---- LDS path: a workgroup owns a row, staged once in LDS as f32 ------------------------
-template <Dt D>
-__device__ __forceinline__ void softmax_row_in_lds(const void *in, void *out, int64_t row, int64_t cols,
-                                                   float *rowBuf, float *scratch, bool vec) {
-  using E = Elem<D>;
-  const int64_t base = row * cols;
-  float m = kMaxInit;
-  // Vector path: element i of 16-byte vector v lives at rowBuf[i * vecs + v], so
-  // neighbouring lanes touch neighbouring LDS words (no bank conflicts).
-  const int64_t vecs = cols / E::kPerVec;
-  if (vec) {
-    const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(in) + base * E::kBytes);
-    for (int64_t v = threadIdx.x; v < vecs; v += kThreads) {
-      float f[E::kPerVec];
-      E::unpack(src[v], f);
-#pragma unroll
-      for (int i = 0; i < E::kPerVec; ++i) {
-        rowBuf[i * vecs + v] = f[i];
-        m = fmaxf(m, f[i]);
-      }
-    }
-  } else {
-    for (int64_t c = threadIdx.x; c < cols; c += kThreads) {
-      const float f = E::load(in, base + c);
-      rowBuf[c] = f;
-      m = fmaxf(m, f);
-    }
-  }
-  m = block_reduce(m, true, scratch); // its barriers also publish rowBuf
-  float s = 0.0f;
-  // each thread revisits exactly the elements it wrote: no barrier needed until the sum
-  if (vec) {
-    for (int64_t v = threadIdx.x; v < vecs; v += kThreads)
-#pragma unroll
-      for (int i = 0; i < E::kPerVec; ++i) {
-        const float e = fast_exp(rowBuf[i * vecs + v] - m);
-        rowBuf[i * vecs + v] = e;
-        s += e;
-      }
-  } else {
-    for (int64_t c = threadIdx.x; c < cols; c += kThreads) {
-      const float e = fast_exp(rowBuf[c] - m);
-      rowBuf[c] = e;
-      s += e;
-    }
-  }
-  s = block_reduce(s, false, scratch);
-  // normalised like the other two paths: one IEEE reciprocal per row, then multiplies (an f32 rounding away
-  // from e / s at most, the same on every path, so a row's last bit does not depend on its length class)
-  const float inv = 1.0f / s;
-  if (vec) {
-    u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + base * E::kBytes);
-    for (int64_t v = threadIdx.x; v < vecs; v += kThreads) {
-      float f[E::kPerVec];
-#pragma unroll
-      for (int i = 0; i < E::kPerVec; ++i)
-        f[i] = rowBuf[i * vecs + v] * inv;
-      dst[v] = E::pack(f);
-    }
-  } else {
-    for (int64_t c = threadIdx.x; c < cols; c += kThreads)
-      E::store(out, base + c, rowBuf[c] * inv);
-  }
-  __syncthreads(); // rowBuf is reused by the next row
-}
-
 // ---- any length: workgroup per row, the input read twice -----------------------------------
 // The streaming form of test/Integration/Dialect/XeGPU/WG/softmax_intra_sg_cross_lane.mlir:135-175:
 // one pass carries a running maximum m and a running sum s of exp(x - m), rescaling s by
@@ -498,27 +546,68 @@ __device__ __forceinline__ void softmax_row_streamed(const void *in, void *out, 
   }
 }
 
-template <Dt D>
+template <Dt D, int kLanes, bool kStream>
+__device__ __forceinline__ void softmax_lanes(const void *in, void *out, int64_t rows, int64_t cols, int per) {
+  if (per <= 1)
+    softmax_rows_by_lanes<D, kLanes, 1, kStream>(in, out, rows, cols);
+  else if (per == 2)
+    softmax_rows_by_lanes<D, kLanes, 2, kStream>(in, out, rows, cols);
+  else if (per == 3)
+    softmax_rows_by_lanes<D, kLanes, 3, kStream>(in, out, rows, cols);
+  else
+    softmax_rows_by_lanes<D, kLanes, 4, kStream>(in, out, rows, cols);
+}
+
+template <Dt D, int kMaxThreads>
 __device__ __forceinline__ void softmax_kernel(const void *in, void *out, int64_t rows, int64_t cols) {
   using E = Elem<D>;
   __shared__ float scratch[kWaves];
-  __shared__ __attribute__((aligned(16))) float rowBuf[kLdsCols];
+  __shared__ f32x4 part[2][kMaxWaves / 4];
   const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 &&
                        (cols % E::kPerVec) == 0;
-  if (aligned && cols <= int64_t(kRegChunks) * kWave * E::kPerVec) {
-    // non-temporal accesses: measured faster hot and cold
-    if constexpr (D == Dt::F16) {
-      if (cols == int64_t(kRegChunks) * kWave * 8)
+  const int64_t pieces = (cols + E::kPerVec - 1) / E::kPerVec;
+  if (cols < E::kPerVec) {
+    softmax_rows_of_a_lane<D>(in, out, rows, cols);
+    return;
+  }
+  if constexpr (D == Dt::F16 && kMaxThreads == kThreads)
+    if (aligned && pieces > kWave && pieces <= kRegChunks * kWave) { // non-temporal accesses: measured faster hot and cold
+      if (pieces == kRegChunks * kWave)
         softmax_f16_rows_in_regs<true>(in, out, rows, cols);
       else
         softmax_f16_rows_in_regs<false>(in, out, rows, cols);
-    } else if (rows >= kTwoRowsFrom)
-      softmax_rows_in_regs<D, true, 2>(in, out, rows, cols);
+      return;
+    }
+  if (pieces <= 4 * kWave && (pieces <= kWave || rows >= kManyRows)) {
+    int lanes = 4;
+    while (4 * lanes < pieces || (lanes < pieces && lanes < kWave && rows * lanes < kManyRows * kWave))
+      lanes *= 2;
+    const int per = int(pieces + lanes - 1) / lanes;
+    // Non-temporal accesses from rows of 32 lanes on (of 16 where rows are whole pieces): 20000 x 1001 f32 28.6 us, 30.6
+    // with ordinary ones.  Rows shorter than that share cache lines, which ordinary accesses keep until all of a line
+    // is there: 200001 x 77 bf16 25.4 -> 16.5, 10^6 x 40 f32 99 -> 61.
+    switch (lanes) {
+    case 4: softmax_lanes<D, 4, false>(in, out, rows, cols, per); break;
+    case 8: softmax_lanes<D, 8, false>(in, out, rows, cols, per); break;
+    case 16:
+      if (cols % E::kPerVec == 0)
+        softmax_lanes<D, 16, true>(in, out, rows, cols, per);
+      else
+        softmax_lanes<D, 16, false>(in, out, rows, cols, per);
+      break;
+    case 32: softmax_lanes<D, 32, true>(in, out, rows, cols, per); break;
+    default: softmax_lanes<D, 64, true>(in, out, rows, cols, per); break;
+    }
+  } else if (pieces <= 4 * int64_t(blockDim.x)) {
+    const int per = int(pieces + blockDim.x - 1) / int(blockDim.x);
+    if (per <= 1)
+      softmax_rows_by_workgroup<D, 1>(in, out, rows, cols, part);
+    else if (per == 2)
+      softmax_rows_by_workgroup<D, 2>(in, out, rows, cols, part);
+    else if (per == 3)
+      softmax_rows_by_workgroup<D, 3>(in, out, rows, cols, part);
     else
-      softmax_rows_in_regs<D, true, 1>(in, out, rows, cols);
-  } else if (cols <= kLdsCols) {
-    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
-      softmax_row_in_lds<D>(in, out, row, cols, rowBuf, scratch, aligned);
+      softmax_rows_by_workgroup<D, 4>(in, out, rows, cols, part);
   } else {
     for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
       softmax_row_streamed<D>(in, out, row, cols, scratch, aligned);
@@ -527,19 +616,17 @@ __device__ __forceinline__ void softmax_kernel(const void *in, void *out, int64_
 
 } // namespace
 
-// 8 wavefronts per SIMD (64 registers per lane) so two rows per wavefront still
-// leave room for full occupancy.
-#define IMEX_SOFTMAX_BOUNDS __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
+// 8 wavefronts per SIMD (64 registers per lane).  The _shared kernels are the operators under the launch that gives every
+// group of lanes one row, workgroups of up to 1024 lanes included.
+#define IMEX_SOFTMAX(name, T, D, threads)                                                                          \
+  extern "C" __global__ __launch_bounds__(threads) __attribute__((amdgpu_waves_per_eu(8, 8))) void name(            \
+      const T *in, T *out, int64_t rows, int64_t cols) {                                                            \
+    softmax_kernel<D, threads>(in, out, rows, cols);                                                                \
+  }
 
-extern "C" __global__ IMEX_SOFTMAX_BOUNDS void imex_softmax_f32(const float *in, float *out, int64_t rows,
-                                                                int64_t cols) {
-  softmax_kernel<Dt::F32>(in, out, rows, cols);
-}
-extern "C" __global__ IMEX_SOFTMAX_BOUNDS void imex_softmax_f16(const uint16_t *in, uint16_t *out, int64_t rows,
-                                                                int64_t cols) {
-  softmax_kernel<Dt::F16>(in, out, rows, cols);
-}
-extern "C" __global__ IMEX_SOFTMAX_BOUNDS void imex_softmax_bf16(const uint16_t *in, uint16_t *out, int64_t rows,
-                                                                 int64_t cols) {
-  softmax_kernel<Dt::BF16>(in, out, rows, cols);
-}
+IMEX_SOFTMAX(imex_softmax_f32, float, Dt::F32, kThreads)
+IMEX_SOFTMAX(imex_softmax_f16, uint16_t, Dt::F16, kThreads)
+IMEX_SOFTMAX(imex_softmax_bf16, uint16_t, Dt::BF16, kThreads)
+IMEX_SOFTMAX(imex_softmax_f32_shared, float, Dt::F32, kMaxWaves * kWave)
+IMEX_SOFTMAX(imex_softmax_f16_shared, uint16_t, Dt::F16, kMaxWaves * kWave)
+IMEX_SOFTMAX(imex_softmax_bf16_shared, uint16_t, Dt::BF16, kMaxWaves * kWave)

@@ -34,7 +34,7 @@ extern const unsigned char imex_blob_attention[], imex_blob_attention_end[];
 namespace {
 
 enum class Module { Eltwise, Softmax, Reduce, Transpose, Gemm, GemmSmall, GemmUnaligned, Fusion, Attention };
-enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, RowSum, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention };
+enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention };
 
 struct Entry {
   const char *name;
@@ -67,6 +67,9 @@ const Entry kEntries[] = {
     {"imex_softmax_f32", "(in: f32*, out: f32*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxRows32, 2},
     {"imex_softmax_f16", "(in: f16*, out: f16*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxRows16, 2},
     {"imex_softmax_bf16", "(in: bf16*, out: bf16*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxRows16, 2},
+    {"imex_softmax_f32_shared", "(in: f32*, out: f32*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxShared32, 2},
+    {"imex_softmax_f16_shared", "(in: f16*, out: f16*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxShared16, 2},
+    {"imex_softmax_bf16_shared", "(in: bf16*, out: bf16*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxShared16, 2},
     {"imex_rowsum_f32", "(in: f32*, out: f32*, rows: i64, cols: i64, init: f32)", Module::Reduce, Shape::RowSum, 2},
     {"imex_rowmean_f32", "(in: f32*, out: f32*, rows: i64, cols: i64)", Module::Reduce, Shape::RowSum, 2},
     {"imex_reduce_outer_f32", "(in: f32*, out: f32*, outer: i64, inner: i64, init: f32)", Module::Reduce,
@@ -279,6 +282,20 @@ const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   return find(name)->name;
 }
 
+// The operator's own launch is one for wavefronts (four per workgroup) or workgroups of 256 that have a row each: right
+// for f16 rows that wavefronts walk (65 .. 128 whole 16-byte pieces) and for rows that fit nobody's registers (more than
+// 4096 pieces).  Every other row goes to as many lanes as suit its length: 65536 x 32 bf16 20.5 us with a wavefront
+// per row, 3.2 so; 2500 x 8191 55.3 with 256 lanes of the streaming form, 18.8; 16384 x 1024 f32 24.4 / 23.1.
+const char *softmaxVariant(const Entry *e, int64_t rows, int64_t cols) {
+  const int64_t perVec = e->shape == Shape::SoftmaxRows16 ? 8 : 4, pieces = (cols + perVec - 1) / perVec;
+  const bool walked = cols % perVec == 0 && pieces > 64 && pieces <= 128 && strcmp(e->name, "imex_softmax_f16") == 0;
+  if (rows == 0 || cols == 0 || walked || pieces > 4096)
+    return e->name;
+  char name[96];
+  snprintf(name, sizeof name, "%s_shared", e->name);
+  return find(name)->name;
+}
+
 extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *dims, int ndims) {
   const Entry *e = find(kernel);
   if (!e || ndims != e->ndims || (ndims > 0 && !dims))
@@ -294,6 +311,9 @@ extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *d
   case Shape::ReduceOuter:
   case Shape::ReduceOuter16:
     return reduceVariant(e, dims[0], dims[1]);
+  case Shape::SoftmaxRows32:
+  case Shape::SoftmaxRows16:
+    return softmaxVariant(e, dims[0], dims[1]);
   default:
     return e->name;
   }
@@ -331,11 +351,9 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     break;
   case Shape::SoftmaxRows32:
   case Shape::SoftmaxRows16: {
-    // Rows of up to 128 x 16 B stay in registers, one per wavefront (four per workgroup); longer rows take
-    // a workgroup each.  The kernels stride over the rows, so any grid is correct.  f32 and bf16 register
-    // rows: one pass (two rows per wavefront from 16384 rows on).  f16 register rows: a wavefront walks
-    // its rows with the next row's loads in flight, and 2048 workgroups give every wavefront slot of the
-    // chip (256 CUs x 4 SIMDs x 8) one wavefront.
+    // Any grid is correct, the kernels stride over the rows.  f16 rows of 65 .. 128 whole 16-byte pieces: a
+    // wavefront walks its rows with the next row's loads in flight, and 2048 workgroups give every wavefront
+    // slot of the chip (256 CUs x 4 SIMDs x 8) one wavefront.
     const int64_t regCols = e->shape == Shape::SoftmaxRows16 ? 1024 : 512;
     const bool f16 = std::strcmp(e->name, "imex_softmax_f16") == 0;
     if (dims[1] > regCols)
@@ -346,6 +364,25 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
       grid[0] = ceilDiv(dims[0], dims[0] >= 16384 ? 8 : 4);
     if (dims[1] == 0)
       grid[0] = 0;
+    break;
+  }
+  case Shape::SoftmaxShared32:
+  case Shape::SoftmaxShared16: { // one row for every group of lanes: the kernels' own rule (softmax_kernel in softmax.hip)
+    const int64_t rows = dims[0], cols = dims[1], perVec = e->shape == Shape::SoftmaxShared16 ? 8 : 4;
+    const int64_t pieces = (cols + perVec - 1) / perVec;
+    if (cols == 0)
+      grid[0] = 0;
+    else if (cols < perVec)
+      grid[0] = ceilDiv(rows, 256);
+    else if (pieces <= 256 && (pieces <= 64 || rows >= 2048)) {
+      int64_t lanes = 4;
+      while (4 * lanes < pieces || (lanes < pieces && lanes < 64 && rows * lanes < 2048 * 64))
+        lanes *= 2;
+      grid[0] = ceilDiv(rows, 256 / lanes);
+    } else {
+      grid[0] = static_cast<size_t>(std::min<int64_t>(rows, 1048560));
+      block[0] = pieces <= 1024 ? 256 : pieces <= 2048 ? 512 : pieces <= 4096 ? 1024 : 256;
+    }
     break;
   }
   case Shape::RowSum: // workgroup per row above 2048 columns, else wavefront per row

@@ -245,6 +245,38 @@ def test_softmax_nan_and_infinite_rows(host, orc, stream, dtype, cols):
     assert np.all(np.abs(got[ok] - ref[ok]) <= 1e-3 * np.abs(ref[ok]) + (2.0 ** -24 if dtype == "f16" else 0.0))
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,pieces", [(40001, 0.75), (40001, 1), (70000, 4), (70000, 4.25), (9001, 8.75), (9001, 16.5),
+                                         (4500, 32.25), (4500, 63.75), (2049, 64.25), (2049, 129.5), (2048, 256), (2047, 255.75),
+                                         (3000, 256.25), (3, 1023.75), (5, 1024.25), (5, 3072.5), (3, 4095.75), (2, 4096.25)])
+def test_softmax_rows_of_any_length_and_address(host, orc, stream, rows, pieces, dtype):
+    """Rows at the edges of the kernel's splits (16-byte pieces per row: less than one, a lane's four, a wavefront's
+    256, a workgroup's 1024, 2048 and 4096), from buffers that start one element behind a 16-byte boundary, and the
+    elements on either side of the result untouched.  Tolerances: those of test_softmax_shapes; bf16 outputs are
+    the oracle's value or its neighbour (one rounding, 2^-8, of quotients that differ by f32 roundings)."""
+    per, width = (4, 4) if dtype == "f32" else (8, 2)
+    cols = int(pieces * per)
+    say("softmax %s %dx%d, unaligned" % (dtype, rows, cols))
+    x = orc.fill_normal(rows * cols, dtype, rows + cols, 0.0, 2.0)
+    raw = np.zeros(rows * cols + 2, x.dtype)
+    raw[1:-1] = x
+    d_in, d_out = stream.to_device(raw), stream.to_device(np.full_like(raw, 7))
+    stream.launch("imex_softmax_" + dtype, [rows, cols], [host.Ptr(d_in + width), host.Ptr(d_out + width), rows, cols])
+    stream.wait()
+    got = stream.from_device(d_out, (rows * cols + 2,), raw.dtype)
+    stream.free(d_in), stream.free(d_out)
+    assert got[0] == 7 and got[-1] == 7
+    got, x = got[1:-1].reshape(rows, cols), x.reshape(rows, cols)
+    if dtype == "f32":
+        ref = orc.softmax_f32(x)
+        assert np.max(np.abs(got - ref) / np.maximum(ref, 1e-30)) < 5e-5
+    elif dtype == "f16":
+        assert close_16(orc, got, orc.softmax_16(x, "f16"), "f16")
+    else:
+        ref = orc.softmax_16(x, "bf16")
+        assert np.max(np.abs(got.astype(np.int32) - ref.astype(np.int32))) <= 1
+
+
 @pytest.mark.parametrize("rows,cols", [(1000, 1024), (1000, 1016), (37, 1024), (4097, 1024), (5, 8)])
 def test_softmax_f16_rows_in_registers_any_grid(host, orc, stream, rows, cols):
     """The f16 register path walks its rows with the next row's loads in flight: a wavefront that takes one
