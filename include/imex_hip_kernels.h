@@ -39,6 +39,8 @@
  *       benchmarks/transpose/transpose2d_gpu.mlir.in:4-11 dims = {rows, cols}
  *   imex_transpose3d_b16 / _b32    (in, out, d0:i64, d1:i64, d2:i64)
  *       benchmarks/transpose/transpose3d_gpu.mlir.in:4-11 dims = {d0, d1, d2}
+ *   imex_transpose2d_b16_any, imex_transpose2d_b32_any, imex_transpose3d_b16_any, imex_transpose3d_b32_any
+ *       the same for rows that are no whole 16-byte vectors                   dims as above
  *   imex_loop_fusion_f32 / _f16 / _bf16   (a, b, out, n:i64)         out = (log a + |b|) - a
  *       benchmarks/kLoopFusion/kLoopFusion.mlir.in:4-30  dims = {n}
  *   imex_input_fusion_f32 / _f16 / _bf16  (a, b, out, rows:i64, cols:i64)

@@ -36,14 +36,16 @@
 //    through LDS and out: a workgroup always has a tile's reads in flight (4096 x 4096 streaming
 //    from HBM: 22.9 us against 24.0 us with one workgroup per tile).  The same walk for the 16-bit
 //    256 x 256 tile (512 lanes, so that two tiles fit the registers) gained 1.5 % and is not used.
-// Shapes or bases that break 16-byte alignment use the scalar 64 x 64 tile path
-// of the same kernel.
+//  * Shapes or bases that break 16-byte alignment: 8 x 8 (4 x 4) blocks at any address, moved back inside at the
+//    edges (tile_unaligned).  Bound by HBM transactions: row segments that are no whole lines cost two partly used
+//    ones each (16-bit 5000 x 4097: 22.1 us, 3.7 TB/s; 5000 x 4096 would take 13.7 at 6 TB/s; one element at a time
+//    before: 150 us with buffers that are not in the caches).
 //
 // Arguments: 2-D (in, out, rows: i64, cols: i64); 3-D (in, out, d0, d1, d2: i64).
 // Launch: block (256,1,1); one workgroup per tile, grid 2-D (ceil(cols/C),
 // ceil(rows/R), 1), 3-D (ceil(d2/C), ceil(d0/R), d1) with (R, C) as above -- for 32-bit
-// problems of whole 128 x 128 tiles at most 512 workgroups in all; any
-// other grid is also correct (workgroups stride over the tiles).
+// problems of whole 128 x 128 tiles at most 512 workgroups in all; the _any kernels one
+// workgroup per 512-byte x 128-byte tile; any other grid is also correct (workgroups stride over the tiles).
 
 #include "device_common.h"
 
@@ -237,7 +239,77 @@ __device__ __forceinline__ void tile16_quarters(const uint16_t *__restrict__ in,
   }
 }
 
-// ---- any shape / alignment ------------------------------------------------------
+// ---- any sizes and addresses, from 8 rows and 8 columns of 16-bit (4 x 4 of 32-bit) elements on --------------------
+// The scheme of tile16_fast and Tile32 on blocks of B x B elements (B to a 16-byte vector) whose rows and columns need
+// not be aligned: 16-byte loads and stores take any element's address.  A block that would stick out of the matrix is
+// moved back inside instead -- it starts at rows - B or cols - B, and the elements it shares with the block before are
+// written twice with the same value -- so there are no partial vectors anywhere.  Ordinary accesses, not non-temporal
+// ones: neighbouring row segments share cache lines, which the caches put together.
+template <typename T> struct Block;
+template <> struct Block<uint16_t> {
+  static constexpr int B = 8;
+  typedef uint32_t Vec __attribute__((ext_vector_type(4), aligned(2)));
+  // column c of the block whose rows are x[0 .. 7]
+  static __device__ __forceinline__ u32x4 column(const u32x4 (&x)[8], int c) {
+    const uint32_t pick = c & 1 ? 0x07060302u : 0x05040100u; // the high or the low halves of a word of two rows
+    u32x4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      v[q] = __builtin_amdgcn_perm(x[2 * q + 1][c >> 1], x[2 * q][c >> 1], pick);
+    return v;
+  }
+};
+template <> struct Block<uint32_t> {
+  static constexpr int B = 4;
+  typedef uint32_t Vec __attribute__((ext_vector_type(4), aligned(4)));
+  static __device__ __forceinline__ u32x4 column(const u32x4 (&x)[4], int c) {
+    return u32x4{x[0][c], x[1][c], x[2][c], x[3][c]};
+  }
+};
+
+template <typename T, int R, int C>
+__device__ __forceinline__ void tile_unaligned(const T *__restrict__ in, T *__restrict__ out, const View &v, int64_t r0,
+                                               int64_t c0, u32x4 *tile) {
+  typedef Block<T> Blk;
+  typedef typename Blk::Vec Vec;
+  constexpr int B = Blk::B, G = R / B, CG = C / B;   // 16-byte groups per LDS row, column blocks
+  constexpr int BP = kThreads / CG, LP = G / BP;     // row blocks per pass, passes
+  constexpr int CP = kThreads / G, SP = C / CP;      // store: output rows per pass, passes
+  static_assert(G >= 16 && (G & (G - 1)) == 0 && LP >= 1 && LP * BP == G, "whole passes, and 16 groups or more to swizzle");
+  const int rowsLeft = int(min(v.rows - r0, int64_t(R))), colsLeft = int(min(v.cols - c0, int64_t(C)));
+  const int cg = threadIdx.x % CG, bb = threadIdx.x / CG;
+  u32x4 x[LP][B];
+  const T *src = in + r0 * v.ldIn + c0;
+  const int col = cg * B < colsLeft ? min(cg * B, colsLeft - B) : 0; // (may lie in the tile before)
+#pragma unroll
+  for (int p = 0; p < LP; ++p) {
+    const int row = (bb + BP * p) * B;
+    if (row < rowsLeft && cg * B < colsLeft) {
+      const T *from = src + min(row, rowsLeft - B) * v.ldIn + col;
+#pragma unroll
+      for (int j = 0; j < B; ++j)
+        x[p][j] = *reinterpret_cast<const Vec *>(from + j * v.ldIn);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < LP; ++p) {
+    const int pos = (bb + BP * p) ^ (cg & 15);
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+      tile[(cg * B + k) * G + pos] = Blk::column(x[p], k);
+  }
+  lds_barrier();
+  const int g = threadIdx.x % G, cc = threadIdx.x / G;
+  T *dst = out + c0 * v.ldOut + r0 + min(g * B, rowsLeft - B);
+#pragma unroll
+  for (int p = 0; p < SP; ++p) {
+    const int c = cc + CP * p, block = c / B * B; // LDS row, first column of its block
+    if (block < colsLeft && g * B < rowsLeft)
+      *reinterpret_cast<Vec *>(dst + (min(block, colsLeft - B) + c % B) * v.ldOut) = tile[c * G + (g ^ (c / B & 15))];
+  }
+}
+
+// ---- fewer rows or columns than that ------------------------------------------------------
 template <typename T, int kTile>
 __device__ __forceinline__ void tile_scalar(const T *__restrict__ in, T *__restrict__ out, const View &v,
                                             int64_t r0, int64_t c0, T (*tile)[kTile + 1]) {
@@ -271,6 +343,26 @@ __device__ __forceinline__ void for_each_tile(const View &v, int64_t planes, Bod
     const int64_t ty = rem % tilesY;
     const int64_t tx = (ty + rem / tilesY) % tilesX;
     body(plane, ty * R, tx * C);
+    __syncthreads(); // the tile has left LDS before the next one is staged
+  }
+}
+
+// The same tiles in another order: workgroups go to the 8 XCDs in turn, and each XCD takes its own eighth of the tiles,
+// down the tile rows of one tile column after the other.  Row segments that share a cache line -- neighbours, where
+// rows are no whole lines -- then meet in one L2, which writes the line once (16-bit 4001 x 4096: 15.5 us, 19.7
+// by diagonals; 32-bit 9999 x 6001: 109 / 134).
+template <int R, int C, typename Body>
+__device__ __forceinline__ void for_each_tile_by_xcd(const View &v, int64_t planes, Body body) {
+  const int64_t tilesX = (v.cols + C - 1) / C, tilesY = (v.rows + R - 1) / R;
+  const int64_t perPlane = tilesX * tilesY, total = perPlane * planes, share = (total + 7) / 8;
+  const int64_t first = (int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  const int64_t stride = int64_t(gridDim.x) * gridDim.y * gridDim.z;
+  for (int64_t t = first; t < 8 * share; t += stride) {
+    const int64_t u = (t & 7) * share + (t >> 3);
+    if (u >= total)
+      continue; // the last XCD's share may be the smaller one
+    const int64_t plane = u / perPlane, rem = u % perPlane;
+    body(plane, rem % tilesY * R, rem / tilesY * C);
     __syncthreads(); // the tile has left LDS before the next one is staged
   }
 }
@@ -323,6 +415,23 @@ __device__ __forceinline__ void pipelined_tiles(const T *in, T *out, const View 
   }
 }
 
+// Any sizes and addresses.  Tiles of 512-byte output segments by 128 bytes of input rows: with whole lines shared
+// between neighbours the write side gains from long segments more than the read side loses (16-bit 9999 x 6001, by
+// diagonals: 256 x 64 64.3 us, 128 x 128 76.8, 256 x 128 67.5, 64 x 64 93.7, 512 x 32 64.3).
+template <typename T>
+__device__ __forceinline__ void transpose_any(const T *in, T *out, const View &v, int64_t planes, int64_t inPlane,
+                                              int64_t outPlane, char *lds) {
+  constexpr int R = 512 / sizeof(T), C = 128 / sizeof(T);
+  if (v.rows >= Block<T>::B && v.cols >= Block<T>::B)
+    for_each_tile_by_xcd<R, C>(v, planes, [&](int64_t plane, int64_t r0, int64_t c0) {
+      tile_unaligned<T, R, C>(in + plane * inPlane, out + plane * outPlane, v, r0, c0, reinterpret_cast<u32x4 *>(lds));
+    });
+  else
+    for_each_tile<64, 64>(v, planes, [&](int64_t plane, int64_t r0, int64_t c0) {
+      tile_scalar<T, 64>(in + plane * inPlane, out + plane * outPlane, v, r0, c0, reinterpret_cast<T(*)[65]>(lds));
+    });
+}
+
 // planes: number of 2-D problems (1, or d1 for the 3-D reversal) with element
 // strides inPlane / outPlane between them.
 template <typename T>
@@ -337,9 +446,7 @@ __device__ __forceinline__ void transpose_block(const T *in, T *out, const View 
                     inPlane % kVec == 0 && outPlane % kVec == 0;
   const bool big = v.rows * v.cols * planes >= kBigProblem;
   if (!fast) {
-    for_each_tile<64, 64>(v, planes, [&](int64_t plane, int64_t r0, int64_t c0) {
-      tile_scalar<T, 64>(in + plane * inPlane, out + plane * outPlane, v, r0, c0, reinterpret_cast<T(*)[65]>(lds));
-    });
+    transpose_any(in, out, v, planes, inPlane, outPlane, lds);
   } else if constexpr (sizeof(T) == 4) {
     if (big && v.rows % 128 == 0 && v.cols % 128 == 0)
       pipelined_tiles<128, 128, Tile32<128, 128>>(in, out, v, planes, inPlane, outPlane, reinterpret_cast<u32x4 *>(lds));
@@ -393,4 +500,31 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose3d_b32(cons
 extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose3d_b16(const uint16_t *in, uint16_t *out,
                                                                            int64_t d0, int64_t d1, int64_t d2) {
   transpose_block<uint16_t>(in, out, View{d0, d2, d1 * d2, d1 * d0}, d1, d2, d0);
+}
+
+// The operators for sizes that are no whole 16-byte vectors, with the LDS of these tiles only: four workgroups on a
+// CU where the kernels above leave room for two (16-bit 9999 x 6001: 59.9 us, 79.9 with 64 KiB of LDS and
+// 128 x 128 tiles; 307.8 one element at a time).
+extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose2d_b32_any(const uint32_t *in, uint32_t *out,
+                                                                               int64_t rows, int64_t cols) {
+  __shared__ __attribute__((aligned(16))) char lds[64 * 65 * 4];
+  transpose_any<uint32_t>(in, out, View{rows, cols, cols, rows}, 1, 0, 0, lds);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose2d_b16_any(const uint16_t *in, uint16_t *out,
+                                                                               int64_t rows, int64_t cols) {
+  __shared__ __attribute__((aligned(16))) char lds[512 * 64];
+  transpose_any<uint16_t>(in, out, View{rows, cols, cols, rows}, 1, 0, 0, lds);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose3d_b32_any(const uint32_t *in, uint32_t *out,
+                                                                               int64_t d0, int64_t d1, int64_t d2) {
+  __shared__ __attribute__((aligned(16))) char lds[64 * 65 * 4];
+  transpose_any<uint32_t>(in, out, View{d0, d2, d1 * d2, d1 * d0}, d1, d2, d0, lds);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose3d_b16_any(const uint16_t *in, uint16_t *out,
+                                                                               int64_t d0, int64_t d1, int64_t d2) {
+  __shared__ __attribute__((aligned(16))) char lds[512 * 64];
+  transpose_any<uint16_t>(in, out, View{d0, d2, d1 * d2, d1 * d0}, d1, d2, d0, lds);
 }

@@ -491,6 +491,28 @@ def test_transpose_large_tiles_ragged(host, orc, stream, rows, cols, dtype):
     assert np.array_equal(got, x.T)
 
 
+@pytest.mark.parametrize("rows,planes,cols", [(8, 1, 9), (9, 1, 8), (4, 1, 5), (7, 1, 300), (256, 1, 65), (257, 1, 64), (255, 3, 63),
+                                              (264, 1, 1001), (1001, 1, 264), (129, 2, 33), (513, 5, 191), (4097, 1, 4001)])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_transpose_of_any_size_and_address(host, orc, stream, rows, planes, cols, dtype):
+    """Sizes at the edges of the blocks and tiles for rows that are no whole 16-byte vectors, from buffers that start
+    one element behind a 16-byte boundary; both kernels of the operator, the elements around the result untouched."""
+    n, width, bits = rows * planes * cols, 4 if dtype == "f32" else 2, 32 if dtype == "f32" else 16
+    say("transpose %s %dx%dx%d, unaligned" % (dtype, rows, planes, cols))
+    raw = orc.fill_bits(n + 2, dtype, rows + cols).view(np.uint32 if dtype == "f32" else np.uint16)
+    want = raw[1:-1].reshape(rows, planes, cols).transpose(2, 1, 0)
+    dims = [rows, cols] if planes == 1 else [rows, planes, cols]
+    name = "imex_transpose%dd_b%d" % (len(dims), bits)
+    for grid in (None, (3, 1, 1)):  # the catalogue's choice; the operator itself, its workgroups walking the tiles
+        d_in, d_out = stream.to_device(raw), stream.to_device(np.full_like(raw, 7))
+        stream.launch(name, dims, [host.Ptr(d_in + width), host.Ptr(d_out + width), *dims], grid=grid)
+        stream.wait()
+        got = stream.from_device(d_out, raw.shape, raw.dtype)
+        stream.free(d_in), stream.free(d_out)
+        assert got[0] == 7 and got[-1] == 7
+        assert np.array_equal(got[1:-1].reshape(want.shape), want)
+
+
 @pytest.mark.parametrize("rows,cols", [(4096, 4224), (128, 131072), (8192, 4096)])
 def test_transpose_b32_whole_tiles_pipelined(host, orc, stream, rows, cols):
     """32-bit problems made of whole 128 x 128 tiles: at most 512 workgroups, each walking two or more tiles
