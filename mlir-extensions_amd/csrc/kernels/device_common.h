@@ -85,6 +85,34 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 #undef IMEX_DPP_REDUCE
 
+// Reductions over groups of 4 .. 64 neighbouring lanes, the result in every lane of the group.
+template <int kLanes> __device__ __forceinline__ float lanes_sum(float v) {
+  if constexpr (kLanes == kWave)
+    return wave_sum(v);
+  v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0xB1, 0xf, 0xf, true));  // lane ^ 1
+  v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x4E, 0xf, 0xf, true));  // lane ^ 2
+  if constexpr (kLanes > 4)
+    v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x141, 0xf, 0xf, true)); // mirrored within eight
+  if constexpr (kLanes > 8)
+    v += u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x140, 0xf, 0xf, true)); // mirrored within sixteen
+  if constexpr (kLanes > 16)
+    v += u2f(__builtin_amdgcn_ds_swizzle(f2u(v), 0x401f)); // lane ^ 16
+  return v;
+}
+template <int kLanes> __device__ __forceinline__ float lanes_max(float v) {
+  if constexpr (kLanes == kWave)
+    return wave_max(v);
+  v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0xB1, 0xf, 0xf, true)));
+  v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x4E, 0xf, 0xf, true)));
+  if constexpr (kLanes > 4)
+    v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x141, 0xf, 0xf, true)));
+  if constexpr (kLanes > 8)
+    v = fmaxf(v, u2f(__builtin_amdgcn_mov_dpp(f2u(v), 0x140, 0xf, 0xf, true)));
+  if constexpr (kLanes > 16)
+    v = fmaxf(v, u2f(__builtin_amdgcn_ds_swizzle(f2u(v), 0x401f)));
+  return v;
+}
+
 // Element traits for kernels that exist in f32, f16 and bf16 forms: scalar get / put through
 // f32, and a 16-byte vector (u32x4) unpacked to / packed from kPerVec f32 values.  16-bit values
 // widen exactly and narrow with round-to-nearest-even.  (In a namespace of their own: kernels with

@@ -34,7 +34,7 @@ extern const unsigned char imex_blob_attention[], imex_blob_attention_end[];
 namespace {
 
 enum class Module { Eltwise, Softmax, Reduce, Transpose, Gemm, GemmSmall, GemmUnaligned, Fusion, Attention };
-enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention };
+enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention };
 
 struct Entry {
   const char *name;
@@ -72,6 +72,8 @@ const Entry kEntries[] = {
     {"imex_softmax_bf16_shared", "(in: bf16*, out: bf16*, rows: i64, cols: i64)", Module::Softmax, Shape::SoftmaxShared16, 2},
     {"imex_rowsum_f32", "(in: f32*, out: f32*, rows: i64, cols: i64, init: f32)", Module::Reduce, Shape::RowSum, 2},
     {"imex_rowmean_f32", "(in: f32*, out: f32*, rows: i64, cols: i64)", Module::Reduce, Shape::RowSum, 2},
+    {"imex_rowsum_f32_short", "(in: f32*, out: f32*, rows: i64, cols: i64, init: f32)", Module::Reduce, Shape::RowSumShort, 2},
+    {"imex_rowmean_f32_short", "(in: f32*, out: f32*, rows: i64, cols: i64)", Module::Reduce, Shape::RowSumShort, 2},
     {"imex_reduce_outer_f32", "(in: f32*, out: f32*, outer: i64, inner: i64, init: f32)", Module::Reduce,
      Shape::ReduceOuter, 2},
     {"imex_reduce_outer_f16", "(in: f16*, out: f16*, outer: i64, inner: i64, init: f32)", Module::Reduce,
@@ -332,6 +334,10 @@ extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *d
   case Shape::SoftmaxRows32:
   case Shape::SoftmaxRows16:
     return softmaxVariant(e, dims[0], dims[1]);
+  case Shape::RowSum: // rows that fit a wavefront's four pieces per lane (131072 x 32: 20.9 -> 4.1 us; 1000 x 1000: 3.6 -> 3.3)
+    if (dims[1] < 4 || dims[1] > 1024)
+      return e->name;
+    return strcmp(e->name, "imex_rowsum_f32") == 0 ? "imex_rowsum_f32_short" : "imex_rowmean_f32_short";
   case Shape::Transpose2D32:
   case Shape::Transpose2D16:
   case Shape::Transpose3D32:
@@ -411,6 +417,14 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
   case Shape::RowSum: // workgroup per row above 2048 columns, else wavefront per row
     grid[0] = dims[1] > 2048 ? static_cast<size_t>(dims[0]) : ceilDiv(dims[0], 4);
     break;
+  case Shape::RowSumShort: { // up to four 16-byte pieces of a row per lane
+    int64_t lanes = 4;
+    while (lanes < 64 && 16 * lanes < dims[1])
+      lanes *= 2;
+    grid[0] = dims[1] >= 4 && dims[1] <= 1024 ? ceilDiv(dims[0], 256 / lanes)
+                                             : dims[1] > 2048 ? static_cast<size_t>(dims[0]) : ceilDiv(dims[0], 4);
+    break;
+  }
   case Shape::ReduceOuter:
   case Shape::ReduceOuter16: { // 256 lanes x v vectors of 4 (8) outputs, v = 8, 4, 2, 1: the widest that leaves 512 workgroups
     const int64_t inner = dims[1], perVec = e->shape == Shape::ReduceOuter ? 1024 : 2048;

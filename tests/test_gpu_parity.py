@@ -316,6 +316,21 @@ def test_rowsum_golden_and_exact(host, orc, stream):
         assert np.array_equal(host.rowsum(stream, xi, init=3.0), orc.rowsum_f32(xi, init=3.0)), (rows, cols)
 
 
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 63, 64, 65, 129, 256, 511, 513, 1023, 1024, 1025, 1030, 2049, 3001, 4096, 4099])
+def test_row_sums_of_any_length_and_address(host, orc, stream, cols):
+    """Rows at the edges of the lane groups (four 16-byte pieces a lane, 4 .. 64 lanes) and of the longer forms, from a
+    buffer that starts one element behind a 16-byte boundary.  Integer values: the sums are exact in any order."""
+    rows = 333
+    x = orc.fill_int(rows * cols, "f32", cols, -8, 8)
+    d_in, d_out = stream.to_device(np.concatenate([np.float32([np.nan]), x, np.float32([np.nan])])), stream.alloc(rows * 4)
+    x = x.reshape(rows, cols)
+    for name, rest, want in (("rowsum", [3.0], orc.rowsum_f32(x, init=3.0)), ("rowmean", [], orc.rowmean_f32(x))):
+        stream.launch("imex_%s_f32" % name, [rows, cols], [host.Ptr(d_in + 4), d_out, rows, cols, *rest])
+        stream.wait()
+        assert np.array_equal(stream.from_device(d_out, (rows,), np.float32), want), name
+    stream.free(d_in), stream.free(d_out)
+
+
 def test_rowsum_config_8192x8192(host, orc, stream):
     x = orc.fill_uniform(8192 * 8192, "f32", 20243, 0.0, 1.0).reshape(8192, 8192)
     got, ref = host.rowsum(stream, x), orc.rowsum_f32(x)
