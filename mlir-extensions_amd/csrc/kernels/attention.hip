@@ -36,6 +36,7 @@
 // Arguments: (Q, K, V, Out, sm_scale: f32, ZH: i64, N_CTX: i64)   dims = {ZH, N_CTX}
 //   ZH = batch * heads; all four tensors [(ZH*N_CTX), 64]; sm_scale > 0.  N_CTX need not divide the
 //   tiles: queries past the end are not stored, keys past the end get a score of -inf.
+// imex_flash_attention_fwd_f16_q32 / _q64 / _q128 / _q256 are the operator with one tiling each.
 // Launch: grid (ceil(N_CTX / q), ZH, 1) with q = 64, 128 or 256 and block (512,1,1), or q = 256
 // and block (1024,1,1).  Other launches (and a scale <= 0, or misaligned tensors) take the
 // one-query-per-lane reference loop of the same kernel (grid-stride, any grid and block).
@@ -48,8 +49,6 @@ namespace {
 
 constexpr int kMaxThreads = 1024; // 8 or 16 wavefronts per workgroup
 constexpr int D = 64;                 // head dimension
-constexpr int BN = 64;                // keys per tile; a ring stage holds one K and one V tile per key group
-constexpr int kTileBytes = BN * D * 2;          // 8 KiB
 constexpr int kLdsBytes = 128 * 1024;           // the ring: 2 stages of 64 KiB, 4 of 32 KiB or 8 of 16 KiB
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -65,6 +64,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, in
 }
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+// the larger of this lane's value and the one that lane l+32 (or l-32) holds
+__device__ __forceinline__ float max_of_halves(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false); // the lower half's, the upper half's
+  return fmaxf(u2f(both[0]), u2f(both[1]));
 }
 // the value lane l+32 (or l-32) holds
 __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 64); }
@@ -105,7 +109,7 @@ __device__ __forceinline__ void attention_scalar(const uint16_t *Q, const uint16
 // all keys of its head); fewer key groups mean smaller ring stages and therefore a deeper ring.
 // kRagged: N_CTX is not a multiple of the workgroup's 32 QB queries or of its 64 KG-key blocks; the
 // padding logic below is compiled in only then.
-template <int QB, int KG, bool kRagged>
+template <int QB, int KG, int KB, bool kRagged, bool kScoresAhead = false>
 __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
                                                 const uint16_t *__restrict__ V, uint16_t *__restrict__ Out,
                                                 float scale, int64_t N, char *lds) {
@@ -113,10 +117,12 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int kWaves = QB * KG;
+  constexpr int BN = 32 * KB;                      // keys per tile
+  constexpr int kTileBytes = BN * D * 2;           // 4 or 8 KiB
   constexpr int kStageBytes = 2 * KG * kTileBytes; // K tiles of all key groups, then their V tiles
   constexpr int kStages = kLdsBytes / kStageBytes; // 2, 4 or 8
   constexpr int kAhead = kStages - 1;              // blocks in flight ahead of the one being multiplied
-  constexpr int kCopies = 64 * KG / (8 * kWaves);  // 1 KiB (8-row) copies per wavefront, stage and operand
+  constexpr int kCopies = BN * KG / (8 * kWaves);  // 1 KiB (8-row) copies per wavefront, stage and operand
   const int wq = wave % QB, wk = wave / QB;
   const int qi = lane & 31, half = lane >> 5;
   // Workgroups go to the 8 XCDs round-robin in launch order, and each XCD has its own L2.  Renumber
@@ -144,23 +150,23 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   for (int ds = 0; ds < 4; ++ds)
     qf[ds] = *reinterpret_cast<const f16x8 *>(Q + qRow * D + ds * 16 + half * 8);
 
-  // -- global -> LDS copies.  A stage is [K tile 0 .. KG-1][V tile 0 .. KG-1], each 64
+  // -- global -> LDS copies.  A stage is [K tile 0 .. KG-1][V tile 0 .. KG-1], each BN
   // rows of 128 bytes; one copy = 8 rows.  16-byte chunk c of row r is stored at
   //   K: c ^ ((r ^ (r>>3 & 3)) & 7)   (conflict-free 128-bit fragment reads; same for r and r+32)
   //   V: c ^ (((r>>1) & 1) << 2)     (conflict-free transpose reads)
   // applied on the global side, since a direct copy fixes the lane's LDS position.
   const __amdgpu_buffer_rsrc_t kRsrc = make_rsrc(K + head0 * D, N * D * 2);
   const __amdgpu_buffer_rsrc_t vRsrc = make_rsrc(V + head0 * D, N * D * 2);
-  const int iters = int((N + KG * BN - 1) / (KG * BN));            // key blocks of 64 KG keys
-  const int lastRows = int(N - int64_t(iters - 1) * (KG * BN));    // keys in the last block: 1 .. 64 KG
+  const int iters = int((N + KG * BN - 1) / (KG * BN));            // key blocks of BN KG keys
+  const int lastRows = int(N - int64_t(iters - 1) * (KG * BN));    // keys in the last block: 1 .. BN KG
   const bool raggedKeys = kRagged && lastRows != KG * BN;
   int kVoff[kCopies], vVoff[kCopies];   // per-lane byte offsets inside a block
   int kVoffT[kCopies], vVoffT[kCopies]; // the same for the last block, rows clamped to its last key
 #pragma unroll
   for (int c = 0; c < kCopies; ++c) {
-    // wavefront w copies rows [8 kCopies w, 8 kCopies (w+1)) of the stage's 64 KG K rows and of its V rows
-    const int row = wave * (8 * kCopies) + c * 8 + (lane >> 3); // key within the stage's block of 64 KG keys
-    const int r = row & 63;                          // row within its tile
+    // wavefront w copies rows [8 kCopies w, 8 kCopies (w+1)) of the stage's BN KG K rows and of its V rows
+    const int row = wave * (8 * kCopies) + c * 8 + (lane >> 3); // key within the stage's block of BN KG keys
+    const int r = row & (BN - 1);                          // row within its tile
     const int kc = (lane & 7) ^ ((r ^ ((r >> 3) & 3)) & 7);
     const int vc = (lane & 7) ^ (((r >> 1) & 1) << 2);
     kVoff[c] = (row * D + kc * 8) * 2;
@@ -169,17 +175,21 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
     kVoffT[c] = (rowT * D + kc * 8) * 2;
     vVoffT[c] = (rowT * D + vc * 8) * 2;
   }
-  auto dma_stage = [&](int block, int stage) { // keys [64 KG block, 64 KG (block + 1)) into ring stage `stage`
+  auto dma_k = [&](int block, int stage) { // keys [BN KG block, BN KG (block + 1)) into ring stage `stage`
     LdsChar *dst = ldsBase + stage * kStageBytes + wave * (kCopies * 1024);
-    const int soff = block * (KG * BN * D * 2);
     const bool tail = raggedKeys && block == iters - 1; // uniform
 #pragma unroll
     for (int c = 0; c < kCopies; ++c)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kRsrc, dst + c * 1024, 16, tail ? kVoffT[c] : kVoff[c], soff, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kRsrc, dst + c * 1024, 16, tail ? kVoffT[c] : kVoff[c],
+                                               block * (KG * BN * D * 2), 0, 0);
+  };
+  auto dma_v = [&](int block, int stage) { // the same keys' rows of V
+    LdsChar *dst = ldsBase + stage * kStageBytes + KG * kTileBytes + wave * (kCopies * 1024);
+    const bool tail = raggedKeys && block == iters - 1;
 #pragma unroll
     for (int c = 0; c < kCopies; ++c)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vRsrc, dst + KG * kTileBytes + c * 1024, 16,
-                                               tail ? vVoffT[c] : vVoff[c], soff, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vRsrc, dst + c * 1024, 16, tail ? vVoffT[c] : vVoff[c],
+                                               block * (KG * BN * D * 2), 0, 0);
   };
 
   // -- LDS read addresses (relative to this wavefront's K / V tile of a stage)
@@ -215,72 +225,75 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   float l = 0.0f;              // running sum of p over THIS lane's keys only
   const float c = scale * 1.44269504088896341f;
 
-  // The ring always holds kAhead blocks in flight (past the end the last block is simply fetched
-  // again, into stages nobody reads any more), so "block `it` has landed" is one fixed vmcnt.
+  // S^T = K . Q^T for this wavefront's BN keys of a stage (the first product of each chain takes a
+  // literal zero accumulator, so no registers are cleared)
+  auto scores = [&](f32x16(&s)[KB], const char *st) {
+    const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    f16x8 kf[KB][4];
 #pragma unroll
-  for (int b = 0; b < kAhead; ++b)
-    dma_stage(min(b, iters - 1), b);
-  int cur = 0; // ring stage of block `it`
-  for (int it = 0; it < iters; ++it) {
-    wait_vmcnt<(kAhead - 1) * 2 * kCopies>(); // block `it` has landed (this wavefront's copies)
-    __builtin_amdgcn_s_barrier();             // ... everyone's; and everyone is done reading block it-1
-    __builtin_amdgcn_sched_barrier(0);
-    dma_stage(min(it + kAhead, iters - 1), cur == 0 ? kStages - 1 : cur - 1); // into the stage block it-1 occupied
-    const char *st = lds + cur * kStageBytes;
-
-    // S^T = K . Q^T for this wavefront's 64 keys (the first product of each chain takes a
-    // literal zero accumulator, so no registers are cleared)
-    f32x16 s[2];
-    {
-      const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      f16x8 kf[2][4];
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int ds = 0; ds < 4; ++ds)
-          kf[kb][ds] = *reinterpret_cast<const f16x8 *>(st + kRd[ds] + kb * 32 * 128);
-      // the two accumulator chains alternate, so no MFMA waits for the one just issued
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds)
+        kf[kb][ds] = *reinterpret_cast<const f16x8 *>(st + kRd[ds] + kb * 32 * 128);
+    // the two accumulator chains alternate, so no MFMA waits for the one just issued
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kb][ds], qf[ds], ds == 0 ? zero : s[kb], 0, 0, 0);
-    }
-    // keys of this wavefront's tile that exist: fewer than 64 only in the last block of a ragged N_CTX
+    for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kb][ds], qf[ds], ds == 0 ? zero : s[kb], 0, 0, 0);
+  };
+  // block `it`, its scores in s and its V tile in stage st: online softmax, O^T += V^T . P^T
+  auto attend = [&](f32x16(&s)[KB], int it, const char *st) {
+    // keys of this wavefront's tile that exist: fewer than BN only in the last block of a ragged N_CTX
     const int nValid = int(N) - (it * (KG * BN) + wk * BN);
     if (kRagged && nValid < BN) { // uniform over the wavefront
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           s[kb][r] = kb * 32 + (r >> 2) * 8 + half * 4 + (r & 3) < nValid ? s[kb][r] : -__builtin_inff();
     }
-    // online softmax over the keys; this lane owns 32 of the query's 64 scores
-    float mx = s[0][0];
+    // online softmax over the keys; this lane owns half of the query's BN scores
+    // four chains of additions and maxima where few wavefronts would wait for one; one where many issue (16 x 4096: 83 us, 86)
+    constexpr int kChains = kScoresAhead ? 4 : 1;
+    float part[kChains];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int r = 0; r < kChains; ++r)
+      part[r] = s[0][r];
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        mx = fmaxf(mx, s[kb][r]);
-    mx = fmaxf(mx, other_half(mx));
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int r = kb ? 0 : kChains; r < 16; ++r)
+        part[r % kChains] = fmaxf(part[r % kChains], s[kb][r]);
+    float mx = part[0];
+#pragma unroll
+    for (int r = 1; r < kChains; ++r)
+      mx = fmaxf(mx, part[r]);
+    mx = max_of_halves(mx);
     const float mRun = fmaxf(m, mx * c);
     // a key group that has seen no key yet (ragged N_CTX shorter than its first tile) stays at -inf;
     // 0 stands in for it below so that -inf - -inf never forms: every p and alpha is then exp2(-inf) = 0
     const float mNew = kRagged && mRun == -__builtin_inff() ? 0.0f : mRun;
     const float alpha = __builtin_amdgcn_exp2f(m - mNew);
     m = mRun;
-    float sum = 0.0f;
-    f16x8 pf[4];
+    float sum[kChains];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
+    for (int r = 0; r < kChains; ++r)
+      sum[r] = 0.0f;
+    f16x8 pf[2 * KB];
+#pragma unroll
+    for (int kk = 0; kk < 2 * KB; ++kk) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kk >> 1][(kk & 1) * 8 + e], c, -mNew)); // one fused op per score
         pf[kk][e] = static_cast<_Float16>(p); // the reference truncates P to f16 before P.V (:262-265)
-        sum += p;                             // ... and sums the untruncated f32 values (:243-247)
+        sum[e % kChains] += p;                      // ... and sums the untruncated f32 values (:243-247)
       }
     }
-    l = l * alpha + sum;
+    #pragma unroll
+    for (int r = 1; r < kChains; ++r)
+      sum[0] += sum[r];
+    l = l * alpha + sum[0];
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) { // the running max moved for some query of this wavefront
 #pragma unroll
       for (int db = 0; db < 2; ++db)
@@ -290,7 +303,7 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
     }
     // O^T += V^T . P^T
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
+    for (int kk = 0; kk < 2 * KB; ++kk) {
 #pragma unroll
       for (int db = 0; db < 2; ++db) {
         const char *p = st + vRd[db] + kk * 16 * 128;
@@ -300,7 +313,60 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
         o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[kk], o[db], 0, 0, 0);
       }
     }
-    cur = cur == kStages - 1 ? 0 : cur + 1;
+  };
+
+  if constexpr (kScoresAhead) {
+    // The scores of block it + 1 are formed while block `it` goes through the softmax, so a block costs no wait for its
+    // own K reads and first products.  K(it + 1) and V(it) are there when block `it` begins; the copies in flight
+    // are pairs of these.
+    dma_k(0, 0);
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      dma_k(min(b + 1, iters - 1), b + 1);
+      dma_v(min(b, iters - 1), b);
+    }
+    wait_vmcnt<kAhead * 2 * kCopies>(); // K(0) has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16 s[KB], next[KB];
+    scores(s, lds);
+    int cur = 0; // ring stage of V(it)
+    for (int it = 0; it < iters; ++it) {
+      __builtin_amdgcn_sched_barrier(0);        // everything read from LDS so far has been used
+      wait_vmcnt<(kAhead - 1) * 2 * kCopies>(); // K(it + 1), V(it) have landed
+      __builtin_amdgcn_s_barrier();             // ... everyone's; and everyone is done with K(it), V(it - 1) ...
+      __builtin_amdgcn_sched_barrier(0);
+      dma_k(min(it + kStages, iters - 1), cur); // ... whose places these go to
+      dma_v(min(it + kAhead, iters - 1), cur == 0 ? kStages - 1 : cur - 1);
+      const int after = cur == kStages - 1 ? 0 : cur + 1;
+      scores(next, lds + after * kStageBytes); // (past the last block: of whatever the ring holds, not used)
+      attend(s, it, lds + cur * kStageBytes);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        s[kb] = next[kb];
+      cur = after;
+    }
+  } else {
+    // The ring always holds kAhead blocks in flight (past the end the last block is simply fetched
+    // again, into stages nobody reads any more), so "block `it` has landed" is one fixed vmcnt.
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      dma_k(min(b, iters - 1), b);
+      dma_v(min(b, iters - 1), b);
+    }
+    int cur = 0; // ring stage of block `it`
+    for (int it = 0; it < iters; ++it) {
+      wait_vmcnt<(kAhead - 1) * 2 * kCopies>(); // block `it` has landed (this wavefront's copies)
+      __builtin_amdgcn_s_barrier();             // ... everyone's; and everyone is done reading block it-1
+      __builtin_amdgcn_sched_barrier(0);
+      const int before = cur == 0 ? kStages - 1 : cur - 1; // the stage block it-1 occupied
+      dma_k(min(it + kAhead, iters - 1), before);
+      dma_v(min(it + kAhead, iters - 1), before);
+      f32x16 s[KB];
+      scores(s, lds + cur * kStageBytes);
+      attend(s, it, lds + cur * kStageBytes);
+      cur = cur == kStages - 1 ? 0 : cur + 1;
+    }
   }
   wait_vmcnt<0>();
   l += other_half(l); // both key halves of the lane pair
@@ -355,6 +421,14 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   }
 }
 
+// What the tiled path takes, of the arguments and of the launch.
+__device__ __forceinline__ bool attention_shaped(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
+                                                 const uint16_t *Out, float scale, int64_t ZH, int64_t N) {
+  return N > 0 && N < (int64_t(1) << 24) && scale > 0.0f && gridDim.y == ZH && gridDim.z == 1 &&
+         ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+           reinterpret_cast<uintptr_t>(Out)) & 15) == 0;
+}
+
 } // namespace
 
 extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_fwd_f16(const uint16_t *Q,
@@ -366,32 +440,60 @@ extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_f
   // The launch says how many queries a workgroup takes (ceil(N_CTX / gridDim.x) = 64, 128 or 256) and
   // with how many wavefronts.  The tiled path assumes a positive scale (it takes the row maximum
   // before scaling) and 32-bit byte offsets inside one head.
-  const bool shaped = N_CTX > 0 && N_CTX < (int64_t(1) << 24) && sm_scale > 0.0f && gridDim.y == ZH && gridDim.z == 1 &&
-                      ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) |
-                        reinterpret_cast<uintptr_t>(V) | reinterpret_cast<uintptr_t>(Out)) & 15) == 0;
+  const bool shaped = attention_shaped(Q, K, V, Out, sm_scale, ZH, N_CTX);
   const int64_t gx = gridDim.x;
   const bool even = N_CTX % 256 == 0; // every tiling divides it
   if (shaped && blockDim.x == 512 && gx == (N_CTX + 63) / 64) {
     if (even)
-      attention_tiled<2, 4, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<2, 4, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<2, 4, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<2, 4, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 512 && gx == (N_CTX + 127) / 128) {
     if (even)
-      attention_tiled<4, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<4, 2, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<4, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<4, 2, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 512 && gx == (N_CTX + 255) / 256) {
     if (even)
-      attention_tiled<8, 1, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 1, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<8, 1, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 1, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 1024 && gx == (N_CTX + 255) / 256) {
     if (even)
-      attention_tiled<8, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 2, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<8, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 2, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else {
     attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
   }
 }
+
+// One tiling each, for problems whose tilings by the rule above leave CUs idle or run a nearly empty last round
+// (attentionVariant in KernelCatalog.cpp).  32 queries are eight key groups of 32-key tiles; it is the form for few
+// heads, bound by the 1 MiB of K and V (N_CTX 4096) that one CU's copies bring in: 1 x 4096 27.6 -> 20.0 us, 2 x 4096
+// 27.8 -> 21.1.  64 and 128 queries are the forms above with the next block's scores formed ahead: 5 x 3001 24.2 -> 21.9,
+// 8 x 2048 17.4 -> 16.4, 4 x 4096 28.9 -> 27.4.
+template <int QB, int KG, int KB, bool kScoresAhead>
+__device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
+                                                     uint16_t *Out, float scale, int64_t ZH, int64_t N, char *lds) {
+  constexpr int64_t kQueries = 32 * QB;
+  if (!attention_shaped(Q, K, V, Out, scale, ZH, N) || blockDim.x != QB * KG * kWave ||
+      gridDim.x != (N + kQueries - 1) / kQueries)
+    attention_scalar(Q, K, V, Out, scale, ZH, N);
+  else if (N % 256 == 0)
+    attention_tiled<QB, KG, KB, false, kScoresAhead>(Q, K, V, Out, scale, N, lds);
+  else
+    attention_tiled<QB, KG, KB, true, kScoresAhead>(Q, K, V, Out, scale, N, lds);
+}
+
+#define IMEX_ATTENTION_TILING(QUERIES, QB, KG, KB, AHEAD)                                                              \
+  extern "C" __global__ __launch_bounds__(QB *KG *kWave) void imex_flash_attention_fwd_f16_q##QUERIES(                \
+      const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH,             \
+      int64_t N_CTX) {                                                                                                \
+    __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];                                                      \
+    attention_one_tiling<QB, KG, KB, AHEAD>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);                                  \
+  }
+IMEX_ATTENTION_TILING(32, 1, 8, 1, true)
+IMEX_ATTENTION_TILING(64, 2, 4, 2, true)
+IMEX_ATTENTION_TILING(128, 4, 2, 2, true)
+IMEX_ATTENTION_TILING(256, 8, 2, 2, false)

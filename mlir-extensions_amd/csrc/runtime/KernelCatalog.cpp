@@ -34,7 +34,7 @@ extern const unsigned char imex_blob_attention[], imex_blob_attention_end[];
 namespace {
 
 enum class Module { Eltwise, Softmax, Reduce, Transpose, Gemm, GemmSmall, GemmUnaligned, Fusion, Attention };
-enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention };
+enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention, AttentionTiling };
 
 struct Entry {
   const char *name;
@@ -116,6 +116,18 @@ const Entry kEntries[] = {
     {"imex_flash_attention_fwd_f16",
      "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
      Shape::Attention, 2},
+    {"imex_flash_attention_fwd_f16_q32",
+     "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
+     Shape::AttentionTiling, 2},
+    {"imex_flash_attention_fwd_f16_q64",
+     "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
+     Shape::AttentionTiling, 2},
+    {"imex_flash_attention_fwd_f16_q128",
+     "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
+     Shape::AttentionTiling, 2},
+    {"imex_flash_attention_fwd_f16_q256",
+     "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
+     Shape::AttentionTiling, 2},
     {"imex_gemm_f16_f16_f32", "(A: f16*, B: f16*, C: f32*, M: i64, N: i64, K: i64)", Module::Gemm, Shape::Gemm, 3},
     {"imex_gemm_f16_f16_f32_acc", "(A: f16*, B: f16*, C: f32*, M: i64, N: i64, K: i64)", Module::Gemm, Shape::Gemm, 3},
     {"imex_gemm_bf16_bf16_f32", "(A: bf16*, B: bf16*, C: f32*, M: i64, N: i64, K: i64)", Module::Gemm, Shape::Gemm, 3},
@@ -316,6 +328,41 @@ const char *transposeVariant(const Entry *e, const int64_t *dims) {
   return find(name)->name;
 }
 
+// The operator's own launch takes the most queries per workgroup that give every CU a workgroup.  That leaves CUs idle
+// where 64 queries are too many for it, and runs a second, partly empty round where the next larger tiling would do in
+// one.  A tiling costs its rounds of 256 workgroups, in microseconds at 4096 keys.  1 x 4096 27.6 -> 20.0 us (32 queries),
+// 12 x 1500 27.0 -> 20.3 (128), 6 x 4096 53.1 -> 42.5 (128), 12 x 4096 85.1 -> 68.3 (256).  Heads of fewer than 768 keys
+// stay (16 x 512 7.4 us, 7.9 with 32 queries), as do problems that fill more than one round with 256 queries; the 64
+// queries that form scores ahead gain from 2048 keys on (8 x 2048 17.4 -> 16.4, 16 x 1024 10.4 -> 10.9).
+const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
+  struct Tiling {
+    const char *suffix;
+    int64_t queries;
+    double cost;
+  };
+  constexpr Tiling kTilings[] = {{"_q32", 32, 22.0}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
+  auto workgroups = [&](int64_t queries) { return (N + queries - 1) / queries * ZH; };
+  if (N < 768 || N >= (int64_t(1) << 24) || ZH == 0 || ZH > 256 || workgroups(256) > 256)
+    return e->name;
+  int64_t own = 256; // as imexHipKernelLaunchShape
+  while (own > 64 && workgroups(own) < 256)
+    own /= 2;
+  const Tiling *best = nullptr;
+  double least = 0.0;
+  for (const Tiling &t : kTilings) {
+    const double cost = double((workgroups(t.queries) + 255) / 256) * t.cost;
+    if (!best || cost < least) {
+      best = &t;
+      least = cost;
+    }
+  }
+  if (best->queries == own && (own != 64 || N < 2048))
+    return e->name;
+  char name[96];
+  snprintf(name, sizeof name, "%s%s", e->name, best->suffix);
+  return find(name)->name;
+}
+
 extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *dims, int ndims) {
   const Entry *e = find(kernel);
   if (!e || ndims != e->ndims || (ndims > 0 && !dims))
@@ -343,6 +390,8 @@ extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *d
   case Shape::Transpose3D32:
   case Shape::Transpose3D16:
     return transposeVariant(e, dims);
+  case Shape::Attention:
+    return attentionVariant(e, dims[0], dims[1]);
   default:
     return e->name;
   }
@@ -504,6 +553,17 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
       grid[1] = static_cast<size_t>(ZH);
       if (queries == 256)
         block[0] = 1024;
+    } else {
+      grid[0] = ceilDiv(ZH * N, 512); // one lane per query
+    }
+    break;
+  }
+  case Shape::AttentionTiling: { // the tiling that the name ends in
+    const int64_t ZH = dims[0], N = dims[1], queries = atoi(strrchr(e->name, '_') + 2);
+    block[0] = queries == 256 ? 1024 : 512;
+    if (N > 0 && N < (int64_t(1) << 24) && ZH > 0 && ZH <= 65535) {
+      grid[0] = ceilDiv(N, queries);
+      grid[1] = static_cast<size_t>(ZH);
     } else {
       grid[0] = ceilDiv(ZH * N, 512); // one lane per query
     }

@@ -769,6 +769,28 @@ def test_flash_attention_ragged_context(host, orc, stream, zh, n_ctx, scale):
         assert attention_close(out[rows], ref, orc), (queries, threads)
 
 
+@pytest.mark.parametrize("queries", [32, 64, 128, 256])
+@pytest.mark.parametrize("zh,n_ctx", [(1, 1), (2, 33), (3, 255), (2, 512), (1, 769), (2, 1537)])
+def test_flash_attention_one_tiling(host, orc, stream, queries, zh, n_ctx):
+    """The kernels with one tiling each: fewer keys than key groups, one more than a tile, one fewer than a block of
+    256, whole blocks, several blocks with a ragged last one; every row, and the rows behind Out untouched."""
+    n = zh * n_ctx
+    q = orc.fill_uniform(n * 64, "f16", 87, -2, 2).reshape(n, 64)
+    k = orc.fill_uniform(n * 64, "f16", 88, -2, 2).reshape(n, 64)
+    v = orc.fill_uniform(n * 64, "f16", 89, -1, 1).reshape(n, 64)
+    rows = np.arange(n) if n <= 1200 else np.unique(np.concatenate([np.arange(0, n, 5), [n_ctx - 1, n_ctx % n, n - 1]]))
+    guard = np.full((n + 256, 64), 0x7e01, np.uint16)
+    d_q, d_k, d_v, d_o = (stream.to_device(t) for t in (q, k, v, guard))
+    say("attention %dx%d, %d queries per workgroup" % (zh, n_ctx, queries))
+    stream.launch("imex_flash_attention_fwd_f16_q%d" % queries, [zh, n_ctx], [d_q, d_k, d_v, d_o, 0.5, zh, n_ctx])
+    stream.wait()
+    out = stream.from_device(d_o, (n + 256, 64), np.uint16)
+    for p in (d_q, d_k, d_v, d_o):
+        stream.free(p)
+    assert np.all(out[n:] == 0x7e01), "wrote behind Out"
+    assert attention_close(out[rows], orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows), orc)
+
+
 def test_flash_attention_negative_scale_takes_the_reference_loop(host, orc, stream):
     """The tiled path takes the row maximum before scaling, which needs a positive scale; any
     other scale runs the one-lane-per-query loop of the same kernel."""
