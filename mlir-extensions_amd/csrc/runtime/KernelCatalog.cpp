@@ -171,6 +171,10 @@ const Entry *find(const char *name) {
 
 size_t ceilDiv(int64_t a, int64_t b) { return static_cast<size_t>((a + b - 1) / b); }
 
+// The grid of a form whose problem has `groups` workgroups of work.  HIP takes fewer than 2^32 lanes per dimension of a
+// launch, and the kernels stride over what a smaller grid leaves out.  (A multiple of 8: as many for each XCD.)
+size_t gridFor(size_t groups, size_t block) { return std::min(groups, ((size_t(1) << 32) - 1) / block / 8 * 8); }
+
 // What the MFMA paths of the GEMM kernels take (mfma_takes in gemm_tile.h): 16-byte aligned rows, and operands
 // addressed through one 32-bit-offset buffer descriptor below 2 GiB.
 bool mfmaTakes(bool transA, bool transB, int64_t M, int64_t N, int64_t K) {
@@ -451,12 +455,12 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     if (cols == 0)
       grid[0] = 0;
     else if (cols < perVec)
-      grid[0] = ceilDiv(rows, 256);
+      grid[0] = gridFor(ceilDiv(rows, 256), 256);
     else if (pieces <= 256 && (pieces <= 64 || rows >= 2048)) {
       int64_t lanes = 4;
       while (4 * lanes < pieces || (lanes < pieces && lanes < 64 && rows * lanes < 2048 * 64))
         lanes *= 2;
-      grid[0] = ceilDiv(rows, 256 / lanes);
+      grid[0] = gridFor(ceilDiv(rows, 256 / lanes), 256);
     } else {
       grid[0] = static_cast<size_t>(std::min<int64_t>(rows, 1048560));
       block[0] = pieces <= 1024 ? 256 : pieces <= 2048 ? 512 : pieces <= 4096 ? 1024 : 256;
@@ -470,8 +474,9 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     int64_t lanes = 4;
     while (lanes < 64 && 16 * lanes < dims[1])
       lanes *= 2;
-    grid[0] = dims[1] >= 4 && dims[1] <= 1024 ? ceilDiv(dims[0], 256 / lanes)
-                                             : dims[1] > 2048 ? static_cast<size_t>(dims[0]) : ceilDiv(dims[0], 4);
+    grid[0] = gridFor(dims[1] >= 4 && dims[1] <= 1024 ? ceilDiv(dims[0], 256 / lanes)
+                                                      : dims[1] > 2048 ? static_cast<size_t>(dims[0]) : ceilDiv(dims[0], 4),
+                      256);
     break;
   }
   case Shape::ReduceOuter:
@@ -486,13 +491,13 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     const int64_t perVec = e->shape == Shape::ReduceTall32 ? 4 : 8;
     const bool vec = dims[1] % perVec == 0;
     block[0] = vec ? 128 : 320;
-    grid[0] = ceilDiv(dims[1], vec ? 8 * perVec : 64);
+    grid[0] = gridFor(ceilDiv(dims[1], vec ? 8 * perVec : 64), block[0]);
     break;
   }
   case Shape::ReduceDeep32:
   case Shape::ReduceDeep16: { // a lane per 16-byte vector, or per output
     const int64_t perVec = e->shape == Shape::ReduceDeep32 ? 4 : 8;
-    grid[0] = ceilDiv(dims[1], dims[1] % perVec == 0 ? 256 * perVec : 256);
+    grid[0] = gridFor(ceilDiv(dims[1], dims[1] % perVec == 0 ? 256 * perVec : 256), 256);
     break;
   }
   case Shape::Transpose2D32:
@@ -534,8 +539,8 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
   case Shape::TransposeAny16: { // a workgroup per tile of 512 bytes of output rows x 128 bytes of input rows, for each XCD the same number
     const int64_t bytes = e->shape == Shape::TransposeAny32 ? 4 : 2, planes = e->ndims == 3 ? dims[1] : 1;
     const size_t perPlane = ceilDiv(dims[0], 512 / bytes) * ceilDiv(dims[e->ndims - 1], 128 / bytes);
-    const size_t most = size_t(1) << 24;
-    grid[0] = perPlane == 0 || planes == 0 ? 0 : perPlane >= most ? most : std::min(most, (perPlane * size_t(planes) + 7) / 8 * 8);
+    const size_t most = size_t(1) << 24; // (the product of two large counts would overflow)
+    grid[0] = gridFor(planes == 0 ? 0 : perPlane >= most ? most : (perPlane * size_t(planes) + 7) / 8 * 8, 256);
     break;
   }
   case Shape::Attention: {
@@ -565,7 +570,7 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
       grid[0] = ceilDiv(N, queries);
       grid[1] = static_cast<size_t>(ZH);
     } else {
-      grid[0] = ceilDiv(ZH * N, 512); // one lane per query
+      grid[0] = gridFor(ceilDiv(ZH * N, 512), block[0]); // one lane per query
     }
     break;
   }
@@ -610,17 +615,19 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     const char *suffix = strrchr(e->name, '_') + 2;
     const int tileM = atoi(suffix), tileN = tileM == 128 && !strchr(suffix, 'x') ? 128 : 64;
     block[0] = 512;
-    grid[0] = mfmaTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
-                  ? ceilDiv(M, tileM) * ceilDiv(N, tileN)
-                  : ceilDiv(M, 128) * ceilDiv(N, 128);
+    grid[0] = gridFor(mfmaTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
+                          ? ceilDiv(M, tileM) * ceilDiv(N, tileN)
+                          : ceilDiv(M, 128) * ceilDiv(N, 128),
+                      512);
     break;
   }
   case Shape::GemmUnaligned: {
     const int64_t M = dims[0], N = dims[1], K = dims[2], tile = atoi(strrchr(e->name, '_') + 2);
     block[0] = 512;
-    grid[0] = unalignedTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
-                  ? ceilDiv(M, tile) * ceilDiv(N, tile)
-                  : ceilDiv(M, 128) * ceilDiv(N, 128);
+    grid[0] = gridFor(unalignedTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
+                          ? ceilDiv(M, tile) * ceilDiv(N, tile)
+                          : ceilDiv(M, 128) * ceilDiv(N, 128),
+                      512);
     break;
   }
   case Shape::GemmStreamK: {

@@ -2,6 +2,7 @@
 symbol include/*.h declares, the launch-shape table, the statistics, the runner
 utilities and the stdout+abort error convention (no GPU compute calls here)."""
 import ctypes as C
+import itertools
 import os
 import re
 import subprocess
@@ -196,6 +197,25 @@ def test_param_desc_packing(host):
     assert C.cast(descs[0].data, C.POINTER(C.c_void_p))[0] == 0x1000
     assert C.cast(descs[1].data, C.POINTER(C.c_int64))[0] == 7
     assert C.cast(descs[2].data, C.POINTER(C.c_float))[0] == 2.5
+
+
+def test_launch_shapes_of_every_form_fit_a_launch(host):
+    """HIP takes fewer than 2^32 lanes per dimension of a launch: every further form of an operator has a grid within
+    that at any size (it strides over the rest), none of it empty, and the transposes' a multiple of the 8 XCDs."""
+    forms = [n for n in host.kernel_names() if re.search(r"_(shared|l\d+|short|tall|deep|any|[tuq]\d+(x\d+)?)$", n)]
+    assert len(forms) > 60
+    sizes = [1, 8, 9, 4096, 65537, (1 << 24) - 1, 1 << 24, (1 << 28) + 8, (1 << 34) + 4]
+    for name in forms:
+        ndims = next(k for k in (1, 2, 3) if host.kernels().imexHipKernelLaunchShape(
+            name.encode(), (C.c_int64 * 3)(1, 1, 1), k, (C.c_size_t * 3)(), (C.c_size_t * 3)(), None) == 0)
+        for dims in itertools.product(sizes, repeat=ndims):
+            grid, block, _ = host.launch_shape(name, list(dims))
+            assert all(g >= 1 and g * b < 1 << 32 for g, b in zip(grid, block)), (name, dims, grid, block)
+            if name.endswith("_any"):
+                assert grid[0] % 8 == 0
+    # many planes of one small tile; a lane per output
+    assert host.launch_shape("imex_transpose3d_b16_any", [8, 1 << 24, 9])[0][0] == (1 << 24) - 8
+    assert host.launch_shape("imex_reduce_outer_f32_deep", [2, (1 << 32) + 1])[0][0] == (1 << 24) - 8
 
 
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
