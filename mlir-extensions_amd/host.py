@@ -260,6 +260,8 @@ class _Plan:
     def __init__(self, stream, name, dims):
         name = variant(name, dims)
         grid, block, smem = launch_shape(name, dims)
+        if max(grid) >= 1 << 32:  # gpuLaunchKernel's own check; the shape below is 32 bits wide
+            raise ValueError("%s at %s: a grid of %s is outside [1, 2^32)" % (name, list(dims), grid))
         self.types = signature_types(name)
         self.kernel = None if 0 in grid else stream.kernel(name)
         self.shape = (C.c_uint32 * 7)(*grid, *block, smem)

@@ -235,6 +235,17 @@ def test_plan_packs_arguments_as_the_kernel_declares_them(host):
             plan.pack(bad)
 
 
+def test_plan_refuses_a_grid_that_no_launch_takes(host):
+    """A grid of 2^32 workgroups and more is an error, as it is for gpuLaunchKernel, not its low 32 bits."""
+    class Resolver:
+        def kernel(self, name):
+            return 1
+    rows = (1 << 34) + 4  # a workgroup per four rows: 2^32 + 1
+    assert host.launch_shape("imex_rowsum_f32", [rows, 2000])[0][0] == (1 << 32) + 1
+    with pytest.raises(ValueError, match="outside"):
+        host._Plan(Resolver(), "imex_rowsum_f32", [rows, 2000])
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
