@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import operator
 import os
 import re
 import struct
@@ -270,11 +271,15 @@ class _Plan:
 
     def pack(self, args):
         """The arguments' values as imexHipLaunchValues takes them; _pack_params' errors for wrong ones."""
-        if len(args) == len(self.types) and all(isinstance(args[i], Ptr) for i in self.pointers):
-            try:
-                return self.packer.pack(*args)
-            except (struct.error, OverflowError):
-                pass  # a value that needs converting (an index given as 2.0), or one no conversion fits
+        if len(args) == len(self.types):
+            for i in self.pointers:
+                if not isinstance(args[i], Ptr):
+                    break
+            else:
+                try:
+                    return self.packer.pack(*args)
+                except (struct.error, OverflowError):
+                    pass  # a value that needs converting (an index given as 2.0), or one no conversion fits
         descs, keep = _pack_params(args, self.types)
         return b"".join(C.string_at(d.data, d.size).ljust(8, b"\0") for d in descs[:len(self.types)])
 
@@ -363,7 +368,8 @@ class Stream:
         None when the launch shape is empty).  `grid` / `block` replace the catalogue's, and with one of
         them given it is `name` itself that is launched; otherwise the variant the catalogue advises."""
         if grid is None and block is None and not deps:
-            plan = self._plans.get((name, *dims)) or self._plan(name, dims)
+            # (operator.index: 64.0 equals 64 as a key, but is no dim)
+            plan = self._plans.get((name, *map(operator.index, dims))) or self._plan(name, dims)
             if plan.kernel is None:
                 return None
             return self.rt.imexHipLaunchValues(self.handle, plan.kernel, plan.shape, plan.pack(args), len(plan.types))

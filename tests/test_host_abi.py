@@ -246,6 +246,27 @@ def test_plan_refuses_a_grid_that_no_launch_takes(host):
         host._Plan(Resolver(), "imex_rowsum_f32", [rows, 2000])
 
 
+def test_launch_takes_the_dims_that_launch_shape_takes(host):
+    """Whole numbers of any integer type, and nothing else -- also where the plan of an equal number is kept."""
+    launched = []
+
+    class Runtime:
+        def imexHipLaunchValues(self, *args):
+            launched.append(args)
+            return 7
+    s = host.Stream.__new__(host.Stream)
+    s.rt, s.handle, s._plans, s.kernel = Runtime(), 1, {}, lambda name: 1
+    p = host.Ptr(0x1000)
+    for n in (64, np.int64(64), np.uint8(64)):
+        assert s.launch("imex_relu_f32", [n], [p, p, 64]) == 7
+    for n in (64.0, np.float32(64), "64"):
+        with pytest.raises(TypeError):
+            host.launch_shape("imex_relu_f32", [n])
+        with pytest.raises(TypeError):
+            s.launch("imex_relu_f32", [n], [p, p, 64])
+    assert len(launched) == 3 and len(s._plans) == 1
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
