@@ -367,26 +367,27 @@ class Stream:
         """gpuModuleLoad + gpuKernelGet + gpuLaunchKernel; returns the event (or
         None when the launch shape is empty).  `grid` / `block` replace the catalogue's, and with one of
         them given it is `name` itself that is launched; otherwise the variant the catalogue advises."""
-        if grid is None and block is None and not deps:
+        if grid is None and block is None:
             # (operator.index: 64.0 equals 64 as a key, but is no dim)
             plan = self._plans.get((name, *map(operator.index, dims))) or self._plan(name, dims)
             if plan.kernel is None:
                 return None
-            return self.rt.imexHipLaunchValues(self.handle, plan.kernel, plan.shape, plan.pack(args), len(plan.types))
-        if grid is None and block is None:
-            name = variant(name, dims)
-        cat_grid, cat_block, smem = launch_shape(name, dims)
-        grid = tuple(grid) if grid is not None else cat_grid
-        block = tuple(block) if block is not None else cat_block
-        if 0 in grid:
-            return None
-        fn = self.kernel(name)
-        descs, keep = _pack_params(args, signature_types(name))
+            if not deps:
+                return self.rt.imexHipLaunchValues(self.handle, plan.kernel, plan.shape, plan.pack(args),
+                                                   len(plan.types))
+            fn, types, shape = plan.kernel, plan.types, plan.shape
+        else:
+            cat_grid, cat_block, smem = launch_shape(name, dims)
+            grid = tuple(grid) if grid is not None else cat_grid
+            block = tuple(block) if block is not None else cat_block
+            if 0 in grid:
+                return None
+            fn, types, shape = self.kernel(name), signature_types(name), (*grid[:3], *block[:3], smem)
+        descs, keep = _pack_params(args, types)
         evs = (EventDesc * (len(deps or []) + 1))()
         for i, e in enumerate(deps or []):
             evs[i].event = e
-        ev = self.rt.gpuLaunchKernel(self.handle, fn, grid[0], grid[1], grid[2], block[0], block[1], block[2],
-                                     smem, C.cast(descs, C.c_void_p), C.cast(evs, C.c_void_p))
+        ev = self.rt.gpuLaunchKernel(self.handle, fn, *shape, C.cast(descs, C.c_void_p), C.cast(evs, C.c_void_p))
         del keep
         return ev
 

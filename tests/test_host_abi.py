@@ -267,6 +267,28 @@ def test_launch_takes_the_dims_that_launch_shape_takes(host):
     assert len(launched) == 3 and len(s._plans) == 1
 
 
+def test_launch_with_dependencies_uses_the_kept_plan(host):
+    """The kernel of a size is resolved once, whether a launch waits for events of other streams or not, and both go
+    to the variant the catalogue advises under its launch shape."""
+    launched, resolved = [], []
+
+    class Runtime:
+        def imexHipLaunchValues(self, handle, fn, shape, values, count):
+            launched.append((fn, tuple(shape)))
+
+        def gpuLaunchKernel(self, handle, fn, *rest):
+            launched.append((fn, rest[:7]))
+    s = host.Stream.__new__(host.Stream)
+    s.rt, s.handle, s._plans, s.kernel = Runtime(), 1, {}, lambda name: resolved.append(name) or name
+    p = host.Ptr(0x1000)
+    for deps in (None, [0x20], [0x20, 0x30]):
+        s.launch("imex_rowsum_f32", [300, 40], [p, p, 300, 40, 0.0], deps=deps)
+    name = host.variant("imex_rowsum_f32", [300, 40])
+    grid, block, smem = host.launch_shape(name, [300, 40])
+    assert name != "imex_rowsum_f32" and resolved == [name]
+    assert launched == [(name, (*grid, *block, smem))] * 3
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
