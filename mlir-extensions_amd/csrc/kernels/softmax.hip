@@ -9,12 +9,16 @@
 //  * rows of up to 256 pieces of 16 bytes (2048 16-bit / 1024 f32 elements) belong to 4 .. 64 lanes of a wavefront,
 //    up to four pieces a lane, so a wavefront has up to sixteen rows at once; max and sum are reductions on the VALU's
 //    cross-lane paths (DPP), no LDS.  Longer rows, up to 4096 pieces, and more than 64 pieces where there are fewer
-//    than 2048 rows to give to wavefronts, belong to a workgroup.  Either way a row stays in registers from its one
-//    read to its one write, and neither its length nor its address need be multiples of anything.
-//    Bound by HBM on whole pieces (f32 16384 x 1024: 23.1 us, 5.8 TB/s; one and two rows per wavefront before: 24.4;
-//    bf16 8192 x 2000, staged in LDS before: 16.8 -> 13.2); odd rows cost a second transaction per request on both
-//    sides (bf16 6000 x 3001: 35.1 -> 17.2 us, 4.2 TB/s, with buffers that are not in the caches; one element at a
-//    time through LDS before), short ones are cut to size (bf16 65536 x 32: 20.5 -> 3.2; 200001 x 77: 119 -> 16.5).
+//    than 1024 rows to give to wavefronts (f32 1500 x 1200: 4.1 us, 5.4 with a workgroup each), belong to a workgroup.
+//    Either way a row stays in registers from its one read to its one write, and neither its length nor its address
+//    need be multiples of anything.
+//    Bound by HBM on whole pieces (f32 16384 x 1024 from HBM: 23.8 us, 5.6 TB/s; bf16 8192 x 2000: 13.6); odd rows cost
+//    a second transaction per request on both sides (bf16 6000 x 3001 with changing buffers: 17 us, 4.2 TB/s; one element
+//    at a time through LDS 35.1), short ones are cut to size (bf16 65536 x 32: 3.2, with a wavefront each 20.5;
+//    200001 x 77: 119 / 16.5).
+//  * f32 and bf16 rows of 65 .. 128 whole pieces, up to 8192 rows (16384 from 96 pieces on): a wavefront has a row, from
+//    16384 rows on two, in the operator's own kernel.  f32 16384 x 384: 9.0 us, 10.8 on 32 lanes per row; bf16 2047 x
+//    1000: 3.9, 5.5 with a workgroup per row.
 //  * f16 rows of 65 .. 128 whole pieces: a wavefront walks rows w, w + W, ... with the next row's loads in
 //    flight while it computes the current one, and the arithmetic is written for the instruction count (packed f16
 //    maximum, mixed-precision FMAs straight from and into the f16 halves, one reciprocal per row): about 6 vector
@@ -27,9 +31,10 @@
 //
 // Arguments: (in, out, rows: i64, cols: i64).
 // Launch: any grid >= 1 is correct (workgroups stride over the rows), with block (256,1,1); the _shared forms also
-// take (512,1,1) and (1024,1,1) for rows of a workgroup, and the catalogue's launch of these gives every group of lanes
-// one row and a workgroup's row the smallest block that holds it (bf16 6000 x 3001: 17.3 us with 256 lanes, 23.8 with
-// 512, 43.5 with 1024).
+// take any whole number of wavefronts up to (1024,1,1) for rows of a workgroup, and the catalogue's launch of these gives
+// every group of lanes one row and a workgroup's row the lanes that it fills with as few pieces each as 256, 512 or 1024
+// lanes would have (bf16 6000 x 3001: 17.3 us with 256 lanes, 23.8 with 512, 43.5 with 1024; 8192 x 2400, two pieces
+// each: 16.5 with 192 lanes, 18.2 with 256).
 
 #include "device_common.h"
 
@@ -41,7 +46,9 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kRegChunks = 2;          // 16-byte chunks per lane and row of the f16 walk
 constexpr int kMaxWaves = 16;          // of a workgroup that has a long row
-constexpr int64_t kManyRows = 2048;    // wavefronts' worth of rows from which a lane takes up to four pieces of one
+constexpr int64_t kTwoRowsFrom = 16384; // rows from which a wavefront takes two: every wavefront slot of the chip is then filled
+constexpr int64_t kManyRows = 2048;    // wavefronts' worth of rows from which a lane takes several pieces of one
+constexpr int64_t kWaveRows = 1024;    // rows of 65 .. 256 pieces from which a wavefront has one, not a workgroup
 
 enum class Dt { F32, F16, BF16 };
 
@@ -152,10 +159,7 @@ template <Dt D, int kPieces, bool kStream> struct RowPieces {
     u32x4 raw[kPieces];
 #pragma unroll
     for (int c = 0; c < kPieces; ++c)
-      if constexpr (kStream)
-        raw[c] = __builtin_nontemporal_load(reinterpret_cast<const Vec *>(row + start[c] * E::kBytes));
-      else
-        raw[c] = *reinterpret_cast<const Vec *>(row + start[c] * E::kBytes);
+      raw[c] = *reinterpret_cast<const Vec *>(row + start[c] * E::kBytes);
     float m = kMaxInit;
 #pragma unroll
     for (int c = 0; c < kPieces; ++c) {
@@ -223,7 +227,12 @@ template <Dt D, int kPieces>
 __device__ __forceinline__ void softmax_rows_by_workgroup(const void *in, void *out, int64_t rows, int64_t cols,
                                                           f32x4 (&part)[2][kMaxWaves / 4]) {
   const int64_t rowBytes = cols * Elem<D>::kBytes;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), quads = blockDim.x / kWave / 4;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), tid = threadIdx.x;
+  const int waves = blockDim.x / kWave, quads = (waves + 3) / 4;
+  if (tid >= waves && tid < quads * 4) { // places of wavefronts that the last quad lacks
+    reinterpret_cast<float *>(part[0])[tid] = kMaxInit;
+    reinterpret_cast<float *>(part[1])[tid] = 0.0f;
+  }
   RowPieces<D, kPieces, true> r(threadIdx.x, blockDim.x, int(cols));
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
     float m = wave_max(r.load_and_max(static_cast<const char *>(in) + row * rowBytes));
@@ -270,6 +279,79 @@ __device__ __forceinline__ void softmax_rows_of_a_lane(const void *in, void *out
     for (int i = 0; i < E::kPerVec - 1; ++i)
       if (i < cols)
         E::store(out, row * cols + i, x[i] * inv);
+  }
+}
+
+// ---- 65 .. 128 whole vectors: a wavefront owns kRowsPerWave rows ---------------------------
+// One row with ordinary loads (f32 8192 x 512 in the caches: 3.8 us, 6.5 with non-temporal ones), two of the large problems
+// with non-temporal ones.
+template <Dt D, bool kStreamIn, int kRowsPerWave>
+__device__ __forceinline__ void softmax_rows_in_regs(const void *in, void *out, int64_t rows, int64_t cols) {
+  using E = Elem<D>;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int64_t vecsPerRow = cols / E::kPerVec;
+  const int64_t rowBytes = cols * E::kBytes;
+  const int64_t groups = (rows + kRowsPerWave - 1) / kRowsPerWave;
+  for (int64_t g = int64_t(blockIdx.x) * kWaves + wave; g < groups; g += int64_t(gridDim.x) * kWaves) {
+    float x[kRowsPerWave][kRegChunks][E::kPerVec];
+    u32x4 raw[kRowsPerWave][kRegChunks];
+    // all loads of both rows first
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const int64_t row = g * kRowsPerWave + r;
+      const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(in) + row * rowBytes);
+#pragma unroll
+      for (int c = 0; c < kRegChunks; ++c) {
+        const int64_t v = int64_t(c) * kWave + lane;
+        if (row < rows && v < vecsPerRow)
+          raw[r][c] = load128<kStreamIn>(src + v);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const int64_t row = g * kRowsPerWave + r;
+      if (row >= rows)
+        continue; // uniform across the wavefront
+      float m = kMaxInit;
+#pragma unroll
+      for (int c = 0; c < kRegChunks; ++c) {
+        const bool live = int64_t(c) * kWave + lane < vecsPerRow;
+        if (live)
+          E::unpack(raw[r][c], x[r][c]);
+#pragma unroll
+        for (int i = 0; i < E::kPerVec; ++i) {
+          x[r][c][i] = live ? x[r][c][i] : kMaxInit;
+          m = fmaxf(m, x[r][c][i]);
+        }
+      }
+      m = wave_max(m);
+      float s = 0.0f;
+#pragma unroll
+      for (int c = 0; c < kRegChunks; ++c) {
+        const bool live = int64_t(c) * kWave + lane < vecsPerRow;
+#pragma unroll
+        for (int i = 0; i < E::kPerVec; ++i) {
+          x[r][c][i] = live ? fast_exp(x[r][c][i] - m) : 0.0f;
+          s += x[r][c][i];
+        }
+      }
+      s = wave_sum(s);
+      // one IEEE division per row, then multiplies (differs from z / s by at
+      // most an f32 rounding, far inside the 1e-3 bar)
+      const float inv = 1.0f / s;
+      u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + row * rowBytes);
+#pragma unroll
+      for (int c = 0; c < kRegChunks; ++c) {
+        const int64_t v = int64_t(c) * kWave + lane;
+        if (v < vecsPerRow) {
+#pragma unroll
+          for (int i = 0; i < E::kPerVec; ++i)
+            x[r][c][i] = x[r][c][i] * inv;
+          store128<true>(E::pack(x[r][c]), dst + v);
+        }
+      }
+    }
   }
 }
 
@@ -542,27 +624,37 @@ __device__ __forceinline__ void softmax_kernel(const void *in, void *out, int64_
     softmax_rows_of_a_lane<D>(in, out, rows, cols);
     return;
   }
-  if constexpr (D == Dt::F16 && kMaxThreads == kThreads)
-    if (aligned && pieces > kWave && pieces <= kRegChunks * kWave) { // non-temporal accesses: measured faster hot and cold
-      if (pieces == kRegChunks * kWave)
-        softmax_f16_rows_in_regs<true>(in, out, rows, cols);
+  if constexpr (kMaxThreads == kThreads)
+    if (aligned && pieces > kWave && pieces <= kRegChunks * kWave) {
+      if constexpr (D == Dt::F16) {
+        if (pieces == kRegChunks * kWave)
+          softmax_f16_rows_in_regs<true>(in, out, rows, cols);
+        else
+          softmax_f16_rows_in_regs<false>(in, out, rows, cols);
+      } else if (rows >= kTwoRowsFrom)
+        softmax_rows_in_regs<D, true, 2>(in, out, rows, cols);
       else
-        softmax_f16_rows_in_regs<false>(in, out, rows, cols);
+        softmax_rows_in_regs<D, false, 1>(in, out, rows, cols);
       return;
     }
-  if (pieces <= 4 * kWave && (pieces <= kWave || rows >= kManyRows)) {
+  // Ordinary loads, non-temporal stores: 8192 x 1024 f32 over again, its input in the caches, takes 9.5 us where
+  // non-temporal loads took 12.0, and the same 13.4 on buffers that are not (8192 x 4096: 39.6 / 43.4, from HBM
+  // 46.8 / 44.8).  Rows of up to 16 lanes (of 8 where they are whole pieces) share cache lines, which ordinary stores
+  // keep until all of a line is there: 200001 x 77 bf16 25.4 -> 16.5, 10^6 x 40 f32 99 -> 61.
+  if (pieces <= 4 * kWave &&
+      (pieces <= kWave || rows >= kWaveRows || (kMaxThreads == kThreads && pieces <= kRegChunks * kWave))) {
+    // up to four pieces a lane, two where that wastes no lanes (f16 30000 x 400 from HBM: 10.7 us, 12.3 with four)
+    const bool whole = cols % E::kPerVec == 0;
     int lanes = 4;
-    while (4 * lanes < pieces || (lanes < pieces && lanes < kWave && rows * lanes < kManyRows * kWave))
+    while (lanes < kWave && (4 * lanes < pieces || (lanes < pieces && rows * lanes < kManyRows * kWave) ||
+                             (whole && pieces > 48 && 2 * lanes < pieces)))
       lanes *= 2;
     const int per = int(pieces + lanes - 1) / lanes;
-    // Non-temporal accesses from rows of 32 lanes on (of 16 where rows are whole pieces): 20000 x 1001 f32 28.6 us, 30.6
-    // with ordinary ones.  Rows shorter than that share cache lines, which ordinary accesses keep until all of a line
-    // is there: 200001 x 77 bf16 25.4 -> 16.5, 10^6 x 40 f32 99 -> 61.
     switch (lanes) {
     case 4: softmax_lanes<D, 4, false>(in, out, rows, cols, per); break;
     case 8: softmax_lanes<D, 8, false>(in, out, rows, cols, per); break;
     case 16:
-      if (cols % E::kPerVec == 0)
+      if (whole)
         softmax_lanes<D, 16, true>(in, out, rows, cols, per);
       else
         softmax_lanes<D, 16, false>(in, out, rows, cols, per);

@@ -307,13 +307,15 @@ const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
 }
 
 // The operator's own launch is one for wavefronts (four per workgroup) or workgroups of 256 that have a row each: right
-// for f16 rows that wavefronts walk (65 .. 128 whole 16-byte pieces) and for rows that fit nobody's registers (more than
-// 4096 pieces).  Every other row goes to as many lanes as suit its length: 65536 x 32 bf16 20.5 us with a wavefront
-// per row, 3.2 so; 2500 x 8191 55.3 with 256 lanes of the streaming form, 18.8; 16384 x 1024 f32 24.4 / 23.1.
+// for rows of 65 .. 128 whole 16-byte pieces -- the f16 ones that wavefronts walk; f32 and bf16 up to 8192 rows, 16384 from
+// 96 pieces on (f32 16384 x 384: 9.0 us, 10.8 with shared wavefronts; 30000 x 512: 23.9 / 22.6) -- and for rows that fit
+// nobody's registers (more than 4096 pieces).  Every other row goes to as many lanes as suit its length: 65536 x 32 bf16
+// 20.5 us with a wavefront per row, 3.2 so; 2500 x 8191 55.3 with 256 lanes of the streaming form, 18.8.
 const char *softmaxVariant(const Entry *e, int64_t rows, int64_t cols) {
   const int64_t perVec = e->shape == Shape::SoftmaxRows16 ? 8 : 4, pieces = (cols + perVec - 1) / perVec;
-  const bool walked = cols % perVec == 0 && pieces > 64 && pieces <= 128 && strcmp(e->name, "imex_softmax_f16") == 0;
-  if (rows == 0 || cols == 0 || walked || pieces > 4096)
+  const bool f16 = strcmp(e->name, "imex_softmax_f16") == 0;
+  const bool own = cols % perVec == 0 && pieces <= 128 && pieces > 64 && (f16 || rows <= (pieces >= 96 ? 16384 : 8192));
+  if (rows == 0 || cols == 0 || own || pieces > 4096)
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s_shared", e->name);
@@ -456,14 +458,16 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
       grid[0] = 0;
     else if (cols < perVec)
       grid[0] = gridFor(ceilDiv(rows, 256), 256);
-    else if (pieces <= 256 && (pieces <= 64 || rows >= 2048)) {
+    else if (pieces <= 256 && (pieces <= 64 || rows >= 1024)) {
       int64_t lanes = 4;
-      while (4 * lanes < pieces || (lanes < pieces && lanes < 64 && rows * lanes < 2048 * 64))
+      while (lanes < 64 && (4 * lanes < pieces || (lanes < pieces && rows * lanes < 2048 * 64) ||
+                            (cols % perVec == 0 && pieces > 48 && 2 * lanes < pieces)))
         lanes *= 2;
       grid[0] = gridFor(ceilDiv(rows, 256 / lanes), 256);
     } else {
       grid[0] = static_cast<size_t>(std::min<int64_t>(rows, 1048560));
-      block[0] = pieces <= 1024 ? 256 : pieces <= 2048 ? 512 : pieces <= 4096 ? 1024 : 256;
+      const int64_t most = pieces <= 1024 ? 256 : pieces <= 2048 ? 512 : 1024, per = (pieces + most - 1) / most;
+      block[0] = pieces > 4096 ? 256 : ceilDiv((pieces + per - 1) / per, 64) * 64;
     }
     break;
   }

@@ -277,6 +277,35 @@ def test_softmax_rows_of_any_length_and_address(host, orc, stream, rows, pieces,
         assert np.max(np.abs(got.astype(np.int32) - ref.astype(np.int32))) <= 1
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,pieces", [(2500, 0.5), (700, 20.25), (1500, 65), (20003, 96), (300, 100.5), (1023, 129), (1024, 129),
+                                         (40, 300), (7, 641), (5, 1025), (4, 1537), (3, 2049), (3, 4096), (2, 4100)])
+def test_softmax_forms_by_their_own_names(host, orc, stream, rows, pieces, dtype):
+    """The operator itself and its _shared form, each by its own name under its own launch shape and on two workgroups
+    that walk all rows (a C caller need not take the advice of imexHipKernelVariant).  Tolerances: those of
+    test_softmax_rows_of_any_length_and_address."""
+    cols = int(pieces * (4 if dtype == "f32" else 8))
+    x = orc.fill_normal(rows * cols, dtype, 3 * rows + cols, 0.0, 2.0).reshape(rows, cols)
+    ref = orc.softmax_f32(x) if dtype == "f32" else orc.softmax_16(x, dtype)
+    blank = np.zeros_like(x)
+    d_in, d_out = stream.to_device(x), stream.alloc(x.nbytes)
+    for name in ("imex_softmax_" + dtype, "imex_softmax_%s_shared" % dtype):
+        grid, block, _ = host.launch_shape(name, [rows, cols])
+        for g in (grid, (2, 1, 1)):
+            say("%s %dx%d grid %s block %s" % (name, rows, cols, g, block))
+            stream.copy(d_out, blank.ctypes.data, x.nbytes)
+            stream.launch(name, [rows, cols], [d_in, d_out, rows, cols], grid=g, block=block)
+            stream.wait()
+            got = stream.from_device(d_out, (rows, cols), x.dtype)
+            if dtype == "f32":
+                assert np.max(np.abs(got - ref) / np.maximum(ref, 1e-30)) < 5e-5
+            elif dtype == "f16":
+                assert close_16(orc, got, ref, "f16")
+            else:
+                assert np.max(np.abs(got.astype(np.int32) - ref.astype(np.int32))) <= 1
+    stream.free(d_in), stream.free(d_out)
+
+
 @pytest.mark.parametrize("rows,cols", [(1000, 1024), (1000, 1016), (37, 1024), (4097, 1024), (5, 8)])
 def test_softmax_f16_rows_in_registers_any_grid(host, orc, stream, rows, cols):
     """The f16 register path walks its rows with the next row's loads in flight: a wavefront that takes one

@@ -218,6 +218,25 @@ def test_launch_shapes_of_every_form_fit_a_launch(host):
     assert host.launch_shape("imex_reduce_outer_f32_deep", [2, (1 << 32) + 1])[0][0] == (1 << 24) - 8
 
 
+def test_softmax_launch_rules(host):
+    """Rows of 65 .. 128 whole pieces stay with the operator's wavefronts as far as these are the faster form; a workgroup's
+    row gets whole wavefronts that hold it in at most four pieces per lane."""
+    choice = lambda dt, rows, pieces: host.variant("imex_softmax_" + dt, [rows, pieces * (4 if dt == "f32" else 8)])
+    for dt in ("f32", "bf16"):
+        own, shared = "imex_softmax_" + dt, "imex_softmax_%s_shared" % dt
+        assert [choice(dt, 8192, n) for n in (64, 65, 128, 129)] == [shared, own, own, shared]
+        assert [choice(dt, rows, n) for rows, n in ((8193, 95), (8193, 96), (16384, 96), (16385, 96))] == [shared, own, own, shared]
+        assert host.variant(own, [100, 65 * 8 + 1]) == shared
+    assert choice("f16", 1 << 20, 128) == "imex_softmax_f16" and choice("f16", 1 << 20, 64) == "imex_softmax_f16_shared"
+    for pieces in range(257, 4097):
+        grid, block, _ = host.launch_shape("imex_softmax_f32_shared", [3000, 4 * pieces - 3])
+        assert grid == (3000, 1, 1) and block[0] % 64 == 0 and block[0] <= 1024
+        assert pieces <= 4 * block[0] and -(-pieces // block[0]) == -(-pieces // (256 if pieces <= 1024 else 512 if pieces <= 2048 else 1024))
+    # a wavefront per row from 1024 rows of up to 256 pieces on
+    assert host.launch_shape("imex_softmax_f32_shared", [1024, 800])[0] == (256, 1, 1)
+    assert host.launch_shape("imex_softmax_f32_shared", [1023, 800])[0] == (1023, 1, 1)
+
+
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
     """Stream.launch's fast path: 8 bytes per argument, an f32 in the low four, with _pack_params' conversions and errors."""
     class Resolver:
