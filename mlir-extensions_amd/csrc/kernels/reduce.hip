@@ -274,6 +274,17 @@ __device__ __forceinline__ void reduce_outer_vec(const void *__restrict__ in, vo
   }
 }
 
+template <io::Dt D>
+__device__ __forceinline__ void reduce_outer_by_element(const void *in, void *out, int64_t outer, int64_t inner, float init) {
+  using E = io::Elem<D>;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < inner; i += int64_t(gridDim.x) * blockDim.x) {
+    float acc = init;
+    for (int64_t o = 0; o < outer; ++o)
+      acc = acc + E::get(in, o * inner + i);
+    E::put(out, i, acc);
+  }
+}
+
 // 16-bit inputs widen to f32, are added in f32 in slice order and rounded once at the end (the
 // reference's policy for 16-bit element types on the GPU, docs/Transforms/BF16ToGpu.md:17-26;
 // benchmarks/reduce/reduce.dtypes.in lists f32, f16, bf16).
@@ -294,12 +305,7 @@ __device__ __forceinline__ void reduce_outer(const void *in, void *out, int64_t 
     else
       reduce_outer_vec<D, 1>(in, out, outer, inner, init);
   } else {
-    for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < inner; i += int64_t(gridDim.x) * kThreads) {
-      float acc = init;
-      for (int64_t o = 0; o < outer; ++o)
-        acc = acc + E::get(in, o * inner + i);
-      E::put(out, i, acc);
-    }
+    reduce_outer_by_element<D>(in, out, outer, inner, init);
   }
 }
 
@@ -419,6 +425,10 @@ __device__ __forceinline__ void reduce_outer_deep_entry(const void *in, void *ou
   using E = io::Elem<D>;
   if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 && inner % E::kPerVec == 0)
     reduce_outer_deep<D, true>(in, out, outer, inner, init);
+  else if (outer <= 2 && inner % E::kPerVec == 0)
+    // a buffer off the 16-byte grid under the vectors' launch: a lane walks several outputs, and sixteen loads of one or
+    // two slices each cost more than they hide (bf16 1 x 65536: 5.4 us, 3.3 so)
+    reduce_outer_by_element<D>(in, out, outer, inner, init);
   else
     reduce_outer_deep<D, false>(in, out, outer, inner, init);
 }
@@ -589,12 +599,7 @@ __device__ __forceinline__ void reduce_outer_tall_entry(const void *in, void *ou
   else if (fits && blockDim.x == kTallElemThreads)
     reduce_outer_tall<D, false>(in, out, outer, inner, init, lds);
   else
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < inner; i += int64_t(gridDim.x) * blockDim.x) {
-      float acc = init;
-      for (int64_t o = 0; o < outer; ++o)
-        acc = acc + E::get(in, o * inner + i);
-      E::put(out, i, acc);
-    }
+    reduce_outer_by_element<D>(in, out, outer, inner, init);
 }
 
 extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_f32_tall(const float *in, float *out,

@@ -442,6 +442,31 @@ def test_reduce_outer_forms_bit_exact(host, orc, stream, form, dtype, outer, inn
     stream.free(d_out)
 
 
+@pytest.mark.parametrize("form", ["_tall", "_deep"])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,inner", [(1, 4104), (2, 520), (131, 520)])
+def test_reduce_outer_forms_at_any_address(host, orc, stream, form, dtype, outer, inner):
+    """Slices of whole 16-byte vectors in a buffer that starts one element behind a 16-byte boundary, and a result that
+    does: the loops that stand in for the vector forms add in the same order."""
+    width = 4 if dtype == "f32" else 2
+    x = orc.fill_uniform(outer * inner, dtype, 92, -1.0, 1.0)
+    wide = (x if dtype == "f32" else orc.to_float(x, dtype)).reshape(outer, inner)
+    want = orc.reduce_outer_f32(wide, 0.25)
+    want = want if dtype == "f32" else orc.from_float(want, dtype)
+    name = "imex_reduce_outer_" + dtype + form
+    for shift_in, shift_out in ((1, 0), (0, 1), (1, 1)):
+        say("%s %dx%d, bases %d and %d elements off" % (name, outer, inner, shift_in, shift_out))
+        fill = np.full(inner + 2, 3, x.dtype)
+        d_in = stream.to_device(np.concatenate([np.zeros(shift_in, x.dtype), x]))
+        d_out = stream.to_device(fill)
+        stream.launch(name, [outer, inner], [host.Ptr(d_in + shift_in * width), host.Ptr(d_out + shift_out * width), outer, inner, 0.25])
+        stream.wait()
+        got = stream.from_device(d_out, fill.shape, fill.dtype)
+        stream.free(d_in), stream.free(d_out)
+        assert np.array_equal(got[shift_out:shift_out + inner], want), (name, shift_in, shift_out)
+        assert np.all(got[:shift_out] == 3) and np.all(got[shift_out + inner:] == 3)
+
+
 def test_reduce_outer_benchmark_shape_and_any_grid(host, orc, stream):
     """32x16x512x512 (the reference suite's reduce shape, README.md:335): integer-valued inputs
     make the sum exact; then the same kernel on a grid of 7 workgroups, which must stride."""
