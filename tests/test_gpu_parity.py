@@ -360,6 +360,20 @@ def test_row_sums_of_any_length_and_address(host, orc, stream, cols):
     stream.free(d_in), stream.free(d_out)
 
 
+@pytest.mark.parametrize("cols", [4, 63, 129, 300, 1023])
+def test_short_row_sums_walk(host, orc, stream, cols):
+    """The forms whose lanes share a wavefront, on three workgroups that walk all rows.  Integer values: exact sums."""
+    rows = 1501
+    x = orc.fill_int(rows * cols, "f32", cols, -8, 8).reshape(rows, cols)
+    d_in, d_out = stream.to_device(x), stream.alloc(rows * 4)
+    for name, rest, want in (("rowsum", [3.0], orc.rowsum_f32(x, init=3.0)), ("rowmean", [], orc.rowmean_f32(x))):
+        say("%s %dx%d, three workgroups" % (name, rows, cols))
+        stream.launch("imex_%s_f32_short" % name, [rows, cols], [d_in, d_out, rows, cols, *rest], grid=(3, 1, 1))
+        stream.wait()
+        assert np.array_equal(stream.from_device(d_out, (rows,), np.float32), want), name
+    stream.free(d_in), stream.free(d_out)
+
+
 def test_rowsum_config_8192x8192(host, orc, stream):
     x = orc.fill_uniform(8192 * 8192, "f32", 20243, 0.0, 1.0).reshape(8192, 8192)
     got, ref = host.rowsum(stream, x), orc.rowsum_f32(x)
@@ -845,6 +859,27 @@ def test_flash_attention_one_tiling(host, orc, stream, queries, zh, n_ctx):
     assert attention_close(out[rows], orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows), orc)
 
 
+@pytest.mark.parametrize("queries", [32, 64, 128, 256])
+def test_flash_attention_one_tiling_at_any_address(host, orc, stream, queries):
+    """A tensor that starts one element behind a 16-byte boundary takes the reference loop of the same kernel."""
+    zh, n_ctx = 2, 130
+    n = zh * n_ctx
+    q, k, v = (orc.fill_uniform(n * 64, "f16", seed, -1, 1).reshape(n, 64) for seed in (87, 88, 89))
+    want = orc.flash_attention_rows(q, k, v, n_ctx, 0.5, np.arange(n))
+    for which in range(4):
+        say("attention, %d queries per workgroup, tensor %d off the 16-byte grid" % (queries, which))
+        host_bufs = [q.ravel(), k.ravel(), v.ravel(), np.full(n * 64, 0x7e01, np.uint16)]
+        host_bufs = [np.concatenate([np.zeros(int(i == which), np.uint16), t]) for i, t in enumerate(host_bufs)]
+        bufs = [stream.to_device(t) for t in host_bufs]
+        stream.launch("imex_flash_attention_fwd_f16_q%d" % queries, [zh, n_ctx],
+                      [host.Ptr(p + 2 * (i == which)) for i, p in enumerate(bufs)] + [0.5, zh, n_ctx])
+        stream.wait()
+        out = stream.from_device(bufs[3], host_bufs[3].shape, np.uint16)[int(which == 3):].reshape(n, 64)
+        for p in bufs:
+            stream.free(p)
+        assert attention_close(out, want, orc)
+
+
 def test_flash_attention_negative_scale_takes_the_reference_loop(host, orc, stream):
     """The tiled path takes the row maximum before scaling, which needs a positive scale; any
     other scale runs the one-lane-per-query loop of the same kernel."""
@@ -1149,6 +1184,34 @@ def test_gemm_unaligned_rows(host, orc, stream, tile, M, N, K):
             assert np.array_equal(orc.half_to_float(np.ascontiguousarray(got)), want), name
         else:
             assert np.array_equal(got, want + (7 if which == "acc" else 0)), name
+
+
+@pytest.mark.parametrize("tile,M,N,K", [("_t128", 260, 392, 136), ("_t128x64", 260, 200, 136), ("_t64", 136, 200, 264),
+                                        ("_t32", 104, 136, 264), ("_t16", 40, 200, 520), ("_u128", 259, 391, 135),
+                                        ("_u64", 135, 199, 263)])
+def test_gemm_tiles_walk_and_any_address(host, orc, stream, tile, M, N, K):
+    """The kernels with one tile size on two workgroups that walk all tiles (their LDS and their partial tiles are used
+    again), and with each operand's and the result's base one element behind a 16-byte boundary (the aligned forms take
+    their vector-ALU loop there).  Integer operands give the exact f32 sum in any order."""
+    for which in ("plain", "acc", "ta", "tb"):
+        name = "imex_gemm_" + {"plain": "f16_f16_f32", "acc": "f16_f16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb"}[which] + tile
+        m = (M + 7) // 8 * 8 if which == "ta" and tile[1] == "t" else M
+        a, b = orc.fill_int(m * K, "f16", 95, -3, 3).reshape(m, K), orc.fill_int(K * N, "f16", 96, -3, 3).reshape(K, N)
+        want = orc.half_to_float(a).astype(np.int64) @ orc.half_to_float(b).astype(np.int64) + (7 if which == "acc" else 0)
+        ins = [(a.T if which == "ta" else a).ravel(), (b.T if which == "tb" else b).ravel(), np.full(m * N, 7, np.float32)]
+        full = host.launch_shape(name, [m, N, K])[0]
+        for shifted, grid in ((None, (2, 1, 1)), (0, full), (1, full), (2, full)):
+            say("%s %dx%dx%d grid %s, buffer %s off the 16-byte grid" % (name, m, N, K, grid, shifted))
+            padded = [np.concatenate([np.zeros(int(i == shifted), t.dtype), t, np.full(64, 9, t.dtype)]) for i, t in enumerate(ins)]
+            bufs = [stream.to_device(t) for t in padded]
+            stream.launch(name, [m, N, K], [host.Ptr(p + t.itemsize * (i == shifted)) for i, (p, t) in enumerate(zip(bufs, ins))] + [m, N, K],
+                          grid=grid)
+            stream.wait()
+            got = stream.from_device(bufs[2], padded[2].shape, np.float32)[int(shifted == 2):]
+            for p in bufs:
+                stream.free(p)
+            assert np.array_equal(got[:m * N].reshape(m, N).astype(np.int64), want), (name, shifted, grid)
+            assert np.all(got[m * N:] == 9), (name, shifted, grid)
 
 
 @pytest.mark.parametrize("which", ["", "_ta", "_tb"])
@@ -1540,3 +1603,45 @@ def test_mfma_ceiling_kernel_computes_what_it_says(host, stream, mode):
             assert np.all(np.abs(have - want) <= 1e-4 * np.abs(want).max() + 1e-4), (g, w)
     assert not np.any(host.mfma_lds_ceiling(stream, 2, 7, mode=1))
     assert host.mfma_lds_ceiling(stream, 1, 0).shape == (1, 512) and not np.any(host.mfma_lds_ceiling(stream, 1, 0))
+
+
+# =============================== Launches by kept plans =====================
+@pytest.mark.parametrize("rows,cols", [(64, 2000), (3, 77), (200, 512)])
+def test_kept_plans_hold_each_operator_to_its_own_bar(host, orc, stream, rows, cols):
+    """Stream.launch twice per operator and size, with other buffers the second time, so that the second launch packs its
+    arguments for a plan that is kept: every result within the operator's own bar, exact where the operator is."""
+    n, k8 = rows * cols, (cols + 7) // 8 * 8
+    for seed in (501, 502):
+        f = orc.fill_uniform(n, "f32", seed, 0.5, 2.0).reshape(rows, cols)
+        h = orc.fill_normal(n, "f16", seed, 0.0, 2.0).reshape(rows, cols)
+        g = orc.fill_uniform(n, "f32", seed + 10, -3.0, 3.0).reshape(rows, cols)
+        a = orc.fill_uniform(rows * k8, "f16", seed, -1.0, 1.0).reshape(rows, k8)
+        b = orc.fill_uniform(k8 * 64, "f16", seed + 10, -1.0, 1.0).reshape(k8, 64)
+        exact = orc.half_to_float(a).astype(np.float64) @ orc.half_to_float(b).astype(np.float64)
+        sums = f.astype(np.float64).sum(axis=1)
+        bits = lambda want: (lambda got: np.array_equal(got.view(np.uint32 if got.itemsize == 4 else np.uint16),
+                                                        want.view(np.uint32 if want.itemsize == 4 else np.uint16)))
+        for name, dims, ins, out, rest, ok in (
+                ("imex_relu_f32", [n], [g], (n,), [n], bits(orc.relu_f32(g.ravel()))),
+                ("imex_silu_f16", [n], [h], (n,), [n], bits(orc.silu_16(h.ravel(), "f16"))),
+                ("imex_softmax_f16", [rows, cols], [h], (rows, cols), [rows, cols],
+                 lambda got: close_16(orc, got, orc.softmax_16(h, "f16"), "f16")),
+                # f32 sums of positive terms: `cols` roundings of at most 2^-24 each
+                ("imex_rowsum_f32", [rows, cols], [f], (rows,), [rows, cols, 0.0],
+                 lambda got: np.all(np.abs(got - sums) <= cols * 2.0 ** -24 * sums)),
+                ("imex_reduce_outer_f32", [rows, cols], [g], (cols,), [rows, cols, 0.25], bits(orc.reduce_outer_f32(g, 0.25))),
+                ("imex_transpose2d_b16", [rows, cols], [h], (cols, rows), [rows, cols], bits(orc.transpose2d(h))),
+                ("imex_loop_fusion_f32", [n], [f, g], (n,), [n], bits(orc.loop_fusion_f32(f.ravel(), g.ravel()))),
+                # k8 additions, each rounded by at most 2^-24 of a partial sum; those of uniform products stay below sqrt(k8)
+                ("imex_gemm_f16_f16_f32", [rows, 64, k8], [a, b], (rows, 64), [rows, 64, k8],
+                 lambda got: np.max(np.abs(got - exact)) <= k8 ** 1.5 * 2.0 ** -24)):
+            say("%s %s, seed %d" % (name, dims, seed))
+            dtype = np.uint16 if name.endswith(("f16", "b16")) else np.float32
+            blank = np.full(out, 7, dtype)
+            bufs = [stream.to_device(t) for t in ins] + [stream.to_device(blank)]
+            stream.launch(name, dims, bufs + rest)
+            stream.wait()
+            got = stream.from_device(bufs[-1], out, dtype)
+            for p in bufs:
+                stream.free(p)
+            assert ok(got), (name, seed)
