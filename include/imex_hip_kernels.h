@@ -135,9 +135,12 @@ const char *imexHipKernelSignature(int index);
 const void *imexHipKernelModule(const char *kernel, size_t *size);
 
 /* The catalogue kernel to launch for the operator `kernel` on a problem of the given dims: one with the same
- * arguments and results that is faster at that size, or `kernel` itself (also for dims the kernel does not take).
- * Every such kernel is correct at every size, as `kernel` itself is; this is advice, not a requirement.  NULL if
- * the name is unknown. */
+ * arguments that is faster at that size, or `kernel` itself (also for dims the kernel does not take).  Every such
+ * kernel is correct at every size, as `kernel` itself is; this is advice, not a requirement.  Results: the _any,
+ * _tall and _deep forms give `kernel`'s bit for bit; the _shared, _short, _q*, _t* and _u* forms add in another order
+ * and agree within the rounding of f32 sums.  Products of rows that are not 16-byte aligned are bit for bit the
+ * sequential sum only as `kernel` itself, which is what is named below K = 192 and 2^23 multiply-adds.  NULL if the
+ * name is unknown. */
 const char *imexHipKernelVariant(const char *kernel, const int64_t *dims, int ndims);
 
 /* Grid (in workgroups), block and dynamic shared memory for `kernel` on a

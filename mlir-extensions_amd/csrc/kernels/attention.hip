@@ -21,16 +21,17 @@
 // plain register loops plus ONE exchange between lane l and l+32 per block of
 // keys.
 //
-// Workgroup = QB query blocks of 32 x KG key groups, one wavefront each: 64, 128 or 256
-// queries of one (batch, head) as (QB, KG) = (2,4), (4,2), (8,1) with 512 threads, or 256
+// Workgroup = QB query blocks of 32 x KG key groups, one wavefront each: 32, 64, 128 or 256
+// queries of one (batch, head) as (QB, KG) = (1,8), (2,4), (4,2), (8,1) with 512 threads, or 256
 // queries as (8,2) with 1024 threads.  Wavefront w takes query block w % QB and every KG-th
-// 64-key tile, group w / QB; partial (m, l, O) of the key groups are merged through LDS at the
-// end.  Every workgroup walks all keys of its head, so K / V traffic from L2 falls with the
+// key tile, group w / QB -- tiles of 64 keys, of 32 (KB = 1 block of 32) with 32 queries, where
+// eight groups of 64-key tiles would leave the ring one stage; partial (m, l, O) of the key
+// groups are merged through LDS at the end.  Every workgroup walks all keys of its head, so K / V traffic from L2 falls with the
 // queries per workgroup; key groups exist to keep all CUs busy on small problems (the
 // reference's 2 x 2 x 4096 x 64 gives one 64-query workgroup per CU) and, in the 1024-thread
 // form, to put four wavefronts on every SIMD (the tiled path needs 114 registers).  The launch
 // says which: N_CTX / gridDim.x queries per workgroup, blockDim.x threads.  K and V blocks of
-// 64 KG keys go from global memory straight into an LDS ring (buffer_load ... lds) of 2, 4 or
+// 64 KG (32 queries: 256) keys go from global memory straight into an LDS ring (buffer_load ... lds) of 2, 4 or
 // 8 stages, up to seven blocks ahead.
 //
 // Arguments: (Q, K, V, Out, sm_scale: f32, ZH: i64, N_CTX: i64)   dims = {ZH, N_CTX}
@@ -38,7 +39,7 @@
 //   tiles: queries past the end are not stored, keys past the end get a score of -inf.
 // imex_flash_attention_fwd_f16_q32 / _q64 / _q128 / _q256 are the operator with one tiling each.
 // Launch: grid (ceil(N_CTX / q), ZH, 1) with q = 64, 128 or 256 and block (512,1,1), or q = 256
-// and block (1024,1,1).  Other launches (and a scale <= 0, or misaligned tensors) take the
+// and block (1024,1,1); the forms with one tiling take theirs only, _q256 with block (1024,1,1).  Other launches (and a scale <= 0, or misaligned tensors) take the
 // one-query-per-lane reference loop of the same kernel (grid-stride, any grid and block).
 
 #include "device_common.h"
@@ -316,9 +317,11 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   };
 
   if constexpr (kScoresAhead) {
-    // The scores of block it + 1 are formed while block `it` goes through the softmax, so a block costs no wait for its
-    // own K reads and first products.  K(it + 1) and V(it) are there when block `it` begins; the copies in flight
-    // are pairs of these.
+    // The scores of block it + 1 are formed before block `it` goes through the softmax, so the softmax does not wait for
+    // the last products of its own scores.  The K reads are still waited for, in front of the products of either
+    // order: a wavefront issues in order, and these come first.  K(it + 1) and V(it) are there when block `it` begins;
+    // the copies in flight are pairs of these.  Past the end the last block is fetched again, as below: two K and one V
+    // blocks more on a two-stage ring, 3 on 32 (64 queries, 4096 keys).
     dma_k(0, 0);
 #pragma unroll
     for (int b = 0; b < kAhead; ++b) {

@@ -216,12 +216,12 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
   __builtin_amdgcn_s_barrier();
   IMEX_FENCE();
   read(0, 0);
-  // Step t: slab t + 1 has landed and everybody has step t's fragments in registers, so the slot they came from
-  // ... is free one step later (it is the one slab t + S - 1 went into at step t - 1's barrier).
+  // Step t: everybody's fragments of step t - 1 were in registers before the barrier of that step, so its slot takes slab
+  // t + S - 1; slab t + 1 has landed at the barrier of this one.
   int cur = 0; // slot of step t
   auto step = [&](int p, int t) {
     const int nxt = cur + 1 == S ? 0 : cur + 1, free = cur == 0 ? S - 1 : cur - 1;
-    dma(t + S - 1, free); // slot of step t - 1: its fragments were in registers before the barrier at the end of t - 1
+    dma(t + S - 1, free);
     wait_vmcnt<(S - 2) * kCopies>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();

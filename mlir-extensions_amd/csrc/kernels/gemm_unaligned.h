@@ -13,7 +13,7 @@
 //   LDS         two slots: slab t + 2 is written to the slot that step t's fragments have been read from.
 //
 // Bound by the latency of a step (load, LDS write, barrier, fragment reads), as gemm_small.h is; the vector-ALU loop
-// that took these shapes before spent 2.8 us on every sixteen k, most of it waiting for one element's load after the
+// that took these shapes before spent 4.4 us on every sixteen k, most of it waiting for one element's load after the
 // other.  A step of 64 k takes 0.37 us on 64 x 64 tiles (0.19 with direct copies).  1001 x 1003 x 999 f16: 276 us before,
 // 10.7 here; 4097 x 4097 x 1001: 91.5 us, 368 TFLOP/s.
 

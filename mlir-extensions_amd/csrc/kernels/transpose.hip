@@ -38,8 +38,9 @@
 //    256 x 256 tile (512 lanes, so that two tiles fit the registers) gained 1.5 % and is not used.
 //  * Shapes or bases that break 16-byte alignment: 8 x 8 (4 x 4) blocks at any address, moved back inside at the
 //    edges (tile_unaligned).  Bound by HBM transactions: row segments that are no whole lines cost two partly used
-//    ones each (16-bit 5000 x 4097: 22.1 us, 3.7 TB/s; 5000 x 4096 would take 13.7 at 6 TB/s; one element at a time
-//    before: 150 us with buffers that are not in the caches).
+//    ones each (16-bit 5000 x 4097: 22.1 us with buffers that are not in the caches, 3.7 TB/s, where 5000 x 4096 would
+//    take 13.7 at 6 TB/s; 14.4 us over a few buffer sets that the 256 MiB cache holds in part; one element at a time
+//    150 and 119).
 //
 // Arguments: 2-D (in, out, rows: i64, cols: i64); 3-D (in, out, d0, d1, d2: i64).
 // Launch: block (256,1,1); one workgroup per tile, grid 2-D (ceil(cols/C),

@@ -13,7 +13,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
-#include <cstdlib>
 #include <cstring>
 #include <iterator>
 
@@ -34,7 +33,13 @@ extern const unsigned char imex_blob_attention[], imex_blob_attention_end[];
 namespace {
 
 enum class Module { Eltwise, Softmax, Reduce, Transpose, Gemm, GemmSmall, GemmUnaligned, Fusion, Attention };
-enum class Shape { Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16, RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16, Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm, GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16, Attention, AttentionTiling };
+enum class Shape {
+  Eltwise32, Eltwise16, Fusion32, Fusion16, SoftmaxRows32, SoftmaxRows16, SoftmaxShared32, SoftmaxShared16,
+  RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16,
+  Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm,
+  GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16,
+  Attention, AttentionTiling
+};
 
 struct Entry {
   const char *name;
@@ -246,13 +251,22 @@ constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 1500, 6200, 560, 1250, fal
                                    {"_t16", 16, 64, 256, 1100, 2000, 418, 633, false}};
 
 // The same for rows that are not 16-byte aligned, fitted to 70 random problems (M 1 .. 4096, N 64 .. 4096, K 64 .. 2048;
-// the choice was the faster tile on every one).  The operator itself is a loop on the vector ALUs there, 2.8 us for
+// the choice was the faster tile on every one).  The operator itself is a loop on the vector ALUs there, 4.4 us for
 // every sixteen k: 1001 x 1003 x 999 276 us, 10.7 here; 7 x 225 x 1897 346 / 13.8; 1 x 825 x 75 17.4 / 4.1.
 constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -1030, 6410, 742, 760, false},
                                         {"_u64", 64, 64, 64, 2230, 1790, 366, 344, true}};
 // Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit.
 constexpr double kUnalignedFrom = double(1 << 23);
 constexpr int64_t kUnalignedFromK = 192;
+
+// The tile that the name of a GemmSmall or GemmUnaligned entry ends in.
+const GemmTile &tileOf(const Entry *e) {
+  const char *suffix = strrchr(e->name, '_');
+  for (const GemmTile &t : kUnalignedTiles)
+    if (strcmp(t.suffix, suffix) == 0)
+      return t;
+  return *std::find_if(std::begin(kGemmTiles), std::end(kGemmTiles), [&](const GemmTile &t) { return strcmp(t.suffix, suffix) == 0; });
+}
 
 const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
   const bool transA = e->shape == Shape::GemmTA, transB = e->shape == Shape::GemmTB;
@@ -340,13 +354,14 @@ const char *transposeVariant(const Entry *e, const int64_t *dims) {
 // 12 x 1500 27.0 -> 20.3 (128), 6 x 4096 53.1 -> 42.5 (128), 12 x 4096 85.1 -> 68.3 (256).  Heads of fewer than 768 keys
 // stay (16 x 512 7.4 us, 7.9 with 32 queries), as do problems that fill more than one round with 256 queries; the 64
 // queries that form scores ahead gain from 2048 keys on (8 x 2048 17.4 -> 16.4, 16 x 1024 10.4 -> 10.9).
+struct Tiling {
+  const char *suffix;
+  int64_t queries;
+  double cost;
+};
+constexpr Tiling kTilings[] = {{"_q32", 32, 22.0}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
+
 const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
-  struct Tiling {
-    const char *suffix;
-    int64_t queries;
-    double cost;
-  };
-  constexpr Tiling kTilings[] = {{"_q32", 32, 22.0}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
   auto workgroups = [&](int64_t queries) { return (N + queries - 1) / queries * ZH; };
   if (N < 768 || N >= (int64_t(1) << 24) || ZH == 0 || ZH > 256 || workgroups(256) > 256)
     return e->name;
@@ -568,7 +583,10 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     break;
   }
   case Shape::AttentionTiling: { // the tiling that the name ends in
-    const int64_t ZH = dims[0], N = dims[1], queries = atoi(strrchr(e->name, '_') + 2);
+    const int64_t ZH = dims[0], N = dims[1];
+    const int64_t queries = std::find_if(std::begin(kTilings), std::end(kTilings), [&](const Tiling &t) {
+                              return strcmp(t.suffix, strrchr(e->name, '_')) == 0;
+                            })->queries;
     block[0] = queries == 256 ? 1024 : 512;
     if (N > 0 && N < (int64_t(1) << 24) && ZH > 0 && ZH <= 65535) {
       grid[0] = ceilDiv(N, queries);
@@ -616,20 +634,20 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
   }
   case Shape::GemmSmall: { // one workgroup per tile of the size that the name ends in
     const int64_t M = dims[0], N = dims[1], K = dims[2];
-    const char *suffix = strrchr(e->name, '_') + 2;
-    const int tileM = atoi(suffix), tileN = tileM == 128 && !strchr(suffix, 'x') ? 128 : 64;
+    const GemmTile &tile = tileOf(e);
     block[0] = 512;
     grid[0] = gridFor(mfmaTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
-                          ? ceilDiv(M, tileM) * ceilDiv(N, tileN)
+                          ? ceilDiv(M, tile.tileM) * ceilDiv(N, tile.tileN)
                           : ceilDiv(M, 128) * ceilDiv(N, 128),
                       512);
     break;
   }
   case Shape::GemmUnaligned: {
-    const int64_t M = dims[0], N = dims[1], K = dims[2], tile = atoi(strrchr(e->name, '_') + 2);
+    const int64_t M = dims[0], N = dims[1], K = dims[2];
+    const GemmTile &tile = tileOf(e);
     block[0] = 512;
     grid[0] = gridFor(unalignedTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
-                          ? ceilDiv(M, tile) * ceilDiv(N, tile)
+                          ? ceilDiv(M, tile.tileM) * ceilDiv(N, tile.tileN)
                           : ceilDiv(M, 128) * ceilDiv(N, 128),
                       512);
     break;

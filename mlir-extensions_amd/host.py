@@ -366,7 +366,8 @@ class Stream:
     def launch(self, name, dims, args, deps=None, grid=None, block=None):
         """gpuModuleLoad + gpuKernelGet + gpuLaunchKernel; returns the event (or
         None when the launch shape is empty).  `grid` / `block` replace the catalogue's, and with one of
-        them given it is `name` itself that is launched; otherwise the variant the catalogue advises."""
+        them given it is `name` itself that is launched; otherwise the variant the catalogue advises, whose sums
+        may be added in another order (imex_hip_kernels.h says which)."""
         if grid is None and block is None:
             # (operator.index: 64.0 equals 64 as a key, but is no dim)
             plan = self._plans.get((name, *map(operator.index, dims))) or self._plan(name, dims)
