@@ -9,16 +9,16 @@
 //  * rows of up to 256 pieces of 16 bytes (2048 16-bit / 1024 f32 elements) belong to 4 .. 64 lanes of a wavefront,
 //    up to four pieces a lane, so a wavefront has up to sixteen rows at once; max and sum are reductions on the VALU's
 //    cross-lane paths (DPP), no LDS.  Longer rows, up to 4096 pieces, and more than 64 pieces where there are fewer
-//    than 1024 rows to give to wavefronts (f32 1500 x 1200: 4.1 us, 5.4 with a workgroup each), belong to a workgroup.
+//    than 1024 rows to give to wavefronts (f32 1500 x 1000 from HBM: 4.1 us, 5.3 with a workgroup each), belong to a workgroup.
 //    Either way a row stays in registers from its one read to its one write, and neither its length nor its address
 //    need be multiples of anything.
-//    Bound by HBM on whole pieces (f32 16384 x 1024 from HBM: 23.8 us, 5.6 TB/s; bf16 8192 x 2000: 13.6); odd rows cost
+//    Bound by HBM on whole pieces (f32 16384 x 1024 from HBM: 24.3 us, 5.5 TB/s; bf16 8192 x 2000: 13.6); odd rows cost
 //    a second transaction per request on both sides (bf16 6000 x 3001 with changing buffers: 17 us, 4.2 TB/s; one element
 //    at a time through LDS 35.1), short ones are cut to size (bf16 65536 x 32: 3.2, with a wavefront each 20.5;
 //    200001 x 77: 119 / 16.5).
 //  * f32 and bf16 rows of 65 .. 128 whole pieces, up to 8192 rows (16384 from 96 pieces on): a wavefront has a row, from
 //    16384 rows on two, in the operator's own kernel.  f32 16384 x 384: 9.0 us, 10.8 on 32 lanes per row; bf16 2047 x
-//    1000: 3.9, 5.5 with a workgroup per row.
+//    1000 from HBM: 3.3, 5.5 with a workgroup per row.
 //  * f16 rows of 65 .. 128 whole pieces: a wavefront walks rows w, w + W, ... with the next row's loads in
 //    flight while it computes the current one, and the arithmetic is written for the instruction count (packed f16
 //    maximum, mixed-precision FMAs straight from and into the f16 halves, one reciprocal per row): about 6 vector
@@ -637,13 +637,13 @@ __device__ __forceinline__ void softmax_kernel(const void *in, void *out, int64_
         softmax_rows_in_regs<D, false, 1>(in, out, rows, cols);
       return;
     }
-  // Ordinary loads, non-temporal stores: 8192 x 1024 f32 over again, its input in the caches, takes 9.5 us where
-  // non-temporal loads took 12.0, and the same 13.4 on buffers that are not (8192 x 4096: 39.6 / 43.4, from HBM
-  // 46.8 / 44.8).  Rows of up to 16 lanes (of 8 where they are whole pieces) share cache lines, which ordinary stores
+  // Ordinary loads, non-temporal stores: 8192 x 1024 f32 over again, its input in the caches, takes 8.9 us where
+  // non-temporal loads took 12.1, and the same 13.3 on buffers that are not (8192 x 4096: 39.6 / 43.7, from HBM
+  // 47.1 / 45.1).  Rows of up to 16 lanes (of 8 where they are whole pieces) share cache lines, which ordinary stores
   // keep until all of a line is there: 200001 x 77 bf16 25.4 -> 16.5, 10^6 x 40 f32 99 -> 61.
   if (pieces <= 4 * kWave &&
       (pieces <= kWave || rows >= kWaveRows || (kMaxThreads == kThreads && pieces <= kRegChunks * kWave))) {
-    // up to four pieces a lane, two where that wastes no lanes (f16 30000 x 400 from HBM: 10.7 us, 12.3 with four)
+    // up to four pieces a lane, two where that wastes no lanes (f16 30000 x 400 from HBM: 10.4 us, 12.3 with four)
     const bool whole = cols % E::kPerVec == 0;
     int lanes = 4;
     while (lanes < kWave && (4 * lanes < pieces || (lanes < pieces && rows * lanes < kManyRows * kWave) ||
