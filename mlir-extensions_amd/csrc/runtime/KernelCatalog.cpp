@@ -475,8 +475,8 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
       grid[0] = gridFor(ceilDiv(rows, 256), 256);
     else if (pieces <= 256 && (pieces <= 64 || rows >= 1024)) {
       int64_t lanes = 4;
-      while (lanes < 64 && (4 * lanes < pieces || (lanes < pieces && rows * lanes < 2048 * 64) ||
-                            (cols % perVec == 0 && pieces > 48 && 2 * lanes < pieces)))
+      while (lanes < 64 && (4 * lanes < pieces || (lanes < pieces && rows * lanes <= 2048 * 64) ||
+                            (cols % perVec == 0 && pieces > 48 && pieces != 64 && 2 * lanes < pieces)))
         lanes *= 2;
       grid[0] = gridFor(ceilDiv(rows, 256 / lanes), 256);
     } else {
