@@ -40,7 +40,8 @@ constexpr int kThreads = 256;
 // [0x3f330000, ...), c = table centre of z's 1/16 sub-interval, r = z/c - 1,
 // log x = k ln2 + log c + r + r^2 (A2 + A1 r + A0 r^2); all in f64 with IEEE
 // operations, one final rounding).  A host build of this function agrees with
-// libm's logf on every positive finite f32.
+// libm's logf on every positive finite f32, with its products and sums rounded
+// separately and fused: fused it is five f64 instructions shorter.
 // ---------------------------------------------------------------------------
 struct LogfEntry {
   double invc, logc;
@@ -56,28 +57,25 @@ __device__ const LogfEntry kLogfTable[16] = {
     {0x1.886e6037841edp-1, 0x1.1058bc8a07ee1p-2},  {0x1.767dcf5534862p-1, 0x1.4043057b6ee09p-2},
 };
 
-// The arithmetic of logf on the bits of a positive normal number (libm's main path).
-__device__ __forceinline__ float logf_libm_core(uint32_t ix, const LogfEntry *table) {
+// The arithmetic of logf on the bits of a positive normal number (libm's main path), before its one rounding to f32.
+constexpr double kLn2 = 0x1.62e42fefa39efp-1;
+__device__ __forceinline__ double logf_libm_core(uint32_t ix, const LogfEntry *table) {
   const uint32_t tmp = ix - 0x3f330000u;
   const int i = (tmp >> 19) & 15;
   const int k = static_cast<int32_t>(tmp) >> 23;
   const uint32_t iz = ix - (tmp & 0xff800000u);
   const double invc = table[i].invc, logc = table[i].logc;
   const double z = static_cast<double>(u2f(iz));
-  const double r = z * invc - 1.0;
-  const double y0 = logc + static_cast<double>(k) * 0x1.62e42fefa39efp-1;
+  const double r = __builtin_fma(z, invc, -1.0);
+  const double y0 = __builtin_fma(static_cast<double>(k), kLn2, logc);
   const double r2 = r * r;
-  double y = 0x1.5575b0be00b6ap-2 * r + -0x1.ffffef20a4123p-2;
-  y = -0x1.00ea348b88334p-2 * r2 + y;
-  y = y * r2 + (y0 + r);
-  return static_cast<float>(y);
+  double y = __builtin_fma(0x1.5575b0be00b6ap-2, r, -0x1.ffffef20a4123p-2);
+  y = __builtin_fma(-0x1.00ea348b88334p-2, r2, y);
+  return __builtin_fma(y, r2, y0 + r);
 }
 
-// Positive, normal, finite and not 1.0: what libm sends straight down its main path.
-__device__ __forceinline__ bool logf_ordinary(float x) {
-  const uint32_t ix = f2u(x);
-  return ix - 0x00800000u < 0x7f800000u - 0x00800000u && ix != 0x3f800000u;
-}
+// Positive, normal and finite: what libm sends down its main path, and 1.0, for which that path gives its +0 too.
+__device__ __forceinline__ bool logf_ordinary(float x) { return f2u(x) - 0x00800000u < 0x7f800000u - 0x00800000u; }
 
 __device__ __forceinline__ float logf_libm(float x, const LogfEntry *table) {
   uint32_t ix = f2u(x);
@@ -95,29 +93,53 @@ __device__ __forceinline__ float logf_libm(float x, const LogfEntry *table) {
     ix = f2u(x * 0x1p23f);      // subnormal: normalise
     ix -= 23u << 23;
   }
-  return logf_libm_core(ix, table);
+  return static_cast<float>(logf_libm_core(ix, table));
 }
 
-__device__ __forceinline__ void stage_table(LogfEntry *lds) {
-  if (threadIdx.x < 16)
-    lds[threadIdx.x] = kLogfTable[threadIdx.x];
-  __syncthreads();
-}
+// The logarithms of a kernel, with what they need in LDS.  kMantissa is 0 for any f32.  A value widened from a 16-bit
+// type has a mantissa of 7 (bf16) or 10 (f16) bits, and log x = k ln2 + log m: the f64 logarithms of all 128 (1024)
+// mantissas, from the arithmetic above, leave one fused multiply-add and the rounding per element, where the general
+// form has twelve f64 instructions and conversions (a host build agrees with libm's logf on every bf16 and f16 value).
+// Without them the logarithms bound the 16-bit chains: loop fusion of 64 M bf16 78.3 -> 64.0 us (6.0 TB/s), of 11.3 M
+// 20.5 -> 15.1, of 4.6 M f16 11.2 -> 8.7.
+template <int kMantissa> struct Logarithms {
+  LogfEntry entry[16];
+  double mantissa[kMantissa ? 1 << kMantissa : 1];
+
+  // by all threads of the workgroup; readable after a barrier
+  __device__ __forceinline__ void stage() {
+    if (threadIdx.x < 16)
+      entry[threadIdx.x] = kLogfTable[threadIdx.x];
+    if constexpr (kMantissa != 0)
+      for (uint32_t m = threadIdx.x; m < 1u << kMantissa; m += blockDim.x)
+        mantissa[m] = logf_libm_core(0x3f800000u | m << (23 - kMantissa), kLogfTable);
+  }
+  // kOrdinary: the caller has checked logf_ordinary() in every lane of the wavefront, so that this is straight-line code
+  // (libm's special cases cost a masked region per element, which keeps the f64 chains of a vector's elements from
+  // interleaving).
+  template <bool kOrdinary> __device__ __forceinline__ float of(float x) const {
+    if constexpr (!kOrdinary)
+      return logf_libm(x, entry);
+    else if constexpr (kMantissa == 0)
+      return static_cast<float>(logf_libm_core(f2u(x), entry));
+    const uint32_t ix = f2u(x);
+    const double k = static_cast<int32_t>(ix >> 23) - 127;
+    return static_cast<float>(__builtin_fma(k, kLn2, mantissa[ix >> (23 - kMantissa) & ((1u << kMantissa) - 1)]));
+  }
+};
+template <Dt D> constexpr int kMantissaOf = D == Dt::F32 ? 0 : D == Dt::F16 ? 10 : 7;
 
 // the chains, on f32 values
-// kOrdinary: the caller has checked logf_ordinary() for the logarithm's argument in every lane of the
-// wavefront, so the chain is straight-line code (libm's special cases cost a masked region per element,
-// which keeps the f64 chains of a vector's elements from interleaving).
-template <bool kOrdinary = false>
-__device__ __forceinline__ float loop_chain(float a, float b, const LogfEntry *table) {
-  const float t1 = kOrdinary ? logf_libm_core(f2u(a), table) : logf_libm(a, table);
+template <bool kOrdinary = false, typename Logs>
+__device__ __forceinline__ float loop_chain(float a, float b, const Logs &logs) {
+  const float t1 = logs.template of<kOrdinary>(a);
   const float t2 = __builtin_fabsf(b);
   const float t3 = t1 + t2;
   return t3 - a;
 }
-template <bool kOrdinary = false>
-__device__ __forceinline__ float input_chain(float a, float b, const LogfEntry *table) {
-  const float t1 = kOrdinary ? logf_libm_core(f2u(b), table) : logf_libm(b, table);
+template <bool kOrdinary = false, typename Logs>
+__device__ __forceinline__ float input_chain(float a, float b, const Logs &logs) {
+  const float t1 = logs.template of<kOrdinary>(b);
   const float t2 = __builtin_fabsf(a);
   return t1 + t2;
 }
@@ -130,9 +152,9 @@ __device__ __forceinline__ float input_chain(float a, float b, const LogfEntry *
 // workgroups is what shortens it.
 constexpr int64_t kSmallFusion = int64_t(1) << 22; // elements
 
-template <Dt D, int kVecs>
+template <Dt D, int kVecs, typename Logs>
 __device__ __forceinline__ void loop_fusion_pass(const void *__restrict__ a, const void *__restrict__ b,
-                                                 void *__restrict__ out, int64_t n, const LogfEntry *table) {
+                                                 void *__restrict__ out, int64_t n, const Logs &logs) {
   using E = Elem<D>;
   constexpr int kVecsPerThread = kVecs;
   constexpr int64_t kElemsPerBlock = int64_t(kThreads) * kVecsPerThread * E::kPerVec;
@@ -162,17 +184,17 @@ __device__ __forceinline__ void loop_fusion_pass(const void *__restrict__ a, con
         if (__builtin_amdgcn_ballot_w64(!ordinary) == 0) { // uniform over the wavefront
 #pragma unroll
           for (int i = 0; i < E::kPerVec; ++i)
-            fa[i] = loop_chain<true>(fa[i], fb[i], table);
+            fa[i] = loop_chain<true>(fa[i], fb[i], logs);
         } else {
 #pragma unroll
           for (int i = 0; i < E::kPerVec; ++i)
-            fa[i] = loop_chain(fa[i], fb[i], table);
+            fa[i] = loop_chain(fa[i], fb[i], logs);
         }
         store128<true>(E::pack(fa), po + j * kThreads + threadIdx.x);
       }
     } else {
       for (int64_t i = base + threadIdx.x; i < base + kElemsPerBlock && i < n; i += kThreads)
-        E::put(out, i, loop_chain(E::get(a, i), E::get(b, i), table));
+        E::put(out, i, loop_chain(E::get(a, i), E::get(b, i), logs));
     }
   }
 }
@@ -180,12 +202,24 @@ __device__ __forceinline__ void loop_fusion_pass(const void *__restrict__ a, con
 template <Dt D>
 __device__ __forceinline__ void loop_fusion(const void *__restrict__ a, const void *__restrict__ b,
                                             void *__restrict__ out, int64_t n) {
-  __shared__ LogfEntry table[16];
-  stage_table(table);
-  if (n < kSmallFusion)
-    loop_fusion_pass<D, 1>(a, b, out, n, table);
-  else
-    loop_fusion_pass<D, 4>(a, b, out, n, table);
+  __shared__ Logarithms<kMantissaOf<D>> logs;
+  if (n < kSmallFusion) {
+    // (f16: 1024 mantissas are as many logarithms as a workgroup of 2048 elements saves)
+    if constexpr (D == Dt::F16) {
+      __shared__ Logarithms<0> plain;
+      plain.stage();
+      __syncthreads();
+      loop_fusion_pass<D, 1>(a, b, out, n, plain);
+    } else {
+      logs.stage();
+      __syncthreads();
+      loop_fusion_pass<D, 1>(a, b, out, n, logs);
+    }
+    return;
+  }
+  logs.stage();
+  __syncthreads();
+  loop_fusion_pass<D, 4>(a, b, out, n, logs);
 }
 
 // ---- kInputFusion: chain + column sums ------------------------------------------------
@@ -232,7 +266,7 @@ __device__ __forceinline__ float add_in_row_order(float acc, const float *t, int
 template <Dt D, int kCols, int kTileElems = ::kTileElems>
 __device__ __forceinline__ void input_fusion_cols(const void *__restrict__ a, const void *__restrict__ b,
                                                   void *__restrict__ out, int64_t rows, int64_t cols,
-                                                  const LogfEntry *table, float *tile) {
+                                                  const Logarithms<0> &logs, float *tile) {
   using E = Elem<D>;
   constexpr int kTileRows = kTileElems / kCols;
   constexpr int kPerLane = kTileElems / kThreads;
@@ -260,12 +294,12 @@ __device__ __forceinline__ void input_fusion_cols(const void *__restrict__ a, co
 #pragma unroll
         for (int u = 0; u < kPerLane; ++u)
           if (worker && r0 + (u * kThreads) / kCols < rows) // passes that lie wholly below the last row are skipped
-            t[u * kThreads + tid] = input_chain<true>(xa[u], xb[u], table);
+            t[u * kThreads + tid] = input_chain<true>(xa[u], xb[u], logs);
       } else {
 #pragma unroll
         for (int u = 0; u < kPerLane; ++u)
           if (worker && r0 + (u * kThreads) / kCols < rows)
-            t[u * kThreads + tid] = input_chain(xa[u], xb[u], table);
+            t[u * kThreads + tid] = input_chain(xa[u], xb[u], logs);
       }
       __syncthreads(); // the tile is complete; the other buffer was consumed before the previous barrier
       if (tid < kCols && c0 + tid < cols) {
@@ -407,7 +441,7 @@ __device__ __forceinline__ void tile_handover() {
 template <Dt D, typename S>
 __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, const void *__restrict__ b,
                                                     void *__restrict__ out, int64_t rows, int64_t cols,
-                                                    const LogfEntry *table, float *tile) {
+                                                    const Logarithms<0> &logs, float *tile) {
   using E = Elem<D>;
   constexpr int kCols = S::kCols, kTileRows = S::kTileRows, kWorkers = S::kWork, kPer = S::kPer;
   constexpr int kGroupPasses = S::kGroupPasses;
@@ -466,11 +500,11 @@ __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, 
               if (__builtin_amdgcn_ballot_w64(!ordinary) == 0) { // uniform over the wavefront
 #pragma unroll
                 for (int i = 0; i < kPer; ++i)
-                  fa[i] = input_chain<true>(fa[i], fb[i], table);
+                  fa[i] = input_chain<true>(fa[i], fb[i], logs);
               } else {
 #pragma unroll
                 for (int i = 0; i < kPer; ++i)
-                  fa[i] = input_chain(fa[i], fb[i], table);
+                  fa[i] = input_chain(fa[i], fb[i], logs);
               }
 #pragma unroll
               for (int i = 0; i < kPer; ++i)
@@ -512,30 +546,31 @@ __device__ __forceinline__ int input_fusion_block_cols(int64_t cols) {
 template <Dt D>
 __device__ __forceinline__ void input_fusion(const void *__restrict__ a, const void *__restrict__ b,
                                              void *__restrict__ out, int64_t rows, int64_t cols) {
-  __shared__ LogfEntry table[16];
+  __shared__ Logarithms<0> logs;
   __shared__ __attribute__((aligned(16))) float tile[2 * kStreamTileFloats];
-  stage_table(table);
+  logs.stage();
+  __syncthreads();
   // The launch says which form: 576 or 320 lanes ask for a streaming one, which needs whole aligned vectors.
   const bool vectors = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
                        cols % Elem<D>::kPerVec == 0;
   if (blockDim.x == kStreamThreads && vectors && input_fusion_streams<D>(rows, cols)) {
-    input_fusion_stream<D, WideShape<D>>(a, b, out, rows, cols, table, tile);
+    input_fusion_stream<D, WideShape<D>>(a, b, out, rows, cols, logs, tile);
     return;
   }
   if (blockDim.x == kNarrowThreads && input_fusion_narrow(cols)) {
-    input_fusion_stream<D, NarrowShape<D>>(a, b, out, rows, cols, table, tile);
+    input_fusion_stream<D, NarrowShape<D>>(a, b, out, rows, cols, logs, tile);
     return;
   }
   switch (input_fusion_block_cols(cols)) {
-  case 64: input_fusion_cols<D, 64>(a, b, out, rows, cols, table, tile); break;
-  case 32: input_fusion_cols<D, 32>(a, b, out, rows, cols, table, tile); break;
-  case 16: input_fusion_cols<D, 16>(a, b, out, rows, cols, table, tile); break;
-  case 8: input_fusion_cols<D, 8>(a, b, out, rows, cols, table, tile); break;
+  case 64: input_fusion_cols<D, 64>(a, b, out, rows, cols, logs, tile); break;
+  case 32: input_fusion_cols<D, 32>(a, b, out, rows, cols, logs, tile); break;
+  case 16: input_fusion_cols<D, 16>(a, b, out, rows, cols, logs, tile); break;
+  case 8: input_fusion_cols<D, 8>(a, b, out, rows, cols, logs, tile); break;
   default:
     if (rows <= 1024)
-      input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, table, tile);
+      input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, tile);
     else
-      input_fusion_cols<D, 4>(a, b, out, rows, cols, table, tile);
+      input_fusion_cols<D, 4>(a, b, out, rows, cols, logs, tile);
     break;
   }
 }

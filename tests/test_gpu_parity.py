@@ -703,6 +703,20 @@ def test_loop_fusion_16bit(host, orc, stream, dtype):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n", [1 << 16, (1 << 22) + 8192 + 5])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_loop_fusion_16bit_every_logarithm(host, orc, stream, dtype, n):
+    """Every 16-bit pattern under the logarithm, in order, so that whole wavefronts hold ordinary numbers and others zeros,
+    infinities, NaN and negative ones; with one and with four vectors per lane and a tail: the oracle's bits (of a NaN,
+    that it is one)."""
+    a = np.resize(np.arange(1 << 16, dtype=np.uint16), n)
+    b = orc.fill_uniform(n, dtype, 49, -2.0, 2.0)
+    got = orc.to_float(host.loop_fusion(stream, a, b, dtype), dtype)
+    want = orc.to_float(orc.from_float(orc.loop_fusion_f32(orc.to_float(a, dtype), orc.to_float(b, dtype)), dtype), dtype)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got.view(np.uint32)[~np.isnan(want)], want.view(np.uint32)[~np.isnan(want)])
+
+
 # from 2048 x 4096 on the launch asks for the streaming form (576 lanes): whole tiles, ragged rows and a partial
 # last block of columns, and a column count that is not made of whole vectors (the kernel falls back by itself)
 # below 4096 columns: four columns per workgroup, 64-row tiles, eight tiles' loads together (one group, several
