@@ -47,6 +47,8 @@
  *   imex_input_fusion_f32 / _f16 / _bf16  (a, b, out, rows:i64, cols:i64)
  *       out[j] = sum_i (log b[i,j] + |a[i,j]|)
  *       benchmarks/kInputFusion/kInputFusion.mlir.in:6-40 dims = {rows, cols}
+ *   imex_input_fusion_f32_tall, imex_input_fusion_f16_tall, imex_input_fusion_bf16_tall
+ *       the same for more than a few rows                                      dims = {rows, cols}
  *   imex_flash_attention_fwd_f16   (Q, K, V, Out, sm_scale:f32, ZH:i64, N_CTX:i64)
  *       softmax(sm_scale Q K^T) V per (batch, head), head dim 64, tensors [(ZH*N_CTX), 64]
  *       WG/flash_attention_fwd.mlir:25-307               dims = {ZH, N_CTX}

@@ -5,12 +5,15 @@
 // What bounds it is the chain of dependent additions of a column: a lone wavefront issues one instruction every four
 // cycles or so whatever it is, so a row costs four cycles for its addition and four for every other instruction that
 // the adding wavefront runs per row (measured, cycles per row: additions alone 4.2; with a 32-bit LDS read each 8.8 ..
-// 10; with a 128-bit read per four rows and one wait per sixteen 5.3; a 16-bit value widened by the adder 10.9).  So
-// the work is split between wavefronts of one workgroup: workers load, widen, evaluate and write f32 values to LDS
-// COLUMN by column, and one wavefront does nothing but add, a lane per column, four rows per LDS read.  A lane of a
-// worker loads the same 8 or 16 bytes of four consecutive rows and so holds four consecutive values of every column it
-// touches: the change of layout costs no instruction.  One barrier per tile of rows hands a tile over and the other one
-// back.  Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them.
+// 10; with a 128-bit read per four rows 7.4, and here, with one wait per sixteen rows, 6.3; a 16-bit value widened by the
+// adder 10.9).  So the work is split between the wavefronts of a workgroup: workers load, widen, evaluate and write f32
+// values to LDS COLUMN by column, and one wavefront does nothing but add, a lane per column, four rows per LDS read.  A
+// lane of a worker loads the same 8 bytes of four consecutive rows and so holds four consecutive values of every column
+// it touches: the change of layout costs no instruction.  One barrier per tile of rows hands a tile over and the other
+// one back; loads run one tile ahead (two tiles ahead were slower, f32 fused chain of 1500 x 2048 9.1 / 10.0 us).
+// Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them
+// (f32 sums of 8192 x 4096 34.4 us, 41.8 in launch order; ordinary loads: non-temporal ones lose the line, fused chain of
+// f32 8192 x 512 50 us against 32).
 #ifndef IMEX_HIP_COLUMN_CHAIN_H
 #define IMEX_HIP_COLUMN_CHAIN_H
 
@@ -18,35 +21,49 @@
 
 namespace imexhip {
 
-// kInputs matrices; kLanes lanes of a worker cover a row's segment with kWords 32-bit words each; kWorkers wavefronts of
-// workers; loads run kAhead tiles ahead of the one that is evaluated.
-template <io::Dt D, int kInputs_, int kLanes_, int kWords_, int kWorkers_, int kAhead_> struct ColumnChain {
+// Lanes per row segment (of 8 bytes each), by the 32-byte segments of a row.  Chains on one CU get in each other's way
+// (their additions fill a SIMD each, whether 8 or 64 lanes have a column), so: the narrowest segments of which every CU
+// gets one.  f32 sums of 8192 x 256 25.1 us with 4 lanes, 26.6 with 8, 29.5 with 16; 6481 x 2832 40.4, 21.9, 23.8; 964 x
+// 26136 61.8, 37.6, 27.0.
+__device__ __forceinline__ int chain_lanes(int64_t segments) { return segments <= 256 ? 4 : segments <= 512 ? 8 : 16; }
+// Eight workers where a CU gets one segment of 128 bytes (f16 sums of 5914 x 13936: 45.3 us with four, 31.8 with eight),
+// four where it gets more of them, so that these share it (128 x 32768: 6.5 with eight, 3.9 with four).
+__device__ __forceinline__ int wide_chain_workers(int64_t segments) { return segments <= 4 * 256 ? 8 : 4; }
+
+// What the chains take: a segment of columns, and a tile's rows (256 at most) within 32-bit offsets of its first one.
+template <io::Dt D> __device__ __forceinline__ bool chains_take(int64_t rows, int64_t cols) {
+  return cols * io::Elem<D>::kBytes >= 32 && cols * io::Elem<D>::kBytes < int64_t(1) << 22 && rows < int64_t(1) << 31;
+}
+
+// kInputs matrices; kLanes lanes of a worker cover a row's segment with 8 bytes each; kWorkers wavefronts of workers.
+template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain {
   using E = io::Elem<D>;
-  static constexpr int kInputs = kInputs_, kLanes = kLanes_, kWords = kWords_, kWorkers = kWorkers_, kAhead = kAhead_;
-  static constexpr int kPer = kWords * 4 / E::kBytes;           // columns per lane
+  static constexpr int kInputs = kInputs_, kLanes = kLanes_, kWorkers = kWorkers_;
+  static constexpr int kPer = 8 / E::kBytes;                    // columns per lane
   static constexpr int kCols = kLanes * kPer;                   // columns per workgroup, a lane of the adder each
   static constexpr int kRowsPerWave = 4 * (kWave / kLanes);     // rows of a tile that one worker wavefront takes
   static constexpr int kTileRows = kWorkers * kRowsPerWave;
   static constexpr int kThreads = (kWorkers + 1) * kWave;
-  // Floats from one column of a tile to the next.  128-bit LDS accesses are served sixteen lanes at a time over 64
-  // banks.  The adder's lanes read at c * pitch: an odd number of 4-word groups serves sixteen lanes without conflict,
-  // two for eight.  A worker's sixteen lanes write four rows-of-four of four column groups, kPer * pitch apart: with
-  // 16 words (modulo 64) between these they land on sixteen different groups.
+  // Floats from one column of a tile to the next, and where a column keeps its rows: four rows (a "quad") are 16 bytes,
+  // and quad q of a column that lane group j wrote is at place q ^ swizzle(j) within its four.  128-bit LDS accesses
+  // are served sixteen lanes at a time over 64 banks.  The adder's sixteen lanes read one quad of sixteen columns:
+  // conflict-free with 4 words (modulo 64) from column to column, and with 8 where there are eight columns.  A worker's
+  // sixteen lanes write 16 / kLanes quads of min(16, kLanes) column groups, kPer columns apart: 4 kPer words (or 16), and
+  // groups that meet after 16 / kPer of them (there are no more than four per place) trade quads.
   static constexpr int kPad = kCols <= 8 ? 8 : 4;
   static constexpr int kPitch = kTileRows + kPad;
+  static constexpr bool kSwizzled = kLanes * kPer > 16;
+  static __device__ __forceinline__ int swizzle(int group) {
+    return kSwizzled ? group * kPer / 16 * (kLanes < 16 ? 16 / kLanes : 1) : 0;
+  }
   static constexpr int kTileFloats = kCols * kPitch;
   static constexpr int kLdsFloats = 2 * kTileFloats;
-  static_assert(kCols <= kWave && kTileRows % 64 == 0, "a lane per column; the adder takes sixteen rows at a time, four deep");
+  static_assert(kCols <= kWave && kTileRows % 64 == 0 && kTileRows <= 256, "a lane per column; the adder takes sixteen rows at a time, four deep");
 
-  typedef uint32_t Raw __attribute__((ext_vector_type(kWords), aligned(E::kBytes))); // at any element's address
+  typedef uint32_t Raw __attribute__((ext_vector_type(2), aligned(2))); // at any element's address
   struct Tile {
     Raw v[kInputs][4];
   };
-
-  static __device__ __forceinline__ bool takes(int64_t rows, int64_t cols) {
-    // a tile's rows are addressed with 32-bit offsets from its first one
-    return cols >= kCols && cols * E::kBytes < (int64_t(1) << 31) / kTileRows && rows < (int64_t(1) << 40);
-  }
 
   // prologue(): run by every thread while the first loads are in flight; what it leaves in LDS is there for eval.
   // eval(const Raw (&words)[kInputs], float (&f)[kPer]): one row's values of this lane's columns.
@@ -55,40 +72,35 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWords_, int kWorkers_, int k
                                              float *lds, Prologue prologue, Eval eval) {
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t pitch = static_cast<uint32_t>(cols * E::kBytes);
-    const int64_t tiles = (rows + kTileRows - 1) / kTileRows;
-    const int lastRows = static_cast<int>(rows - (tiles - 1) * kTileRows); // of the last tile
-    const int64_t blocks = (cols + kCols - 1) / kCols;
+    const int tiles = static_cast<int>((rows + kTileRows - 1) / kTileRows);
+    const int lastRows = static_cast<int>(rows - int64_t(tiles - 1) * kTileRows); // of the last tile
+    const uint32_t blocks = static_cast<uint32_t>((cols + kCols - 1) / kCols);
     bool first = true;
-    for (int64_t w = blockIdx.x; w < blocks; w += gridDim.x) {
+    for (uint32_t w = blockIdx.x; w < blocks; w += gridDim.x) {
       // Workgroup w runs on XCD w % 8: the XCDs take contiguous shares of the segments.  (The last block of columns
       // starts early enough to be whole; columns that two workgroups share get the same value from both.)
-      const int64_t share = blocks / 8, extra = blocks % 8, x = w % 8;
-      const int64_t block = x * share + min(x, extra) + w / 8;
-      const int64_t c0 = min(block * kCols, cols - kCols);
+      const uint32_t xcd = w % 8, block = xcd * (blocks / 8) + min(xcd, blocks % 8) + w / 8;
+      const int64_t c0 = min(block * kCols, static_cast<uint32_t>(cols) - kCols);
       if (wave < kWorkers) {
         const int quad = wave * (kWave / kLanes) + lane / kLanes; // rows 4 quad .. 4 quad + 3 of a tile
         const int col = (lane % kLanes) * kPer;
         const char *base[2] = {static_cast<const char *>(a) + c0 * E::kBytes, static_cast<const char *>(b) + c0 * E::kBytes};
-        uint32_t at[4], atLast[4]; // rows past the end re-read the last one; they are never added
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          at[i] = static_cast<uint32_t>(4 * quad + i) * pitch + col * E::kBytes;
-          atLast[i] = static_cast<uint32_t>(min(4 * quad + i, lastRows - 1)) * pitch + col * E::kBytes;
-        }
-        auto load = [&](int64_t t, Tile &tile) { // tiles past the end: the last one again, never evaluated
+        const uint32_t at = static_cast<uint32_t>(4 * quad) * pitch + col * E::kBytes;
+        auto load = [&](int t, Tile &tile) { // tiles past the end: the last one again, never evaluated
           const bool last = t >= tiles - 1;
-          const int64_t start = (last ? tiles - 1 : t) * kTileRows * int64_t(pitch);
+          const int64_t start = int64_t(last ? tiles - 1 : t) * kTileRows * int64_t(pitch);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const uint32_t o = last ? atLast[i] : at[i];
+            // rows past the end re-read the last one; they are never added
+            const uint32_t o = last ? static_cast<uint32_t>(min(4 * quad + i, lastRows - 1)) * pitch + col * E::kBytes : at + i * pitch;
 #pragma unroll
             for (int n = 0; n < kInputs; ++n)
-              tile.v[n][i] = __builtin_nontemporal_load(reinterpret_cast<const Raw *>(base[n] + start + o));
+              tile.v[n][i] = *reinterpret_cast<const Raw *>(base[n] + start + o);
           }
         };
-        auto put = [&](int64_t t, const Tile &tile) {
+        auto put = [&](int t, const Tile &tile) {
           if (t < tiles - 1 || 4 * (quad - lane / kLanes) < lastRows) { // uniform: a wavefront wholly past the end has nothing to do
-            float *dst = lds + (t & 1) * kTileFloats + col * kPitch + 4 * quad;
+            float *dst = lds + (t & 1) * kTileFloats + col * kPitch + 4 * (quad ^ swizzle(lane % kLanes));
             float f[4][kPer];
             eval(tile.v, f);
 #pragma unroll
@@ -97,23 +109,19 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWords_, int kWorkers_, int k
           }
           handover(); // tile t is complete; the adder is done with tile t - 1, whose place tile t + 1 goes to
         };
-        Tile ring[kAhead + 1];
-        if (tiles > 0) {
-#pragma unroll
-          for (int u = 0; u < kAhead; ++u)
-            load(u, ring[u]);
-        }
+        Tile even, odd; // the loads of a tile are on their way while the one before it is evaluated
+        if (tiles > 0)
+          load(0, even);
         if (first) {
           prologue();
           handover();
         }
-        for (int64_t t = 0; t < tiles; t += kAhead + 1) {
-#pragma unroll
-          for (int u = 0; u <= kAhead; ++u) {
-            if (t + u < tiles) { // uniform
-              load(t + u + kAhead, ring[(u + kAhead) % (kAhead + 1)]);
-              put(t + u, ring[u]);
-            }
+        for (int t = 0; t < tiles; t += 2) {
+          load(t + 1, odd);
+          put(t, even);
+          if (t + 1 < tiles) { // uniform
+            load(t + 2, even);
+            put(t + 1, odd);
           }
         }
       } else {
@@ -125,60 +133,94 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWords_, int kWorkers_, int k
         const int col = lane % kCols;
         float acc = init;
         if (tiles > 0) {
-          constexpr int kGroups = kTileRows / 16; // of sixteen rows, four LDS reads each, three groups ahead
+          // Four groups of sixteen rows in registers: while one is added, the three after it are on their way.
+          typedef __attribute__((address_space(3))) const float LdsFloat;
+          typedef __attribute__((address_space(3))) const f32x4 LdsVec;
           f32x4 x[4][4];
-          const float *p = lds + col * kPitch;
-          auto read = [&](f32x4(&v)[4], int g) {
+          LdsFloat *place[4]; // of the first four quads of the 64 rows that are read
+          auto start = [&](int t) {
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-              v[q] = *reinterpret_cast<const f32x4 *>(p + g * 16 + q * 4);
+              place[q] = (LdsFloat *)lds + (t & 1) * kTileFloats + col * kPitch + 4 * (q ^ swizzle(col / kPer));
           };
-          auto add = [&](f32x4(&v)[4]) {
-            asm volatile("" : "+v"(v[3])); // one wait, for the youngest of the four reads
+          auto read = [&](int g, int at = 0) { // the g-th group of the 64 rows `at` rows on
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              x[g][q] = *(LdsVec *)(place[q] + at + g * 16);
+            __builtin_amdgcn_sched_barrier(0);
+          };
+          auto add = [&](int g) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              acc = acc + v[q].x;
-              acc = acc + v[q].y;
-              acc = acc + v[q].z;
-              acc = acc + v[q].w;
+              acc = acc + x[g][q].x;
+              acc = acc + x[g][q].y;
+              acc = acc + x[g][q].z;
+              acc = acc + x[g][q].w;
             }
+            __builtin_amdgcn_sched_barrier(0);
           };
+          auto landed = [] { // all reads but those of the three youngest groups: one wait per group, not one per read
+            __builtin_amdgcn_s_waitcnt(0xc07f | 12 << 8);
+            __builtin_amdgcn_sched_barrier(0);
+          };
+          start(0);
           handover(); // tile 0 is complete
+          read(0);
+          read(1);
+          read(2);
+          for (int t = 0; t + 1 < tiles; ++t) {
 #pragma unroll
-          for (int g = 0; g < 3; ++g)
-            read(x[g], g);
-          for (int64_t t = 0; t + 1 < tiles; ++t) {
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-              if (g + 3 == kGroups) {
+            for (int at = 0; at < kTileRows; at += 64) {
+              read(3, at);
+              landed();
+              add(0);
+              if (at + 64 == kTileRows) {
                 handover(); // everything of tile t is in registers; tile t + 1 is complete
-                p = lds + ((t + 1) & 1) * kTileFloats + col * kPitch;
+                start(t + 1);
               }
-              read(x[(g + 3) % 4], (g + 3) % kGroups);
-              add(x[g % 4]);
-              __builtin_amdgcn_sched_barrier(0);
+              const int next = (at + 64) % kTileRows;
+              read(0, next);
+              landed();
+              add(1);
+              read(1, next);
+              landed();
+              add(2);
+              read(2, next);
+              landed();
+              add(3);
             }
           }
-          // the last tile: 1 .. kTileRows rows
-          int g = 0;
-          for (; 16 * g + 64 <= lastRows; g += 4) {
+          int left = lastRows;
+#pragma unroll 1
+          for (; left >= 64; left -= 64) {
+            read(3);
+            landed();
+            add(0);
+            if (left > 64) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              read(x[(u + 3) % 4], min(g + u + 3, kGroups - 1));
-              add(x[u]);
+              for (int q = 0; q < 4; ++q)
+                place[q] += 64;
             }
+            read(0); // (past the last row: some rows again, not added)
+            landed();
+            add(1);
+            read(1);
+            landed();
+            add(2);
+            read(2);
+            landed();
+            add(3);
           }
+          read(3);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if (u == 0 && 16 * g + 48 < lastRows)
-              read(x[3], g + 3);
-            if (16 * (g + u) + 16 <= lastRows) { // uniform, as the others
-              add(x[u]);
+          for (int g = 0; g < 4; ++g) {
+            if (left >= 16 * g + 16) { // uniform
+              add(g);
             } else {
 #pragma unroll
               for (int r = 0; r < 15; ++r)
-                if (16 * (g + u) + r < lastRows)
-                  acc = acc + x[u][r / 4][r % 4];
+                if (16 * g + r < left)
+                  acc = acc + x[g][r / 4][r % 4];
             }
           }
         }

@@ -24,8 +24,10 @@
 // block (320,1,1), grid ceil(cols / 4); from 2048 rows and 128 row segments of 128 bytes on block (576,1,1),
 // grid ceil(cols * element bytes / 128); otherwise block (256,1,1), grid ceil(cols / c), a workgroup per
 // block of c = 64 .. 8 columns (the widest that leaves 512 workgroups).  A launch with 256 lanes always gets
-// the last form.  Workgroups stride, so any grid is correct.
+// the last form.  The _tall forms: block (320,1,1) up to 256 segments of 32 bytes in a row, else (576,1,1); grid a
+// workgroup per segment of 32, 64 or 128 bytes (chain_lanes in column_chain.h).  Workgroups stride, so any grid is correct.
 
+#include "column_chain.h"
 #include "device_common.h"
 
 using namespace imexhip;
@@ -43,7 +45,7 @@ constexpr int kThreads = 256;
 // libm's logf on every positive finite f32, with its products and sums rounded
 // separately and fused: fused it is five f64 instructions shorter.
 // ---------------------------------------------------------------------------
-struct LogfEntry {
+struct alignas(16) LogfEntry {
   double invc, logc;
 };
 __device__ const LogfEntry kLogfTable[16] = {
@@ -77,23 +79,15 @@ __device__ __forceinline__ double logf_libm_core(uint32_t ix, const LogfEntry *t
 // Positive, normal and finite: what libm sends down its main path, and 1.0, for which that path gives its +0 too.
 __device__ __forceinline__ bool logf_ordinary(float x) { return f2u(x) - 0x00800000u < 0x7f800000u - 0x00800000u; }
 
+// Any x, without a branch: libm's special cases are selected at the end.
 __device__ __forceinline__ float logf_libm(float x, const LogfEntry *table) {
-  uint32_t ix = f2u(x);
-  if (ix == 0x3f800000u)
-    return 0.0f;
-  if (ix - 0x00800000u >= 0x7f800000u - 0x00800000u) {
-    if (ix * 2 == 0)
-      return -__builtin_inff(); // log(+-0)
-    if (ix == 0x7f800000u)
-      return x;                 // log(inf)
-    if (ix * 2 > 0xff000000u)
-      return x + x;             // NaN: quieted, sign and payload kept
-    if (ix & 0x80000000u)
-      return u2f(0xffc00000u);  // log of a negative number: libm's (x - x) / 0, the x86 default NaN
-    ix = f2u(x * 0x1p23f);      // subnormal: normalise
-    ix -= 23u << 23;
-  }
-  return static_cast<float>(logf_libm_core(ix, table));
+  const uint32_t ix = f2u(x);
+  const uint32_t normal = ix < 0x00800000u ? f2u(x * 0x1p23f) - (23u << 23) : ix; // subnormals: normalised
+  float y = static_cast<float>(logf_libm_core(normal, table));
+  y = ix >= 0x7f800000u ? u2f(0xffc00000u) : y; // log of a negative number: libm's (x - x) / 0, the x86 default NaN
+  y = ix == 0x7f800000u ? x : y;                // log(inf)
+  y = ix * 2 > 0xff000000u ? x + x : y;         // NaN: quieted, sign and payload kept
+  return ix * 2 == 0 ? -__builtin_inff() : y;   // log(+-0)
 }
 
 // The logarithms of a kernel, with what they need in LDS.  kMantissa is 0 for any f32.  A value widened from a 16-bit
@@ -263,10 +257,10 @@ __device__ __forceinline__ float add_in_row_order(float acc, const float *t, int
   return acc;
 }
 
-template <Dt D, int kCols, int kTileElems = ::kTileElems>
+template <Dt D, int kCols, int kTileElems = ::kTileElems, typename Logs>
 __device__ __forceinline__ void input_fusion_cols(const void *__restrict__ a, const void *__restrict__ b,
                                                   void *__restrict__ out, int64_t rows, int64_t cols,
-                                                  const Logarithms<0> &logs, float *tile) {
+                                                  const Logs &logs, float *tile) {
   using E = Elem<D>;
   constexpr int kTileRows = kTileElems / kCols;
   constexpr int kPerLane = kTileElems / kThreads;
@@ -537,6 +531,83 @@ __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, 
   }
 }
 
+// ---- kInputFusion by column chains (column_chain.h) -------------------------------------------
+// Any number of columns and rows, at any address: the forms above read 4 .. 64 columns of a row per workgroup element by
+// element unless the rows are whole 16-byte vectors and there are 2048 of them and 128 segments of 128 bytes, and were
+// bound by the latency of those loads or, 16-bit inputs, by the logarithms.  bf16 5550 x 5932 449 -> 42 us (floor 21 for its
+// bytes), f32 3785 x 3480 155 -> 27 (17), f16 1052 x 5433 76 -> 11, f32 8192 x 512 87 -> 31 (the chain alone: 22), f32
+// 8192 x 8192 106 -> 91 (85).  Two workers per SIMD on segments of 64 and 128 bytes: one took 29 and 82 us on f16 3785 x
+// 3480 and f32 5550 x 5932, two take 19 and 60.
+template <Dt D, int kLanes, int kWorkers, typename Logs>
+__device__ __forceinline__ void input_fusion_chains(const void *__restrict__ a, const void *__restrict__ b,
+                                                    void *__restrict__ out, int64_t rows, int64_t cols, Logs &logs, float *lds) {
+  using C = ColumnChain<D, 2, kLanes, kWorkers>;
+  using E = Elem<D>;
+  constexpr int kPer = C::kPer;
+  C::run(a, b, out, rows, cols, 0.0f, lds, [&] { logs.stage(); }, [&](const typename C::Raw(&v)[2][4], float(&f)[4][kPer]) {
+    float x[4][kPer]; // under the logarithm
+    uint32_t least = ~0u, most = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        if constexpr (D == Dt::F32) {
+          f[i][w] = u2f(v[0][i][w]);
+          x[i][w] = u2f(v[1][i][w]);
+        } else {
+          f[i][2 * w] = E::widen(v[0][i][w] & 0xffffu);
+          f[i][2 * w + 1] = E::widen(v[0][i][w] >> 16);
+          x[i][2 * w] = E::widen(v[1][i][w] & 0xffffu);
+          x[i][2 * w + 1] = E::widen(v[1][i][w] >> 16);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        least = min(least, f2u(x[i][e]));
+        most = max(most, f2u(x[i][e]));
+      }
+    }
+    // uniform over the wavefront: all of them logf_ordinary()
+    if (__builtin_amdgcn_ballot_w64(least < 0x00800000u || most >= 0x7f800000u) == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < kPer; ++e)
+          f[i][e] = input_chain<true>(f[i][e], x[i][e], logs);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < kPer; ++e)
+          f[i][e] = input_chain(f[i][e], x[i][e], logs);
+    }
+  });
+}
+
+// Four workers for segments of 32 bytes, eight for 64 (wide_chain_workers() for 128).  Other launches, and what the chains
+// do not take, go by blocks of columns.
+template <Dt D>
+__device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, const void *__restrict__ b,
+                                                  void *__restrict__ out, int64_t rows, int64_t cols) {
+  __shared__ __attribute__((aligned(16))) float lds[ColumnChain<D, 2, 16, 8>::kLdsFloats];
+  __shared__ Logarithms<kMantissaOf<D>> logs;
+  const int64_t segments = (cols * Elem<D>::kBytes + 31) / 32;
+  const int lanes = chain_lanes(segments), workers = lanes == 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
+  if (!chains_take<D>(rows, cols) || int(blockDim.x) != (workers + 1) * kWave) {
+    logs.stage();
+    __syncthreads();
+    input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
+  } else if (lanes == 4) {
+    input_fusion_chains<D, 4, 4>(a, b, out, rows, cols, logs, lds);
+  } else if (lanes == 8) {
+    input_fusion_chains<D, 8, 8>(a, b, out, rows, cols, logs, lds);
+  } else if (workers == 8) {
+    input_fusion_chains<D, 16, 8>(a, b, out, rows, cols, logs, lds);
+  } else {
+    input_fusion_chains<D, 16, 4>(a, b, out, rows, cols, logs, lds);
+  }
+}
+
 // Columns per workgroup: as many as still leave every CU a couple of workgroups (wide blocks read
 // longer row segments), down to 4.
 __device__ __forceinline__ int input_fusion_block_cols(int64_t cols) {
@@ -585,6 +656,10 @@ __device__ __forceinline__ void input_fusion(const void *__restrict__ a, const v
   extern "C" __global__ __launch_bounds__(kStreamThreads) void imex_input_fusion_##SUFFIX(                                 \
       const CTYPE *a, const CTYPE *b, CTYPE *out, int64_t rows, int64_t cols) {                                      \
     input_fusion<DT>(a, b, out, rows, cols);                                                                         \
+  }                                                                                                                  \
+  extern "C" __global__ __launch_bounds__(576) void imex_input_fusion_##SUFFIX##_tall(          \
+      const CTYPE *a, const CTYPE *b, CTYPE *out, int64_t rows, int64_t cols) {                                      \
+    input_fusion_tall<DT>(a, b, out, rows, cols);                                                                    \
   }
 
 IMEX_FUSION_KERNELS(f32, Dt::F32, float)

@@ -27,6 +27,7 @@
 //   reduce_outer: grid (ceil(inner / (1024 v)), 1, 1), v = 8, 4, 2 or 1: the largest that leaves
 //           512 workgroups (any other grid works too, the workgroups stride).
 
+#include "column_chain.h"
 #include "device_common.h"
 
 using namespace imexhip;
@@ -453,169 +454,60 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16_de
 
 // ---- outer-dimension sum, many slices of few outputs -------------------------------------------------
 // With 4 .. 32 KiB of every slice per workgroup, a tall matrix (column sums of [8192, 4096]: 4 workgroups of the
-// form above) leaves the chip idle and waits for one slice's latency per four slices.  What bounds it is the chain:
-// the additions of one output are ordered, so a column costs `outer` dependent additions (6 cycles each from a lone
-// wavefront) whatever is done -- the rest is keeping that chain fed and free of other instructions.  A workgroup
-// owns the columns of a 128-byte segment (32 f32, 64 16-bit ones) and walks all slices in chunks of 64: copier
-// wavefronts bring the chunks from global memory straight into a ring of LDS (1 KiB = eight slices per copy, seven
-// chunks = 56 KiB in flight), and ONE wavefront does nothing but add, a lane per column, sixteen slices' reads ahead
-// of the additions.  One barrier per chunk hands a chunk over and the oldest one back.
-// Slices that are not made of whole 16-byte vectors are copied element by element (one slice of 64 columns per
-// copy; the copy itself widens a 2-byte element to a word), by four copier wavefronts.
-// 8192 x 4096 f32: 980 us in the plain form, now 45 (floor 21 for its bytes; the chain alone is 8192 x 6.3 cycles = 22);
-// 700 x 3001 f32: 651 -> 7.3; bf16 4429 x 544: 505 -> 34.  A wavefront that copies for itself between its additions
-// took 76 us on the first: 22 cycles per slice where these take 12.
-typedef __attribute__((address_space(3))) char LdsChar;
-constexpr int kTallRing = 64 * 1024; // bytes of LDS
-constexpr int kTallRows = 64;        // slices per chunk
-constexpr int kTallVecThreads = 128, kTallElemThreads = 320;
-
-template <io::Dt D> __device__ __forceinline__ void add_slice(float &acc, uint32_t raw) {
-  if constexpr (D == io::Dt::F32)
-    acc = acc + u2f(raw);
-  else if constexpr (D == io::Dt::BF16)
-    acc = acc + u2f(raw << 16);
-  else // the f16 operand widens inside the instruction (exactly), times 1.0, plus acc: one rounding
-    asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(raw));
-}
-
-template <int N> __device__ __forceinline__ void chunk_landed() { // this wavefront's copies, all but the N youngest
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-  __builtin_amdgcn_s_barrier();
-}
-
-template <io::Dt D, bool kVec>
-__device__ __forceinline__ void reduce_outer_tall(const void *__restrict__ in, void *__restrict__ out, int64_t outer,
-                                                  int64_t inner, float init, char *lds) {
+// form above) leaves the chip idle and waits for one slice's latency per four slices.  Column chains instead
+// (column_chain.h), whose workers have nothing to do but widen: the additions of one output are ordered, so a column costs
+// `outer` dependent additions whatever is done, 2.7 ns each here.  f32 8192 x 4096: 980 us in the plain form, 45.2 with a
+// 32-bit LDS read for every addition, 36.1 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 14.3;
+// bf16 8192 x 4096 58.0 -> 26.9, where the adder widened as well; f16 2000 x 1001 16.6 -> 8.4, 500 x 20000 9.5 -> 5.9.
+template <io::Dt D, int kLanes, int kWorkers>
+__device__ __forceinline__ void reduce_outer_chains(const void *in, void *out, int64_t outer, int64_t inner, float init, float *lds) {
+  using C = ColumnChain<D, 1, kLanes, kWorkers>;
   using E = io::Elem<D>;
-  constexpr int kCols = kVec ? 128 / E::kBytes : 64;
-  constexpr int kSlice = kVec ? 128 : 256;               // bytes of a slice's segment in LDS
-  constexpr int kElem = kVec ? E::kBytes : 4;            // bytes of an element in LDS
-  constexpr int kChunk = kTallRows * kSlice;             // 8 or 16 KiB
-  constexpr int kRing = kTallRing / kChunk;              // 8 or 4 chunks
-  constexpr int kCopiers = (kVec ? kTallVecThreads : kTallElemThreads) / kWave - 1;
-  constexpr int kCopies = kVec ? kTallRows / 8 : kTallRows / kCopiers; // per copier and chunk: 8 or 16
-  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int pitch = int(inner * E::kBytes);
-  const int chunks = int((outer + kTallRows - 1) / kTallRows), lastRows = int(outer - int64_t(chunks - 1) * kTallRows);
-  for (int64_t c0 = int64_t(blockIdx.x) * kCols; c0 < inner; c0 += int64_t(gridDim.x) * kCols) {
-    if (wave != 0) {
-      // Columns past the end re-read the last ones, slices past the end the last one (never added); chunks past the
-      // end go through a descriptor of size zero, so that every chunk is the same number of copies.
-      const int first = kVec ? lane >> 3 : (wave - 1) * kCopies; // slice of this lane's first copy within a chunk
-      const int col = kVec ? int(min((lane & 7) * 16 + c0 * E::kBytes, int64_t(pitch) - 16))
-                           : int(min(c0 + lane, inner - 1) * E::kBytes);
-      constexpr int kStep = kVec ? 8 : 1; // slices per copy
-      auto fetch = [&](int k) {
-        const char *base = static_cast<const char *>(in) + int64_t(k) * kTallRows * pitch;
-        const __amdgpu_buffer_rsrc_t rsrc =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(base), 0, k < chunks ? 0x7ffffff0 : 0, 0x00020000);
-        LdsChar *dst = (LdsChar *)lds + (k & (kRing - 1)) * kChunk + (kVec ? 0 : first * kSlice);
-        if (k != chunks - 1) {
-          const int voff = kVec ? first * pitch + col : col;
-          int soff = kVec ? 0 : first * pitch;
+  C::run(in, nullptr, out, outer, inner, init, lds, [] {}, [](const typename C::Raw(&v)[1][4], float(&f)[4][C::kPer]) {
 #pragma unroll
-          for (int u = 0; u < kCopies; ++u, soff += kStep * pitch)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst + u * kStep * kSlice, kVec ? 16 : E::kBytes, voff, soff, 0, 0);
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        if constexpr (D == io::Dt::F32) {
+          f[i][w] = u2f(v[0][i][w]);
         } else {
-#pragma unroll
-          for (int u = 0; u < kCopies; ++u)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, dst + u * kStep * kSlice, kVec ? 16 : E::kBytes,
-                                                     min(first + u * kStep, lastRows - 1) * pitch + col, 0, 0, 0);
+          f[i][2 * w] = E::widen(v[0][i][w] & 0xffffu);
+          f[i][2 * w + 1] = E::widen(v[0][i][w] >> 16);
         }
-      };
-      for (int k = 0; k < kRing - 1; ++k)
-        fetch(k);
-      for (int k = 0; k < chunks; ++k) {
-        chunk_landed<(kRing - 2) * kCopies>(); // chunk k is there; the adder has taken chunk k - 1, whose place ...
-        fetch(k + kRing - 1);                  // ... this one goes to
       }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else if (chunks > 0) {
-      const int at = (lane % kCols) * kElem;
-      uint32_t x[16], y[16];
-      auto read = [&](uint32_t(&v)[16], int k, int q) { // slices 16 q .. 16 q + 15 of chunk k
-        const char *p = lds + (k & (kRing - 1)) * kChunk + q * (16 * kSlice) + at;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          v[r] = kElem == 4 ? *reinterpret_cast<const uint32_t *>(p + r * kSlice)
-                            : *reinterpret_cast<const uint16_t *>(p + r * kSlice);
-      };
-      float acc = init;
-      auto add = [&](const uint32_t(&v)[16]) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          add_slice<D>(acc, v[r]);
-      };
-      auto next_chunk = [&] { // everything read so far is in registers
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      next_chunk();
-      read(x, 0, 0);
-      for (int k = 0; k + 1 < chunks; ++k) {
-        read(y, k, 1);
-        add(x);
-        read(x, k, 2);
-        add(y);
-        read(y, k, 3);
-        add(x);
-        next_chunk();
-        read(x, k + 1, 0);
-        add(y);
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) { // the last chunk: 1 .. 64 slices
-        if (16 * q + 16 <= lastRows) {
-          add(x);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 15; ++r)
-            if (16 * q + r < lastRows)
-              add_slice<D>(acc, x[r]);
-        }
-        if (q < 3)
-          read(x, chunks - 1, q + 1);
-      }
-      if (lane < kCols && c0 + lane < inner)
-        E::put(out, c0 + lane, acc);
-    } else if (lane < kCols && c0 + lane < inner) {
-      E::put(out, c0 + lane, init);
-    }
-    __syncthreads(); // the ring is free for the next columns
-  }
+  });
 }
 
-// 128 lanes ask for the 16-byte form, 320 for the element form, which takes any slices.  Other launches, and slices of
-// 32 MiB and more (offsets inside a chunk are 31 bits), add slice by slice as the kernel without the suffix does.
+// Four workers for segments of 32 and 64 bytes, wide_chain_workers() for 128.  Other launches, and what the chains do not
+// take, add slice by slice as the kernel without the suffix does.
 template <io::Dt D>
-__device__ __forceinline__ void reduce_outer_tall_entry(const void *in, void *out, int64_t outer, int64_t inner, float init) {
-  using E = io::Elem<D>;
-  __shared__ __attribute__((aligned(16))) char lds[kTallRing];
-  const bool fits = inner * E::kBytes < (int64_t(1) << 31) / kTallRows && outer < (int64_t(1) << 31);
-  if (fits && blockDim.x == kTallVecThreads && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && inner % E::kPerVec == 0)
-    reduce_outer_tall<D, true>(in, out, outer, inner, init, lds);
-  else if (fits && blockDim.x == kTallElemThreads)
-    reduce_outer_tall<D, false>(in, out, outer, inner, init, lds);
-  else
+__device__ __forceinline__ void reduce_outer_tall(const void *in, void *out, int64_t outer, int64_t inner, float init) {
+  __shared__ __attribute__((aligned(16))) float lds[ColumnChain<D, 1, 16, 8>::kLdsFloats];
+  const int64_t segments = (inner * io::Elem<D>::kBytes + 31) / 32;
+  const int lanes = chain_lanes(segments), workers = lanes == 16 ? wide_chain_workers(segments) : 4;
+  if (!chains_take<D>(outer, inner) || int(blockDim.x) != (workers + 1) * kWave)
     reduce_outer_by_element<D>(in, out, outer, inner, init);
+  else if (lanes == 4)
+    reduce_outer_chains<D, 4, 4>(in, out, outer, inner, init, lds);
+  else if (lanes == 8)
+    reduce_outer_chains<D, 8, 4>(in, out, outer, inner, init, lds);
+  else if (workers == 8)
+    reduce_outer_chains<D, 16, 8>(in, out, outer, inner, init, lds);
+  else
+    reduce_outer_chains<D, 16, 4>(in, out, outer, inner, init, lds);
 }
 
-extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_f32_tall(const float *in, float *out,
-                                                                                 int64_t outer, int64_t inner,
-                                                                                 float init) {
-  reduce_outer_tall_entry<io::Dt::F32>(in, out, outer, inner, init);
+extern "C" __global__ __launch_bounds__(576) void imex_reduce_outer_f32_tall(const float *in, float *out, int64_t outer,
+                                                                            int64_t inner, float init) {
+  reduce_outer_tall<io::Dt::F32>(in, out, outer, inner, init);
 }
 
-extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_f16_tall(const uint16_t *in, uint16_t *out,
-                                                                                 int64_t outer, int64_t inner,
-                                                                                 float init) {
-  reduce_outer_tall_entry<io::Dt::F16>(in, out, outer, inner, init);
+extern "C" __global__ __launch_bounds__(576) void imex_reduce_outer_f16_tall(const uint16_t *in, uint16_t *out, int64_t outer,
+                                                                            int64_t inner, float init) {
+  reduce_outer_tall<io::Dt::F16>(in, out, outer, inner, init);
 }
 
-extern "C" __global__ __launch_bounds__(kTallElemThreads) void imex_reduce_outer_bf16_tall(const uint16_t *in, uint16_t *out,
-                                                                                  int64_t outer, int64_t inner,
-                                                                                  float init) {
-  reduce_outer_tall_entry<io::Dt::BF16>(in, out, outer, inner, init);
+extern "C" __global__ __launch_bounds__(576) void imex_reduce_outer_bf16_tall(const uint16_t *in, uint16_t *out, int64_t outer,
+                                                                            int64_t inner, float init) {
+  reduce_outer_tall<io::Dt::BF16>(in, out, outer, inner, init);
 }

@@ -38,7 +38,7 @@ enum class Shape {
   RowSum, RowSumShort, ReduceOuter, ReduceOuter16, ReduceTall32, ReduceTall16, ReduceDeep32, ReduceDeep16,
   Transpose2D32, Transpose2D16, Transpose3D32, Transpose3D16, TransposeAny32, TransposeAny16, Gemm,
   GemmStreamK, GemmTA, GemmTB, GemmSmall, GemmUnaligned, GemmFixed4k, ColumnThreads, ColumnThreads16,
-  Attention, AttentionTiling
+  ColumnChains, ColumnChains16, Attention, AttentionTiling
 };
 
 struct Entry {
@@ -118,6 +118,12 @@ const Entry kEntries[] = {
      Shape::ColumnThreads16, 2},
     {"imex_input_fusion_bf16", "(a: bf16*, b: bf16*, out: bf16*, rows: i64, cols: i64)", Module::Fusion,
      Shape::ColumnThreads16, 2},
+    {"imex_input_fusion_f32_tall", "(a: f32*, b: f32*, out: f32*, rows: i64, cols: i64)", Module::Fusion,
+     Shape::ColumnChains, 2},
+    {"imex_input_fusion_f16_tall", "(a: f16*, b: f16*, out: f16*, rows: i64, cols: i64)", Module::Fusion,
+     Shape::ColumnChains16, 2},
+    {"imex_input_fusion_bf16_tall", "(a: bf16*, b: bf16*, out: bf16*, rows: i64, cols: i64)", Module::Fusion,
+     Shape::ColumnChains16, 2},
     {"imex_flash_attention_fwd_f16",
      "(Q: f16*, K: f16*, V: f16*, Out: f16*, sm_scale: f32, ZH: i64, N_CTX: i64)", Module::Attention,
      Shape::Attention, 2},
@@ -179,6 +185,9 @@ size_t ceilDiv(int64_t a, int64_t b) { return static_cast<size_t>((a + b - 1) / 
 // The grid of a form whose problem has `groups` workgroups of work.  HIP takes fewer than 2^32 lanes per dimension of a
 // launch, and the kernels stride over what a smaller grid leaves out.  (A multiple of 8: as many for each XCD.)
 size_t gridFor(size_t groups, size_t block) { return std::min(groups, ((size_t(1) << 32) - 1) / block / 8 * 8); }
+
+// How many 32-byte segments of a row a workgroup of column chains takes (chain_lanes in column_chain.h).
+int chainWidth(size_t segments) { return segments <= 256 ? 1 : segments <= 512 ? 2 : 4; }
 
 // What the MFMA paths of the GEMM kernels take (mfma_takes in gemm_tile.h): 16-byte aligned rows, and operands
 // addressed through one 32-bit-offset buffer descriptor below 2 GiB.
@@ -297,26 +306,31 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
   return variant ? variant->name : e->name;
 }
 
-// Which form of the outer-dimension sum a problem should take, from two estimates in microseconds fitted to 670
-// timed problems (7 .. 4096 slices of 256 .. 2 Mi outputs, all types, whole vectors and not; the choice is within 2.5 %
-// of the fastest form in the mean, 5.6 x faster than the plain form throughout).
-//   plain  whole vectors and enough of them that a workgroup reads 8 KiB and more of every slice (512 workgroups);
-//   tall   a segment of 128 bytes (64 columns where the slices are no whole vectors) costs its load plus the chain of
-//          its additions, 512 of them at a time; 3.2 TB/s at most;
-//   deep   a slice costs its share of sixteen slices' latency; 6.5 (5) TB/s at most.
-// 8192 x 4096 f32: plain 980, tall 45, deep 520 us; 512 x 131072: 73, 64, 45; 238 x 209827 (no whole vectors): 350, 70, 40.
+// Which form of the outer-dimension sum a problem should take, from two estimates in microseconds fitted to 700
+// timed problems (4 .. 9000 slices of 64 .. 4 Mi outputs, all types, whole vectors and not, from HBM; the choice is within
+// 0.2 % of the faster of tall and deep in the mean; near a tie deep, f32 300 x 80000 26.4 / 25.4).
+//   plain  whole vectors and slices of 5 MiB (16-bit: 8 MiB) and more (f32 12 x 1051744: plain 11.7, deep 10.4; 12 x
+//          1408680: 13.0, 13.5; f16 15 x 2283888: 18.3, 12.6);
+//   tall   a launch, a slice's share of the chain, and what a CU pays for further workgroups; 5.6 TB/s at most;
+//   deep   a slice costs its share of sixteen slices' latency, which its bytes hide little of; 7.3 (6.0) TB/s at most.
+// 8192 x 4096 f32: plain 980, tall 36, deep 520 us; 568 x 197848: tall 102, deep 66; bf16 389 x 129280: 30, 32.
 const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const bool f32 = e->shape == Shape::ReduceOuter;
-  const int64_t perVec = f32 ? 4 : 8;
+  const int64_t perVec = f32 ? 4 : 8, slice = inner * (f32 ? 4 : 2);
   const bool vec = inner % perVec == 0;
-  if (outer == 0 || inner == 0 || (vec && inner >= 512 * 2 * 256 * perVec))
+  if (outer == 0 || inner == 0 || (vec && slice >= (f32 ? int64_t(5) << 20 : int64_t(8) << 20)))
     return e->name;
-  const double bytes = double(outer) * double(inner) * (f32 ? 4 : 2);
-  const double rounds = std::max(1.0, double(ceilDiv(inner, vec ? 8 * perVec : 64)) / 512.0);
-  const double tall = 0.7 + std::max(rounds * (3.35 + double(outer) * (f32 ? 0.0046 : 0.0058)), bytes / 3.15e6);
-  const double deep = 2.6 + std::max(double(outer) * (vec ? 0.0615 : f32 ? 0.0304 : 0.0169), bytes / (vec ? 6.5e6 : 5.0e6));
+  const double bytes = double(outer) * double(slice);
+  const size_t segments = ceilDiv(slice, 32);
+  const int width = chainWidth(segments);
+  const double more = std::max(0.0, double(ceilDiv(segments, width)) / 256.0 - 1.0);
+  const double step = width == 1 ? 0.0026 : width == 2 ? 0.0030 : f32 ? 0.0038 : 0.0043;
+  const double tall = 3.04 + std::max(0.77 * more + double(outer) * step * (1.0 + 1.63 * more), bytes / 5.6e6);
+  const double wait = double(outer) * (vec ? 0.0517 : f32 ? 0.0220 : 0.0143), move = bytes / (vec ? 7.35e6 : 6.04e6);
+  const double deep = 2.61 + std::max(wait, move) + (vec ? 0.72 : 0.55) * std::min(wait, move);
+  const bool chains = slice >= 32 && slice < int64_t(1) << 22 && outer < int64_t(1) << 31; // chains_take in column_chain.h
   char name[96];
-  snprintf(name, sizeof name, "%s%s", e->name, tall < deep ? "_tall" : "_deep");
+  snprintf(name, sizeof name, "%s%s", e->name, chains && tall < 0.96 * deep ? "_tall" : "_deep");
   return find(name)->name;
 }
 
@@ -384,6 +398,22 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
   return find(name)->name;
 }
 
+// The fused chain with column sums: column chains, but for a few rows, where the operator's own launch has a shorter way to
+// its first and only additions.  By 300 timed problems (2 .. 12000 rows of 16 .. 300000 columns): below 2048 columns
+// from 128 rows on (f16 124 x 81: own 4.1 us, chains 4.4; f32 827 x 1592 23.2 / 6.2); rows that take workgroups of 128-byte
+// segments more than one round from 72 (f32) or 24 rows on (f32 33 x 25520 9.9 / 10.8; f16 20 x 37008 8.7 / 9.5; bf16 5550 x
+// 5932 449 / 42); rows in between always (f32 2 x 7024 6.6 / 3.8).
+const char *inputFusionVariant(const Entry *e, int64_t rows, int64_t cols) {
+  const bool f32 = e->shape == Shape::ColumnThreads;
+  const int64_t bytes = cols * (f32 ? 4 : 2);
+  if (rows == 0 || rows >= int64_t(1) << 31 || bytes >= int64_t(1) << 22 || // chains_take in column_chain.h
+      (cols < 2048 ? rows < 128 || bytes < 32 : bytes > 256 * 128 && rows < (f32 ? 72 : 24)))
+    return e->name;
+  char name[96];
+  snprintf(name, sizeof name, "%s_tall", e->name);
+  return find(name)->name;
+}
+
 extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *dims, int ndims) {
   const Entry *e = find(kernel);
   if (!e || ndims != e->ndims || (ndims > 0 && !dims))
@@ -411,6 +441,9 @@ extern "C" const char *imexHipKernelVariant(const char *kernel, const int64_t *d
   case Shape::Transpose3D32:
   case Shape::Transpose3D16:
     return transposeVariant(e, dims);
+  case Shape::ColumnThreads:
+  case Shape::ColumnThreads16:
+    return inputFusionVariant(e, dims[0], dims[1]);
   case Shape::Attention:
     return attentionVariant(e, dims[0], dims[1]);
   default:
@@ -503,14 +536,6 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     const int64_t inner = dims[1], perVec = e->shape == Shape::ReduceOuter ? 1024 : 2048;
     const int64_t v = inner >= 512 * 8 * perVec ? 8 : inner >= 512 * 4 * perVec ? 4 : inner >= 512 * 2 * perVec ? 2 : 1;
     grid[0] = ceilDiv(inner, perVec * v);
-    break;
-  }
-  case Shape::ReduceTall32:
-  case Shape::ReduceTall16: { // a workgroup per 128-byte segment; slices of no whole 16-byte vectors: per 64 columns
-    const int64_t perVec = e->shape == Shape::ReduceTall32 ? 4 : 8;
-    const bool vec = dims[1] % perVec == 0;
-    block[0] = vec ? 128 : 320;
-    grid[0] = gridFor(ceilDiv(dims[1], vec ? 8 * perVec : 64), block[0]);
     break;
   }
   case Shape::ReduceDeep32:
@@ -618,6 +643,19 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     // otherwise a workgroup per block of 64 .. 8 columns: the widest that leaves 512 workgroups
     const int64_t block_cols = cols >= 64 * 512 ? 64 : cols >= 32 * 512 ? 32 : cols >= 16 * 512 ? 16 : cols >= 8 * 512 ? 8 : 4;
     grid[0] = ceilDiv(cols, block_cols);
+    break;
+  }
+  case Shape::ReduceTall32:
+  case Shape::ReduceTall16:
+  case Shape::ColumnChains:
+  case Shape::ColumnChains16: { // a workgroup per segment of 32, 64 or 128 bytes: the kernels' own rule (chain_lanes in column_chain.h)
+    const bool f32 = e->shape == Shape::ReduceTall32 || e->shape == Shape::ColumnChains;
+    const bool reduce = e->shape == Shape::ReduceTall32 || e->shape == Shape::ReduceTall16;
+    const int64_t perSegment = f32 ? 8 : 16;
+    const size_t segments = ceilDiv(dims[1], perSegment);
+    const int64_t times = chainWidth(segments);
+    block[0] = (times == 4 && segments <= 4 * 256) || (times == 2 && !reduce) ? 576 : 320; // eight workers or four
+    grid[0] = gridFor(ceilDiv(dims[1], times * perSegment), block[0]);
     break;
   }
   case Shape::Gemm:

@@ -768,6 +768,50 @@ def test_input_fusion_any_grid(host, orc, stream, shape, block):
         stream.free(p)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,segments,extra", [(1, 1, 0), (255, 1, 1), (256, 3, -1), (257, 256, 0), (1000, 256, -7),
+                                                 (127, 256, 1), (129, 512, 0), (271, 511, 3), (128, 512, 1),
+                                                 (513, 515, 5), (64, 1024, 9), (0, 4, 0)])
+def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra):
+    """The fused chain and the plain sum down the columns around the tiles of rows (128, 256) and the widths of a
+    workgroup's segment (32, 64 and 128 bytes: up to 256, up to 512 and more 32-byte segments in a row), with buffers on and
+    one element off the 16-byte grid, on the catalogue's grid, on five workgroups and with lanes that the chains do not
+    take: the additions are in row order, so the results are the oracle's bits.  Zeros, infinities, NaN, negative and
+    subnormal numbers stand under the logarithm of some columns."""
+    width = 4 if dtype == "f32" else 2
+    cols = segments * (32 // width) + extra
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    a = orc.fill_uniform(max(rows * cols, 1), dtype, 53, -5.0, 5.0)[:rows * cols].reshape(rows, cols)
+    b = orc.fill_uniform(max(rows * cols, 1), dtype, 54, 0.01, 40.0)[:rows * cols].reshape(rows, cols)
+    if rows > 2 and cols > 16:
+        b[rows // 2, :6] = narrow(np.float32([0.0, -0.0, np.inf, -3.0, np.nan, 1e-40]))
+        b[-1, -2:] = narrow(np.float32([1e-39, 1.0]))
+    zeros = lambda init: np.full(cols, init, np.float32)
+    want = {"input_fusion": narrow(orc.input_fusion_f32(wide(a), wide(b)) if rows else zeros(0.0)),
+            "reduce_outer": narrow(orc.reduce_outer_f32(wide(a), 0.25) if rows else zeros(0.25))}
+    for shift in (0, 1):
+        at = lambda t: stream.to_device(np.concatenate([np.zeros(shift, t.dtype), t.ravel(), np.zeros(8, t.dtype)]))
+        d_a, d_b = at(a), at(b)
+        fill = np.full(cols + 16, 3, a.dtype)
+        d_out = stream.to_device(fill)
+        p_a, p_b, p_out = (host.Ptr(p + shift * width) for p in (d_a, d_b, d_out))
+        for op, args in (("input_fusion", [p_a, p_b, p_out, rows, cols]), ("reduce_outer", [p_a, p_out, rows, cols, 0.25])):
+            name = "imex_%s_%s_tall" % (op, dtype)
+            for launch in ({}, {"grid": (5, 1, 1)}, {"block": (256, 1, 1)}):
+                say("%s %dx%d, %d off, %s" % (name, rows, cols, shift, launch))
+                stream.copy(d_out, fill.ctypes.data, fill.nbytes)
+                stream.launch(name, [rows, cols], args, **launch)
+                stream.wait()
+                got = stream.from_device(d_out, fill.shape, fill.dtype)
+                res, ref = wide(got[shift:shift + cols]), wide(want[op])
+                assert np.array_equal(np.isnan(res), np.isnan(ref)), (name, launch)
+                assert np.array_equal(got[shift:shift + cols][~np.isnan(ref)], want[op][~np.isnan(ref)]), (name, launch)
+                assert np.all(got[:shift] == 3) and np.all(got[shift + cols:] == 3), (name, launch)
+        for p in (d_a, d_b, d_out):
+            stream.free(p)
+
+
 # ============================ flash attention ===============================
 def attention_close(got_bits, ref_bits, orc):
     """The reference checks its kernel with allclose (atol 1e-4, rtol 1e-3) on a constant
