@@ -88,8 +88,25 @@
  *   imex_gemm_bf16_bias_silu_bf16_t128, imex_gemm_bf16_bias_silu_bf16_t128x64,
  *   imex_gemm_bf16_bias_silu_bf16_t64,
  *   imex_gemm_bf16_bias_silu_bf16_t32, imex_gemm_bf16_bias_silu_bf16_t16
- *       the operator without the suffix, same arguments, on tiles of 128 x 128, 128 x 64, 64 x 64, 32 x 64 and 16 x 64
- *       outputs: what imexHipKernelVariant names for problems that would leave most of the chip idle
+ *   imex_gemm_f16_f16_f32_t256x128, imex_gemm_f16_f16_f32_t128x64s,
+ *   imex_gemm_f16_f16_f32_t16x32, imex_gemm_f16_f16_f32_t16x16
+ *   imex_gemm_f16_f16_f32_acc_t256x128, imex_gemm_f16_f16_f32_acc_t128x64s,
+ *   imex_gemm_f16_f16_f32_acc_t16x32, imex_gemm_f16_f16_f32_acc_t16x16
+ *   imex_gemm_bf16_bf16_f32_t256x128, imex_gemm_bf16_bf16_f32_t128x64s,
+ *   imex_gemm_bf16_bf16_f32_t16x32, imex_gemm_bf16_bf16_f32_t16x16
+ *   imex_gemm_bf16_bf16_f32_acc_t256x128, imex_gemm_bf16_bf16_f32_acc_t128x64s,
+ *   imex_gemm_bf16_bf16_f32_acc_t16x32, imex_gemm_bf16_bf16_f32_acc_t16x16
+ *   imex_gemm_f16_f16_f16_t256x128, imex_gemm_f16_f16_f16_t128x64s,
+ *   imex_gemm_f16_f16_f16_t16x32, imex_gemm_f16_f16_f16_t16x16
+ *   imex_gemm_f16_f16_f32_tb_t256x128, imex_gemm_f16_f16_f32_tb_t128x64s,
+ *   imex_gemm_f16_f16_f32_tb_t16x32, imex_gemm_f16_f16_f32_tb_t16x16
+ *   imex_gemm_f16_f16_f32_ta_t256x128, imex_gemm_f16_f16_f32_ta_t128x64s,
+ *   imex_gemm_f16_f16_f32_ta_t16x32, imex_gemm_f16_f16_f32_ta_t16x16
+ *   imex_gemm_bf16_bias_silu_bf16_t256x128, imex_gemm_bf16_bias_silu_bf16_t128x64s,
+ *   imex_gemm_bf16_bias_silu_bf16_t16x32, imex_gemm_bf16_bias_silu_bf16_t16x16
+ *       the operator without the suffix, same arguments, on tiles of 256 x 128, 128 x 128, 128 x 64 (s: two workgroups to
+ *       a CU), 64 x 64, 32 x 64, 16 x 64, 16 x 32 and 16 x 16 outputs: what imexHipKernelVariant names for problems that
+ *       would leave much of the chip idle
  *                                                          dims = {M, N, K}
  *   imex_gemm_f16_f16_f32_u128, imex_gemm_f16_f16_f32_u64
  *   imex_gemm_f16_f16_f32_acc_u128, imex_gemm_f16_f16_f32_acc_u64

@@ -14,8 +14,10 @@
 //               (TN) elements whose 32-byte pairs trade places with the k row (pair_swizzle);
 //   registers   the fragments of step t + 1 are read while step t is multiplied (one barrier per step);
 //   result      the product is taken transposed (a lane holds four consecutive columns of a row); the KG partial
-//               tiles meet in LDS (pitch TN + 4 floats: no bank conflicts on either side), are added in group
-//               order and leave as four consecutive columns per lane, whole lines per row.
+//               tiles meet in LDS (pitch TN + 4 floats: no bank conflicts on either side; one after the other where
+//               they do not fit side by side), are added in group order and leave as four consecutive columns per
+//               lane, whole lines per row.
+//   edges       rows and columns past the end go out of the descriptor's range: nothing moves for them.
 //
 // Steps past the end of K are fetched through a descriptor of size zero (nothing moves, LDS gets zeros).
 // Operands whose rows are not 16-byte aligned take gemm_blocked, as in gemm_tile.h, or the kernels of gemm_unaligned.h.
@@ -80,7 +82,7 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
       for (int q = 0; q < kCopies; ++q) {
         const int id = wave * kCopies + q, slab = id / (TR / 8), row = (id % (TR / 8)) * 8 + (lane >> 3);
         const int k = slab * 64 + (((lane & 7) ^ ((row >> 1) & 7)) << 3);
-        voff[q] = int((int64_t(min(row, last)) * ld + k) * 2);
+        voff[q] = row <= last ? int((int64_t(row) * ld + k) * 2) : kOutOfRange;
         voffT[q] = k < kRem ? voff[q] : kOutOfRange;
       }
       step = BK * 2;
@@ -93,8 +95,8 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
       for (int q = 0; q < kCopies; ++q) {
         const int row = (wave * kCopies + q) * (1024 / kRow) + lane / kChunks, chunk = lane % kChunks;
         const int pair = (chunk >> 1) ^ pair_swizzle<TR / 16>(row);
-        const int64_t col = min(int64_t(pair * 16 + (chunk & 1) * 8), ld - 8 - first); // ld % 8 == 0
-        voff[q] = int((int64_t(row) * ld + col) * 2);
+        const int64_t col = pair * 16 + (chunk & 1) * 8; // ld % 8 == 0: a piece is inside or not
+        voff[q] = first + col < ld ? int((int64_t(row) * ld + col) * 2) : kOutOfRange;
         voffT[q] = row < kRem ? voff[q] : kOutOfRange;
       }
       step = int(BK * ld * 2);
@@ -105,10 +107,10 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0, kt < steps ? range : 0, 0x00020000);
     const bool tail = kt == steps - 1;
+    const int at = kt < steps ? kt * step : 0; // (never beyond the descriptor's range)
 #pragma unroll
     for (int q = 0; q < kCopies; ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds + image + dst + q * 1024, 16, tail ? voffT[q] : voff[q],
-                                               kt * step, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds + image + dst + q * 1024, 16, tail ? voffT[q] : voff[q], at, 0, 0);
   }
   // fragment f (16 rows from w0 + 16 f), 32-wide slice s of the step
   __device__ __forceinline__ typename T::Frag read(const char *lds, int image, int f, int s) const {
@@ -130,7 +132,9 @@ template <int TMv, int TNv, int WMCv, int WNCv, int KGv, int Sv> struct SmallSha
   static constexpr int FI = TM / WMC / 16, FJ = TN / WNC / 16;
   static constexpr int kStageBytes = (TM + TN) * BK * 2;
   static constexpr int kPitch = TN + 4; // floats per row of a partial tile in LDS
-  static constexpr int kMergeBytes = KG * TM * kPitch * 4;
+  // the partial tiles of all key groups side by side, or one after the other where these would not fit
+  static constexpr bool kMergeInPlace = KG * TM * kPitch * 4 > 160 * 1024;
+  static constexpr int kMergeBytes = (kMergeInPlace ? 1 : KG) * TM * kPitch * 4;
   static constexpr int kLds = S * kStageBytes > kMergeBytes ? S * kStageBytes : kMergeBytes;
   static constexpr int kWavesPerEu = kLds <= 80 * 1024 ? 4 : 2; // two workgroups on a CU where LDS has room for two
   static_assert(WMC * WNC * KG == kWaves && BK % 64 == 0 && kLds <= 160 * 1024, "eight wavefronts, one CU's LDS");
@@ -147,13 +151,27 @@ __device__ __forceinline__ void merge_and_store(const f32x4 (&acc)[P::FI][P::FJ]
   // partial tiles side by side in LDS: lane holds row lane % 16, columns (lane / 16) * 4 .. + 3 of a block
   float *part = reinterpret_cast<float *>(lds);
   {
-    float *mine = part + kg * (P::TM * P::kPitch) + (wm * (P::TM / P::WMC) + (lane & 15)) * P::kPitch +
-                  wn * (P::TN / P::WNC) + (lane >> 4) * 4;
+    float *mine = part + (P::kMergeInPlace ? 0 : kg) * (P::TM * P::kPitch) +
+                  (wm * (P::TM / P::WMC) + (lane & 15)) * P::kPitch + wn * (P::TN / P::WNC) + (lane >> 4) * 4;
+    auto put = [&](bool add) {
 #pragma unroll
-    for (int i = 0; i < FI; ++i)
+      for (int i = 0; i < FI; ++i)
 #pragma unroll
-      for (int j = 0; j < FJ; ++j)
-        *reinterpret_cast<f32x4 *>(mine + i * 16 * P::kPitch + j * 16) = acc[i][j];
+        for (int j = 0; j < FJ; ++j) {
+          f32x4 *at = reinterpret_cast<f32x4 *>(mine + i * 16 * P::kPitch + j * 16);
+          *at = add ? acc[i][j] + *at : acc[i][j];
+        }
+    };
+    if constexpr (P::kMergeInPlace) {
+      static_assert(P::KG == 2);
+      if (kg == 1) // uniform over the wavefront
+        put(false);
+      __syncthreads();
+      if (kg == 0)
+        put(true);
+    } else {
+      put(false);
+    }
   }
   __syncthreads();
   constexpr int kVecs = P::TM * P::TN / 4;
@@ -164,7 +182,7 @@ __device__ __forceinline__ void merge_and_store(const f32x4 (&acc)[P::FI][P::FJ]
       const int r = v / (P::TN / 4), c = (v % (P::TN / 4)) * 4;
       f32x4 sum = *reinterpret_cast<const f32x4 *>(part + r * P::kPitch + c);
 #pragma unroll
-      for (int g = 1; g < P::KG; ++g)
+      for (int g = 1; g < (P::kMergeInPlace ? 1 : P::KG); ++g)
         sum += *reinterpret_cast<const f32x4 *>(part + g * (P::TM * P::kPitch) + r * P::kPitch + c);
       if (m0 + r < M && n0 + c < N)
         store_columns(epi, m0 + r, n0 + c, N, sum);
@@ -196,18 +214,25 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
 #pragma unroll
     for (int j = 0; j < FJ; ++j)
       acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  typename T::Frag af[2][FI], bf[2][FJ];
+  // With eight A fragments per wavefront there is room for one set of them: each is replaced by the next step's as soon
+  // as its products are issued.
+  constexpr bool kOneA = FI >= 8;
+  typename T::Frag af[kOneA ? 1 : 2][FI], bf[2][FJ];
   auto dma = [&](int kt, int slot) {
     opA.dma(ldsBase, slot * P::kStageBytes + kImageA, kt, steps);
     opB.dma(ldsBase, slot * P::kStageBytes + kImageB, kt, steps);
   };
-  auto read = [&](int p, int slot) {
-#pragma unroll
-    for (int i = 0; i < FI; ++i)
-      af[p][i] = opA.read(lds, slot * P::kStageBytes + kImageA, i, kg);
+  auto read_a = [&](int p, int slot, int i) { af[kOneA ? 0 : p][i] = opA.read(lds, slot * P::kStageBytes + kImageA, i, kg); };
+  auto read_b = [&](int p, int slot) {
 #pragma unroll
     for (int j = 0; j < FJ; ++j)
       bf[p][j] = opB.read(lds, slot * P::kStageBytes + kImageB, j, kg);
+  };
+  auto read = [&](int p, int slot) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+      read_a(p, slot, i);
+    read_b(p, slot);
   };
 #pragma unroll
   for (int t = 0; t < S - 1; ++t)
@@ -226,15 +251,30 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     IMEX_FENCE();
-    read(p ^ 1, nxt);
-    IMEX_FENCE();
+    if constexpr (kOneA) {
+      read_b(p ^ 1, nxt);
+      IMEX_FENCE();
 #pragma unroll
-    for (int j = 0; j < FJ; ++j)
+      for (int i = 0; i < FI; ++i) {
 #pragma unroll
-      for (int s = 0; s < FI; ++s) {
-        const int i = (j & 1) ? FI - 1 - s : s;
-        acc[i][j] = T::mfma(bf[p][j], af[p][i], acc[i][j]);
+        for (int s = 0; s < FJ; ++s) {
+          const int j = (i & 1) ? FJ - 1 - s : s;
+          acc[i][j] = T::mfma(bf[p][j], af[0][i], acc[i][j]);
+        }
+        read_a(0, nxt, i);
+        IMEX_FENCE();
       }
+    } else {
+      read(p ^ 1, nxt);
+      IMEX_FENCE();
+#pragma unroll
+      for (int j = 0; j < FJ; ++j)
+#pragma unroll
+        for (int s = 0; s < FI; ++s) {
+          const int i = (j & 1) ? FI - 1 - s : s;
+          acc[i][j] = T::mfma(bf[p][j], af[p][i], acc[i][j]);
+        }
+    }
     cur = nxt;
   };
   int t = 0;

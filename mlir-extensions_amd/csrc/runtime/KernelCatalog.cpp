@@ -57,6 +57,10 @@ struct Entry {
       {NAME "_t64", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                               \
       {NAME "_t32", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                               \
       {NAME "_t16", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                               \
+      {NAME "_t256x128", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                          \
+      {NAME "_t128x64s", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                          \
+      {NAME "_t16x32", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                            \
+      {NAME "_t16x16", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                            \
       {NAME "_u128", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3},                                      \
       {NAME "_u64", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3}
 
@@ -238,26 +242,29 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
   return begin;
 }
 
-// Which tile a GEMM should take.  What one workgroup costs was fitted to 400 random problems (M 1 .. 4096, N 64 ..
-// 11008, K 64 .. 4096, all eight operators, every tile timed on each): a launch takes `constant`, a workgroup `setup`
-// (first slab, result) plus `step` per K step, and every further workgroup that a CU gets costs `setup` again and
-// `stepMore` per step -- less than the sum of the two where two workgroups share a CU (64 x 64: counted by the
-// fraction, the others by whole rounds of 256 workgroups).  Nanoseconds.  The tile with the least estimate is within
-// 1.3 % of the fastest one in the mean over those problems (90 % of them within 4 %), 2.9 x faster than 256 x 256
-// tiles throughout; examples, 256 x 256 / chosen: 256 x 256 x 256 10.5 / 3.5 us (16 x 64), 1000^3 27.5 / 7.9 (64 x 64),
-// 16 x 11008 x 4096 73 / 17.1 (64 x 64), 2048^3 40.5 / 23.7 (128 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with
-// 128 x 128 tiles.
+// Which tile a GEMM should take.  What one workgroup costs was fitted to 750 random problems (M 1 .. 4096, N 64 ..
+// 11008, K 64 .. 4096, all eight operators, operands from beyond the L2s, every tile timed on each): a launch takes
+// `constant`, a workgroup `setup` (first slab, result) plus `step` per K step, and every further workgroup that a CU gets
+// costs `setup` again and `stepMore` per step -- less than the sum of the two where workgroups share a CU (64 x 64: counted
+// by the fraction, the others by whole rounds of 256 workgroups).  Nanoseconds.  The tile with the least estimate is within
+// 0.2 % of the fastest one in the mean over those problems (at worst 11 %); examples, 256 x 256 / chosen: 256 x 256 x 256
+// 10.5 / 3.5 us (16 x 16), 1000^3 27.5 / 7.4 (64 x 64), 16 x 1680 x 3992 67.6 / 9.8 (16 x 16), 2414 x 2104 x 2208 49.1 / 36.4
+// (256 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with 128 x 128 tiles.
 struct GemmTile {
   const char *suffix;
   int tileM, tileN, stepK, constant, setup, step, stepMore;
   bool shared;
 };
-constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 1500, 6200, 560, 1250, false},
-                                   {"_t128", 128, 128, 64, 0, 4200, 445, 590, false},
-                                   {"_t128x64", 128, 64, 64, 300, 3300, 290, 375, false},
-                                   {"_t64", 64, 64, 64, 1750, 1350, 187, 246, true},
-                                   {"_t32", 32, 64, 128, 1000, 2200, 244, 383, false},
-                                   {"_t16", 16, 64, 256, 1100, 2000, 418, 633, false}};
+constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 4401, 8420, 610, 708, false},
+                                   {"_t256x128", 256, 128, 64, 1238, 6567, 875, 956, false},
+                                   {"_t128", 128, 128, 64, 1185, 4352, 507, 553, false},
+                                   {"_t128x64", 128, 64, 64, 660, 2993, 270, 391, false},
+                                   {"_t128x64s", 128, 64, 64, 1479, 1683, 378, 311, false},
+                                   {"_t64", 64, 64, 64, 1621, 1810, 267, 278, true},
+                                   {"_t32", 32, 64, 128, 780, 1678, 367, 339, false},
+                                   {"_t16", 16, 64, 256, 837, 2221, 591, 722, false},
+                                   {"_t16x32", 16, 32, 256, 1799, 573, 489, 397, false},
+                                   {"_t16x16", 16, 16, 256, 2285, 485, 379, 282, false}};
 
 // The same for rows that are not 16-byte aligned, fitted to 70 random problems (M 1 .. 4096, N 64 .. 4096, K 64 .. 2048;
 // the choice was the faster tile on every one).  The operator itself is a loop on the vector ALUs there, 4.4 us for

@@ -1165,7 +1165,7 @@ def test_gemm_ragged_tiles(host, orc, stream, M, N, K):
     assert np.max(np.abs(orc.bfloat_to_float(fused)[rows] - ref)) <= 5e-3 * np.max(np.abs(ref)) + 2.0 ** -9
 
 
-@pytest.mark.parametrize("tile", ["", "_t128", "_t128x64", "_t64", "_t32", "_t16"])
+@pytest.mark.parametrize("tile", ["", "_t256x128", "_t128", "_t128x64", "_t128x64s", "_t64", "_t32", "_t16", "_t16x32", "_t16x16"])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (64, 64, 256), (127, 136, 72), (129, 264, 520), (520, 72, 1032)])
 def test_gemm_every_tile_integers_exact(host, orc, stream, tile, M, N, K):
     """Each tile size (\"\": 256 x 256) on shapes below, at and beyond its edges in M, N and K, for every operand
@@ -1246,6 +1246,7 @@ def test_gemm_unaligned_rows(host, orc, stream, tile, M, N, K):
 
 @pytest.mark.parametrize("tile,M,N,K", [("_t128", 260, 392, 136), ("_t128x64", 260, 200, 136), ("_t64", 136, 200, 264),
                                         ("_t32", 104, 136, 264), ("_t16", 40, 200, 520), ("_u128", 259, 391, 135),
+                                        ("_t256x128", 520, 264, 136), ("_t16x32", 40, 104, 520), ("_t16x16", 24, 56, 776),
                                         ("_u64", 135, 199, 263)])
 def test_gemm_tiles_walk_and_any_address(host, orc, stream, tile, M, N, K):
     """The kernels with one tile size on two workgroups that walk all tiles (their LDS and their partial tiles are used
