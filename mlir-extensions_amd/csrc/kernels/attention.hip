@@ -21,17 +21,17 @@
 // plain register loops plus ONE exchange between lane l and l+32 per block of
 // keys.
 //
-// Workgroup = QB query blocks of 32 x KG key groups, one wavefront each: 32, 64, 128 or 256
-// queries of one (batch, head) as (QB, KG) = (1,8), (2,4), (4,2), (8,1) with 512 threads, or 256
+// Workgroup = QB query blocks of 32 x KG key groups, one wavefront each: 64, 128 or 256
+// queries of one (batch, head) as (QB, KG) = (2,4), (4,2), (8,1) with 512 threads, or 256
 // queries as (8,2) with 1024 threads.  Wavefront w takes query block w % QB and every KG-th
-// key tile, group w / QB -- tiles of 64 keys, of 32 (KB = 1 block of 32) with 32 queries, where
-// eight groups of 64-key tiles would leave the ring one stage; partial (m, l, O) of the key
-// groups are merged through LDS at the end.  Every workgroup walks all keys of its head, so K / V traffic from L2 falls with the
+// key tile of 64 keys, group w / QB; partial (m, l, O) of the key groups are merged through LDS
+// at the end.  (32 queries and eight key groups: "every wavefront its own keys" below.)  Every
+// workgroup walks all keys of its head, so K / V traffic from L2 falls with the
 // queries per workgroup; key groups exist to keep all CUs busy on small problems (the
 // reference's 2 x 2 x 4096 x 64 gives one 64-query workgroup per CU) and, in the 1024-thread
 // form, to put four wavefronts on every SIMD (the tiled path needs 114 registers).  The launch
 // says which: N_CTX / gridDim.x queries per workgroup, blockDim.x threads.  K and V blocks of
-// 64 KG (32 queries: 256) keys go from global memory straight into an LDS ring (buffer_load ... lds) of 2, 4 or
+// 64 KG keys go from global memory straight into an LDS ring (buffer_load ... lds) of 2, 4 or
 // 8 stages, up to seven blocks ahead.
 //
 // Arguments: (Q, K, V, Out, sm_scale: f32, ZH: i64, N_CTX: i64)   dims = {ZH, N_CTX}
@@ -50,7 +50,8 @@ namespace {
 
 constexpr int kMaxThreads = 1024; // 8 or 16 wavefronts per workgroup
 constexpr int D = 64;                 // head dimension
-constexpr int kLdsBytes = 128 * 1024;           // the ring: 2 stages of 64 KiB, 4 of 32 KiB or 8 of 16 KiB
+constexpr int kRingBytes = 128 * 1024;          // 2 stages of 64 KiB, 4 of 32 KiB or 8 of 16 KiB
+constexpr int kLdsBytes = 16 * 34 * 64 * 4;     // the ring, and after it the partial results of sixteen wavefronts
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -104,13 +105,67 @@ __device__ __forceinline__ void attention_scalar(const uint16_t *Q, const uint16
   }
 }
 
+// ---- results ---------------------------------------------------------------------------------
+// The partial results of the key groups meet in LDS (whose tiles nobody copies or reads any more), and every wavefront
+// merges its share of them: 8 / KG of the eight groups of four rows that a query block of 32 has.  (One wavefront per
+// query block merging all of it is as fast for two key groups, 8 x 3000 35.0 against 35.8 us, but not for four, 16 x 768
+// 8.93 against 8.74, or eight.)
+template <int QB, int KG>
+__device__ __forceinline__ void merge_and_store(const f32x16 (&o)[2], float m, float l, uint16_t *__restrict__ Out,
+                                                int64_t firstRow, int64_t endRow, char *lds, int wave, int wq, int wk,
+                                                int lane, bool ragged) {
+  constexpr int kSlot = 34 * 64; // floats per wavefront: 32 accumulator rows, four to a vector, m, l
+  constexpr int kUnits = 8 / KG; // of four rows, per wavefront
+  float *all = reinterpret_cast<float *>(lds);
+  __syncthreads(); // the ring is free
+  {
+    float *mine = all + (wq * KG + wk) * kSlot;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) // rows of the accumulator's block u / 4
+      *reinterpret_cast<f32x4 *>(mine + (u * 64 + lane) * 4) =
+          f32x4{o[u >> 2][(u & 3) * 4], o[u >> 2][(u & 3) * 4 + 1], o[u >> 2][(u & 3) * 4 + 2], o[u >> 2][(u & 3) * 4 + 3]};
+    mine[32 * 64 + lane] = m;
+    mine[33 * 64 + lane] = l;
+  }
+  __syncthreads();
+  const int qb = wave / KG, first = wave % KG * kUnits; // the query block and the units this wavefront merges
+  const float *of = all + qb * (KG * kSlot);
+  float a[KG], mAll = -__builtin_inff(), lAll = 0.0f;
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    a[g] = of[g * kSlot + 32 * 64 + lane];
+    mAll = fmaxf(mAll, a[g]);
+  }
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    a[g] = __builtin_amdgcn_exp2f(a[g] - mAll); // a group without a key: 0
+    lAll += of[g * kSlot + 33 * 64 + lane] * a[g];
+  }
+  const float inv = 1.0f / lAll;
+  const int64_t row = firstRow + qb * 32 + (lane & 31);
+#pragma unroll
+  for (int j = 0; j < kUnits; ++j) {
+    const int u = first + j; // lane holds, for its query, d = u*8 + (lane/32)*4 .. +3
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int g = 0; g < KG; ++g)
+      acc += *reinterpret_cast<const f32x4 *>(of + g * kSlot + (u * 64 + lane) * 4) * a[g];
+    f16x4 out4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      out4[e] = static_cast<_Float16>(acc[e] * inv);
+    if (!ragged || row < endRow)
+      *reinterpret_cast<f16x4 *>(Out + row * D + u * 8 + (lane >> 5) * 4) = out4;
+  }
+}
+
 // ---- MFMA path ---------------------------------------------------------------------------
 // QB = 32-query blocks per workgroup, KG = key groups: QB x KG wavefronts (8 or 16).  More query
 // blocks mean fewer workgroups but proportionally less K / V traffic from L2 (every workgroup walks
 // all keys of its head); fewer key groups mean smaller ring stages and therefore a deeper ring.
 // kRagged: N_CTX is not a multiple of the workgroup's 32 QB queries or of its 64 KG-key blocks; the
 // padding logic below is compiled in only then.
-template <int QB, int KG, int KB, bool kRagged, bool kScoresAhead = false>
+template <int QB, int KG, bool kRagged, bool kScoresAhead = false>
 __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
                                                 const uint16_t *__restrict__ V, uint16_t *__restrict__ Out,
                                                 float scale, int64_t N, char *lds) {
@@ -118,10 +173,10 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int kWaves = QB * KG;
-  constexpr int BN = 32 * KB;                      // keys per tile
-  constexpr int kTileBytes = BN * D * 2;           // 4 or 8 KiB
+  constexpr int KB = 2, BN = 32 * KB;              // keys per tile
+  constexpr int kTileBytes = BN * D * 2;           // 8 KiB
   constexpr int kStageBytes = 2 * KG * kTileBytes; // K tiles of all key groups, then their V tiles
-  constexpr int kStages = kLdsBytes / kStageBytes; // 2, 4 or 8
+  constexpr int kStages = kRingBytes / kStageBytes; // 2, 4 or 8
   constexpr int kAhead = kStages - 1;              // blocks in flight ahead of the one being multiplied
   constexpr int kCopies = BN * KG / (8 * kWaves);  // 1 KiB (8-row) copies per wavefront, stage and operand
   const int wq = wave % QB, wk = wave / QB;
@@ -158,6 +213,7 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   // applied on the global side, since a direct copy fixes the lane's LDS position.
   const __amdgpu_buffer_rsrc_t kRsrc = make_rsrc(K + head0 * D, N * D * 2);
   const __amdgpu_buffer_rsrc_t vRsrc = make_rsrc(V + head0 * D, N * D * 2);
+  const __amdgpu_buffer_rsrc_t nothing = make_rsrc(K + head0 * D, 0);
   const int iters = int((N + KG * BN - 1) / (KG * BN));            // key blocks of BN KG keys
   const int lastRows = int(N - int64_t(iters - 1) * (KG * BN));    // keys in the last block: 1 .. BN KG
   const bool raggedKeys = kRagged && lastRows != KG * BN;
@@ -176,21 +232,27 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
     kVoffT[c] = (rowT * D + kc * 8) * 2;
     vVoffT[c] = (rowT * D + vc * 8) * 2;
   }
+  // Blocks past the end: through a descriptor of size zero with four key groups (nothing moves, but the copies count: 4 x
+  // 4096 28.5 -> 28.2 us); the last block again with fewer, whose two query blocks and more per key group hide it, and
+  // which the choice of a descriptor costs more (12 x 1500 20.1, 20.3).
+  constexpr bool kSkip = KG >= 4;
   auto dma_k = [&](int block, int stage) { // keys [BN KG block, BN KG (block + 1)) into ring stage `stage`
     LdsChar *dst = ldsBase + stage * kStageBytes + wave * (kCopies * 1024);
-    const bool tail = raggedKeys && block == iters - 1; // uniform
+    const int b = kSkip ? block : min(block, iters - 1);
+    const bool tail = raggedKeys && b == iters - 1; // uniform
 #pragma unroll
     for (int c = 0; c < kCopies; ++c)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kRsrc, dst + c * 1024, 16, tail ? kVoffT[c] : kVoff[c],
-                                               block * (KG * BN * D * 2), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b < iters ? kRsrc : nothing, dst + c * 1024, 16, tail ? kVoffT[c] : kVoff[c],
+                                               b < iters ? b * (KG * BN * D * 2) : 0, 0, 0);
   };
   auto dma_v = [&](int block, int stage) { // the same keys' rows of V
     LdsChar *dst = ldsBase + stage * kStageBytes + KG * kTileBytes + wave * (kCopies * 1024);
-    const bool tail = raggedKeys && block == iters - 1;
+    const int b = kSkip ? block : min(block, iters - 1);
+    const bool tail = raggedKeys && b == iters - 1;
 #pragma unroll
     for (int c = 0; c < kCopies; ++c)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vRsrc, dst + c * 1024, 16, tail ? vVoffT[c] : vVoff[c],
-                                               block * (KG * BN * D * 2), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b < iters ? vRsrc : nothing, dst + c * 1024, 16, tail ? vVoffT[c] : vVoff[c],
+                                               b < iters ? b * (KG * BN * D * 2) : 0, 0, 0);
   };
 
   // -- LDS read addresses (relative to this wavefront's K / V tile of a stage)
@@ -320,13 +382,12 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
     // The scores of block it + 1 are formed before block `it` goes through the softmax, so the softmax does not wait for
     // the last products of its own scores.  The K reads are still waited for, in front of the products of either
     // order: a wavefront issues in order, and these come first.  K(it + 1) and V(it) are there when block `it` begins;
-    // the copies in flight are pairs of these.  Past the end the last block is fetched again, as below: two K and one V
-    // blocks more on a two-stage ring, 3 on 32 (64 queries, 4096 keys).
+    // the copies in flight are pairs of these.  Past the end as below.
     dma_k(0, 0);
 #pragma unroll
     for (int b = 0; b < kAhead; ++b) {
-      dma_k(min(b + 1, iters - 1), b + 1);
-      dma_v(min(b, iters - 1), b);
+      dma_k(b + 1, b + 1);
+      dma_v(b, b);
     }
     wait_vmcnt<kAhead * 2 * kCopies>(); // K(0) has landed
     __builtin_amdgcn_s_barrier();
@@ -339,8 +400,8 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
       wait_vmcnt<(kAhead - 1) * 2 * kCopies>(); // K(it + 1), V(it) have landed
       __builtin_amdgcn_s_barrier();             // ... everyone's; and everyone is done with K(it), V(it - 1) ...
       __builtin_amdgcn_sched_barrier(0);
-      dma_k(min(it + kStages, iters - 1), cur); // ... whose places these go to
-      dma_v(min(it + kAhead, iters - 1), cur == 0 ? kStages - 1 : cur - 1);
+      dma_k(it + kStages, cur); // ... whose places these go to
+      dma_v(it + kAhead, cur == 0 ? kStages - 1 : cur - 1);
       const int after = cur == kStages - 1 ? 0 : cur + 1;
       scores(next, lds + after * kStageBytes); // (past the last block: of whatever the ring holds, not used)
       attend(s, it, lds + cur * kStageBytes);
@@ -350,12 +411,11 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
       cur = after;
     }
   } else {
-    // The ring always holds kAhead blocks in flight (past the end the last block is simply fetched
-    // again, into stages nobody reads any more), so "block `it` has landed" is one fixed vmcnt.
+    // The ring always holds kAhead blocks in flight (also past the end), so "block `it` has landed" is one fixed vmcnt.
 #pragma unroll
     for (int b = 0; b < kAhead; ++b) {
-      dma_k(min(b, iters - 1), b);
-      dma_v(min(b, iters - 1), b);
+      dma_k(b, b);
+      dma_v(b, b);
     }
     int cur = 0; // ring stage of block `it`
     for (int it = 0; it < iters; ++it) {
@@ -363,8 +423,8 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
       __builtin_amdgcn_s_barrier();             // ... everyone's; and everyone is done reading block it-1
       __builtin_amdgcn_sched_barrier(0);
       const int before = cur == 0 ? kStages - 1 : cur - 1; // the stage block it-1 occupied
-      dma_k(min(it + kAhead, iters - 1), before);
-      dma_v(min(it + kAhead, iters - 1), before);
+      dma_k(it + kAhead, before);
+      dma_v(it + kAhead, before);
       f32x16 s[KB];
       scores(s, lds + cur * kStageBytes);
       attend(s, it, lds + cur * kStageBytes);
@@ -374,7 +434,12 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   wait_vmcnt<0>();
   l += other_half(l); // both key halves of the lane pair
 
-  // -- merge the key groups through LDS: groups 1.. hand (m, l, O^T) to group 0
+  if constexpr (KG >= 4) {
+    merge_and_store<QB, KG>(o, m, l, Out, q0 - wq * 32, head0 + N, lds, wave, wq, wk, lane, kRagged);
+    return;
+  }
+
+  // -- two key groups: group 1 hands (m, l, O^T) to group 0 through LDS
   __syncthreads(); // the ring is free
   constexpr int kSlot = 34 * 64; // floats per (query half, key group): 32 accumulator rows, m, l
   float *xchg = reinterpret_cast<float *>(lds) + wq * (KG - 1) * kSlot;
@@ -424,6 +489,170 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   }
 }
 
+// ---- every wavefront its own keys ------------------------------------------------------------
+// Eight wavefronts on 32 queries; wavefront w takes every eighth 32-key tile.  Nobody else reads its tiles, so it
+// copies them into LDS of its own (a place of 4 KiB for K and one for V, filled again as soon as the fragments are in
+// registers) and waits for its own copies only: no barrier in the loop, and the wavefronts of a SIMD drift apart, so that
+// one's products run under the others' exponentials, where the shared ring keeps all of them in step.  68 KiB of LDS and
+// at most 128 registers let two workgroups share a CU.  Against the 32-query form of attention_tiled that it replaced
+// (1 x 4096, 128 workgroups: 20.0 us) and 64 queries (the others): 1 x 4096 14.8 us, 4 x 2048 14.0 -> 11.0, 8 x 1024 10.0
+// -> 7.6, 4 x 512 7.1 -> 5.9, 4 x 264 7.8 -> 5.2, 256 x 32 7.3 -> 4.3; more than one workgroup on a CU is where it ends
+// (16 x 768 8.75 -> 10.0), which walk twice the keys that 64 queries do.  Bound by the softmax's instructions (about 460
+// cycles of issue per tile, two wavefronts on a SIMD) and, at one wavefront's 8 KiB in flight, by the copies' latency.
+// Sixteen wavefronts, or 64 queries per wavefront, were not faster.
+constexpr int kOwnKeys = 32, kOwnTile = kOwnKeys * D * 2;
+constexpr int kOwnWaves = 8, kOwnLds = kOwnWaves * 34 * 64 * 4; // the partial results; the tiles are 8 KiB per wavefront
+
+template <bool kRagged>
+__device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
+                                                   const uint16_t *__restrict__ V, uint16_t *__restrict__ Out,
+                                                   float scale, int64_t N, char *lds) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int qi = lane & 31, half = lane >> 5;
+  uint32_t bx = blockIdx.x, by = blockIdx.y; // renumbered as in attention_tiled
+  {
+    const uint32_t total = gridDim.x * gridDim.y, launched = by * gridDim.x + bx;
+    if (total % 8 == 0) {
+      const uint32_t logical = (launched & 7) * (total >> 3) + (launched >> 3);
+      by = logical / gridDim.x;
+      bx = logical - by * gridDim.x;
+    }
+  }
+  const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 32;
+  const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
+  const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
+
+  // copies, places and fragment addresses: the layouts of attention_tiled for 32-key tiles
+  const __amdgpu_buffer_rsrc_t kRsrc = make_rsrc(K + head0 * D, N * D * 2), vRsrc = make_rsrc(V + head0 * D, N * D * 2);
+  const __amdgpu_buffer_rsrc_t nothing = make_rsrc(K + head0 * D, 0); // past the last tile: nothing moves, but the copies count
+  int kVoff[4], vVoff[4], kVoffT[4], vVoffT[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int r = c * 8 + (lane >> 3), rT = kRagged ? min(r, lastRows - 1) : r;
+    const int kc = (lane & 7) ^ ((r ^ ((r >> 3) & 3)) & 7), vc = (lane & 7) ^ (((r >> 1) & 1) << 2);
+    kVoff[c] = (r * D + kc * 8) * 2;
+    vVoff[c] = (r * D + vc * 8) * 2;
+    kVoffT[c] = (rT * D + kc * 8) * 2;
+    vVoffT[c] = (rT * D + vc * 8) * 2;
+  }
+  char *own = lds + wave * (2 * kOwnTile); // K, V
+  auto dma_k = [&](int i) {
+    LdsChar *dst = (LdsChar *)own;
+    const int tile = wave + i * kOwnWaves;
+    const bool tail = kRagged && tile == tiles - 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < iters ? kRsrc : nothing, dst + c * 1024, 16, tail ? kVoffT[c] : kVoff[c],
+                                               i < iters ? tile * kOwnTile : 0, 0, 0);
+  };
+  auto dma_v = [&](int i) {
+    LdsChar *dst = (LdsChar *)own + kOwnTile;
+    const int tile = wave + i * kOwnWaves;
+    const bool tail = kRagged && tile == tiles - 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < iters ? vRsrc : nothing, dst + c * 1024, 16, tail ? vVoffT[c] : vVoff[c],
+                                               i < iters ? tile * kOwnTile : 0, 0, 0);
+  };
+  dma_k(0);
+  const int64_t qRow = kRagged ? min(q0 + qi, head0 + N - 1) : q0 + qi;
+  f16x8 qf[4]; // loaded between the first copies: the wait for the keys covers them
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds)
+    qf[ds] = *reinterpret_cast<const f16x8 *>(Q + qRow * D + ds * 16 + half * 8);
+  __builtin_amdgcn_sched_barrier(0);
+  dma_v(0);
+  int kRd[4], vRd[2];
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds)
+    kRd[ds] = qi * 128 + ((((ds * 2 + half) ^ qi ^ ((qi >> 3) & 3)) & 7) << 4);
+  {
+    const int t = lane & 15, blk = (lane >> 4) & 1, row = half * 4 + (t >> 2);
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+      vRd[db] = row * 128 + ((((db ^ ((t >> 3) & 1)) << 2) | (blk << 1) | ((t & 3) >> 1)) * 16) + (t & 1) * 8;
+  }
+  f32x16 o[2];
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      o[db][r] = 0.0f;
+  float m = -__builtin_inff(), l = 0.0f;
+  const float c = scale * 1.44269504088896341f;
+  auto landed = [] { // all but the four youngest copies, of one tile
+    wait_vmcnt<4>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto read_done = [] { // the fragments are in registers: their place may be filled again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  for (int i = 0; i < iters; ++i) {
+    landed(); // K(i); V(i) may be on its way
+    f16x8 kf[4];
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+      kf[ds] = *reinterpret_cast<const f16x8 *>(own + kRd[ds]);
+    read_done();
+    dma_k(i + 1);
+    const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    f32x16 s;
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds], qf[ds], ds == 0 ? zero : s, 0, 0, 0);
+    if (kRagged && wave + i * kOwnWaves == tiles - 1 && lastRows < kOwnKeys) { // uniform over the wavefront
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[r] = (r >> 2) * 8 + half * 4 + (r & 3) < lastRows ? s[r] : -__builtin_inff();
+    }
+    // online softmax, as in attention_tiled; while every score so far is -inf, 0 stands in for the maximum
+    float part[2] = {s[0], s[1]};
+#pragma unroll
+    for (int r = 2; r < 16; ++r)
+      part[r & 1] = fmaxf(part[r & 1], s[r]);
+    const float mRun = fmaxf(m, max_of_halves(fmaxf(part[0], part[1])) * c);
+    const float mNew = mRun == -__builtin_inff() ? 0.0f : mRun;
+    const float alpha = __builtin_amdgcn_exp2f(m - mNew);
+    m = mRun;
+    f16x8 pf[2];
+    float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -mNew));
+      pf[r >> 3][r & 7] = static_cast<_Float16>(p);
+      sum[r & 1] += p;
+    }
+    l = l * alpha + (sum[0] + sum[1]);
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) { // the running max moved for some query of this wavefront
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          o[db][r] *= alpha;
+    }
+    landed(); // V(i); K(i + 1) may be on its way
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        const char *p = own + kOwnTile + vRd[db] + kk * 16 * 128;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p + 8 * 128));
+        const f16x8 vf = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[kk], o[db], 0, 0, 0);
+      }
+    read_done();
+    dma_v(i + 1);
+  }
+  wait_vmcnt<0>();
+
+  merge_and_store<1, kOwnWaves>(o, m, l + other_half(l), Out, q0, head0 + N, lds, wave, 0, wave, lane, kRagged);
+}
+
 // What the tiled path takes, of the arguments and of the launch.
 __device__ __forceinline__ bool attention_shaped(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                                  const uint16_t *Out, float scale, int64_t ZH, int64_t N) {
@@ -448,35 +677,33 @@ extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_f
   const bool even = N_CTX % 256 == 0; // every tiling divides it
   if (shaped && blockDim.x == 512 && gx == (N_CTX + 63) / 64) {
     if (even)
-      attention_tiled<2, 4, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<2, 4, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<2, 4, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<2, 4, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 512 && gx == (N_CTX + 127) / 128) {
     if (even)
-      attention_tiled<4, 2, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<4, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<4, 2, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<4, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 512 && gx == (N_CTX + 255) / 256) {
     if (even)
-      attention_tiled<8, 1, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 1, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<8, 1, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 1, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else if (shaped && blockDim.x == 1024 && gx == (N_CTX + 255) / 256) {
     if (even)
-      attention_tiled<8, 2, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
     else
-      attention_tiled<8, 2, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+      attention_tiled<8, 2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
   } else {
     attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
   }
 }
 
 // One tiling each, for problems whose tilings by the rule above leave CUs idle or run a nearly empty last round
-// (attentionVariant in KernelCatalog.cpp).  32 queries are eight key groups of 32-key tiles; it is the form for few
-// heads, bound by the 1 MiB of K and V (N_CTX 4096) that one CU's copies bring in: 1 x 4096 27.6 -> 20.0 us, 2 x 4096
-// 27.8 -> 21.1.  64 and 128 queries are the forms above with the next block's scores formed ahead: 5 x 3001 24.2 -> 21.9,
-// 8 x 2048 17.4 -> 16.4, 4 x 4096 28.9 -> 27.4.
-template <int QB, int KG, int KB, bool kScoresAhead>
+// (attentionVariant in KernelCatalog.cpp).  64 and 128 queries are the forms above with the next block's scores formed
+// ahead: 5 x 3001 24.2 -> 21.9, 8 x 2048 17.4 -> 16.4, 4 x 4096 28.9 -> 27.4.
+template <int QB, int KG, bool kScoresAhead>
 __device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                                      uint16_t *Out, float scale, int64_t ZH, int64_t N, char *lds) {
   constexpr int64_t kQueries = 32 * QB;
@@ -484,19 +711,28 @@ __device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const ui
       gridDim.x != (N + kQueries - 1) / kQueries)
     attention_scalar(Q, K, V, Out, scale, ZH, N);
   else if (N % 256 == 0)
-    attention_tiled<QB, KG, KB, false, kScoresAhead>(Q, K, V, Out, scale, N, lds);
+    attention_tiled<QB, KG, false, kScoresAhead>(Q, K, V, Out, scale, N, lds);
   else
-    attention_tiled<QB, KG, KB, true, kScoresAhead>(Q, K, V, Out, scale, N, lds);
+    attention_tiled<QB, KG, true, kScoresAhead>(Q, K, V, Out, scale, N, lds);
 }
 
-#define IMEX_ATTENTION_TILING(QUERIES, QB, KG, KB, AHEAD)                                                              \
+#define IMEX_ATTENTION_TILING(QUERIES, QB, KG, AHEAD)                                                                  \
   extern "C" __global__ __launch_bounds__(QB *KG *kWave) void imex_flash_attention_fwd_f16_q##QUERIES(                \
       const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH,             \
       int64_t N_CTX) {                                                                                                \
     __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];                                                      \
-    attention_one_tiling<QB, KG, KB, AHEAD>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);                                  \
+    attention_one_tiling<QB, KG, AHEAD>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);                                      \
   }
-IMEX_ATTENTION_TILING(32, 1, 8, 1, true)
-IMEX_ATTENTION_TILING(64, 2, 4, 2, true)
-IMEX_ATTENTION_TILING(128, 4, 2, 2, true)
-IMEX_ATTENTION_TILING(256, 8, 2, 2, false)
+extern "C" __global__ __launch_bounds__(kOwnWaves *kWave, 4) void imex_flash_attention_fwd_f16_q32(
+    const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
+  __shared__ __attribute__((aligned(16))) char lds[kOwnLds];
+  if (!attention_shaped(Q, K, V, Out, sm_scale, ZH, N_CTX) || blockDim.x != kOwnWaves * kWave || gridDim.x != (N_CTX + 31) / 32)
+    attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
+  else if (N_CTX % 32 == 0)
+    attention_own_keys<false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+  else
+    attention_own_keys<true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+}
+IMEX_ATTENTION_TILING(64, 2, 4, true)
+IMEX_ATTENTION_TILING(128, 4, 2, true)
+IMEX_ATTENTION_TILING(256, 8, 2, false)

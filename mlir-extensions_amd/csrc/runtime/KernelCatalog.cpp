@@ -371,20 +371,22 @@ const char *transposeVariant(const Entry *e, const int64_t *dims) {
 
 // The operator's own launch takes the most queries per workgroup that give every CU a workgroup.  That leaves CUs idle
 // where 64 queries are too many for it, and runs a second, partly empty round where the next larger tiling would do in
-// one.  A tiling costs its rounds of 256 workgroups, in microseconds at 4096 keys.  1 x 4096 27.6 -> 20.0 us (32 queries),
-// 12 x 1500 27.0 -> 20.3 (128), 6 x 4096 53.1 -> 42.5 (128), 12 x 4096 85.1 -> 68.3 (256).  Heads of fewer than 768 keys
-// stay (16 x 512 7.4 us, 7.9 with 32 queries), as do problems that fill more than one round with 256 queries; the 64
-// queries that form scores ahead gain from 2048 keys on (8 x 2048 17.4 -> 16.4, 16 x 1024 10.4 -> 10.9).
+// one.  A tiling costs its rounds of 256 workgroups, in microseconds at 4096 keys: 32 queries wherever they fit one round
+// (1 x 4096 27.6 -> 14.8 us, 8 x 1024 10.0 -> 7.6, 16 x 512 7.1 -> 6.0, 4 x 64 6.0 -> 4.2; at 264 workgroups 24 x 333
+// 7.6, 7.7, at 288 48 x 192 6.2, 7.1), 128 where 64 take two (12 x 1500 27.0 -> 20.1, 6 x 4096 53.1 -> 42.5, 64 x 320 14.2
+// -> 9.2, 200 x 128 11.6 -> 7.0), 256 where 128 take two (12 x 4096 85.1 -> 68.3, 100 x 333 19.1 -> 14.1).  Of the two
+// forms with 64 queries the one that forms scores ahead from 768 keys on (16 x 1000 11.1 -> 10.7, 8 x 2048 17.4 -> 16.0;
+// 16 x 700 9.0, 9.2).  Problems that fill more than one round with 256 queries stay.
 struct Tiling {
   const char *suffix;
   int64_t queries;
   double cost;
 };
-constexpr Tiling kTilings[] = {{"_q32", 32, 22.0}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
+constexpr Tiling kTilings[] = {{"_q32", 32, 15.5}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
 
 const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
   auto workgroups = [&](int64_t queries) { return (N + queries - 1) / queries * ZH; };
-  if (N < 768 || N >= (int64_t(1) << 24) || ZH == 0 || ZH > 256 || workgroups(256) > 256)
+  if (N <= 0 || N >= (int64_t(1) << 24) || ZH == 0 || ZH > 256 || workgroups(256) > 256)
     return e->name;
   int64_t own = 256; // as imexHipKernelLaunchShape
   while (own > 64 && workgroups(own) < 256)
@@ -398,7 +400,7 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
       least = cost;
     }
   }
-  if (best->queries == own && (own != 64 || N < 2048))
+  if (best->queries == own && (own != 64 || N < 768))
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s%s", e->name, best->suffix);

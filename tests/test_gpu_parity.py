@@ -917,6 +917,37 @@ def test_flash_attention_one_tiling(host, orc, stream, queries, zh, n_ctx):
     assert attention_close(out[rows], orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows), orc)
 
 
+@pytest.mark.parametrize("zh,n_ctx,tiling", [
+    (1, 31, "_q32"), (1, 32, "_q32"), (7, 225, "_q32"), (256, 32, "_q32"), (16, 512, "_q32"), (32, 256, "_q32"),  # to 256
+    (4, 2048, "_q32"), (1, 3169, "_q32"), (17, 500, ""), (257, 32, ""), (16, 768, "_q64"), (48, 333, "_q128"),
+    (100, 333, "_q256"), (2, 8000, "_q64")])
+def test_flash_attention_tiling_by_size(host, orc, stream, zh, n_ctx, tiling):
+    """The tiling that the catalogue takes on both sides of its lines; wavefronts without a tile, with one that is ragged,
+    with several; infinite keys (scores of -inf for whole tiles) and values beside it: the rows behind Out untouched."""
+    name = "imex_flash_attention_fwd_f16"
+    assert host.variant(name, [zh, n_ctx]) == name + tiling
+    n = zh * n_ctx
+    q, k, v = (orc.fill_uniform(n * 64, "f16", seed, lo, hi).reshape(n, 64)
+               for seed, lo, hi in ((90, 0.25, 2), (91, -2, 2), (92, -1, 1)))
+    head = np.arange(n).reshape(zh, n_ctx)[-1]
+    k[head[:-1][head[:-1] % 3 != 0], 5] = 0xfc00  # -inf times a positive query
+    v[head[0], 9] = 0x7c00
+    rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 200)), head[:40], head[-40:]]))
+    guard = np.full((n + 256, 64), 0x7e01, np.uint16)
+    d_q, d_k, d_v, d_o = (stream.to_device(t) for t in (q, k, v, guard))
+    say("attention %dx%d by size" % (zh, n_ctx))
+    stream.launch(name, [zh, n_ctx], [d_q, d_k, d_v, d_o, 0.5, zh, n_ctx])
+    stream.wait()
+    out = stream.from_device(d_o, (n + 256, 64), np.uint16)
+    for p in (d_q, d_k, d_v, d_o):
+        stream.free(p)
+    assert np.all(out[n:] == 0x7e01), "wrote behind Out"
+    got, ref = orc.half_to_float(out[rows]), orc.half_to_float(orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows))
+    ok = np.isfinite(ref)
+    assert np.array_equal(np.isfinite(got), ok) and np.all(ok[:, :9]) and np.all(ok[:, 10:])
+    assert np.max(np.abs(got[ok] - ref[ok])) <= 2.0 ** -10 + 2.0 ** -11 * np.max(np.abs(ref[ok]))
+
+
 @pytest.mark.parametrize("queries", [32, 64, 128, 256])
 def test_flash_attention_one_tiling_at_any_address(host, orc, stream, queries):
     """A tensor that starts one element behind a 16-byte boundary takes the reference loop of the same kernel."""
