@@ -126,8 +126,9 @@ template <typename T, bool kStrided, int TR, int BK> struct SmallOperand {
   }
 };
 
-template <int TMv, int TNv, int WMCv, int WNCv, int KGv, int Sv> struct SmallShape {
+template <int TMv, int TNv, int WMCv, int WNCv, int KGv, int Sv, bool kRefillv = false> struct SmallShape {
   static constexpr int TM = TMv, TN = TNv, WMC = WMCv, WNC = WNCv, KG = KGv, S = Sv;
+  static constexpr bool kRefill = kRefillv; // a slot is filled again in the step whose fragments were the last read of it
   static constexpr int BK = 32 * KG;
   static constexpr int FI = TM / WMC / 16, FJ = TN / WNC / 16;
   static constexpr int kStageBytes = (TM + TN) * BK * 2;
@@ -235,18 +236,20 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
     read_b(p, slot);
   };
 #pragma unroll
-  for (int t = 0; t < S - 1; ++t)
+  for (int t = 0; t < (P::kRefill ? S : S - 1); ++t)
     dma(t, t);
-  wait_vmcnt<(S - 2) * kCopies>();
+  wait_vmcnt<(P::kRefill ? S - 1 : S - 2) * kCopies>();
   __builtin_amdgcn_s_barrier();
   IMEX_FENCE();
   read(0, 0);
   // Step t: everybody's fragments of step t - 1 were in registers before the barrier of that step, so its slot takes slab
-  // t + S - 1; slab t + 1 has landed at the barrier of this one.
+  // t + S - 1; slab t + 1 has landed at the barrier of this one.  With kRefill the slot of step t takes slab t + S behind
+  // the barrier of step t, at which everybody's fragments of it are in registers.
   int cur = 0; // slot of step t
   auto step = [&](int p, int t) {
     const int nxt = cur + 1 == S ? 0 : cur + 1, free = cur == 0 ? S - 1 : cur - 1;
-    dma(t + S - 1, free);
+    if constexpr (!P::kRefill)
+      dma(t + S - 1, free);
     wait_vmcnt<(S - 2) * kCopies>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -266,6 +269,8 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
       }
     } else {
       read(p ^ 1, nxt);
+      if constexpr (P::kRefill)
+        dma(t + S, cur);
       IMEX_FENCE();
 #pragma unroll
       for (int j = 0; j < FJ; ++j)

@@ -12,16 +12,19 @@ using namespace imexhip_gemm;
 // The last number is the ring's stages.  More of them do not make a K step shorter -- a CU's requests beyond its L2 are
 // what bounds the small tiles (16 x 16 on N = 1680: 0.36 us per 256 k with 3, 4, 8 and 9 stages) -- but the first result
 // later (K = 1024: 3.4, 3.7, 3.8, 4.0 us), so: what lets workgroups share a CU, or what hides the latency of a step.
+// "true" refills a slot in the step that has its fragments in registers, a step sooner than the rest, and so does with a
+// stage less: 128 x 128 (4 stages before) 1616 x 1760 x 3616 33.2 -> 31.9 us, 1064 x 2200 x 424 9.2 -> 8.9; 64 x 64 (5
+// before) 912 x 944 x 520 5.33 -> 5.14, 1000 x 1592 x 1168 the same; 128 x 64 and narrower tiles gain nothing or lose 1 %.
 //   256 x 128  between 128 x 128 tiles for two rounds and 256 x 256 for less than half the chip: 2414 x 2104 x 2208 44.4 us
 //              with 128 x 128, 36.4 so; 892 x 4768 x 3096 60.6 / 47.1; 1704 x 2648 x 4088 A^T 97.6 (64 x 64) / 59.3
 //   128 x 64 s two workgroups on a CU for problems of more than one round: 1542 x 4000 x 720 32.8 -> 26.6
 //   16 x 32, 16 x 16  few rows: a CU gets 40 .. 60 GB/s from beyond its L2, so narrow outputs bring more CUs to the weights:
 //              16 x 1680 x 3992 13.8 us with 16 x 64, 9.8 so; 5 x 2200 x 1160 5.8 -> 4.0
 using Tile256x128 = SmallShape<256, 128, 2, 2, 2, 3>;
-using Tile128 = SmallShape<128, 128, 2, 2, 2, 4>;
+using Tile128 = SmallShape<128, 128, 2, 2, 2, 3, true>;
 using Tile128x64 = SmallShape<128, 64, 2, 2, 2, 4>;
 using Tile128x64Shared = SmallShape<128, 64, 2, 2, 2, 3>;
-using Tile64 = SmallShape<64, 64, 2, 2, 2, 5>;
+using Tile64 = SmallShape<64, 64, 2, 2, 2, 4, true>;
 using Tile32 = SmallShape<32, 64, 1, 2, 4, 4>;
 using Tile16 = SmallShape<16, 64, 1, 1, 8, 3>;
 using Tile16x32 = SmallShape<16, 32, 1, 1, 8, 3>;
