@@ -78,7 +78,8 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
     bool first = true;
     for (uint32_t w = blockIdx.x; w < blocks; w += gridDim.x) {
       // Workgroup w runs on XCD w % 8: the XCDs take contiguous shares of the segments.  (The last block of columns
-      // starts early enough to be whole; columns that two workgroups share get the same value from both.)
+      // starts early enough to be whole.  The columns that it shares with the block before it are stored by that one only,
+      // and what it reads of them is not used: so the result may lie in a row of the matrix itself.)
       const uint32_t xcd = w % 8, block = xcd * (blocks / 8) + min(xcd, blocks % 8) + w / 8;
       const int64_t c0 = min(block * kCols, static_cast<uint32_t>(cols) - kCols);
       if (wave < kWorkers) {
@@ -225,7 +226,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
           }
         }
         __builtin_amdgcn_s_setprio(0);
-        if (lane < kCols)
+        if (lane < kCols && c0 + lane >= int64_t(block) * kCols)
           E::put(out, c0 + lane, acc);
       }
       first = false;

@@ -812,6 +812,34 @@ def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra
             stream.free(p)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,segments,extra", [(300, 3, 1), (140, 300, -3), (130, 514, 7), (70, 1030, 5)])
+def test_column_chains_in_place(host, orc, stream, dtype, rows, segments, extra):
+    """A result that lies in the first or the last row of its own matrix.  On one workgroup the last block of columns, which
+    starts inside the one before it, is walked after that one's sums are stored: they must not come back into its own."""
+    width = 4 if dtype == "f32" else 2
+    cols = segments * (32 // width) + extra
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    a = orc.fill_uniform(rows * cols, dtype, 55, -5.0, 5.0).reshape(rows, cols)
+    b = orc.fill_uniform(rows * cols, dtype, 56, 0.01, 40.0).reshape(rows, cols)
+    d_a, d_b = stream.to_device(a), stream.to_device(b)
+    want = {"input_fusion": narrow(orc.input_fusion_f32(wide(a), wide(b))), "reduce_outer": narrow(orc.reduce_outer_f32(wide(a), 0.25))}
+    for grid in ((1, 1, 1), None):
+        for row in (0, rows - 1):
+            out = host.Ptr(d_a + row * cols * width)
+            for op, args in (("input_fusion", [d_a, d_b, out, rows, cols]), ("reduce_outer", [d_a, out, rows, cols, 0.25])):
+                say("%s %s %dx%d, row %d, grid %s" % (op, dtype, rows, cols, row, grid))
+                stream.copy(d_a, a.ctypes.data, a.nbytes)
+                stream.launch("imex_%s_%s_tall" % (op, dtype), [rows, cols], args, grid=grid)
+                stream.wait()
+                got = stream.from_device(d_a, a.shape, a.dtype)
+                assert np.array_equal(got[row], want[op]), (op, row, grid)
+                assert np.array_equal(np.delete(got, row, 0), np.delete(a, row, 0)), (op, row, grid)
+    for p in (d_a, d_b):
+        stream.free(p)
+
+
 # ============================ flash attention ===============================
 def attention_close(got_bits, ref_bits, orc):
     """The reference checks its kernel with allclose (atol 1e-4, rtol 1e-3) on a constant
