@@ -24,8 +24,10 @@
 // block (320,1,1), grid ceil(cols / 4); from 2048 rows and 128 row segments of 128 bytes on block (576,1,1),
 // grid ceil(cols * element bytes / 128); otherwise block (256,1,1), grid ceil(cols / c), a workgroup per
 // block of c = 64 .. 8 columns (the widest that leaves 512 workgroups).  A launch with 256 lanes always gets
-// the last form.  The _tall forms: block (320,1,1) up to 256 segments of 32 bytes in a row, else (576,1,1); grid a
-// workgroup per segment of 32, 64 or 128 bytes (chain_lanes in column_chain.h).  Workgroups stride, so any grid is correct.
+// the last form, one with fewer a lane per column.  The _tall forms, by the 32-byte segments of a row (chain_lanes in
+// column_chain.h): up to 256 block (320,1,1), up to 1024 (576,1,1), beyond that (320,1,1); grid a workgroup per segment
+// of 32, 64 (257 .. 512) or 128 bytes.  With any other block they go as the forms with 256 lanes or fewer.  Workgroups
+// stride, so any grid is correct.
 
 #include "column_chain.h"
 #include "device_common.h"
@@ -102,8 +104,8 @@ template <int kMantissa> struct Logarithms {
 
   // by all threads of the workgroup; readable after a barrier
   __device__ __forceinline__ void stage() {
-    if (threadIdx.x < 16)
-      entry[threadIdx.x] = kLogfTable[threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < 16; i += blockDim.x)
+      entry[i] = kLogfTable[i];
     if constexpr (kMantissa != 0)
       for (uint32_t m = threadIdx.x; m < 1u << kMantissa; m += blockDim.x)
         mantissa[m] = logf_libm_core(0x3f800000u | m << (23 - kMantissa), kLogfTable);
@@ -255,6 +257,19 @@ __device__ __forceinline__ float add_in_row_order(float acc, const float *t, int
   for (; r < n; ++r)
     acc = acc + t[r * stride];
   return acc;
+}
+
+// A lane per column: for launches with fewer lanes than the tiles below are filled by.
+template <Dt D, typename Logs>
+__device__ __forceinline__ void input_fusion_by_element(const void *__restrict__ a, const void *__restrict__ b,
+                                                        void *__restrict__ out, int64_t rows, int64_t cols, const Logs &logs) {
+  using E = Elem<D>;
+  for (int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; c < cols; c += int64_t(gridDim.x) * blockDim.x) {
+    float acc = 0.0f;
+    for (int64_t r = 0; r < rows; ++r)
+      acc = acc + input_chain(E::get(a, r * cols + c), E::get(b, r * cols + c), logs);
+    E::put(out, c, acc);
+  }
 }
 
 template <Dt D, int kCols, int kTileElems = ::kTileElems, typename Logs>
@@ -585,7 +600,7 @@ __device__ __forceinline__ void input_fusion_chains(const void *__restrict__ a, 
 }
 
 // Four workers for segments of 32 bytes, eight for 64 (wide_chain_workers() for 128).  Other launches, and what the chains
-// do not take, go by blocks of columns.
+// do not take, go by blocks of columns, or a lane per column.
 template <Dt D>
 __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, const void *__restrict__ b,
                                                   void *__restrict__ out, int64_t rows, int64_t cols) {
@@ -596,7 +611,10 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
   if (!chains_take<D>(rows, cols) || int(blockDim.x) != (workers + 1) * kWave) {
     logs.stage();
     __syncthreads();
-    input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
+    if (blockDim.x < kThreads)
+      input_fusion_by_element<D>(a, b, out, rows, cols, logs);
+    else
+      input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 4) {
     input_fusion_chains<D, 4, 4>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 8) {
@@ -621,6 +639,10 @@ __device__ __forceinline__ void input_fusion(const void *__restrict__ a, const v
   __shared__ __attribute__((aligned(16))) float tile[2 * kStreamTileFloats];
   logs.stage();
   __syncthreads();
+  if (blockDim.x < kThreads) {
+    input_fusion_by_element<D>(a, b, out, rows, cols, logs);
+    return;
+  }
   // The launch says which form: 576 or 320 lanes ask for a streaming one, which needs whole aligned vectors.
   const bool vectors = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
                        cols % Elem<D>::kPerVec == 0;

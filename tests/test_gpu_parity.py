@@ -813,6 +813,32 @@ def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(150, 41), (130, 2100), (40, 5000), (129, 3)])
+def test_input_fusion_with_any_block(host, orc, stream, dtype, rows, cols):
+    """Launches with fewer lanes than a form's tiles are filled by, with a number that no form asks for, and on two
+    workgroups: the oracle's bits, also for the numbers that libm does not send down its main path."""
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    a = orc.fill_uniform(rows * cols, dtype, 57, -5.0, 5.0).reshape(rows, cols)
+    b = orc.fill_uniform(rows * cols, dtype, 58, 0.01, 40.0).reshape(rows, cols)
+    b[rows // 2, :2] = narrow(np.float32([0.0, np.inf]))
+    want = narrow(orc.input_fusion_f32(wide(a), wide(b)))
+    d_a, d_b, d_out = stream.to_device(a), stream.to_device(b), stream.alloc(cols * a.itemsize)
+    junk = orc.fill_uniform(cols, dtype, 59, 100.0, 200.0)
+    for form in ("", "_tall"):
+        for lanes in (1, 8, 64, 192, 255, 384, 512):
+            for grid in (None, (2, 1, 1)):
+                name = "imex_input_fusion_" + dtype + form
+                stream.copy(d_out, junk.ctypes.data, junk.nbytes)
+                stream.launch(name, [rows, cols], [d_a, d_b, d_out, rows, cols], grid=grid, block=(lanes, 1, 1))
+                stream.wait()
+                got = stream.from_device(d_out, (cols,), a.dtype)
+                assert np.array_equal(got, want), (name, lanes, grid)
+    for p in (d_a, d_b, d_out):
+        stream.free(p)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,segments,extra", [(300, 3, 1), (140, 300, -3), (130, 514, 7), (70, 1030, 5)])
 def test_column_chains_in_place(host, orc, stream, dtype, rows, segments, extra):
     """A result that lies in the first or the last row of its own matrix.  On one workgroup the last block of columns, which
