@@ -608,7 +608,7 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
   __shared__ Logarithms<kMantissaOf<D>> logs;
   const int64_t segments = (cols * Elem<D>::kBytes + 31) / 32;
   const int lanes = chain_lanes(segments), workers = lanes == 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
-  if (!chains_take<D>(rows, cols) || int(blockDim.x) != (workers + 1) * kWave) {
+  if (!chains_take<D>(rows, cols) || cols * Elem<D>::kBytes < 32 || int(blockDim.x) != (workers + 1) * kWave) {
     logs.stage();
     __syncthreads();
     if (blockDim.x < kThreads)

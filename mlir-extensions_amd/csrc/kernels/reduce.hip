@@ -459,11 +459,11 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16_de
 // `outer` dependent additions whatever is done, 2.7 ns each here.  f32 8192 x 4096: 980 us in the plain form, 45.2 with a
 // 32-bit LDS read for every addition, 36.1 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 14.3;
 // bf16 8192 x 4096 58.0 -> 26.9, where the adder widened as well; f16 2000 x 1001 16.6 -> 8.4, 500 x 20000 9.5 -> 5.9.
-template <io::Dt D, int kLanes, int kWorkers>
+template <io::Dt D, int kLanes, int kWorkers, bool kShort = false>
 __device__ __forceinline__ void reduce_outer_chains(const void *in, void *out, int64_t outer, int64_t inner, float init, float *lds) {
   using C = ColumnChain<D, 1, kLanes, kWorkers>;
   using E = io::Elem<D>;
-  C::run(in, nullptr, out, outer, inner, init, lds, [] {}, [](const typename C::Raw(&v)[1][4], float(&f)[4][C::kPer]) {
+  C::template run<kShort>(in, nullptr, out, outer, inner, init, lds, [] {}, [](const typename C::Raw(&v)[1][4], float(&f)[4][C::kPer]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -487,6 +487,8 @@ __device__ __forceinline__ void reduce_outer_tall(const void *in, void *out, int
   const int lanes = chain_lanes(segments), workers = lanes == 16 ? wide_chain_workers(segments) : 4;
   if (!chains_take<D>(outer, inner) || int(blockDim.x) != (workers + 1) * kWave)
     reduce_outer_by_element<D>(in, out, outer, inner, init);
+  else if (inner * io::Elem<D>::kBytes < 8)
+    reduce_outer_chains<D, 4, 4, true>(in, out, outer, inner, init, lds);
   else if (lanes == 4)
     reduce_outer_chains<D, 4, 4>(in, out, outer, inner, init, lds);
   else if (lanes == 8)

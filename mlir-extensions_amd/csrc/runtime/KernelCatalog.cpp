@@ -320,7 +320,8 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
 //          1408680: 13.0, 13.5; f16 15 x 2283888: 18.3, 12.6);
 //   tall   a launch, a slice's share of the chain, and what a CU pays for further workgroups; 5.6 TB/s at most;
 //   deep   a slice costs its share of sixteen slices' latency, which its bytes hide little of; 7.3 (6.0) TB/s at most.
-// 8192 x 4096 f32: plain 980, tall 36, deep 520 us; 568 x 197848: tall 102, deep 66; bf16 389 x 129280: 30, 32.
+// 8192 x 4096 f32: plain 980, tall 37, deep 540 us; 568 x 197848: tall 102, deep 66; bf16 389 x 129280: 30, 32.  Below 64
+// outputs (1 .. 15, 8 .. 10^5 slices) tall is never slower than deep by more than 0.1 us: 64 x 4 both 3.3, 256 x 4 3.3 / 8.5.
 const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const bool f32 = e->shape == Shape::ReduceOuter;
   const int64_t perVec = f32 ? 4 : 8, slice = inner * (f32 ? 4 : 2);
@@ -335,7 +336,7 @@ const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const double tall = 3.04 + std::max(0.77 * more + double(outer) * step * (1.0 + 1.63 * more), bytes / 5.6e6);
   const double wait = double(outer) * (vec ? 0.0517 : f32 ? 0.0220 : 0.0143), move = bytes / (vec ? 7.35e6 : 6.04e6);
   const double deep = 2.61 + std::max(wait, move) + (vec ? 0.72 : 0.55) * std::min(wait, move);
-  const bool chains = slice >= 32 && slice < int64_t(1) << 22 && outer < int64_t(1) << 31; // chains_take in column_chain.h
+  const bool chains = bytes >= 8.0 && slice < int64_t(1) << 22 && outer < int64_t(1) << 31; // chains_take in column_chain.h
   char name[96];
   snprintf(name, sizeof name, "%s%s", e->name, chains && tall < 0.96 * deep ? "_tall" : "_deep");
   return find(name)->name;

@@ -839,6 +839,35 @@ def test_input_fusion_with_any_block(host, orc, stream, dtype, rows, cols):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cols", range(1, 17))
+def test_reduce_outer_narrow_rows(host, orc, stream, dtype, cols):
+    """Rows of less than a 32-byte segment, down to one element: by the catalogue's choice, which takes the chains for tall
+    ones, and by the chains themselves, with matrices of less than 8 bytes, lanes that start inside another's columns, loads
+    that run past a row and the matrix's end in the middle of a tile and behind it; on and off the 16-byte grid; the
+    oracle's bits, and nothing written beside them."""
+    name, width = "imex_reduce_outer_" + dtype, 4 if dtype == "f32" else 2
+    assert host.variant(name, [8192, cols]) == name + "_tall"
+    for rows in (1, 2, 3, 5, 255, 256, 257, 258, 259, 700, 8195):
+        x = orc.fill_uniform(rows * cols, dtype, 93, -1.0, 1.0)
+        want = orc.reduce_outer_f32((x if dtype == "f32" else orc.to_float(x, dtype)).reshape(rows, cols), 0.25)
+        want = want if dtype == "f32" else orc.from_float(want, dtype)
+        for shift in (0, 1):
+            # NaN in front of the matrix and behind it: what is read past its ends must not be added
+            nan = np.full(8, np.nan, np.float32) if dtype == "f32" else np.full(8, 0x7fff, np.uint16)
+            d_in = stream.to_device(np.concatenate([nan[:shift], x, nan]))
+            fill = np.full(cols + 8, 3, x.dtype)
+            for form in ("", "_tall"):
+                d_out = stream.to_device(fill)
+                stream.launch(name + form, [rows, cols], [host.Ptr(d_in + shift * width), host.Ptr(d_out + shift * width), rows, cols, 0.25])
+                stream.wait()
+                got = stream.from_device(d_out, fill.shape, fill.dtype)
+                stream.free(d_out)
+                assert np.array_equal(got[shift:shift + cols], want), (name + form, rows, shift)
+                assert np.all(got[:shift] == 3) and np.all(got[shift + cols:] == 3), (name + form, rows, shift)
+            stream.free(d_in)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,segments,extra", [(300, 3, 1), (140, 300, -3), (130, 514, 7), (70, 1030, 5)])
 def test_column_chains_in_place(host, orc, stream, dtype, rows, segments, extra):
     """A result that lies in the first or the last row of its own matrix.  On one workgroup the last block of columns, which
