@@ -30,10 +30,16 @@ __device__ __forceinline__ int chain_lanes(int64_t segments) { return segments <
 // four where it gets more of them, so that these share it (128 x 32768: 6.5 with eight, 3.9 with four).
 __device__ __forceinline__ int wide_chain_workers(int64_t segments) { return segments <= 4 * 256 ? 8 : 4; }
 
-// What the chains take: 8 bytes or more, and a tile's rows (256 at most) within 32-bit offsets of its first one.
+// What the chains take: a tile's rows (256 at most) within 32-bit offsets of its first one.
 template <io::Dt D> __device__ __forceinline__ bool chains_take(int64_t rows, int64_t cols) {
-  return cols > 0 && cols * io::Elem<D>::kBytes < int64_t(1) << 22 && rows < int64_t(1) << 31 &&
-         rows * cols * io::Elem<D>::kBytes >= 8;
+  return cols > 0 && cols * io::Elem<D>::kBytes < int64_t(1) << 22 && rows < int64_t(1) << 31;
+}
+
+// blockDim.x of a launch by workgroups that are all of one size, as one scalar load of the kernel's hidden arguments (whose
+// layout is the code object's, version 5): blockDim.x itself is a vector load that every wavefront waits for before it
+// knows its form, 0.2 .. 0.3 us of a launch (fused chain of bf16 26 x 880 3.54 -> 3.28 us, f16 105 x 328 4.15 -> 3.87).
+__device__ __forceinline__ int lanes_launched() {
+  return ((const uint32_t *)__builtin_amdgcn_implicitarg_ptr())[3] & 0xffff;
 }
 
 // kInputs matrices; kLanes lanes of a worker cover a row's segment with 8 bytes each; kWorkers wavefronts of workers.
@@ -45,6 +51,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   static constexpr int kRowsPerWave = 4 * (kWave / kLanes);     // rows of a tile that one worker wavefront takes
   static constexpr int kTileRows = kWorkers * kRowsPerWave;
   static constexpr int kThreads = (kWorkers + 1) * kWave;
+  static constexpr bool kNarrow = kInputs == 1 && kLanes == 4; // takes rows of less than a segment too
   // Floats from one column of a tile to the next, and where a column keeps its rows: four rows (a "quad") are 16 bytes,
   // and quad q of a column that lane group j wrote is at place q ^ swizzle(j) within its four.  128-bit LDS accesses
   // are served sixteen lanes at a time over 64 banks.  The adder's sixteen lanes read one quad of sixteen columns:
@@ -75,7 +82,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   template <bool kShort = false, typename Prologue, typename Eval>
   static __device__ __forceinline__ void run(const void *a, const void *b, void *out, int64_t rows, int64_t cols, float init,
                                              float *lds, Prologue prologue, Eval eval) {
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t pitch = static_cast<uint32_t>(cols * E::kBytes);
     const int tiles = static_cast<int>((rows + kTileRows - 1) / kTileRows);
     const int lastRows = static_cast<int>(rows - int64_t(tiles - 1) * kTileRows); // of the last tile
@@ -86,10 +93,16 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
       // starts early enough to be whole.  The columns that it shares with the block before it are stored by that one only,
       // and what it reads of them is not used: so the result may lie in a row of the matrix itself.)
       const uint32_t xcd = w % 8, block = xcd * (blocks / 8) + min(xcd, blocks % 8) + w / 8;
-      const int64_t c0 = min(block * kCols, static_cast<uint32_t>(max(cols, int64_t(kCols))) - kCols);
+      const int64_t c0 = min(block * kCols, static_cast<uint32_t>(kNarrow ? max(cols, int64_t(kCols)) : cols) - kCols);
+      // (The compiler must not take a role's addresses out of this loop: they would stay in registers under the other role,
+      // 16 of the f32 sums' 109 and 13 of the bf16 fused chain's 135.  Four workgroups of five wavefronts on a CU leave a
+      // wavefront 96 -- f32 sums of 128 x 32768 8.0 us with three of them, 5.7 so -- and three 128: fused chain of f16 1606 x
+      // 17080 48.5, 33.8; bf16 382 x 47034 21.7, 16.9.)
+      int lane = threadIdx.x & (kWave - 1);
+      asm volatile("" : "+v"(lane));
       if (wave < kWorkers) {
         const int quad = wave * (kWave / kLanes) + lane / kLanes; // rows 4 quad .. 4 quad + 3 of a tile
-        const int col = kShort ? 0 : min((lane % kLanes) * kPer, static_cast<int>(cols) - kPer);
+        const int col = kShort ? 0 : kNarrow ? min((lane % kLanes) * kPer, static_cast<int>(cols) - kPer) : (lane % kLanes) * kPer;
         const char *base[2] = {static_cast<const char *>(a) + c0 * E::kBytes, static_cast<const char *>(b) + c0 * E::kBytes};
         const uint32_t at = static_cast<uint32_t>(4 * quad) * pitch;
         const int64_t end = rows * int64_t(pitch) - 8; // kShort: the last address of a load
@@ -242,7 +255,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
           }
         }
         __builtin_amdgcn_s_setprio(0);
-        if (lane < kCols && c0 + lane >= int64_t(block) * kCols && c0 + lane < cols)
+        if (lane < kCols && c0 + lane >= int64_t(block) * kCols && (!kNarrow || lane < cols))
           E::put(out, c0 + lane, acc);
       }
       first = false;

@@ -102,12 +102,12 @@ template <int kMantissa> struct Logarithms {
   LogfEntry entry[16];
   double mantissa[kMantissa ? 1 << kMantissa : 1];
 
-  // by all threads of the workgroup; readable after a barrier
+  // by all threads of the workgroup, 16 or more; readable after a barrier
   __device__ __forceinline__ void stage() {
-    for (uint32_t i = threadIdx.x; i < 16; i += blockDim.x)
-      entry[i] = kLogfTable[i];
+    if (threadIdx.x < 16)
+      entry[threadIdx.x] = kLogfTable[threadIdx.x];
     if constexpr (kMantissa != 0)
-      for (uint32_t m = threadIdx.x; m < 1u << kMantissa; m += blockDim.x)
+      for (uint32_t m = threadIdx.x; m < 1u << kMantissa; m += lanes_launched())
         mantissa[m] = logf_libm_core(0x3f800000u | m << (23 - kMantissa), kLogfTable);
   }
   // kOrdinary: the caller has checked logf_ordinary() in every lane of the wavefront, so that this is straight-line code
@@ -259,12 +259,15 @@ __device__ __forceinline__ float add_in_row_order(float acc, const float *t, int
   return acc;
 }
 
-// A lane per column: for launches with fewer lanes than the tiles below are filled by.
+// A lane per column, for launches with fewer lanes than the tiles below are filled by.
 template <Dt D, typename Logs>
 __device__ __forceinline__ void input_fusion_by_element(const void *__restrict__ a, const void *__restrict__ b,
-                                                        void *__restrict__ out, int64_t rows, int64_t cols, const Logs &logs) {
+                                                        void *__restrict__ out, int64_t rows, int64_t cols, Logs &logs) {
   using E = Elem<D>;
-  for (int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; c < cols; c += int64_t(gridDim.x) * blockDim.x) {
+  for (int i = threadIdx.x; i < 16; i += lanes_launched())
+    logs.entry[i] = kLogfTable[i];
+  __syncthreads();
+  for (int64_t c = int64_t(blockIdx.x) * lanes_launched() + threadIdx.x; c < cols; c += int64_t(gridDim.x) * lanes_launched()) {
     float acc = 0.0f;
     for (int64_t r = 0; r < rows; ++r)
       acc = acc + input_chain(E::get(a, r * cols + c), E::get(b, r * cols + c), logs);
@@ -608,13 +611,14 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
   __shared__ Logarithms<kMantissaOf<D>> logs;
   const int64_t segments = (cols * Elem<D>::kBytes + 31) / 32;
   const int lanes = chain_lanes(segments), workers = lanes == 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
-  if (!chains_take<D>(rows, cols) || cols * Elem<D>::kBytes < 32 || int(blockDim.x) != (workers + 1) * kWave) {
+  if (!chains_take<D>(rows, cols) || cols * Elem<D>::kBytes < 32 || lanes_launched() != (workers + 1) * kWave) {
+    if (lanes_launched() < kThreads) {
+      input_fusion_by_element<D>(a, b, out, rows, cols, logs);
+      return;
+    }
     logs.stage();
     __syncthreads();
-    if (blockDim.x < kThreads)
-      input_fusion_by_element<D>(a, b, out, rows, cols, logs);
-    else
-      input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
+    input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 4) {
     input_fusion_chains<D, 4, 4>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 8) {
@@ -637,20 +641,20 @@ __device__ __forceinline__ void input_fusion(const void *__restrict__ a, const v
                                              void *__restrict__ out, int64_t rows, int64_t cols) {
   __shared__ Logarithms<0> logs;
   __shared__ __attribute__((aligned(16))) float tile[2 * kStreamTileFloats];
-  logs.stage();
-  __syncthreads();
-  if (blockDim.x < kThreads) {
+  if (lanes_launched() < kThreads) {
     input_fusion_by_element<D>(a, b, out, rows, cols, logs);
     return;
   }
+  logs.stage();
+  __syncthreads();
   // The launch says which form: 576 or 320 lanes ask for a streaming one, which needs whole aligned vectors.
   const bool vectors = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
                        cols % Elem<D>::kPerVec == 0;
-  if (blockDim.x == kStreamThreads && vectors && input_fusion_streams<D>(rows, cols)) {
+  if (lanes_launched() == kStreamThreads && vectors && input_fusion_streams<D>(rows, cols)) {
     input_fusion_stream<D, WideShape<D>>(a, b, out, rows, cols, logs, tile);
     return;
   }
-  if (blockDim.x == kNarrowThreads && input_fusion_narrow(cols)) {
+  if (lanes_launched() == kNarrowThreads && input_fusion_narrow(cols)) {
     input_fusion_stream<D, NarrowShape<D>>(a, b, out, rows, cols, logs, tile);
     return;
   }

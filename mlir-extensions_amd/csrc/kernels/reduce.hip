@@ -485,9 +485,10 @@ __device__ __forceinline__ void reduce_outer_tall(const void *in, void *out, int
   __shared__ __attribute__((aligned(16))) float lds[ColumnChain<D, 1, 16, 8>::kLdsFloats];
   const int64_t segments = (inner * io::Elem<D>::kBytes + 31) / 32;
   const int lanes = chain_lanes(segments), workers = lanes == 16 ? wide_chain_workers(segments) : 4;
-  if (!chains_take<D>(outer, inner) || int(blockDim.x) != (workers + 1) * kWave)
+  const int64_t slice = inner * io::Elem<D>::kBytes;
+  if (!chains_take<D>(outer, inner) || lanes_launched() != (workers + 1) * kWave || (slice < 8 && outer * slice < 8))
     reduce_outer_by_element<D>(in, out, outer, inner, init);
-  else if (inner * io::Elem<D>::kBytes < 8)
+  else if (lanes == 4 && slice < 8)
     reduce_outer_chains<D, 4, 4, true>(in, out, outer, inner, init, lds);
   else if (lanes == 4)
     reduce_outer_chains<D, 4, 4>(in, out, outer, inner, init, lds);
