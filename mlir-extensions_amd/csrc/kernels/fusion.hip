@@ -325,73 +325,38 @@ __device__ __forceinline__ void input_fusion_cols(const void *__restrict__ a, co
   }
 }
 
-// ---- kInputFusion on tall, wide matrices: the streaming form --------------------------------
-// With 4 .. 64 columns per workgroup the form above reads 16 .. 64-byte row segments, computes and adds
-// in turn, and is bound by memory latency (17 % of HBM at 8192 x 8192).  Here a workgroup of 576 lanes
-// owns the columns of one 128-byte row segment (32 f32 or 64 16-bit columns).  Its first 512 lanes are
-// workers: 16 bytes per lane and access, 8 lanes per row, 64 rows per access; a tile is 8192 elements
-// (256 or 128 rows), the next tile's loads are issued before this tile's chains are evaluated, and the
-// results go into one of two LDS tiles.  The ninth wavefront does nothing but the ordered additions, one
-// lane per column, a tile behind the workers: one barrier per tile, passed by everybody, hands a tile
-// over and returns the other one.
-// The same structure serves narrow matrices (fewer than 4096 columns, the reference's 512 x 1024 among them):
-// 256 workers + the adder wavefront = 320 lanes own 4 columns, one element per lane and access, 64 rows per
-// tile, eight tiles' loads in flight together.  There the ordered additions are the critical path
-// (a lone wavefront issues a dependent addition every ~8 cycles), and what this form buys is that nothing
-// else is ever on it: the adder never loads or evaluates, and the workers are always a tile ahead.
-constexpr int kStreamWorkers = 512, kStreamThreads = kStreamWorkers + 64;
+// ---- kInputFusion on narrow matrices: the streaming form ------------------------------------
+// With 4 columns per workgroup the form above reads 16-byte row segments, computes and adds in turn, and is bound by
+// memory latency.  Here 256 workers + one adder wavefront = 320 lanes own 4 columns, one element per lane and access, 64
+// rows per tile (a lane's first result is ready after ONE chain), the loads of eight tiles -- 512 rows -- in flight
+// together.  The next group's loads are issued before this group's chains are evaluated; the results go into one of two
+// LDS tiles.  The fifth wavefront does nothing but the ordered additions, one lane per column, a tile behind the
+// workers: one barrier per tile, passed by everybody, hands a tile over and returns the other one.  The ordered additions
+// are the critical path (a lone wavefront issues a dependent addition every ~8 cycles), and what this form buys is that
+// nothing else is ever on it.  Taller matrices go by column chains (below).
 constexpr int kNarrowWorkers = 256, kNarrowThreads = kNarrowWorkers + 64;
-constexpr int kStreamTileElems = 8192;
-constexpr int kStreamTileFloats = 64 * (128 + 16); // the largest padded tile: 64 columns of 128 rows
+constexpr int kNarrowCols = 4, kNarrowRows = kNarrowWorkers / kNarrowCols, kNarrowTilesAhead = 8;
+// A tile lies in LDS COLUMN by column, and row r of column c sits at position r ^ 4 c: the adder still reads four
+// consecutive rows of its column with one 128-bit access.  A 32-bit write is served 32 lanes at a time (0-31, 32-63) over
+// banks that repeat every 32 words: eight rows of four columns, of which the pitch (16 modulo 32 words) puts odd and even
+// ones 16 banks apart and the swizzle the two of a kind 8.
+constexpr int kNarrowPitch = kNarrowRows + 16, kNarrowTileFloats = kNarrowCols * kNarrowPitch;
+// 576 lanes, from 2048 rows and 128 row segments of 128 bytes on: column chains of such segments, eight workers
+constexpr int kStreamThreads = 576;
 constexpr int64_t kStreamFromRows = 2048;
-
-// kLanesPerRow worker lanes cover a row segment, each with one 16-byte vector (kVec) or one element; an access
-// of all workers is a pass, kTilePasses passes make a tile (what is handed to the adder at one barrier), and
-// the loads of kGroupTiles tiles are issued together, one such group ahead of the one being evaluated.
-template <Dt D, int kLanesPerRow, int kWorkers, int kTilePassesT, int kGroupTilesT, bool kVecT> struct StreamShape {
-  static constexpr bool kVec = kVecT;
-  static constexpr int kLanes = kLanesPerRow, kWork = kWorkers, kTilePasses = kTilePassesT, kGroupTiles = kGroupTilesT;
-  static constexpr int kPer = kVec ? Elem<D>::kPerVec : 1;      // elements per lane and access
-  static constexpr int kCols = kLanesPerRow * kPer;             // columns per workgroup
-  static constexpr int kRowsPerPass = kWorkers / kLanesPerRow;
-  static constexpr int kTileRows = kTilePasses * kRowsPerPass;
-  static constexpr int kGroupPasses = kTilePasses * kGroupTiles;
-  // A tile lies in LDS COLUMN by column, kTileRows + 16 floats apart, and row r of column c sits at position
-  // r ^ row_swizzle(c), a multiple of 4 below 32: blocks of four rows trade places inside their block of 32,
-  // so the adder still reads four consecutive rows of its column with one 128-bit access.  Pitch and swizzle
-  // follow from how the LDS serves the two kinds of access (measured with two-lane probes): a 32-bit write is
-  // served 32 lanes at a time (0-31, 32-63) over banks that repeat every 32 words; a 128-bit read sixteen
-  // lanes at a time (0-3 with 12-15, 20-23 and 24-27; 4-11 with 16-19 and 28-31; the same + 32) over banks
-  // that repeat every 64 words.  A worker half-wavefront writes four rows of eight column groups with one
-  // instruction: the pitch (16 modulo 32 words) puts odd and even groups 16 banks apart, the swizzle
-  // 4 x (group index) spreads the four groups of each kind over the four 4-bank blocks.  The adder's sixteen
-  // lanes then read sixteen different 16-byte bank groups for every row block.
-  static constexpr int kColPitch = kTileRows + 16;
-  static __device__ __forceinline__ int row_swizzle(int col) { return 4 * ((col / kPer) & 7); }
-  static constexpr int kTileFloats = kCols * kColPitch;
-  static_assert(kTileRows % 32 == 0 && kTileFloats <= kStreamTileFloats, "the LDS tiles are sized for 9216 floats");
-};
-// wide: 128-byte row segments, 8192-element tiles (256 rows of 32 f32, 128 rows of 64 16-bit columns)
-template <Dt D>
-using WideShape = StreamShape<D, 8, kStreamWorkers, kStreamTileElems / (128 / Elem<D>::kBytes) / (kStreamWorkers / 8), 1, true>;
-// narrow: four columns, one element per lane, 64 rows per tile (a lane's first result is ready after ONE chain),
-// the loads of eight tiles -- 512 rows -- in flight together
-template <Dt D> using NarrowShape = StreamShape<D, 4, kNarrowWorkers, 1, 8, false>;
 
 // what the launch and the kernel both decide on: enough column blocks for the chip, enough rows for a pipeline
 template <Dt D> __device__ __forceinline__ bool input_fusion_streams(int64_t rows, int64_t cols) {
-  return rows >= kStreamFromRows && cols >= int64_t(WideShape<D>::kCols) * 128;
+  return rows >= kStreamFromRows && cols * Elem<D>::kBytes >= 128 * 128;
 }
 // ... and the narrow form wherever the form above would take four columns per workgroup
 __device__ __forceinline__ bool input_fusion_narrow(int64_t cols) { return cols < 8 * 512; }
 
-// acc + c[0] + c[1] + ... + c[n-1], added in that order, for a column c of kTileRows consecutive floats
+// acc + c[0] + c[1] + ... + c[n-1], added in that order, for a column c of kNarrowRows consecutive floats
 // (16-byte aligned, all of them readable): sixteen rows arrive as four 128-bit LDS reads while the previous
 // sixteen are added, so the adder issues 1.25 instructions per row.
 // swz: row r is kept at position r ^ swz (a multiple of 4 below 32: blocks of four rows trade places).
-template <int kTileRows>
-__device__ __forceinline__ float add_column_in_row_order(float acc, const float *c, int n, int swz = 0) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float add_column_in_row_order(float acc, const float *c, int n, int swz) {
   f32x4 x[4], y[4];
   auto read16 = [&](f32x4(&v)[4], int r) {
 #pragma unroll
@@ -412,7 +377,7 @@ __device__ __forceinline__ float add_column_in_row_order(float acc, const float 
   for (; r + 32 <= n; r += 32) {
     read16(y, r + 16);
     add16(x);
-    read16(x, r + 32 < kTileRows ? r + 32 : 0); // past the tile's last row: any readable rows, not added
+    read16(x, r + 32 < kNarrowRows ? r + 32 : 0); // past the tile's last row: any readable rows, not added
     add16(y);
   }
   // x holds rows r .. r + 15; fewer than 32 rows are left
@@ -443,46 +408,35 @@ __device__ __forceinline__ float add_column_in_row_order(float acc, const float 
 // pass it exactly once per tile -- `tiles` times per block of columns, the workers after writing tile t,
 // the adder before reading it -- and once more together when the block of columns is done.  Written as
 // the instruction with the LDS release / acquire around it, not as a call the compiler may treat as
-// convergent across the two branches.  The workgroup must be exactly kWork + 64 lanes (the entry checks).
+// convergent across the two branches.  The workgroup must be exactly kNarrowThreads lanes (the entry checks).
 __device__ __forceinline__ void tile_handover() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-template <Dt D, typename S>
+template <Dt D>
 __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, const void *__restrict__ b,
                                                     void *__restrict__ out, int64_t rows, int64_t cols,
                                                     const Logarithms<0> &logs, float *tile) {
   using E = Elem<D>;
-  constexpr int kCols = S::kCols, kTileRows = S::kTileRows, kWorkers = S::kWork, kPer = S::kPer;
-  constexpr int kGroupPasses = S::kGroupPasses;
-  struct Raw { // what one load brings: a 16-byte vector, or one element already widened
-    u32x4 v;
-    float f;
-  };
   const int tid = threadIdx.x;
-  const int64_t tiles = (rows + kTileRows - 1) / kTileRows;
-  const int64_t groups = (tiles + S::kGroupTiles - 1) / S::kGroupTiles;
-  for (int64_t c0 = int64_t(blockIdx.x) * kCols; c0 < cols; c0 += int64_t(gridDim.x) * kCols) {
-    if (tid < kWorkers) {
-      const int lr = tid / S::kLanes, lc = (tid % S::kLanes) * kPer; // row within a pass, the lane's first column
+  const int64_t tiles = (rows + kNarrowRows - 1) / kNarrowRows;
+  const int64_t groups = (tiles + kNarrowTilesAhead - 1) / kNarrowTilesAhead;
+  for (int64_t c0 = int64_t(blockIdx.x) * kNarrowCols; c0 < cols; c0 += int64_t(gridDim.x) * kNarrowCols) {
+    if (tid < kNarrowWorkers) {
+      const int lr = tid / kNarrowCols, lc = tid % kNarrowCols; // row within a tile, column
       // Rows past the end and, in a partial last block, columns past the end re-read a position inside the
       // matrix instead (their results are never added): the loads are then unconditional, straight-line
       // code, and the wait for a tile's data leaves the next group's loads in flight.
-      const int64_t col = c0 + lc < cols ? c0 + lc : c0; // vectors: cols is a multiple of the vector, all of it or none
-      Raw ca[kGroupPasses], cb[kGroupPasses], na[kGroupPasses], nb[kGroupPasses];
-      auto load_group = [&](int64_t g, Raw(&va)[kGroupPasses], Raw(&vb)[kGroupPasses]) {
+      const int64_t col = c0 + lc < cols ? c0 + lc : c0;
+      float ca[kNarrowTilesAhead], cb[kNarrowTilesAhead], na[kNarrowTilesAhead], nb[kNarrowTilesAhead];
+      auto load_group = [&](int64_t g, float(&va)[kNarrowTilesAhead], float(&vb)[kNarrowTilesAhead]) {
 #pragma unroll
-        for (int p = 0; p < kGroupPasses; ++p) {
-          const int64_t r = min((g * kGroupPasses + p) * S::kRowsPerPass + lr, rows - 1);
-          if constexpr (S::kVec) {
-            va[p].v = load128<true>(reinterpret_cast<const u32x4 *>(static_cast<const char *>(a) + (r * cols + col) * E::kBytes));
-            vb[p].v = load128<true>(reinterpret_cast<const u32x4 *>(static_cast<const char *>(b) + (r * cols + col) * E::kBytes));
-          } else {
-            va[p].f = E::get(a, r * cols + col);
-            vb[p].f = E::get(b, r * cols + col);
-          }
+        for (int p = 0; p < kNarrowTilesAhead; ++p) {
+          const int64_t r = min((g * kNarrowTilesAhead + p) * kNarrowRows + lr, rows - 1);
+          va[p] = E::get(a, r * cols + col);
+          vb[p] = E::get(b, r * cols + col);
         }
       };
       if (groups > 0) // (no rows: nothing to read, the sums are +0.0)
@@ -490,57 +444,32 @@ __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, 
       for (int64_t g = 0; g < groups; ++g) {
         load_group(g + 1 < groups ? g + 1 : g, na, nb); // past the last group: the last one again, unused
 #pragma unroll
-        for (int j = 0; j < S::kGroupTiles; ++j) {
-          const int64_t t = g * S::kGroupTiles + j;
+        for (int j = 0; j < kNarrowTilesAhead; ++j) {
+          const int64_t t = g * kNarrowTilesAhead + j;
           if (t < tiles) { // uniform
-            float *dst = tile + (t & 1) * S::kTileFloats + lc * S::kColPitch;
-#pragma unroll
-            for (int q = 0; q < S::kTilePasses; ++q) {
-              const int p = j * S::kTilePasses + q;
-              float fa[kPer], fb[kPer];
-              if constexpr (S::kVec) {
-                E::unpack(ca[p].v, fa);
-                E::unpack(cb[p].v, fb);
-              } else {
-                fa[0] = ca[p].f;
-                fb[0] = cb[p].f;
-              }
-              bool ordinary = true;
-#pragma unroll
-              for (int i = 0; i < kPer; ++i)
-                ordinary = ordinary && logf_ordinary(fb[i]);
-              if (__builtin_amdgcn_ballot_w64(!ordinary) == 0) { // uniform over the wavefront
-#pragma unroll
-                for (int i = 0; i < kPer; ++i)
-                  fa[i] = input_chain<true>(fa[i], fb[i], logs);
-              } else {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i)
-                  fa[i] = input_chain(fa[i], fb[i], logs);
-              }
-#pragma unroll
-              for (int i = 0; i < kPer; ++i)
-                dst[i * S::kColPitch + q * S::kRowsPerPass + (lr ^ S::row_swizzle(lc + i))] = fa[i];
-            }
+            float *dst = tile + (t & 1) * kNarrowTileFloats + lc * kNarrowPitch + (lr ^ 4 * lc);
+            if (__builtin_amdgcn_ballot_w64(!logf_ordinary(cb[j])) == 0) // uniform over the wavefront
+              *dst = input_chain<true>(ca[j], cb[j], logs);
+            else
+              *dst = input_chain(ca[j], cb[j], logs);
             tile_handover(); // tile t is complete; the adder is done with tile t-1, whose buffer tile t+1 goes into
           }
         }
 #pragma unroll
-        for (int p = 0; p < kGroupPasses; ++p) {
+        for (int p = 0; p < kNarrowTilesAhead; ++p) {
           ca[p] = na[p];
           cb[p] = nb[p];
         }
       }
     } else {
-      const int col = tid - kWorkers;
-      const bool active = col < kCols && c0 + col < cols;
+      const int col = tid - kNarrowWorkers;
+      const bool active = col < kNarrowCols && c0 + col < cols;
       float acc = 0.0f;
       for (int64_t t = 0; t < tiles; ++t) {
         tile_handover(); // tile t is complete
-        const int n = rows - t * kTileRows < kTileRows ? int(rows - t * kTileRows) : kTileRows;
+        const int n = rows - t * kNarrowRows < kNarrowRows ? int(rows - t * kNarrowRows) : kNarrowRows;
         if (active)
-          acc = add_column_in_row_order<kTileRows>(acc, tile + (t & 1) * S::kTileFloats + col * S::kColPitch, n,
-                                                   S::row_swizzle(col));
+          acc = add_column_in_row_order(acc, tile + (t & 1) * kNarrowTileFloats + col * kNarrowPitch, n, 4 * col);
       }
       if (active)
         E::put(out, c0 + col, acc);
@@ -551,8 +480,7 @@ __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, 
 
 // ---- kInputFusion by column chains (column_chain.h) -------------------------------------------
 // Any number of columns and rows, at any address: the forms above read 4 .. 64 columns of a row per workgroup element by
-// element unless the rows are whole 16-byte vectors and there are 2048 of them and 128 segments of 128 bytes, and were
-// bound by the latency of those loads or, 16-bit inputs, by the logarithms.  bf16 5550 x 5932 449 -> 42 us (floor 21 for its
+// element and are bound by the latency of those loads or, 16-bit inputs, by the logarithms.  bf16 5550 x 5932 449 -> 42 us (floor 21 for its
 // bytes), f32 3785 x 3480 155 -> 27 (17), f16 1052 x 5433 76 -> 11, f32 8192 x 512 87 -> 31 (the chain alone: 22), f32
 // 8192 x 8192 106 -> 91 (85).  Two workers per SIMD on segments of 64 and 128 bytes: one took 29 and 82 us on f16 3785 x
 // 3480 and f32 5550 x 5932, two take 19 and 60.
@@ -639,23 +567,24 @@ __device__ __forceinline__ int input_fusion_block_cols(int64_t cols) {
 template <Dt D>
 __device__ __forceinline__ void input_fusion(const void *__restrict__ a, const void *__restrict__ b,
                                              void *__restrict__ out, int64_t rows, int64_t cols) {
+  constexpr int kLdsFloats = ColumnChain<D, 2, 16, 8>::kLdsFloats;
+  static_assert(kLdsFloats >= 2 * kTileElems && kLdsFloats >= 2 * kNarrowTileFloats);
   __shared__ Logarithms<0> logs;
-  __shared__ __attribute__((aligned(16))) float tile[2 * kStreamTileFloats];
+  __shared__ __attribute__((aligned(16))) float tile[kLdsFloats];
   if (lanes_launched() < kThreads) {
     input_fusion_by_element<D>(a, b, out, rows, cols, logs);
     return;
   }
-  logs.stage();
-  __syncthreads();
-  // The launch says which form: 576 or 320 lanes ask for a streaming one, which needs whole aligned vectors.
-  const bool vectors = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 &&
-                       cols % Elem<D>::kPerVec == 0;
-  if (lanes_launched() == kStreamThreads && vectors && input_fusion_streams<D>(rows, cols)) {
-    input_fusion_stream<D, WideShape<D>>(a, b, out, rows, cols, logs, tile);
+  // The launch says which form.
+  if (lanes_launched() == kStreamThreads && chains_take<D>(rows, cols) && input_fusion_streams<D>(rows, cols)) {
+    __shared__ Logarithms<kMantissaOf<D>> all;
+    input_fusion_chains<D, 16, 8>(a, b, out, rows, cols, all, tile);
     return;
   }
+  logs.stage();
+  __syncthreads();
   if (lanes_launched() == kNarrowThreads && input_fusion_narrow(cols)) {
-    input_fusion_stream<D, NarrowShape<D>>(a, b, out, rows, cols, logs, tile);
+    input_fusion_stream<D>(a, b, out, rows, cols, logs, tile);
     return;
   }
   switch (input_fusion_block_cols(cols)) {

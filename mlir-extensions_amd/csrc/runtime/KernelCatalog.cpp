@@ -336,7 +336,7 @@ const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const double tall = 3.04 + std::max(0.77 * more + double(outer) * step * (1.0 + 1.63 * more), bytes / 5.6e6);
   const double wait = double(outer) * (vec ? 0.0517 : f32 ? 0.0220 : 0.0143), move = bytes / (vec ? 7.35e6 : 6.04e6);
   const double deep = 2.61 + std::max(wait, move) + (vec ? 0.72 : 0.55) * std::min(wait, move);
-  const bool chains = bytes >= 8.0 && slice < int64_t(1) << 22 && outer < int64_t(1) << 31; // chains_take in column_chain.h
+  const bool chains = bytes >= 8.0 && slice < int64_t(1) << 26 && outer < int64_t(1) << 31; // chains_take in column_chain.h
   char name[96];
   snprintf(name, sizeof name, "%s%s", e->name, chains && tall < 0.96 * deep ? "_tall" : "_deep");
   return find(name)->name;
@@ -412,11 +412,11 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
 // its first and only additions.  By 300 timed problems (2 .. 12000 rows of 16 .. 300000 columns): below 2048 columns
 // from 128 rows on (f16 124 x 81: own 4.1 us, chains 4.4; f32 827 x 1592 23.2 / 6.2); rows that take workgroups of 128-byte
 // segments more than one round from 72 (f32) or 24 rows on (f32 33 x 25520 9.9 / 10.8; f16 20 x 37008 8.7 / 9.5; bf16 5550 x
-// 5932 449 / 42); rows in between always (f32 2 x 7024 6.6 / 3.8).
+// 5932 449 / 42; f32 72 x 1074784 494 / 299); rows in between always (f32 2 x 7024 6.6 / 3.8).
 const char *inputFusionVariant(const Entry *e, int64_t rows, int64_t cols) {
   const bool f32 = e->shape == Shape::ColumnThreads;
   const int64_t bytes = cols * (f32 ? 4 : 2);
-  if (rows == 0 || rows >= int64_t(1) << 31 || bytes >= int64_t(1) << 22 || // chains_take in column_chain.h
+  if (rows == 0 || rows >= int64_t(1) << 31 || bytes >= int64_t(1) << 26 || // chains_take in column_chain.h
       (cols < 2048 ? rows < 128 || bytes < 32 : bytes > 256 * 128 && rows < (f32 ? 72 : 24)))
     return e->name;
   char name[96];
@@ -634,17 +634,16 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
   case Shape::ColumnThreads:
   case Shape::ColumnThreads16: {
     const int64_t rows = dims[0], cols = dims[1];
-    // From 2048 rows and 128 row segments of 128 bytes on: the streaming form, 576 lanes per segment's
-    // columns (32 f32 or 64 16-bit ones).  The kernel applies the same rule, and falls back by itself when
-    // the rows are not made of whole aligned 16-byte vectors.
+    // From 2048 rows and 128 row segments of 128 bytes on: column chains with 576 lanes per segment's
+    // columns (32 f32 or 64 16-bit ones).  The kernel applies the same rule.
     const int64_t segment_cols = e->shape == Shape::ColumnThreads ? 32 : 64;
     if (rows >= 2048 && cols >= segment_cols * 128) {
       block[0] = 576;
       grid[0] = ceilDiv(cols, segment_cols);
       break;
     }
-    // Fewer than 4096 columns (the reference's 512 x 1024): the same form with 256 workers and the adder
-    // wavefront = 320 lanes per four columns.
+    // Fewer than 4096 columns (the reference's 512 x 1024): 256 workers and the adder wavefront = 320 lanes per
+    // four columns.
     if (cols < 8 * 512) {
       block[0] = 320;
       grid[0] = ceilDiv(cols, 4);

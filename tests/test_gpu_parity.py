@@ -838,6 +838,23 @@ def test_input_fusion_with_any_block(host, orc, stream, dtype, rows, cols):
         stream.free(p)
 
 
+@pytest.mark.parametrize("dtype,rows,cols", [("f32", 73, (1 << 20) + 5), ("f16", 30, (1 << 21) + 3), ("bf16", 66, (1 << 21) + 8)])
+def test_column_chains_rows_of_4_mib(host, orc, stream, dtype, rows, cols):
+    """Rows of 4 MiB and more, in one and in two tiles of 64 rows: offsets inside a tile pass 2^28."""
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    assert host.variant("imex_input_fusion_" + dtype, [rows, cols]) == "imex_input_fusion_%s_tall" % dtype
+    a = orc.fill_uniform(rows * cols, dtype, 61, -5.0, 5.0).reshape(rows, cols)
+    b = orc.fill_uniform(rows * cols, dtype, 62, 0.01, 40.0).reshape(rows, cols)
+    assert np.array_equal(host.input_fusion(stream, a, b, dtype), narrow(orc.input_fusion_f32(wide(a), wide(b))))
+    d_in, d_out = stream.to_device(a), stream.alloc(cols * a.itemsize)
+    stream.launch("imex_reduce_outer_%s_tall" % dtype, [rows, cols], [d_in, d_out, rows, cols, 0.25], grid=(1000, 1, 1))
+    stream.wait()
+    got = stream.from_device(d_out, (cols,), a.dtype)
+    stream.free(d_in), stream.free(d_out)
+    assert np.array_equal(got, narrow(orc.reduce_outer_f32(wide(a), 0.25)))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("cols", range(1, 17))
 def test_reduce_outer_narrow_rows(host, orc, stream, dtype, cols):
