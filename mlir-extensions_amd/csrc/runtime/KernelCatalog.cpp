@@ -313,32 +313,33 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
   return variant ? variant->name : e->name;
 }
 
-// Which form of the outer-dimension sum a problem should take, from two estimates in microseconds fitted to 700
-// timed problems (4 .. 9000 slices of 64 .. 4 Mi outputs, all types, whole vectors and not, from HBM; the choice is within
-// 0.2 % of the faster of tall and deep in the mean; near a tie deep, f32 300 x 80000 26.4 / 25.4).
-//   plain  whole vectors and slices of 5 MiB (16-bit: 8 MiB) and more (f32 12 x 1051744: plain 11.7, deep 10.4; 12 x
-//          1408680: 13.0, 13.5; f16 15 x 2283888: 18.3, 12.6);
-//   tall   a launch, a slice's share of the chain, and what a CU pays for further workgroups; 5.6 TB/s at most;
-//   deep   a slice costs its share of sixteen slices' latency, which its bytes hide little of; 7.3 (6.0) TB/s at most.
-// 8192 x 4096 f32: plain 980, tall 37, deep 540 us; 568 x 197848: tall 102, deep 66; bf16 389 x 129280: 30, 32.  Below 64
+// Which form of the outer-dimension sum a problem should take, from two estimates in microseconds fitted to 1000
+// timed problems (1 .. 20000 slices of 1 .. 8 Mi outputs, all types, whole vectors and not, from HBM and not; the choice is
+// within 0.2 % of the faster of tall and deep in the mean, at worst 12 %; over 350 others within 0.6 % of the fastest form).
+//   plain  whole vectors and slices of 5 MiB (16-bit: 8 MiB) and more, for up to four slices 4 MiB (f32 4 x 1359872 6.8,
+//          deep 8.5; f16 2 x 2999824 8.1, 8.7; f32 7 x 2071552 15.4, 13.5; 12 x 1051744 11.7, 10.4; 6 x 1500000 16.4, 16.0;
+//          f16 15 x 2283888 18.3, 12.6);
+//   tall   a launch, a slice's share of the chain, and what a CU pays for further workgroups; 4.9 TB/s at most;
+//   deep   a slice costs its share of sixteen slices' latency, which its bytes hide little of; 8.0 (5.1) TB/s at most.
+// 8192 x 4096 f32: plain 980, tall 37, deep 540 us; 62 x 32296: tall 4.1, deep 7.0; 568 x 197848: 102, 66.  Below 64
 // outputs (1 .. 15, 8 .. 10^5 slices) tall is never slower than deep by more than 0.1 us: 64 x 4 both 3.3, 256 x 4 3.3 / 8.5.
 const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const bool f32 = e->shape == Shape::ReduceOuter;
   const int64_t perVec = f32 ? 4 : 8, slice = inner * (f32 ? 4 : 2);
   const bool vec = inner % perVec == 0;
-  if (outer == 0 || inner == 0 || (vec && slice >= (f32 ? int64_t(5) << 20 : int64_t(8) << 20)))
+  if (outer == 0 || inner == 0 || (vec && slice >= (outer <= 4 ? int64_t(4) << 20 : f32 ? int64_t(5) << 20 : int64_t(8) << 20)))
     return e->name;
   const double bytes = double(outer) * double(slice);
   const size_t segments = ceilDiv(slice, 32);
   const int width = chainWidth(segments);
   const double more = std::max(0.0, double(ceilDiv(segments, width)) / 256.0 - 1.0);
-  const double step = width == 1 ? 0.0026 : width == 2 ? 0.0030 : f32 ? 0.0038 : 0.0043;
-  const double tall = 3.04 + std::max(0.77 * more + double(outer) * step * (1.0 + 1.63 * more), bytes / 5.6e6);
-  const double wait = double(outer) * (vec ? 0.0517 : f32 ? 0.0220 : 0.0143), move = bytes / (vec ? 7.35e6 : 6.04e6);
-  const double deep = 2.61 + std::max(wait, move) + (vec ? 0.72 : 0.55) * std::min(wait, move);
+  const double step = width == 1 ? 0.00252 : width == 2 ? 0.00363 : f32 ? 0.00112 : 0.00458;
+  const double tall = 3.28 + std::max(0.744 * more + double(outer) * step * (1.0 + (f32 ? 1.77 : 1.17) * more), bytes / 4.91e6);
+  const double wait = double(outer) * (vec ? 0.0375 : f32 ? 0.0236 : 0.0139), move = bytes / (vec ? 8.02e6 : 5.13e6);
+  const double deep = 3.26 + std::max(wait, move) + (vec ? 0.88 : 0.098) * std::min(wait, move);
   const bool chains = bytes >= 8.0 && slice < int64_t(1) << 26 && outer < int64_t(1) << 31; // chains_take in column_chain.h
   char name[96];
-  snprintf(name, sizeof name, "%s%s", e->name, chains && tall < 0.96 * deep ? "_tall" : "_deep");
+  snprintf(name, sizeof name, "%s%s", e->name, chains && tall < deep ? "_tall" : "_deep");
   return find(name)->name;
 }
 

@@ -237,6 +237,23 @@ def test_softmax_launch_rules(host):
     assert host.launch_shape("imex_softmax_f32_shared", [1023, 800])[0] == (1023, 1, 1)
 
 
+def test_reduce_outer_launch_rules(host):
+    """The outer sum's own form for large slices of whole vectors, from 4 MiB for up to four of them; chains for narrow and
+    for tall matrices, a lane per vector (or column) for few slices of many columns."""
+    choice = lambda dt, outer, inner: host.variant("imex_reduce_outer_" + dt, [outer, inner])[len("imex_reduce_outer_" + dt):]
+    mib = 1 << 20
+    for dt, width, least in (("f32", 4, 5), ("f16", 2, 8), ("bf16", 2, 8)):
+        for outer in (1, 4):
+            assert [choice(dt, outer, 4 * mib // width + d) for d in (-8, 0, 1)] == ["_deep", "", "_deep"]
+        for outer in (5, 32):
+            assert [choice(dt, outer, least * mib // width + d) for d in (-8, 0, 1)] == ["_deep", "", "_deep"]
+        for cols in range(1, 17):
+            assert choice(dt, 8192, cols) == choice(dt, 200, cols) == "_tall"
+        assert choice(dt, 8192, 4096) == choice(dt, 64, 2000) == "_tall" and choice(dt, 64, 100000) == "_deep"
+        assert choice(dt, 0, 16) == choice(dt, 16, 0) == ""
+    assert choice("f32", 62, 32296) == "_tall" and choice("f32", 568, 197848) == "_deep"
+
+
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
     """Stream.launch's fast path: 8 bytes per argument, an f32 in the low four, with _pack_params' conversions and errors."""
     class Resolver:
