@@ -423,11 +423,40 @@ def test_rowmean(host, orc, stream):
 @pytest.mark.parametrize("shape", [(32, 16, 64, 64), (10, 20), (7, 1023), (33, 4100), (1, 5), (3, 1, 9),
                                    (5, 512 * 2048 + 4), (3, 512 * 4096 + 1028), (2, 512 * 8192 + 8), (6, 512 * 2048 + 3)])
 def test_reduce_outer_bit_exact(host, orc, stream, shape):
-    """The last four shapes reach the 8, 16 and 32 KiB-per-slice variants with a ragged last
-    workgroup, and the one-lane-per-output path at a size where it strides."""
+    """The catalogue's choice: the operator's own form with 16 and 32 KiB of a slice per workgroup and a ragged last one for
+    3 and 2 slices of whole vectors, a lane per vector or output for the other large ones, column chains for the tall."""
     x = orc.fill_uniform(int(np.prod(shape)), "f32", 77, -1.0, 1.0).reshape(shape)
     got, ref = host.reduce_outer(stream, x, init=0.25), orc.reduce_outer_f32(x, init=0.25)
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("outer,inner,chosen", [(3, 2 * 512 + 1.25, True), (4, 2 * 512, True), (5, 4 * 512 + 3, True), (2, 8 * 512 + 1, True),
+                                                (6, 2.5 * 512, True), (5, 2 * 512 + 0.25, False), (7, 300.125, False),
+                                                (130, 0.5, False), (10, 0.03125, False)])
+def test_reduce_outer_own_launch(host, orc, stream, dtype, outer, inner, chosen):
+    """The operator's own kernel under its own launch; `inner` counts a workgroup's row of 256 16-byte vectors.  What the
+    catalogue leaves to it (slices of 4 MiB and more for up to four of them, of 5 MiB, 16-bit: 8 MiB, beyond that): two, four
+    and eight vectors per lane, with a whole and a ragged last workgroup; and what it gives to the other forms."""
+    name, vec = "imex_reduce_outer_" + dtype, 4 if dtype == "f32" else 8
+    cols = int(inner * 256 * vec) + (1 if inner % 1 == 0.125 else 0)  # (0.125: no whole vectors)
+    if chosen and (dtype == "f32" or inner != 2.5 * 512):
+        assert host.variant(name, [outer, cols]) == name
+    x = orc.fill_uniform(outer * cols, dtype, 94, -1.0, 1.0).reshape(outer, cols)
+    want = orc.reduce_outer_f32(x if dtype == "f32" else orc.to_float(x, dtype), 0.25)
+    want = want if dtype == "f32" else orc.from_float(want, dtype)
+    fill = np.full(cols + 64, 3, x.dtype)
+    d_in, d_out = stream.to_device(x), stream.alloc(fill.nbytes)
+    grid, block, _ = host.launch_shape(name, [outer, cols])
+    for g in (grid, (5, 1, 1)):
+        say("%s %dx%d, grid %s" % (name, outer, cols, g))
+        stream.copy(d_out, fill.ctypes.data, fill.nbytes)
+        stream.launch(name, [outer, cols], [d_in, d_out, outer, cols, 0.25], grid=g, block=block)
+        stream.wait()
+        got = stream.from_device(d_out, fill.shape, fill.dtype)
+        assert np.array_equal(got[:cols], want), (name, g)
+        assert np.all(got[cols:] == 3), (name, g)
+    stream.free(d_in), stream.free(d_out)
 
 
 @pytest.mark.parametrize("form", ["_tall", "_deep"])
@@ -717,10 +746,8 @@ def test_loop_fusion_16bit_every_logarithm(host, orc, stream, dtype, n):
     assert np.array_equal(got.view(np.uint32)[~np.isnan(want)], want.view(np.uint32)[~np.isnan(want)])
 
 
-# from 2048 x 4096 on the launch asks for the streaming form (576 lanes): whole tiles, ragged rows and a partial
-# last block of columns, and a column count that is not made of whole vectors (the kernel falls back by itself)
-# below 4096 columns: four columns per workgroup, 64-row tiles, eight tiles' loads together (one group, several
-# groups, a partial last tile, a partial last block of columns)
+# The catalogue's choice: the operator's own launch for (9, 5) and (513, 4), column chains for the others, (2049, 4098) with
+# rows that are no whole vectors.  (The operator's own launch at such sizes: test_input_fusion_own_launch.)
 @pytest.mark.parametrize("shape", [(512, 1024), (9, 5), (1000, 300), (3, 2049), (1500, 36), (513, 4), (2048, 4096),
                                    (2500, 4100), (2049, 4098)])
 def test_input_fusion_f32_bit_exact(host, orc, stream, shape):
@@ -743,6 +770,38 @@ def test_input_fusion_16bit(host, orc, stream, dtype, shape):
     got = orc.to_float(host.input_fusion(stream, a, b, dtype), dtype)
     want = orc.to_float(orc.from_float(orc.input_fusion_f32(orc.to_float(a, dtype), orc.to_float(b, dtype)), dtype), dtype)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(100, 500), (127, 2047), (3, 17000), (20, 37008), (9, 5), (512, 1024), (700, 41), (1000, 300),
+                                       (1500, 36), (513, 4), (65, 4097), (1030, 5000), (33, 9001), (33, 25520), (129, 33001),
+                                       (2048, 8192), (2500, 8200), (2049, 8202)])
+def test_input_fusion_own_launch(host, orc, stream, dtype, rows, cols):
+    """The operator's own kernel under its own launch, on the catalogue's grid and on three workgroups, where the catalogue
+    leaves a problem to it (the first four) and where it takes the chains: four columns per workgroup with 320 lanes and
+    with 256 (one group of tiles, several, partial ones), blocks of 8, 16, 32 and 64 columns, segments of 128 bytes for
+    many rows."""
+    name = "imex_input_fusion_" + dtype
+    if (rows, cols) in ((100, 500), (127, 2047), (3, 17000), (20, 37008)):
+        assert host.variant(name, [rows, cols]) == name
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    a = orc.fill_uniform(rows * cols, dtype, 65, -5.0, 5.0).reshape(rows, cols)
+    b = orc.fill_uniform(rows * cols, dtype, 66, 0.01, 40.0).reshape(rows, cols)
+    want = orc.input_fusion_f32(wide(a), wide(b))
+    want = want if dtype == "f32" else orc.from_float(want, dtype)
+    fill = np.full(cols + 16, 3, a.dtype)
+    d_a, d_b, d_out = stream.to_device(a), stream.to_device(b), stream.to_device(fill)
+    grid, block, _ = host.launch_shape(name, [rows, cols])
+    for launch in ((grid, block), ((3, 1, 1), block), (grid, (256, 1, 1))):
+        say("%s %dx%d, %s" % (name, rows, cols, launch))
+        stream.copy(d_out, fill.ctypes.data, fill.nbytes)
+        stream.launch(name, [rows, cols], [d_a, d_b, d_out, rows, cols], grid=launch[0], block=launch[1])
+        stream.wait()
+        got = stream.from_device(d_out, fill.shape, fill.dtype)
+        assert np.array_equal(got[:cols], want), (name, launch)
+        assert np.all(got[cols:] == 3), (name, launch)
+    for p in (d_a, d_b, d_out):
+        stream.free(p)
 
 
 @pytest.mark.parametrize("shape,block", [((600, 520), 320), ((2048, 4160), 576), ((2048, 4160), 256), ((600, 520), 256)])
@@ -771,11 +830,12 @@ def test_input_fusion_any_grid(host, orc, stream, shape, block):
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,segments,extra", [(1, 1, 0), (255, 1, 1), (256, 3, -1), (257, 256, 0), (1000, 256, -7),
                                                  (127, 256, 1), (129, 512, 0), (271, 511, 3), (128, 512, 1),
-                                                 (513, 515, 5), (64, 1024, 9), (0, 4, 0)])
+                                                 (513, 515, 5), (64, 1024, 9), (0, 4, 0), (63, 1030, 3), (65, 1030, 1),
+                                                 (128, 1025, 0), (200, 1100, 5), (321, 1025, -1)])
 def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra):
-    """The fused chain and the plain sum down the columns around the tiles of rows (128, 256) and the widths of a
-    workgroup's segment (32, 64 and 128 bytes: up to 256, up to 512 and more 32-byte segments in a row), with buffers on and
-    one element off the 16-byte grid, on the catalogue's grid, on five workgroups and with lanes that the chains do not
+    """The fused chain and the plain sum down the columns around the tiles of rows (256 and 128; 64 beyond 1024 32-byte
+    segments in a row, where every step of the adder's loop hands a tile over) and the widths of a workgroup's segment (32,
+    64 and 128 bytes: up to 256, up to 512 and more segments), with buffers on and one element off the 16-byte grid, on the catalogue's grid, on five workgroups and with lanes that the chains do not
     take: the additions are in row order, so the results are the oracle's bits.  Zeros, infinities, NaN, negative and
     subnormal numbers stand under the logarithm of some columns."""
     width = 4 if dtype == "f32" else 2
