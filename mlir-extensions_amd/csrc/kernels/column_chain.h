@@ -52,7 +52,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   static constexpr int kRowsPerWave = 4 * (kWave / kLanes);     // rows of a tile that one worker wavefront takes
   static constexpr int kTileRows = kWorkers * kRowsPerWave;
   static constexpr int kThreads = (kWorkers + 1) * kWave;
-  static constexpr bool kNarrow = kInputs == 1 && kLanes == 4; // takes rows of less than a segment too
+  static constexpr bool kNarrow = kLanes == 4; // takes rows of less than a segment too
   // Floats from one column of a tile to the next, and where a column keeps its rows: four rows (a "quad") are 16 bytes,
   // and quad q of a column that lane group j wrote is at place q ^ swizzle(j) within its four.  128-bit LDS accesses
   // are served sixteen lanes at a time over 64 banks.  The adder's sixteen lanes read one quad of sixteen columns:
@@ -78,7 +78,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   // kShort: rows of fewer than 8 bytes, which a lane's loads run past: what it finds there is never stored, and at the
   // matrix's end it loads the last 8 bytes instead and moves its row's to the front.  (Rows of 8 .. 31 bytes: lanes whose
   // columns would lie past the end take the row's last ones once more.)  f32 sums of 8192 x 4 24.9 us, with a lane per column
-  // 222; 100000 x 1 266, 1766; bf16 8192 x 8 26.1, 335.
+  // 222; 100000 x 1 266, 1766; bf16 8192 x 8 26.1, 335; fused chain, four columns per workgroup before, f16 9124 x 8 84 -> 34.
   // prologue(): run by every thread while the first loads are in flight; what it leaves in LDS is there for eval.
   // eval(const Raw (&words)[kInputs][4], float (&f)[4][kPer]): four rows' values of this lane's columns.
   template <bool kShort = false, typename Prologue, typename Eval>

@@ -484,13 +484,13 @@ __device__ __forceinline__ void input_fusion_stream(const void *__restrict__ a, 
 // bytes), f32 3785 x 3480 155 -> 27 (17), f16 1052 x 5433 76 -> 11, f32 8192 x 512 87 -> 31 (the chain alone: 22), f32
 // 8192 x 8192 106 -> 91 (85).  Two workers per SIMD on segments of 64 and 128 bytes: one took 29 and 82 us on f16 3785 x
 // 3480 and f32 5550 x 5932, two take 19 and 60.
-template <Dt D, int kLanes, int kWorkers, typename Logs>
+template <Dt D, int kLanes, int kWorkers, bool kShort = false, typename Logs>
 __device__ __forceinline__ void input_fusion_chains(const void *__restrict__ a, const void *__restrict__ b,
                                                     void *__restrict__ out, int64_t rows, int64_t cols, Logs &logs, float *lds) {
   using C = ColumnChain<D, 2, kLanes, kWorkers>;
   using E = Elem<D>;
   constexpr int kPer = C::kPer;
-  C::run(a, b, out, rows, cols, 0.0f, lds, [&] { logs.stage(); }, [&](const typename C::Raw(&v)[2][4], float(&f)[4][kPer]) {
+  C::template run<kShort>(a, b, out, rows, cols, 0.0f, lds, [&] { logs.stage(); }, [&](const typename C::Raw(&v)[2][4], float(&f)[4][kPer]) {
     float x[4][kPer]; // under the logarithm
     uint32_t least = ~0u, most = 0;
 #pragma unroll
@@ -537,9 +537,9 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
                                                   void *__restrict__ out, int64_t rows, int64_t cols) {
   __shared__ __attribute__((aligned(16))) float lds[ColumnChain<D, 2, 16, 8>::kLdsFloats];
   __shared__ Logarithms<kMantissaOf<D>> logs;
-  const int64_t segments = (cols * Elem<D>::kBytes + 31) / 32;
+  const int64_t row = cols * Elem<D>::kBytes, segments = (row + 31) / 32;
   const int lanes = chain_lanes(segments), workers = lanes == 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
-  if (!chains_take<D>(rows, cols) || cols * Elem<D>::kBytes < 32 || lanes_launched() != (workers + 1) * kWave) {
+  if (!chains_take<D>(rows, cols) || (row < 8 && rows * row < 8) || lanes_launched() != (workers + 1) * kWave) {
     if (lanes_launched() < kThreads) {
       input_fusion_by_element<D>(a, b, out, rows, cols, logs);
       return;
@@ -547,6 +547,8 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
     logs.stage();
     __syncthreads();
     input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
+  } else if (lanes == 4 && row < 8) {
+    input_fusion_chains<D, 4, 4, true>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 4) {
     input_fusion_chains<D, 4, 4>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 8) {

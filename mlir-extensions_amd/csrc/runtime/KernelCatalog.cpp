@@ -411,14 +411,15 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
 
 // The fused chain with column sums: column chains, but for a few rows, where the operator's own launch has a shorter way to
 // its first and only additions.  By 300 timed problems (2 .. 12000 rows of 16 .. 300000 columns): below 2048 columns
-// from 128 rows on (f16 124 x 81: own 4.1 us, chains 4.4; f32 827 x 1592 23.2 / 6.2); rows that take workgroups of 128-byte
+// from 128 rows on (f16 124 x 81: own 4.1 us, chains 4.4; f32 827 x 1592 23.2 / 6.2), from 256 on for 16-bit rows of less
+// than a segment (f16 128 x 1 3.9 / 4.8, 300 x 12 5.4 / 4.1, 9124 x 8 84 / 34; f32 100000 x 4 857 / 267); rows that take workgroups of 128-byte
 // segments more than one round from 72 (f32) or 24 rows on (f32 33 x 25520 9.9 / 10.8; f16 20 x 37008 8.7 / 9.5; bf16 5550 x
 // 5932 449 / 42; f32 72 x 1074784 494 / 299); rows in between always (f32 2 x 7024 6.6 / 3.8).
 const char *inputFusionVariant(const Entry *e, int64_t rows, int64_t cols) {
   const bool f32 = e->shape == Shape::ColumnThreads;
   const int64_t bytes = cols * (f32 ? 4 : 2);
   if (rows == 0 || rows >= int64_t(1) << 31 || bytes >= int64_t(1) << 26 || // chains_take in column_chain.h
-      (cols < 2048 ? rows < 128 || bytes < 32 : bytes > 256 * 128 && rows < (f32 ? 72 : 24)))
+      (cols < 2048 ? rows < (f32 || bytes >= 32 ? 128 : 256) : bytes > 256 * 128 && rows < (f32 ? 72 : 24)))
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s_tall", e->name);

@@ -945,6 +945,36 @@ def test_reduce_outer_narrow_rows(host, orc, stream, dtype, cols):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cols", range(1, 17))
+def test_input_fusion_narrow_rows(host, orc, stream, dtype, cols):
+    """The same for the fused chain: rows of less than a segment, by the catalogue's choice, chains from 128 rows on (16-bit
+    rows of less than a segment: 256), and by the chains themselves; infinities and NaN stand beside the matrices and a zero under the last logarithm."""
+    name, width = "imex_input_fusion_" + dtype, 4 if dtype == "f32" else 2
+    line = 256 if width * cols < 32 and width == 2 else 128
+    assert host.variant(name, [line - 1, cols]) == name and host.variant(name, [line, cols]) == name + "_tall"
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    wide = lambda t: (t if dtype == "f32" else orc.to_float(t, dtype)).reshape(-1, cols)
+    for rows in (1, 2, 3, 5, 255, 256, 257, 258, 259, 700, 8195):
+        a = orc.fill_uniform(rows * cols, dtype, 95, -5.0, 5.0)
+        b = orc.fill_uniform(rows * cols, dtype, 96, 0.01, 40.0)
+        b[-1:] = narrow(np.zeros(1, np.float32))
+        want = narrow(orc.input_fusion_f32(wide(a), wide(b)))
+        for shift in (0, 1):
+            beside = narrow(np.resize(np.float32([np.nan, -np.inf, -1.0]), 8))
+            d_a, d_b = (stream.to_device(np.concatenate([beside[:shift], t, beside])) for t in (a, b))
+            fill = np.full(cols + 8, 3, a.dtype)
+            for form in ("", "_tall"):
+                d_out = stream.to_device(fill)
+                stream.launch(name + form, [rows, cols], [host.Ptr(p + shift * width) for p in (d_a, d_b, d_out)] + [rows, cols])
+                stream.wait()
+                got = stream.from_device(d_out, fill.shape, fill.dtype)
+                stream.free(d_out)
+                assert np.array_equal(got[shift:shift + cols], want), (name + form, rows, shift)
+                assert np.all(got[:shift] == 3) and np.all(got[shift + cols:] == 3), (name + form, rows, shift)
+            stream.free(d_a), stream.free(d_b)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,segments,extra", [(300, 3, 1), (140, 300, -3), (130, 514, 7), (70, 1030, 5)])
 def test_column_chains_in_place(host, orc, stream, dtype, rows, segments, extra):
     """A result that lies in the first or the last row of its own matrix.  On one workgroup the last block of columns, which
