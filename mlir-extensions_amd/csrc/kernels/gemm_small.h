@@ -218,6 +218,7 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
   // With eight A fragments per wavefront there is room for one set of them: each is replaced by the next step's as soon
   // as its products are issued.
   constexpr bool kOneA = FI >= 8;
+  static_assert(!(kOneA && P::kRefill), "with one set of A fragments the ring is filled in front of a step's barrier only");
   typename T::Frag af[kOneA ? 1 : 2][FI], bf[2][FJ];
   auto dma = [&](int kt, int slot) {
     opA.dma(ldsBase, slot * P::kStageBytes + kImageA, kt, steps);
