@@ -51,7 +51,8 @@ namespace {
 constexpr int kMaxThreads = 1024; // 8 or 16 wavefronts per workgroup
 constexpr int D = 64;                 // head dimension
 constexpr int kRingBytes = 128 * 1024;          // 2 stages of 64 KiB, 4 of 32 KiB or 8 of 16 KiB
-constexpr int kLdsBytes = 16 * 34 * 64 * 4;     // the ring, and after it the partial results of sixteen wavefronts
+constexpr int kLdsBytes = kRingBytes;           // the ring, and after it the partial results of up to eight wavefronts
+static_assert(kLdsBytes >= 8 * 34 * 64 * 4, "two key groups hand eight of them over, four or eight meet from eight wavefronts");
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -493,11 +494,12 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
 // Eight wavefronts on 32 queries; wavefront w takes every eighth 32-key tile.  Nobody else reads its tiles, so it
 // copies them into LDS of its own (a place of 4 KiB for K and one for V, filled again as soon as the fragments are in
 // registers) and waits for its own copies only: no barrier in the loop, and the wavefronts of a SIMD drift apart, so that
-// one's products run under the others' exponentials, where the shared ring keeps all of them in step.  68 KiB of LDS and
-// at most 128 registers let two workgroups share a CU.  Against the 32-query form of attention_tiled that it replaced
+// one's products run under the others' exponentials, where the shared ring keeps all of them in step.  (68 KiB of LDS and
+// at most 128 registers leave room for a second workgroup on the CU, which the catalogue's rule never puts there: from a
+// second one on, 64 queries walk half the keys.)  Against the 32-query form of attention_tiled that it replaced
 // (1 x 4096, 128 workgroups: 20.0 us) and 64 queries (the others): 1 x 4096 14.8 us, 4 x 2048 14.0 -> 11.0, 8 x 1024 10.0
-// -> 7.6, 4 x 512 7.1 -> 5.9, 4 x 264 7.8 -> 5.2, 256 x 32 7.3 -> 4.3; more than one workgroup on a CU is where it ends
-// (16 x 768 8.75 -> 10.0), which walk twice the keys that 64 queries do.  Bound by the softmax's instructions (about 460
+// -> 7.6, 4 x 512 7.1 -> 5.9, 4 x 264 7.8 -> 5.2, 256 x 32 7.3 -> 4.3; it ends where a CU gets more than one workgroup
+// (16 x 768 8.75 -> 10.0).  Bound by the softmax's instructions (about 460
 // cycles of issue per tile, two wavefronts on a SIMD) and, at one wavefront's 8 KiB in flight, by the copies' latency.
 // Sixteen wavefronts, or 64 queries per wavefront, were not faster.
 constexpr int kOwnKeys = 32, kOwnTile = kOwnKeys * D * 2;
