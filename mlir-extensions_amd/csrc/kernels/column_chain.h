@@ -10,10 +10,13 @@
 // values to LDS COLUMN by column, and one wavefront does nothing but add, a lane per column, four rows per LDS read.  A
 // lane of a worker loads the same 8 bytes of four consecutive rows and so holds four consecutive values of every column
 // it touches: the change of layout costs no instruction.  One barrier per tile of rows hands a tile over and the other
-// one back; loads run one tile ahead (two tiles ahead were slower, f32 fused chain of 1500 x 2048 9.1 / 10.0 us).
-// Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them
-// (f32 sums of 8192 x 4096 34.4 us, 41.8 in launch order; ordinary loads: non-temporal ones lose the line, fused chain of
-// f32 8192 x 512 50 us against 32).
+// one back; loads run one tile ahead (two tiles ahead were slower for the fused chain, whose two inputs take the registers,
+// on 12 MB that the caches hold: f32 1500 x 2048 9.1 / 10.0 us; not tried for one input from HBM).
+// Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them (in launch
+// order / so: f32 sums of 8192 x 4096 42.7 / 37.0 us, 8192 x 2048 44.1 / 25.3, bf16 8192 x 4096 44.5 / 26.3; ordinary loads:
+// non-temporal ones lose the line, fused chain of f32 8192 x 512 50 us against 32).
+// What is left: f32 8192 x 8, one workgroup, takes 24.3 us, 2.6 ns a row behind the launch.  8192 x 2048 hides its loads
+// behind that; 8192 x 4096 does not, 0.58 us per tile of 128 rows, 8 KiB in flight per CU and one memory latency.
 #ifndef IMEX_HIP_COLUMN_CHAIN_H
 #define IMEX_HIP_COLUMN_CHAIN_H
 

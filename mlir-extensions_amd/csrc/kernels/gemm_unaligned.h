@@ -14,8 +14,8 @@
 //
 // Bound by the latency of a step (load, LDS write, barrier, fragment reads), as gemm_small.h is; the vector-ALU loop
 // that took these shapes before spent 4.4 us on every sixteen k, most of it waiting for one element's load after the
-// other.  A step of 64 k takes 0.37 us on 64 x 64 tiles (0.19 with direct copies).  1001 x 1003 x 999 f16: 276 us before,
-// 10.7 here; 4097 x 4097 x 1001: 91.5 us, 368 TFLOP/s.
+// other.  A step of 64 k takes 0.37 us on 64 x 64 tiles (0.27 with direct copies; as the rules of
+// KernelCatalog.cpp have them).  1001 x 1003 x 999 f16: 276 us before, 10.5 here; 4097 x 4097 x 1001: 91.5 us, 368 TFLOP/s.
 
 #ifndef IMEX_HIP_GEMM_UNALIGNED_H
 #define IMEX_HIP_GEMM_UNALIGNED_H

@@ -457,8 +457,8 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16_de
 // form above) leaves the chip idle and waits for one slice's latency per four slices.  Column chains instead
 // (column_chain.h), whose workers have nothing to do but widen: the additions of one output are ordered, so a column costs
 // `outer` dependent additions whatever is done, 2.7 ns each here.  f32 8192 x 4096: 980 us in the plain form, 45.2 with a
-// 32-bit LDS read for every addition, 36.1 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 14.3;
-// bf16 8192 x 4096 58.0 -> 26.9, where the adder widened as well; f16 2000 x 1001 16.6 -> 8.4, 500 x 20000 9.5 -> 5.9.
+// 32-bit LDS read for every addition, 37.0 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 13.9;
+// bf16 8192 x 4096 58.0 -> 26.3, where the adder widened as well; f16 2000 x 1001 16.6 -> 8.1, 500 x 20000 9.5 -> 5.8.
 template <io::Dt D, int kLanes, int kWorkers, bool kShort = false>
 __device__ __forceinline__ void reduce_outer_chains(const void *in, void *out, int64_t outer, int64_t inner, float init, float *lds) {
   using C = ColumnChain<D, 1, kLanes, kWorkers>;
