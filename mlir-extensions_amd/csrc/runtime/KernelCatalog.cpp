@@ -242,35 +242,43 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
   return begin;
 }
 
-// Which tile a GEMM should take.  What one workgroup costs was fitted to 750 random problems (M 1 .. 4096, N 64 ..
-// 11008, K 64 .. 4096, all eight operators, operands from beyond the L2s, every tile timed on each): a launch takes
-// `constant`, a workgroup `setup` (first slab, result) plus `step` per K step, and every further workgroup that a CU gets
-// costs `setup` again and `stepMore` per step -- less than the sum of the two where workgroups share a CU (64 x 64: counted
-// by the fraction, the others by whole rounds of 256 workgroups).  Nanoseconds.  The tile with the least estimate is within
-// 0.2 % of the fastest one in the mean over those problems (at worst 11 %); examples, 256 x 256 / chosen: 256 x 256 x 256
-// 10.5 / 3.5 us (16 x 16), 1000^3 27.5 / 7.4 (64 x 64), 16 x 1680 x 3992 67.6 / 9.8 (16 x 16), 2414 x 2104 x 2208 49.1 / 36.4
-// (256 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with 128 x 128 tiles.
+// Which tile a GEMM should take.  What one workgroup costs was fitted to 4400 random problems (M 1 .. 8192, N 64 ..
+// 11008, K 32 .. 4096, all eight operators, operands from the caches and from beyond the L2s, every tile timed on each): a
+// launch takes `constant`, a workgroup `setup` (first slab) and `store` per byte of a result (storeBytes()) plus `step` per K
+// step, and every further workgroup that a CU gets costs these again and `stepMore` per step -- less than the sum of the two
+// where workgroups share a CU (64 x 64: counted by the fraction, the others by whole rounds of 256 workgroups).
+// Nanoseconds.  The tile with the least estimate is within 0.7 % of the fastest one in the mean over those problems (1.2 %
+// with constants from problems of K >= 64 alone and nothing per byte, which gave short sums too small a share of their time
+// to the result: 2168 x 4064 x 312 with A^T 18.8 us on 128 x 64, 16.6 on 256 x 256; 771 x 880 x 112 4.2 / 3.5 on 64 x 64);
+// examples, 256 x 256 / chosen: 256 x 256 x 256 10.5 / 3.5 us (16 x 16), 1000^3 27.5 / 7.4 (64 x 64), 16 x 1680 x 3992 67.6 /
+// 9.8 (16 x 16), 2414 x 2104 x 2208 49.1 / 36.4 (256 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with 128 x 128 tiles.
 struct GemmTile {
   const char *suffix;
-  int tileM, tileN, stepK, constant, setup, step, stepMore;
+  int tileM, tileN, stepK, constant, setup, store, step, stepMore;
   bool shared;
 };
-constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 4401, 8420, 610, 708, false},
-                                   {"_t256x128", 256, 128, 64, 1238, 6567, 875, 956, false},
-                                   {"_t128", 128, 128, 64, 1185, 4352, 507, 553, false},
-                                   {"_t128x64", 128, 64, 64, 660, 2993, 270, 391, false},
-                                   {"_t128x64s", 128, 64, 64, 1479, 1683, 378, 311, false},
-                                   {"_t64", 64, 64, 64, 1621, 1810, 267, 278, true},
-                                   {"_t32", 32, 64, 128, 780, 1678, 367, 339, false},
-                                   {"_t16", 16, 64, 256, 837, 2221, 591, 722, false},
-                                   {"_t16x32", 16, 32, 256, 1799, 573, 489, 397, false},
-                                   {"_t16x16", 16, 16, 256, 2285, 485, 379, 282, false}};
+constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810, false},
+                                   {"_t256x128", 256, 128, 64, 1238, 5315, 773, 717, 956, false},
+                                   {"_t128", 128, 128, 64, 1068, 3318, 313, 494, 454, false},
+                                   {"_t128x64", 128, 64, 64, 558, 2586, 125, 258, 391, false},
+                                   {"_t128x64s", 128, 64, 64, 1616, 1283, 100, 399, 311, false},
+                                   {"_t64", 64, 64, 64, 1621, 1410, 100, 259, 332, true},
+                                   {"_t32", 32, 64, 128, 814, 1512, 50, 375, 339, false},
+                                   {"_t16", 16, 64, 256, 837, 2121, 25, 574, 722, false},
+                                   {"_t16x32", 16, 32, 256, 1799, 466, 37, 489, 397, false},
+                                   {"_t16x16", 16, 16, 256, 2031, 385, 25, 379, 282, false}};
+
+// Bytes moved for an element of the result: read and written again, or written; the 16-bit result of bias and SiLU counts
+// double for its arithmetic.
+int storeBytes(const Entry *e) {
+  return strstr(e->name, "_acc") ? 8 : strstr(e->name, "f16_f16_f16") ? 2 : 4;
+}
 
 // The same for rows that are not 16-byte aligned, fitted to 70 random problems (M 1 .. 4096, N 64 .. 4096, K 64 .. 2048;
 // the choice was the faster tile on every one).  The operator itself is a loop on the vector ALUs there, 4.4 us for
-// every sixteen k: 1001 x 1003 x 999 276 us, 10.7 here; 7 x 225 x 1897 346 / 13.8; 1 x 825 x 75 17.4 / 4.1.
-constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -1030, 6410, 742, 760, false},
-                                        {"_u64", 64, 64, 64, 2230, 1790, 366, 344, true}};
+// every sixteen k: 1001 x 1003 x 999 276 us, 10.5 here; 7 x 225 x 1897 346 / 13.8; 1 x 825 x 75 17.4 / 4.1.
+constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -1030, 6410, 0, 742, 760, false},
+                                        {"_u64", 64, 64, 64, 2230, 1790, 0, 366, 344, true}};
 // Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit.
 constexpr double kUnalignedFrom = double(1 << 23);
 constexpr int64_t kUnalignedFromK = 192;
@@ -299,7 +307,7 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
     const GemmTile &t = *first;
     const double tiles = double(ceilDiv(M, t.tileM)) * double(ceilDiv(N, t.tileN)), steps = double(ceilDiv(K, t.stepK));
     const double load = t.shared ? std::max(1.0, tiles / 256.0) : std::ceil(tiles / 256.0);
-    const double ns = t.constant + load * t.setup + steps * (t.step + (load - 1.0) * t.stepMore);
+    const double ns = t.constant + load * (t.setup + t.store * storeBytes(e)) + steps * (t.step + (load - 1.0) * t.stepMore);
     if (!best || ns < least) {
       best = &t;
       least = ns;

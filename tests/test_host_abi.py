@@ -254,6 +254,20 @@ def test_reduce_outer_launch_rules(host):
     assert choice("f32", 62, 32296) == "_tall" and choice("f32", 568, 197848) == "_deep"
 
 
+def test_gemm_tile_rules(host):
+    """Tiles by size: few rows narrow ones, ordinary products 64 x 64 and up, short sums with large results 256 x 256 (f32)
+    or 128 x 64 (16-bit), short sums with small results 64 x 64."""
+    tile = lambda kind, *dims: host.variant("imex_gemm_" + kind, list(dims))[len("imex_gemm_" + kind):]
+    assert tile("f16_f16_f32", 4096, 4096, 4096) == tile("bf16_bias_silu_bf16", 4096, 11008, 4096) == ""
+    assert tile("f16_f16_f32_ta", 2168, 4064, 312) == tile("bf16_bf16_f32", 2740, 3360, 216) == ""
+    assert tile("f16_f16_f16", 3000, 1600, 48) == "_t128x64s"
+    assert tile("f16_f16_f32_tb", 1000, 1000, 1000) == tile("f16_f16_f32", 771, 880, 112) == tile("bf16_bf16_f32", 314, 2160, 72) == "_t64"
+    assert tile("bf16_bias_silu_bf16", 923, 992, 120) == "_t64"
+    assert tile("bf16_bias_silu_bf16", 16, 11008, 4096) == "_t16"
+    assert tile("f16_f16_f32", 16, 1680, 3992) == tile("f16_f16_f32", 256, 256, 256) == "_t16x16"
+    assert tile("f16_f16_f32", 1001, 1003, 999) == "_u64"
+
+
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
     """Stream.launch's fast path: 8 bytes per argument, an f32 in the low four, with _pack_params' conversions and errors."""
     class Resolver:
