@@ -10,13 +10,12 @@
 // values to LDS COLUMN by column, and one wavefront does nothing but add, a lane per column, four rows per LDS read.  A
 // lane of a worker loads the same 8 bytes of four consecutive rows and so holds four consecutive values of every column
 // it touches: the change of layout costs no instruction.  One barrier per tile of rows hands a tile over and the other
-// one back; loads run one tile ahead (two tiles ahead were slower for the fused chain, whose two inputs take the registers,
-// on 12 MB that the caches hold: f32 1500 x 2048 9.1 / 10.0 us; not tried for one input from HBM).
+// one back; loads run one tile ahead or three (kAhead).
 // Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them (in launch
 // order / so: f32 sums of 8192 x 4096 42.7 / 37.0 us, 8192 x 2048 44.1 / 25.3, bf16 8192 x 4096 44.5 / 26.3; ordinary loads:
 // non-temporal ones lose the line, fused chain of f32 8192 x 512 50 us against 32).
-// What is left: f32 8192 x 8, one workgroup, takes 24.3 us, 2.6 ns a row behind the launch.  8192 x 2048 hides its loads
-// behind that; 8192 x 4096 does not, 0.58 us per tile of 128 rows, 8 KiB in flight per CU and one memory latency.
+// What is left: f32 8192 x 8, one workgroup, takes 23.7 us, 2.6 ns a row behind the launch.  8192 x 2048 hides its loads
+// behind that (24.7); 8192 x 4096 does not, 33.3 us, 4.3 TB/s in 64-byte pieces of rows 16 KiB apart (rows of 16000 bytes 29.3).
 #ifndef IMEX_HIP_COLUMN_CHAIN_H
 #define IMEX_HIP_COLUMN_CHAIN_H
 
@@ -36,7 +35,7 @@ __device__ __forceinline__ int wide_chain_workers(int64_t segments) { return seg
 // What the chains take: a tile's rows -- 64 where a row has more than 1024 segments, 256 at most -- within 32-bit offsets of
 // its first one.
 template <io::Dt D> __device__ __forceinline__ bool chains_take(int64_t rows, int64_t cols) {
-  return cols > 0 && cols * io::Elem<D>::kBytes < int64_t(1) << 26 && rows < int64_t(1) << 31;
+  return rows > 0 && cols > 0 && cols * io::Elem<D>::kBytes < int64_t(1) << 26 && rows < int64_t(1) << 31;
 }
 
 // blockDim.x of a launch by workgroups that are all of one size, as one scalar load of the kernel's hidden arguments (whose
@@ -55,6 +54,13 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   static constexpr int kRowsPerWave = 4 * (kWave / kLanes);     // rows of a tile that one worker wavefront takes
   static constexpr int kTileRows = kWorkers * kRowsPerWave;
   static constexpr int kThreads = (kWorkers + 1) * kWave;
+  // Tiles whose loads are in flight while one is evaluated.  Three for 64-byte segments of one input, of which a CU has one
+  // workgroup: one 8 KiB tile at a time left it waiting for memory, f32 8192 x 4096 37.2 us, 33.3 so, bf16 8192 x 8000 35.1 /
+  // 29.3 (five: 34.8, 30.2).  One elsewhere: 32-byte segments wait for their additions (4041 x 1792 13.3, with three 14.2),
+  // 128-byte ones of whole 4 KiB rows ask too much of the same channels (8192 x 8192 45.7 / 50.9, of other pitches 5 %
+  // faster), several workgroups on a CU have tiles of each other's in flight (8192 x 12000 65.0 / 75.1) and two inputs
+  // take the registers (fused chain of f32 1500 x 2048 9.1 / 10.0).
+  static constexpr int kAhead = kInputs == 1 && kLanes == 8 ? 3 : 1;
   static constexpr bool kNarrow = kLanes == 4; // takes rows of less than a segment too
   // Floats from one column of a tile to the next, and where a column keeps its rows: four rows (a "quad") are 16 bytes,
   // and quad q of a column that lane group j wrote is at place q ^ swizzle(j) within its four.  128-bit LDS accesses
@@ -92,20 +98,31 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
     const int tiles = static_cast<int>((rows + kTileRows - 1) / kTileRows);
     const int lastRows = static_cast<int>(rows - int64_t(tiles - 1) * kTileRows); // of the last tile
     const uint32_t blocks = static_cast<uint32_t>((cols + kCols - 1) / kCols);
-    bool first = true;
-    for (uint32_t w = blockIdx.x; w < blocks; w += gridDim.x) {
-      // Workgroup w runs on XCD w % 8: the XCDs take contiguous shares of the segments.  (The last block of columns
-      // starts early enough to be whole.  The columns that it shares with the block before it are stored by that one only,
-      // and what it reads of them is not used: so the result may lie in a row of the matrix itself.)
-      const uint32_t xcd = w % 8, block = xcd * (blocks / 8) + min(xcd, blocks % 8) + w / 8;
-      const int64_t c0 = min(block * kCols, static_cast<uint32_t>(kNarrow ? max(cols, int64_t(kCols)) : cols) - kCols);
-      // (The compiler must not take a role's addresses out of this loop: they would stay in registers under the other role,
-      // 16 of the f32 sums' 109 and 13 of the bf16 fused chain's 135.  Four workgroups of five wavefronts on a CU leave a
-      // wavefront 96 -- f32 sums of 128 x 32768 8.0 us with three of them, 5.7 so -- and three 128: fused chain of f16 1606 x
-      // 17080 48.5, 33.8; bf16 382 x 47034 21.7, 16.9.)
-      int lane = threadIdx.x & (kWave - 1);
-      asm volatile("" : "+v"(lane));
-      if (wave < kWorkers) {
+    // Each role walks the blocks in a loop of its own: in one loop around both, the compiler keeps a role's addresses and
+    // tiles in registers under the other role, 16 of the f32 sums' 109 and 13 of the bf16 fused chain's 135.  Four
+    // workgroups of five wavefronts on a CU leave a wavefront 96 -- f32 sums of 128 x 32768 8.0 us with three of them, 5.7
+    // so -- and three 128: fused chain of f16 1606 x 17080 48.5, 33.8; bf16 382 x 47034 21.7, 16.9.
+    const int lane = threadIdx.x & (kWave - 1);
+    auto for_blocks = [&](auto &&role) {
+      bool first = true;
+      for (uint32_t w = blockIdx.x; w < blocks; w += gridDim.x) {
+        // Workgroup w runs on XCD w % 8: the XCDs take contiguous shares of the segments.  (The last block of columns
+        // starts early enough to be whole.  The columns that it shares with the block before it are stored by that one
+        // only, and what it reads of them is not used: so the result may lie in a row of the matrix itself.)
+        // 64-byte segments of rows that are whole 4 KiB meet the same half of their XCD's L2 channels in every row then; so
+        // two XCDs share twice the segments there, a line each in turn (f32 8192 x 4096 34.0 / 33.3 us, 8192 x 3072 32.6 / 31.6).
+        const uint32_t xcd = w % 8, at = w / 8;
+        uint32_t block = xcd * (blocks / 8) + min(xcd, blocks % 8) + at;
+        if (kLanes == 8 && pitch % 4096 == 0 && blocks % 32 == 0)
+          block = xcd / 2 * (blocks / 4) + at / 2 * 4 + xcd % 2 * 2 + at % 2;
+        const int64_t c0 = min(block * kCols, static_cast<uint32_t>(kNarrow ? max(cols, int64_t(kCols)) : cols) - kCols);
+        role(block, c0, first);
+        first = false;
+        handover(); // both tiles are free for the next block of columns
+      }
+    };
+    if (wave < kWorkers) {
+      for_blocks([&](uint32_t, int64_t c0, bool first) {
         const int quad = wave * (kWave / kLanes) + lane / kLanes; // rows 4 quad .. 4 quad + 3 of a tile
         const int col = kShort ? 0 : kNarrow ? min((lane % kLanes) * kPer, static_cast<int>(cols) - kPer) : (lane % kLanes) * kPer;
         const char *base[2] = {static_cast<const char *>(a) + c0 * E::kBytes, static_cast<const char *>(b) + c0 * E::kBytes};
@@ -138,28 +155,44 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
               }
             }
             eval(tile.v, f);
+            // Sixteen rows are added or none: -0 behind the last one leaves a sum as it is, whatever it is.
+            if (t == tiles - 1) { // uniform
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < kPer; ++e)
+                  f[i][e] = 4 * quad + i < lastRows ? f[i][e] : -0.0f;
+            }
 #pragma unroll
             for (int e = 0; e < kPer; ++e)
               *reinterpret_cast<f32x4 *>(dst + e * kPitch) = f32x4{f[0][e], f[1][e], f[2][e], f[3][e]};
           }
           handover(); // tile t is complete; the adder is done with tile t - 1, whose place tile t + 1 goes to
         };
-        Tile even, odd; // the loads of a tile are on their way while the one before it is evaluated
-        if (tiles > 0)
-          load(0, even);
+        Tile ring[kAhead + 1]; // the loads of kAhead tiles are on their way while the one before them is evaluated
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+          load(i, ring[i]);
         if (first) {
           prologue();
           handover();
         }
-        for (int t = 0; t < tiles; t += 2) {
-          load(t + 1, odd);
-          put(t, even);
-          if (t + 1 < tiles) { // uniform
-            load(t + 2, even);
-            put(t + 1, odd);
+        // (whole rounds as one straight line: the loads in flight at every wait are then known exactly)
+        int t = 0;
+        for (; t + kAhead < tiles; t += kAhead + 1) {
+#pragma unroll
+          for (int i = 0; i <= kAhead; ++i) {
+            load(t + i + kAhead, ring[(i + kAhead) % (kAhead + 1)]);
+            put(t + i, ring[i]);
           }
         }
-      } else {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+          if (t + i < tiles) // uniform
+            put(t + i, ring[i]);
+      });
+    } else {
+      for_blocks([&](uint32_t block, int64_t c0, bool first) {
         if (first) {
           prologue();
           handover();
@@ -167,104 +200,93 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
         __builtin_amdgcn_s_setprio(3); // the chain is the critical path
         const int col = lane % kCols;
         float acc = init;
-        if (tiles > 0) {
-          // Four groups of sixteen rows in registers: while one is added, the three after it are on their way.
-          typedef __attribute__((address_space(3))) const float LdsFloat;
-          typedef __attribute__((address_space(3))) const f32x4 LdsVec;
-          f32x4 x[4][4];
-          LdsFloat *place[4]; // of the first four quads of the 64 rows that are read
-          auto start = [&](int t) {
+        // Four groups of sixteen rows in registers: while one is added, the three after it are on their way.
+        typedef __attribute__((address_space(3))) const float LdsFloat;
+        typedef __attribute__((address_space(3))) const f32x4 LdsVec;
+        f32x4 x[4][4];
+        LdsFloat *place[4]; // of the first four quads of the 64 rows that are read
+        auto start = [&](int t) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-              place[q] = (LdsFloat *)lds + (t & 1) * kTileFloats + col * kPitch + 4 * (q ^ swizzle(col / kPer));
-          };
-          auto read = [&](int g, int at = 0) { // the g-th group of the 64 rows `at` rows on
+          for (int q = 0; q < 4; ++q)
+            place[q] = (LdsFloat *)lds + (t & 1) * kTileFloats + col * kPitch + 4 * (q ^ swizzle(col / kPer));
+        };
+        auto read = [&](int g, int at = 0) { // the g-th group of the 64 rows `at` rows on
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-              x[g][q] = *(LdsVec *)(place[q] + at + g * 16);
-            __builtin_amdgcn_sched_barrier(0);
-          };
-          auto add = [&](int g) {
+          for (int q = 0; q < 4; ++q)
+            x[g][q] = *(LdsVec *)(place[q] + at + g * 16);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](int g) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              acc = acc + x[g][q].x;
-              acc = acc + x[g][q].y;
-              acc = acc + x[g][q].z;
-              acc = acc + x[g][q].w;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          };
-          auto landed = [] { // all reads but those of the three youngest groups: one wait per group, not one per read
-            __builtin_amdgcn_s_waitcnt(0xc07f | 12 << 8);
-            __builtin_amdgcn_sched_barrier(0);
-          };
-          start(0);
-          handover(); // tile 0 is complete
-          read(0);
-          read(1);
-          read(2);
-          for (int t = 0; t + 1 < tiles; ++t) {
-#pragma unroll
-            for (int at = 0; at < kTileRows; at += 64) {
-              read(3, at);
-              landed();
-              add(0);
-              if (at + 64 == kTileRows) {
-                handover(); // everything of tile t is in registers; tile t + 1 is complete
-                start(t + 1);
-              }
-              const int next = (at + 64) % kTileRows;
-              read(0, next);
-              landed();
-              add(1);
-              read(1, next);
-              landed();
-              add(2);
-              read(2, next);
-              landed();
-              add(3);
-            }
+          for (int q = 0; q < 4; ++q) {
+            acc = acc + x[g][q].x;
+            acc = acc + x[g][q].y;
+            acc = acc + x[g][q].z;
+            acc = acc + x[g][q].w;
           }
-          int left = lastRows;
-#pragma unroll 1
-          for (; left >= 64; left -= 64) {
-            read(3);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto landed = [] { // all reads but those of the three youngest groups: one wait per group, not one per read
+          __builtin_amdgcn_s_waitcnt(0xc07f | 12 << 8);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        start(0);
+        handover(); // tile 0 is complete
+        read(0);
+        read(1);
+        read(2);
+        for (int t = 0; t + 1 < tiles; ++t) {
+#pragma unroll
+          for (int at = 0; at < kTileRows; at += 64) {
+            read(3, at);
             landed();
             add(0);
-            if (left > 64) {
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                place[q] += 64;
+            if (at + 64 == kTileRows) {
+              handover(); // everything of tile t is in registers; tile t + 1 is complete
+              start(t + 1);
             }
-            read(0); // (past the last row: some rows again, not added)
+            const int next = (at + 64) % kTileRows;
+            read(0, next);
             landed();
             add(1);
-            read(1);
+            read(1, next);
             landed();
             add(2);
-            read(2);
+            read(2, next);
             landed();
             add(3);
           }
-          read(3);
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            if (left >= 16 * g + 16) { // uniform
-              add(g);
-            } else {
-#pragma unroll
-              for (int r = 0; r < 15; ++r)
-                if (16 * g + r < left)
-                  acc = acc + x[g][r / 4][r % 4];
-            }
-          }
         }
+        int left = lastRows;
+#pragma unroll 1
+        for (; left >= 64; left -= 64) {
+          read(3);
+          landed();
+          add(0);
+          if (left > 64) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              place[q] += 64;
+          }
+          read(0); // (past the last row: some rows again, not added)
+          landed();
+          add(1);
+          read(1);
+          landed();
+          add(2);
+          read(2);
+          landed();
+          add(3);
+        }
+        read(3);
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          if (left > 16 * g) // uniform; what the last of them has past the end is -0
+            add(g);
         __builtin_amdgcn_s_setprio(0);
         if (lane < kCols && c0 + lane >= int64_t(block) * kCols && (!kNarrow || lane < cols))
           E::put(out, c0 + lane, acc);
-      }
-      first = false;
-      __syncthreads(); // both tiles are free for the next block of columns
+      });
     }
   }
 

@@ -873,6 +873,29 @@ def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("segments,extra", [(288, 1), (384, 0), (512, 0)])
+def test_column_chains_tiles_ahead(host, orc, stream, dtype, segments, extra):
+    """Sums of 64-byte segments, whose workers have three tiles of 128 rows in flight, over 1 .. 9 tiles and last tiles that
+    end on and beside the sixteen rows that are added at a time; rows of whole 4 KiB too, which pairs of XCDs share line by
+    line.  The oracle's bits, also with a sum of -0 behind which the padding of the last sixteen rows must leave no trace."""
+    cols = segments * (32 // (4 if dtype == "f32" else 2)) + extra
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    a = orc.fill_uniform(1153 * cols, dtype, 63, -5.0, 5.0).reshape(1153, cols)
+    a[:, 5] = narrow(np.full(1, -0.0, np.float32))
+    d_in, d_out = stream.to_device(a), stream.alloc(cols * a.itemsize)
+    for rows in (1, 128, 143, 257, 384, 385, 400, 511, 513, 640, 769, 1000, 1153):
+        say("%d x %d" % (rows, cols))
+        for grid in (None, (7, 1, 1)):
+            stream.launch("imex_reduce_outer_%s_tall" % dtype, [rows, cols], [d_in, d_out, rows, cols, -0.0], grid=grid)
+            stream.wait()
+            got = stream.from_device(d_out, (cols,), a.dtype)
+            want = narrow(orc.reduce_outer_f32(wide(a[:rows]), -0.0))
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (rows, grid)
+    stream.free(d_in), stream.free(d_out)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(150, 41), (130, 2100), (40, 5000), (129, 3)])
 def test_input_fusion_with_any_block(host, orc, stream, dtype, rows, cols):
     """Launches with fewer lanes than a form's tiles are filled by, with a number that no form asks for, and on two
