@@ -7,15 +7,17 @@
 // loads take any address, so a slab goes through registers.
 //
 //   loads       16 bytes per lane at the element's own (2-byte aligned) address, D slabs in flight in registers;
-//   edges       a piece that would stick out of its row -- the last step of a k-contiguous operand, the last tile
-//               column of a strided one -- is loaded from the last 16 bytes of the row and shifted down, zeros
-//               following: no address leaves the matrix, and nothing beyond K is multiplied by anything but zero;
+//   edges       in the last step, a piece that would stick out of its row is loaded from the last 16 bytes of the row and
+//               shifted down, zeros following: no address leaves the matrix, and nothing beyond K is multiplied by
+//               anything but zero.  In the steps before it a strided operand's last pieces run into the next row: what
+//               they find there lies in columns that are never stored.  (Shifting them in every step held up the whole
+//               launch for the last tile column: f16 1001 x 1003 x 999 10.45 us, 9.5 so; A^T 11.7 / 9.7);
 //   LDS         two slots: slab t + 2 is written to the slot that step t's fragments have been read from.
 //
 // Bound by the latency of a step (load, LDS write, barrier, fragment reads), as gemm_small.h is; the vector-ALU loop
 // that took these shapes before spent 4.4 us on every sixteen k, most of it waiting for one element's load after the
 // other.  A step of 64 k takes 0.37 us on 64 x 64 tiles (0.27 with direct copies; as the rules of
-// KernelCatalog.cpp have them).  1001 x 1003 x 999 f16: 276 us before, 10.5 here; 4097 x 4097 x 1001: 91.5 us, 368 TFLOP/s.
+// KernelCatalog.cpp have them).  1001 x 1003 x 999 f16: 276 us before, 9.5 here.
 
 #ifndef IMEX_HIP_GEMM_UNALIGNED_H
 #define IMEX_HIP_GEMM_UNALIGNED_H
@@ -46,9 +48,8 @@ template <typename T, bool kStrided, int TR, int BK> struct UnalignedOperand : S
   int64_t stepBytes;       // bytes per step in memory
   uint32_t off[kCopies];   // per-lane byte offsets from the step's base
   uint32_t offT[kCopies];  // the same for the last step (k-contiguous: from step 0's base)
-  int shift[kCopies];      // places by which the piece has to move down (k-contiguous: in the last step)
+  int shift[kCopies];      // places by which the piece has to move down in the last step
   int put;                 // per-lane LDS address of copy 0 inside the image
-  bool edge;               // strided: this tile sticks out of the rows
 
   // K >= 8, and ld >= 8 where kStrided; ld < 2^22 keeps the offsets below 2^30
   __device__ __forceinline__ void setup(const uint16_t *ptr, int64_t ld, int64_t first, int64_t rows, int w0, int wave,
@@ -59,7 +60,6 @@ template <typename T, bool kStrided, int TR, int BK> struct UnalignedOperand : S
       const int last = int(min(rows - first, int64_t(TR))) - 1;
       from = reinterpret_cast<const char *>(ptr + first * ld);
       stepBytes = BK * 2;
-      edge = false;
 #pragma unroll
       for (int q = 0; q < kCopies; ++q) {
         const int id = wave * kCopies + q, slab = id / (TR / 8), row = (id % (TR / 8)) * 8 + (lane >> 3);
@@ -74,14 +74,13 @@ template <typename T, bool kStrided, int TR, int BK> struct UnalignedOperand : S
       constexpr int kRow = TR * 2, kChunks = kRow / 16; // bytes and 16-byte chunks per k row
       from = reinterpret_cast<const char *>(ptr);
       stepBytes = BK * ld * 2;
-      edge = first + TR > ld;
 #pragma unroll
       for (int q = 0; q < kCopies; ++q) {
         const int row = (wave * kCopies + q) * (1024 / kRow) + lane / kChunks, chunk = lane % kChunks;
         const int pair = (chunk >> 1) ^ pair_swizzle<TR / 16>(row);
         const int64_t col = first + pair * 16 + (chunk & 1) * 8, at = min(col, ld - 8);
         shift[q] = int(col - at);
-        off[q] = (uint32_t(row) * uint32_t(ld) + uint32_t(at)) * 2;
+        off[q] = (uint32_t(row) * uint32_t(ld) + uint32_t(col < ld ? col : at)) * 2; // (another row follows this one)
         offT[q] = (uint32_t(min(row, kRem - 1)) * uint32_t(ld) + uint32_t(at)) * 2;
       }
     }
@@ -100,14 +99,14 @@ template <typename T, bool kStrided, int TR, int BK> struct UnalignedOperand : S
   }
   __device__ __forceinline__ void store(u32x4 (&r)[kCopies], char *image, int slab, int steps, int kRem) const {
     const bool tail = slab == steps - 1;
-    if (kStrided ? tail || edge : tail) {
+    if (tail) {
 #pragma unroll
       for (int q = 0; q < kCopies; ++q) {
         int s = shift[q];
         if constexpr (kStrided) {
           constexpr int kRow = TR * 2;
           const int row = (put + q * 1024) / kRow;
-          s = tail && row >= kRem ? 8 : s;
+          s = row >= kRem ? 8 : s;
         }
         r[q] = shift_down(r[q], s);
       }

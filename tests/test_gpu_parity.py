@@ -1488,6 +1488,24 @@ def test_gemm_unaligned_rows(host, orc, stream, tile, M, N, K):
             assert np.array_equal(got, want + (7 if which == "acc" else 0)), name
 
 
+@pytest.mark.parametrize("tile,M,N,K", [("_u64", 67, 131, 257), ("_u64", 65, 71, 128), ("_u128", 135, 257, 193), ("_u128", 9, 13, 64)])
+def test_gemm_unaligned_last_pieces(host, orc, stream, tile, M, N, K):
+    """A strided operand's pieces at the end of a row run into the next one: infinities at the front of every row reach the
+    results of those columns (rows, for A stored [K,M]) only.  Integer operands, exact sums."""
+    inf = 0x7c00
+    for which in ("plain", "ta"):
+        a = orc.fill_int(M * K, "f16", 95, -1, 1).reshape(M, K)
+        b = orc.fill_int(K * N, "f16", 96, -1, 1).reshape(K, N)
+        b[:, :7] = inf
+        if which == "ta":
+            a[:7] = inf
+        fa, fb = orc.to_float(a, "f16").astype(np.float64), orc.to_float(b, "f16").astype(np.float64)
+        first = 7 if which == "ta" else 0
+        name = "imex_gemm_f16_f16_f32" + ("_ta" if which == "ta" else "") + tile
+        got = _gemm_guarded(host, stream, name, np.ascontiguousarray(a.T) if which == "ta" else a, b, M, N, K)
+        assert np.array_equal(got[first:, 7:], fa[first:] @ fb[:, 7:]), name
+
+
 @pytest.mark.parametrize("tile,M,N,K", [("_t128", 260, 392, 136), ("_t128x64", 260, 200, 136), ("_t64", 136, 200, 264),
                                         ("_t32", 104, 136, 264), ("_t16", 40, 200, 520), ("_u128", 259, 391, 135),
                                         ("_t256x128", 520, 264, 136), ("_t16x32", 40, 104, 520), ("_t16x16", 24, 56, 776),
