@@ -109,13 +109,29 @@
  *       would leave much of the chip idle
  *                                                          dims = {M, N, K}
  *   imex_gemm_f16_f16_f32_u128, imex_gemm_f16_f16_f32_u64
+ *   imex_gemm_f16_f16_f32_u32, imex_gemm_f16_f16_f32_u16x32,
+ *   imex_gemm_f16_f16_f32_u16x16
  *   imex_gemm_f16_f16_f32_acc_u128, imex_gemm_f16_f16_f32_acc_u64
+ *   imex_gemm_f16_f16_f32_acc_u32, imex_gemm_f16_f16_f32_acc_u16x32,
+ *   imex_gemm_f16_f16_f32_acc_u16x16
  *   imex_gemm_bf16_bf16_f32_u128, imex_gemm_bf16_bf16_f32_u64
+ *   imex_gemm_bf16_bf16_f32_u32, imex_gemm_bf16_bf16_f32_u16x32,
+ *   imex_gemm_bf16_bf16_f32_u16x16
  *   imex_gemm_bf16_bf16_f32_acc_u128, imex_gemm_bf16_bf16_f32_acc_u64
+ *   imex_gemm_bf16_bf16_f32_acc_u32, imex_gemm_bf16_bf16_f32_acc_u16x32,
+ *   imex_gemm_bf16_bf16_f32_acc_u16x16
  *   imex_gemm_f16_f16_f16_u128, imex_gemm_f16_f16_f16_u64
+ *   imex_gemm_f16_f16_f16_u32, imex_gemm_f16_f16_f16_u16x32,
+ *   imex_gemm_f16_f16_f16_u16x16
  *   imex_gemm_f16_f16_f32_tb_u128, imex_gemm_f16_f16_f32_tb_u64
+ *   imex_gemm_f16_f16_f32_tb_u32, imex_gemm_f16_f16_f32_tb_u16x32,
+ *   imex_gemm_f16_f16_f32_tb_u16x16
  *   imex_gemm_f16_f16_f32_ta_u128, imex_gemm_f16_f16_f32_ta_u64
+ *   imex_gemm_f16_f16_f32_ta_u32, imex_gemm_f16_f16_f32_ta_u16x32,
+ *   imex_gemm_f16_f16_f32_ta_u16x16
  *   imex_gemm_bf16_bias_silu_bf16_u128, imex_gemm_bf16_bias_silu_bf16_u64
+ *   imex_gemm_bf16_bias_silu_bf16_u32, imex_gemm_bf16_bias_silu_bf16_u16x32,
+ *   imex_gemm_bf16_bias_silu_bf16_u16x16
  *       the operator without the suffix, same arguments, on the matrix cores for operands whose rows are not 16-byte
  *       aligned (tiles of 128 x 128, 64 x 64); f32 sums in another order than the operator's own sequential one
  *                                                          dims = {M, N, K}

@@ -62,7 +62,10 @@ struct Entry {
       {NAME "_t16x32", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                            \
       {NAME "_t16x16", SIGNATURE, Module::GemmSmall, Shape::GemmSmall, 3},                                            \
       {NAME "_u128", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3},                                      \
-      {NAME "_u64", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3}
+      {NAME "_u64", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3},                                       \
+      {NAME "_u32", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3},                                       \
+      {NAME "_u16x32", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3},                                    \
+      {NAME "_u16x16", SIGNATURE, Module::GemmUnaligned, Shape::GemmUnaligned, 3}
 
 const Entry kEntries[] = {
     {"imex_relu_f32", "(in: f32*, out: f32*, n: i64)", Module::Eltwise, Shape::Eltwise32, 1},
@@ -274,11 +277,15 @@ int storeBytes(const Entry *e) {
   return strstr(e->name, "_acc") ? 8 : strstr(e->name, "f16_f16_f16") ? 2 : 4;
 }
 
-// The same for rows that are not 16-byte aligned, fitted to 70 random problems (M 1 .. 4096, N 64 .. 4096, K 64 .. 2048;
-// the choice was the faster tile on every one).  The operator itself is a loop on the vector ALUs there, 4.4 us for
-// every sixteen k: 1001 x 1003 x 999 276 us, 10.5 here; 7 x 225 x 1897 346 / 13.8; 1 x 825 x 75 17.4 / 4.1.
-constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -1030, 6410, 0, 742, 760, false},
-                                        {"_u64", 64, 64, 64, 2230, 1790, 0, 366, 344, true}};
+// The same for rows that are not 16-byte aligned, fitted to 2600 random problems of the seven operators without a bias (M 1 ..
+// 4096, N 64 .. 4096, K 64 .. 2048, N and K odd); over 420 others the choice is 0.5 % from the fastest tile in the mean, and
+// 20 % faster than the better one of 128 x 128 and 64 x 64.  The operator itself is a loop on the vector ALUs there, 4.4 us
+// for every sixteen k: 1001 x 1003 x 999 276 us, 9.5 here (64 x 64); 131 x 133 x 999 8.8 with 64 x 64, 4.7 with 16 x 16.
+constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -568, 4171, 645, 731, 589, false},
+                                        {"_u64", 64, 64, 64, 2399, 413, 233, 350, 306, false},
+                                        {"_u32", 32, 64, 128, 2564, 464, 141, 492, 456, false},
+                                        {"_u16x32", 16, 32, 256, 2842, 0, 105, 591, 611, false},
+                                        {"_u16x16", 16, 16, 256, 2485, 50, 96, 467, 471, false}};
 // Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit.
 constexpr double kUnalignedFrom = double(1 << 23);
 constexpr int64_t kUnalignedFromK = 192;

@@ -1535,6 +1535,16 @@ def test_gemm_tiles_walk_and_any_address(host, orc, stream, tile, M, N, K):
             assert np.all(got[m * N:] == 9), (name, shifted, grid)
 
 
+@pytest.mark.parametrize("tile", ["_u32", "_u16x32", "_u16x16"])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (9, 11, 13), (16, 32, 256), (15, 17, 255), (33, 65, 129), (17, 31, 257), (65, 129, 600)])
+def test_gemm_unaligned_narrow_tiles(host, orc, stream, tile, M, N, K):
+    """The same for the narrow tiles, around their sizes and their steps of 128 and 256 k, and walked by two workgroups."""
+    test_gemm_unaligned_rows(host, orc, stream, tile, M, N, K)
+    test_gemm_unaligned_last_pieces(host, orc, stream, tile, M, N, K)
+    if K > 256:
+        test_gemm_tiles_walk_and_any_address(host, orc, stream, tile, M, N, K)
+
+
 @pytest.mark.parametrize("which", ["", "_ta", "_tb"])
 def test_gemm_unaligned_rows_chosen(host, orc, stream, which):
     """What the operator takes at an ordinary odd size, random operands: against 64 bits within the rounding of 32-bit
