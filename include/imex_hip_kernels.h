@@ -133,7 +133,7 @@
  *   imex_gemm_bf16_bias_silu_bf16_u32, imex_gemm_bf16_bias_silu_bf16_u16x32,
  *   imex_gemm_bf16_bias_silu_bf16_u16x16
  *       the operator without the suffix, same arguments, on the matrix cores for operands whose rows are not 16-byte
- *       aligned (tiles of 128 x 128, 64 x 64); f32 sums in another order than the operator's own sequential one
+ *       aligned (tiles of 128 x 128, 64 x 64, 32 x 64, 16 x 32, 16 x 16); f32 sums in another order than the operator's own sequential one
  *                                                          dims = {M, N, K}
  *   imex_gemm_bf16_bias_silu_bf16_streamk  (A, B, bias, out, M:i64, N:i64, K:i64, workspace, epoch:i64, spin_limit:i64)
  *       the same operator with the last, partial round of tiles split along K over all workgroups (no

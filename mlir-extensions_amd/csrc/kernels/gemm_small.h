@@ -297,10 +297,13 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
 }
 
 // Tile number -> tile, as tile_origin of gemm_tile.h: the workgroups of an XCD (ids congruent mod 8) take a compact
-// band of tiles, four tile rows high.
+// band of tiles, four tile rows high; as many tiles for each XCD, or one more.
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t first_tile_of_xcd(uint32_t xcd, uint32_t tiles) {
+  return xcd * (tiles / kXcds) + min(xcd, tiles % kXcds);
+}
 template <typename P> __device__ __forceinline__ TileOrigin small_tile_origin(uint32_t id, uint32_t tilesM, uint32_t tilesN) {
-  const uint32_t tiles = tilesM * tilesN, whole = tiles / 8 * 8;
-  const uint32_t pid = id < whole ? (id % 8) * (whole / 8) + id / 8 : id;
+  const uint32_t pid = first_tile_of_xcd(id % kXcds, tilesM * tilesN) + id / kXcds;
   const uint32_t group = kGroupM * tilesN, band = pid / group, in = pid - band * group;
   const uint32_t rows = min(tilesM - band * kGroupM, uint32_t(kGroupM));
   uint32_t row = in % kGroupM, col = in / kGroupM;
@@ -313,6 +316,69 @@ template <typename P> __device__ __forceinline__ TileOrigin small_tile_origin(ui
   return TileOrigin{int64_t(band * kGroupM + row) * P::TM, int64_t(col) * P::TN};
 }
 
+// Workgroups without a tile fetch what the other workgroups of their XCD are going to read.  A CU draws no more than 50
+// GB/s from beyond its L2 (a limit on requests: 16 GB/s in 32-byte pieces of rows, 29 in 64-byte ones, 51 in lines) but 180
+// from it, so a few workgroups that walk a long K alone wait for memory while the rest of the chip is idle: that rest brings
+// the operands of an XCD's tiles into its L2, in the order of K, 512 k at a time, as copies into LDS that nobody reads.
+// bf16 16 x 2048 x 4096 from HBM 14.0 -> 7.2 us (6.0 when the L2s have it), from the 256 MiB cache 11.3 -> 7.1; 16 x 1680 x
+// 3992 9.2 -> 6.6.  Nothing depends on it but the time: if workgroups lay elsewhere than on XCD id % 8, lines would be
+// fetched that nobody asks for.
+template <bool kAT, bool kBT, typename P>
+__device__ __forceinline__ void fetch_ahead(const uint16_t *A, const uint16_t *B, uint32_t M, uint32_t N, uint32_t K,
+                                            char *lds, uint32_t id, uint32_t tilesM, uint32_t tilesN, uint32_t workgroups) {
+  constexpr uint32_t kChunk = 512;
+  const uint32_t tiles = tilesM * tilesN, xcd = id % kXcds;
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // the XCD's tiles, this workgroup's number among those of the XCD that fetch, and their wavefronts
+  const uint32_t from = first_tile_of_xcd(xcd, tiles), to = first_tile_of_xcd(xcd + 1, tiles);
+  const uint32_t rank = id / kXcds - (to - from), turns = ((workgroups + kXcds - 1 - xcd) / kXcds - (to - from)) * kWaves;
+  if (turns < 8 * kWaves) // too few: the others would wait for them (200 x 301 x 901 on 247 of 256 workgroups 5 us, 34 so)
+    return;
+  LdsChar *sink = (LdsChar *)lds + wave * 1024;
+  // What the tiles read: rows m0 .. m1 - 1 of A, columns n0 .. n1 - 1 of B, for those of the first band of tile rows and for
+  // the others (of one band, or all columns of more).
+  struct Block {
+    uint32_t m0, m1, n0, n1;
+  };
+  const uint32_t band = kGroupM * tilesN, turnover = min((from / band + 1) * band, to);
+  auto block = [&](uint32_t p, uint32_t end) {
+    if (p >= end)
+      return Block{0, 0, 0, 0};
+    const uint32_t first = p / band, last = (end - 1) / band, rows = min(tilesM - first * kGroupM, uint32_t(kGroupM));
+    const uint32_t col = (p - first * band) / rows, lastCol = first == last ? (end - 1 - first * band) / rows : tilesN - 1;
+    return Block{first * kGroupM * P::TM, min((last + 1) * kGroupM * P::TM, M), first == last ? col * P::TN : 0,
+                 min((lastCol + 1) * P::TN, N)};
+  };
+  const Block blocks[2] = {block(from, turnover), block(turnover, to)};
+  uint32_t turn;
+  // Rows (k-contiguous) or columns (strided) first .. last - 1 of an operand, ks of its k from k0 on: a row, or a k row, for
+  // each wavefront in turn.  (Few instructions per copy: with addresses in 64 bits the copies of 200 bytes and less, 0.15 us
+  // each, took longer than the tiles.)
+  auto fetch = [&](const uint16_t *ptr, bool strided, uint32_t ld, uint32_t first, uint32_t last, uint32_t k0, uint32_t ks) {
+    const uint32_t count = strided ? ks : last - first, bytes = (strided ? last - first : ks) * 2, pitch = ld * 2;
+    if (first >= last || uint64_t(count) * pitch >= kOutOfRange)
+      return;
+    const uint16_t *base = ptr + (strided ? uint64_t(k0) * ld + first : uint64_t(first) * ld + k0);
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0, int((count - 1) * pitch + bytes), 0x00020000);
+    for (; turn < count; turn += turns)
+      for (uint32_t b = 0; b < bytes; b += 1024)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, sink, 16, b + lane * 16 < bytes ? b + lane * 16 : kOutOfRange,
+                                                 turn * pitch, 0, 0);
+    turn -= count;
+  };
+  for (uint32_t k0 = 0; k0 < K; k0 += kChunk) {
+    const uint32_t ks = min(K - k0, kChunk);
+    turn = rank * kWaves + wave;
+#pragma unroll
+    for (const Block &b : blocks) {
+      fetch(A, kAT, kAT ? M : K, b.m0, b.m1, k0, ks);
+      fetch(B, !kBT, kBT ? K : N, b.n0, b.n1, k0, ks);
+    }
+  }
+  wait_vmcnt<0>(); // the copies' place in LDS is given back with the workgroup
+}
+
 template <typename T, bool kAT, bool kBT, typename P, typename Epi>
 __device__ __forceinline__ void gemm_small_entry(const uint16_t *A, const uint16_t *B, int64_t M, int64_t N, int64_t K,
                                                  Epi epi) {
@@ -323,7 +389,12 @@ __device__ __forceinline__ void gemm_small_entry(const uint16_t *A, const uint16
   }
   const int tilesM = int((M + P::TM - 1) / P::TM), tilesN = int((N + P::TN - 1) / P::TN);
   const int tiles = tilesM * tilesN, workgroups = gridDim.x * gridDim.y;
-  for (int id = blockIdx.y * gridDim.x + blockIdx.x; id < tiles; id += workgroups) {
+  int id = blockIdx.y * gridDim.x + blockIdx.x;
+  if (id >= tiles) {
+    fetch_ahead<kAT, kBT, P>(A, B, uint32_t(M), uint32_t(N), uint32_t(K), lds, id, tilesM, tilesN, workgroups);
+    return;
+  }
+  for (; id < tiles; id += workgroups) {
     const TileOrigin o = small_tile_origin<P>(id, tilesM, tilesN);
     gemm_small_tile<T, kAT, kBT, P, Epi>(A, B, M, N, K, epi, lds, o.m0, o.n0);
     if (id + workgroups < tiles)

@@ -2,7 +2,8 @@
 // with tiles of 256 x 128, 128 x 128, 128 x 64, 64 x 64, 32 x 64, 16 x 64, 16 x 32 and 16 x 16 outputs.
 // imexHipKernelVariant says which of them a problem should take.
 //
-// Launch: block (512,1,1); grid (ceil(M / TM) * ceil(N / TN),1,1); workgroups stride, so any grid is correct.
+// Launch: block (512,1,1); grid (ceil(M / TM) * ceil(N / TN),1,1), or 256 workgroups where those without a tile pay as ones
+// that fetch for the others (fetch_ahead; fetchesAhead in KernelCatalog.cpp); workgroups stride, so any grid is correct.
 
 #include "gemm_small.h"
 

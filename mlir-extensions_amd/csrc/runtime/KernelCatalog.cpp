@@ -255,21 +255,38 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
 // to the result: 2168 x 4064 x 312 with A^T 18.8 us on 128 x 64, 16.6 on 256 x 256; 771 x 880 x 112 4.2 / 3.5 on 64 x 64);
 // examples, 256 x 256 / chosen: 256 x 256 x 256 10.5 / 3.5 us (16 x 16), 1000^3 27.5 / 7.4 (64 x 64), 16 x 1680 x 3992 67.6 /
 // 9.8 (16 x 16), 2414 x 2104 x 2208 49.1 / 36.4 (256 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with 128 x 128 tiles.
+//
+// Workgroups that fetch for others (fetch_ahead in gemm_small.h) change what a step costs: stepAhead per step, aheadMib per
+// MiB of operands and `ahead` once, where it is worth more than the launch of 256 workgroups.  From 2100 other problems,
+// operands from beyond the L2s (us without / with, from HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x
+// 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from the 256 MiB cache 11.3 / 7.1 for the second): the launches that
+// get them took 0.90 of their time, and with the tiles chosen by these numbers products of bias and SiLU 0.95, others 0.99.
+// Not below 768 k or 2 MiB, which are there before a helper could fetch them (K = 512 .. 767: 1.00), nor above 32 MiB, which
+// HBM's rate bounds (32 .. 48 MiB: 1.01), with fewer than 96 helpers (176 .. 192 tiles: up to 1.4) or for 128 x 128 tiles and
+// larger, which their own steps bound (above 16 MiB 1.03 .. 1.04).
 struct GemmTile {
   const char *suffix;
   int tileM, tileN, stepK, constant, setup, store, step, stepMore;
   bool shared;
+  int stepAhead, aheadMib, ahead; // (0: as without)
 };
-constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810, false},
-                                   {"_t256x128", 256, 128, 64, 1238, 5315, 773, 717, 956, false},
-                                   {"_t128", 128, 128, 64, 1068, 3318, 313, 494, 454, false},
-                                   {"_t128x64", 128, 64, 64, 558, 2586, 125, 258, 391, false},
-                                   {"_t128x64s", 128, 64, 64, 1616, 1283, 100, 399, 311, false},
-                                   {"_t64", 64, 64, 64, 1621, 1410, 100, 259, 332, true},
-                                   {"_t32", 32, 64, 128, 814, 1512, 50, 375, 339, false},
-                                   {"_t16", 16, 64, 256, 837, 2121, 25, 574, 722, false},
-                                   {"_t16x32", 16, 32, 256, 1799, 466, 37, 489, 397, false},
-                                   {"_t16x16", 16, 16, 256, 2031, 385, 25, 379, 282, false}};
+constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810, false, 0, 0, 0},
+                                   {"_t256x128", 256, 128, 64, 1238, 5315, 773, 717, 956, false, 0, 0, 0},
+                                   {"_t128", 128, 128, 64, 1068, 3318, 313, 494, 454, false, 0, 0, 0},
+                                   {"_t128x64", 128, 64, 64, 558, 2586, 125, 258, 391, false, 0, 0, 0},
+                                   {"_t128x64s", 128, 64, 64, 1616, 1283, 100, 399, 311, false, 0, 0, 0},
+                                   {"_t64", 64, 64, 64, 1621, 1410, 100, 259, 332, true, 181, 23, -171},
+                                   {"_t32", 32, 64, 128, 814, 1512, 50, 375, 339, false, 225, 52, 966},
+                                   {"_t16", 16, 64, 256, 837, 2121, 25, 574, 722, false, 370, 69, 309},
+                                   {"_t16x32", 16, 32, 256, 1799, 466, 37, 489, 397, false, 196, 70, 889},
+                                   {"_t16x16", 16, 16, 256, 2031, 385, 25, 379, 282, false, 146, 94, 761}};
+
+// Whether workgroups without a tile are launched to fetch what the others read.
+bool fetchesAhead(const GemmTile &t, int64_t M, int64_t N, int64_t K) {
+  const double mib = 2.0 * double(K) * (double(M) + double(N)) / (1 << 20);
+  return K >= 768 && mib >= 2.0 && mib <= 32.0 && t.tileM * t.tileN <= 128 * 64 &&
+         ceilDiv(M, t.tileM) * ceilDiv(N, t.tileN) <= 160;
+}
 
 // Bytes moved for an element of the result: read and written again, or written; the 16-bit result of bias and SiLU counts
 // double for its arithmetic.
@@ -281,14 +298,17 @@ int storeBytes(const Entry *e) {
 // 4096, N 64 .. 4096, K 64 .. 2048, N and K odd); over 420 others the choice is 0.5 % from the fastest tile in the mean, and
 // 20 % faster than the better one of 128 x 128 and 64 x 64.  The operator itself is a loop on the vector ALUs there, 4.4 us
 // for every sixteen k: 1001 x 1003 x 999 276 us, 9.5 here (64 x 64); 131 x 133 x 999 8.8 with 64 x 64, 4.7 with 16 x 16.
-constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -568, 4171, 645, 731, 589, false},
-                                        {"_u64", 64, 64, 64, 2399, 413, 233, 350, 306, false},
-                                        {"_u32", 32, 64, 128, 2564, 464, 141, 492, 456, false},
-                                        {"_u16x32", 16, 32, 256, 2842, 0, 105, 591, 611, false},
-                                        {"_u16x16", 16, 16, 256, 2485, 50, 96, 467, 471, false}};
+constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -568, 4171, 645, 731, 589, false, 0, 0, 0},
+                                        {"_u64", 64, 64, 64, 2399, 413, 233, 350, 306, false, 0, 0, 0},
+                                        {"_u32", 32, 64, 128, 2564, 464, 141, 492, 456, false, 0, 0, 0},
+                                        {"_u16x32", 16, 32, 256, 2842, 0, 105, 591, 611, false, 0, 0, 0},
+                                        {"_u16x16", 16, 16, 256, 2485, 50, 96, 467, 471, false, 0, 0, 0}};
 // Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit.
 constexpr double kUnalignedFrom = double(1 << 23);
 constexpr int64_t kUnalignedFromK = 192;
+// The few that are smaller still but have longer sums keep the bits that 64 x 64 tiles give them (101 x 101 x 193 4.9 us, 3.6
+// with 16 x 16).
+constexpr double kUnalignedNarrowFrom = double(1 << 21);
 
 // The tile that the name of a GemmSmall or GemmUnaligned entry ends in.
 const GemmTile &tileOf(const Entry *e) {
@@ -307,6 +327,8 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
         (K < kUnalignedFromK && double(M) * double(N) * double(K) < kUnalignedFrom))
       return e->name;
     first = std::begin(kUnalignedTiles), last = std::end(kUnalignedTiles);
+    if (double(M) * double(N) * double(K) < kUnalignedNarrowFrom)
+      last = first + 2;
   }
   const GemmTile *best = nullptr;
   double least = 0.0;
@@ -314,7 +336,10 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
     const GemmTile &t = *first;
     const double tiles = double(ceilDiv(M, t.tileM)) * double(ceilDiv(N, t.tileN)), steps = double(ceilDiv(K, t.stepK));
     const double load = t.shared ? std::max(1.0, tiles / 256.0) : std::ceil(tiles / 256.0);
-    const double ns = t.constant + load * (t.setup + t.store * storeBytes(e)) + steps * (t.step + (load - 1.0) * t.stepMore);
+    const double once = t.constant + load * (t.setup + t.store * storeBytes(e));
+    double ns = once + steps * (t.step + (load - 1.0) * t.stepMore);
+    if (t.stepAhead && fetchesAhead(t, M, N, K))
+      ns = std::min(ns, once + steps * t.stepAhead + 2.0 * double(K) * (double(M) + double(N)) / (1 << 20) * t.aheadMib + t.ahead);
     if (!best || ns < least) {
       best = &t;
       least = ns;
@@ -700,10 +725,12 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
     const int64_t M = dims[0], N = dims[1], K = dims[2];
     const GemmTile &tile = tileOf(e);
     block[0] = 512;
-    grid[0] = gridFor(mfmaTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)
-                          ? ceilDiv(M, tile.tileM) * ceilDiv(N, tile.tileN)
-                          : ceilDiv(M, 128) * ceilDiv(N, 128),
-                      512);
+    if (mfmaTakes(strstr(e->name, "_ta_") != nullptr, strstr(e->name, "_tb_") != nullptr, M, N, K)) {
+      const size_t tiles = ceilDiv(M, tile.tileM) * ceilDiv(N, tile.tileN);
+      grid[0] = fetchesAhead(tile, M, N, K) ? 256 : gridFor(tiles, 512);
+    } else {
+      grid[0] = gridFor(ceilDiv(M, 128) * ceilDiv(N, 128), 512);
+    }
     break;
   }
   case Shape::GemmUnaligned: {

@@ -1545,6 +1545,34 @@ def test_gemm_unaligned_narrow_tiles(host, orc, stream, tile, M, N, K):
         test_gemm_tiles_walk_and_any_address(host, orc, stream, tile, M, N, K)
 
 
+@pytest.mark.parametrize("tile", ["_t128x64", "_t128x64s", "_t64", "_t32", "_t16", "_t16x32", "_t16x16"])
+@pytest.mark.parametrize("M,N,K", [(40, 232, 4104), (8, 1096, 1032), (1000, 24, 1032), (264, 72, 3592), (336, 112, 2504)])
+def test_gemm_workgroups_that_fetch(host, orc, stream, tile, M, N, K):
+    """Launches with workgroups that have no tile and fetch what the others read: one and several bands of tile rows for an
+    XCD, bands that it shares with the next, tiles that eight does not divide, ragged edges.  Integer operands, exact sums."""
+    launched = 0
+    for which in ("plain", "acc", "ta", "tb", "f16"):
+        kind = {"plain": "bf16_bf16_f32", "acc": "f16_f16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb", "f16": "f16_f16_f16"}[which]
+        name, dtype = "imex_gemm_" + kind + tile, "bf16" if which == "plain" else "f16"
+        n = N - 3 if which == "tb" else N
+        launched += host.launch_shape(name, [M, n, K])[0][0] == 256
+        a, b = orc.fill_int(M * K, dtype, 95, -1, 1).reshape(M, K), orc.fill_int(K * n, dtype, 96, -1, 1).reshape(K, n)
+        want = (orc.to_float(a, dtype) @ orc.to_float(b, dtype)).astype(np.int64) + (7 if which == "acc" else 0)
+        fill = np.full((M + 4, n), 7, np.uint16 if which == "f16" else np.float32)
+        bufs = [stream.to_device(np.ascontiguousarray(a.T) if which == "ta" else a),
+                stream.to_device(np.ascontiguousarray(b.T) if which == "tb" else b), stream.to_device(fill)]
+        for grid in (None, (256, 1, 1), (331, 1, 1)):
+            stream.copy(bufs[2], fill.ctypes.data, fill.nbytes)
+            stream.launch(name, [M, n, K], bufs + [M, n, K], grid=grid or host.launch_shape(name, [M, n, K])[0])
+            stream.wait()
+            got = stream.from_device(bufs[2], fill.shape, fill.dtype)
+            assert np.array_equal((orc.half_to_float(got[:M]) if which == "f16" else got[:M]).astype(np.int64), want), (name, grid)
+            assert np.array_equal(got[M:], fill[M:]), (name, grid)
+        for p in bufs:
+            stream.free(p)
+    assert launched or tile == "_t16x16" and M == 1000 or -(-M // 16) * -(-N // 16) > 160
+
+
 @pytest.mark.parametrize("which", ["", "_ta", "_tb"])
 def test_gemm_unaligned_rows_chosen(host, orc, stream, which):
     """What the operator takes at an ordinary odd size, random operands: against 64 bits within the rounding of 32-bit

@@ -268,6 +268,14 @@ def test_gemm_tile_rules(host):
     assert tile("f16_f16_f32", 1001, 1003, 999) == "_u64"
 
 
+def test_gemm_workgroups_that_fetch_rule(host):
+    """256 workgroups where few tiles walk a long K over operands of 2 .. 32 MiB, a workgroup per tile elsewhere."""
+    grid = lambda tile, *dims: host.launch_shape("imex_gemm_bf16_bias_silu_bf16" + tile, list(dims))[0][0]
+    assert grid("_t16x16", 16, 1680, 3992) == grid("_t32", 128, 2048, 4096) == grid("_t128x64", 1000, 1000, 1024) == 256
+    assert grid("_t16x16", 16, 1680, 760) == 105 and grid("_t16x16", 16, 640, 1024) == 40 and grid("_t64", 16, 8192, 4096) == 128
+    assert grid("_t16x16", 16, 2816, 1024) == 176 and grid("_t128", 1000, 1000, 1024) == 64
+
+
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
     """Stream.launch's fast path: 8 bytes per argument, an f32 in the low four, with _pack_params' conversions and errors."""
     class Resolver:
