@@ -3,13 +3,15 @@ kernel catalogue (imex_hip_kernels.h) and, on top of them, one host function per
 benchmark workload that does what IMEX's JIT'd ``main`` does for it: create a
 stream, gpuMemAlloc, gpuMemCopy in, gpuModuleLoad + gpuKernelGet +
 gpuLaunchKernel with a ParamDesc list, gpuWait, gpuMemCopy out
-(lib/Conversion/GPUXToLLVM/GPUXToLLVMPass.cpp:373-383,508-518,691-710).
+(lib/Conversion/GPUXToLLVM/GPUXToLLVMPass.cpp:373-383,508-518,691-710).  Where
+that is faster the kernel works on pinned host memory instead (_staged).
 
 Nothing here computes on the CPU: if the built libraries are missing the import
 of the runtime raises, and every operator goes through the HIP kernels.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import functools
 import operator
@@ -293,9 +295,12 @@ class Stream:
         self.rt = runtime()
         self.handle = self.rt.gpuCreateStream(None, hip_stream)
         self._plans = {}  # (operator, dims) -> _Plan
+        self._staging = []  # the block that `staging` keeps: [(address, bytes as a numpy array)]
 
     def close(self):
         if self.handle:
+            while self._staging:
+                self.free(self._staging.pop()[0])
             self.rt.gpuStreamDestroy(self.handle)
             self.handle = None
 
@@ -333,6 +338,32 @@ class Stream:
         out = np.empty(shape, dtype=dtype)
         self.copy(out.ctypes.data, ptr, out.nbytes)
         return out
+
+    @contextlib.contextmanager
+    def staging(self, nbytes):
+        """A block of at least `nbytes` of pinned host memory that kernels read and write: (address, numpy
+        bytes), the caller's alone for the `with` block, at whose end no launch that uses it is pending.
+        Allocating and freeing one takes 30 us, so the queue keeps the last one, whose size is a power of two
+        (at most _STAGED_BYTES for the operators below), until it is closed."""
+        try:
+            ptr, block = self._staging.pop()  # atomic: two threads never hold the same block
+        except IndexError:
+            ptr, block = None, b""
+        if len(block) < nbytes:
+            if ptr is not None:
+                self.free(ptr)
+            size = max(1 << 18, 1 << (nbytes - 1).bit_length())
+            ptr = self.alloc(size, shared=True)
+            block = np.frombuffer((C.c_uint8 * size).from_address(ptr), np.uint8)
+        keep = False
+        try:
+            yield ptr, block
+            keep = not self._staging
+        finally:
+            if keep:
+                self._staging.append((ptr, block))
+            else:
+                self.free(ptr)  # waits for the queue
 
     # -- kernels --------------------------------------------------------------
     def kernel(self, name):
@@ -463,11 +494,54 @@ def _check(x, dtype):
         raise TypeError("array of %s does not hold %s elements" % (x.dtype, dtype))
 
 
-def _unary(stream, kernel, x, dtype, dims, extra=(), out_shape=None, out_np=None):
+# Where a kernel reads its operands from pinned host memory and writes its result there, instead of copies to and
+# from buffers allocated on the device, which cost 45..60 us a call before the link carries a byte.  Measured over
+# 1 Ki .. 4 Mi elements, one row to one column, device buffers -> staged:
+#  - at most _STAGED_SMALL bytes, any operator and shape: 57 -> 18 us, 1.9..4.5 times as fast;
+#  - maps, transposes: every element crosses the link once and in runs, 1.2..3 times as fast at all sizes measured
+#    (f16 softmax of 1024 x 2000 473 -> 345 us), hence _STAGED_BYTES, the largest of them;
+#  - 3-D transposes likewise (32^3 154 -> 33), but for runs of a few elements (d0 or d2 under 32) with more than a few planes
+#    between them: 2 x 1000 x 60 87 -> 116, where 65536 x 4 x 4 takes 478 -> 350;
+#  - softmax of rows that a workgroup keeps in registers likewise; one of 262144 columns reads its row again and from few
+#    workgroups (1 x 1048576 f32 1081 -> 2145 us), so rows end at _STAGED_SOFTMAX_COLS (1 x 65536: 95 -> 84);
+#  - sums: chains of dependent loads wait for the link (row sums of 65536 x 1 70 -> 79 us, column sums of 8192 x 32
+#    127 -> 138, 32768 x 32 318 -> 464, f16 2000 x 300 120 -> 125) and little is written back (row sums of 2048 x 2048
+#    557 -> 605), so only runs of 32 (rows) or 512 columns, of at most _STAGED_SUMS bytes: 512 x 1024 162 -> 118, columns
+#    168 -> 124, past that 0.9..1.3 times as fast.
+_STAGED_SMALL = 64 << 10
+_STAGED_SUMS = 5 << 19
+_STAGED_BYTES = 32 << 20
+_STAGED_SOFTMAX_COLS = 65536
+
+
+def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
+    """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes,
+    for nothing, and under the profiler, which times kernels on device memory."""
+    n_out = int(np.prod(out_shape)) * np.dtype(out_np).itemsize  # () is one element
+    total = sum(x.nbytes for x in xs) + n_out
+    if total > max(most, _STAGED_SMALL) or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
+        return None
+    starts, end = [], 0
+    for n in [x.nbytes for x in xs] + [n_out]:
+        starts.append(end)
+        end += -(-n // 256) * 256
+    with stream.staging(end) as (ptr, block):
+        for x, at in zip(xs, starts):
+            block[at:at + x.nbytes].view(x.dtype).reshape(x.shape)[...] = x
+        stream.launch(kernel, dims, [Ptr(ptr + at) for at in starts] + list(dims) + list(extra))
+        stream.wait()
+        return block[starts[-1]:starts[-1] + n_out].view(out_np).reshape(out_shape).copy()
+
+
+def _unary(stream, kernel, x, dtype, dims, extra=(), out_shape=None, out_np=None, staged=_STAGED_BYTES):
+    """`staged`: the most bytes, operand and result, that go through pinned host memory."""
     _check(x, dtype)
     out_shape = x.shape if out_shape is None else out_shape
     out_np = x.dtype if out_np is None else out_np
     n_out = int(np.prod(out_shape)) if len(out_shape) else 1
+    out = _staged(stream, kernel, [x], dims, extra, out_shape, out_np, staged)
+    if out is not None:
+        return out
     d_in = stream.to_device(x)
     d_out = stream.alloc(max(n_out, 1) * np.dtype(out_np).itemsize)
     try:
@@ -489,12 +563,15 @@ def silu(stream, x, dtype="f32"):
     return _unary(stream, "imex_silu_" + dtype, x, dtype, [x.size])
 
 
-def _binary(stream, kernel, a, b, dtype, dims, out_shape):
+def _binary(stream, kernel, a, b, dtype, dims, out_shape, staged=_STAGED_BYTES):
     _check(a, dtype)
     _check(b, dtype)
     if a.shape != b.shape:
         raise ValueError("operand shapes differ: %s vs %s" % (a.shape, b.shape))
     n_out = int(np.prod(out_shape))
+    out = _staged(stream, kernel, [a, b], dims, (), out_shape, a.dtype, staged)
+    if out is not None:
+        return out
     d_a, d_b = stream.to_device(a), stream.to_device(b)
     d_out = stream.alloc(max(n_out, 1) * a.dtype.itemsize)
     try:
@@ -524,7 +601,8 @@ def loop_fusion(stream, a, b, dtype="f32"):
 def input_fusion(stream, a, b, dtype="f32"):
     """benchmarks/kInputFusion/kInputFusion.mlir.in:6-40: out[j] = sum_i (log b[i,j] + |a[i,j]|)"""
     rows, cols = a.shape
-    return _binary(stream, "imex_input_fusion_" + dtype, a, b, dtype, [rows, cols], (cols,))
+    return _binary(stream, "imex_input_fusion_" + dtype, a, b, dtype, [rows, cols], (cols,),
+                   staged=_STAGED_SUMS if cols >= 512 else 0)
 
 
 def flash_attention(stream, q, k, v, zh, n_ctx, sm_scale, queries_per_workgroup=None, threads=512):
@@ -577,19 +655,22 @@ def mfma_lds_ceiling(stream, workgroups, iters, mode=0):
 def softmax(stream, x, dtype="f32"):
     """benchmarks/softmax/softmax_gpu.mlir.in:4-44 (last dim of a 2-D tensor)"""
     rows, cols = x.shape
-    return _unary(stream, "imex_softmax_" + dtype, x, dtype, [rows, cols])
+    return _unary(stream, "imex_softmax_" + dtype, x, dtype, [rows, cols],
+                  staged=_STAGED_BYTES if cols <= _STAGED_SOFTMAX_COLS else 0)
 
 
 def rowsum(stream, x, init=0.0):
     """WG/reduction_2D_1D_cross_sg_cross_lane.mlir:31-37"""
     rows, cols = x.shape
-    return _unary(stream, "imex_rowsum_f32", x, "f32", [rows, cols], extra=[float(init)], out_shape=(rows,))
+    return _unary(stream, "imex_rowsum_f32", x, "f32", [rows, cols], extra=[float(init)], out_shape=(rows,),
+                  staged=_STAGED_SUMS if cols >= 32 else 0)
 
 
 def rowmean(stream, x):
     """WG/reduction_4D_3D_mean_intra_sg_intra_lane.mlir:51-52: mean over the last dimension."""
     rows, cols = x.shape
-    return _unary(stream, "imex_rowmean_f32", x, "f32", [rows, cols], out_shape=(rows,))
+    return _unary(stream, "imex_rowmean_f32", x, "f32", [rows, cols], out_shape=(rows,),
+                  staged=_STAGED_SUMS if cols >= 32 else 0)
 
 
 def reduce_outer(stream, x, init=0.0, dtype="f32"):
@@ -598,7 +679,7 @@ def reduce_outer(stream, x, init=0.0, dtype="f32"):
     outer = x.shape[0]
     inner = int(np.prod(x.shape[1:]))
     return _unary(stream, "imex_reduce_outer_" + dtype, x, dtype, [outer, inner], extra=[float(init)],
-                  out_shape=x.shape[1:])
+                  out_shape=x.shape[1:], staged=_STAGED_SUMS if inner >= 512 else 0)
 
 
 def transpose2d(stream, x):
@@ -614,7 +695,7 @@ def transpose3d(stream, x):
     d0, d1, d2 = x.shape
     bits = x.dtype.itemsize * 8
     return _unary(stream, "imex_transpose3d_b%d" % bits, x, "f32" if bits == 32 else "f16", [d0, d1, d2],
-                  out_shape=(d2, d1, d0))
+                  out_shape=(d2, d1, d0), staged=_STAGED_BYTES if min(d0, d2) >= 32 or d1 <= 4 else 0)
 
 
 def gemm(stream, a, b, c=None, ab_dtype="f16", out_dtype="f32", trans_a=False, trans_b=False):

@@ -361,3 +361,26 @@ def test_adopted_stream_and_graph_replay(host, orc):
     s.close()                                               # must leave the adopted stream alive
     assert hip.hipStreamSynchronize(raw) == 0
     assert hip.hipStreamDestroy(raw) == 0
+
+
+@pytest.mark.parametrize("op,shapes", [
+    ("relu", [(1,), (1023, 17), (2048, 2048), (1, 4194305)]), ("softmax", [(3, 65536), (2, 65537), (130, 2001)]),
+    ("rowsum", [(8191, 1), (8193, 2), (1000, 31), (1001, 32), (1276, 512), (1281, 512)]),
+    ("reduce_outer", [(4097, 4), (70, 511), (71, 512), (1021, 511), (33, 8, 64)]), ("maximum", [(77,), (5, 1001)]),
+    ("input_fusion", [(9, 7), (120, 512), (300, 511)]), ("transpose2d", [(1, 999), (2049, 3), (257, 1031)]),
+    ("transpose3d", [(2, 1000, 60), (32, 7, 33), (31, 700, 5), (900, 4, 9)])])
+def test_operators_on_host_memory(host, op, shapes, monkeypatch):
+    """The same kernel on the same numbers: through pinned host memory and through device buffers the bits are equal,
+    on both sides of each line, whatever block is kept from the sizes before, and a strided operand is packed."""
+    rng, taken = np.random.default_rng(5), []
+    staged = host._staged
+    with host.Stream() as s:
+        for shape in shapes + shapes[:1]:
+            xs = [rng.random(shape, dtype=np.float32) + np.float32(0.1) for _ in range(1 + (op in ("maximum", "input_fusion")))]
+            for ins in (xs, [x[::-1] for x in xs]):
+                monkeypatch.setattr(host, "_staged", lambda *a: None)
+                want = getattr(host, op)(s, *ins)
+                monkeypatch.setattr(host, "_staged", lambda *a: taken.append(staged(*a)) or taken[-1])
+                got = getattr(host, op)(s, *ins)
+                assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32)), shape
+    assert any(t is not None for t in taken)

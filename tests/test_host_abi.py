@@ -347,6 +347,43 @@ def test_launch_with_dependencies_uses_the_kept_plan(host):
     assert launched == [(name, (*grid, *block, smem))] * 3
 
 
+def test_staging_block_of_a_queue(host):
+    """One block per caller at a time, one kept, grown by powers of two, freed when its user fails and with the queue."""
+    live = {}
+
+    class Runtime:
+        def gpuMemAlloc(self, handle, nbytes, alignment, shared):
+            assert shared == 1
+            buf = C.create_string_buffer(nbytes)
+            live[C.addressof(buf)] = buf
+            return C.addressof(buf)
+
+        def gpuMemFree(self, handle, ptr):
+            del live[ptr]
+
+        def gpuStreamDestroy(self, handle):
+            assert not live
+    s = host.Stream.__new__(host.Stream)
+    s.rt, s.handle, s._staging = Runtime(), 1, []
+    with s.staging(100) as (p, block):
+        assert len(block) == 1 << 18 and p in live
+        with s.staging(100) as (q, _):  # a second thread
+            assert q != p and len(live) == 2
+    assert len(live) == 1  # one of the two is kept
+    with s.staging(1 << 18) as (q, _):
+        assert list(live) == [q]
+    with s.staging((1 << 18) + 1) as (q, block):
+        assert list(live) == [q] and len(block) == 1 << 19
+    with pytest.raises(RuntimeError):
+        with s.staging(5) as (q, _):
+            raise RuntimeError
+    assert not live
+    with s.staging(5):
+        pass
+    s.close()
+    assert not live and s.handle is None
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
