@@ -25,7 +25,7 @@
 // queries of one (batch, head) as (QB, KG) = (2,4), (4,2), (8,1) with 512 threads, or 256
 // queries as (8,2) with 1024 threads.  Wavefront w takes query block w % QB and every KG-th
 // key tile of 64 keys, group w / QB; partial (m, l, O) of the key groups are merged through LDS
-// at the end.  (32 queries and eight key groups: "every wavefront its own keys" below.)  Every
+// at the end.  (_q32 and _q64 have eight key groups: "every wavefront its own keys" below.)  Every
 // workgroup walks all keys of its head, so K / V traffic from L2 falls with the
 // queries per workgroup; key groups exist to keep all CUs busy on small problems (the
 // reference's 2 x 2 x 4096 x 64 gives one 64-query workgroup per CU) and, in the 1024-thread
@@ -39,8 +39,8 @@
 //   tiles: queries past the end are not stored, keys past the end get a score of -inf.
 // imex_flash_attention_fwd_f16_q32 / _q64 / _q128 / _q256 are the operator with one tiling each.
 // Launch: grid (ceil(N_CTX / q), ZH, 1) with q = 64, 128 or 256 and block (512,1,1), or q = 256
-// and block (1024,1,1); the forms with one tiling take theirs only, _q256 with block (1024,1,1).  Other launches (and a scale <= 0, or misaligned tensors) take the
-// one-query-per-lane reference loop of the same kernel (grid-stride, any grid and block).
+// and block (1024,1,1); the forms with one tiling take theirs only, _q256 with block (1024,1,1).  Other launches (and a
+// scale <= 0, or misaligned tensors) take the one-query-per-lane reference loop of the same kernel (grid-stride, any grid and block).
 
 #include "device_common.h"
 
@@ -55,6 +55,7 @@ constexpr int kLdsBytes = kRingBytes;           // the ring, and after it the pa
 static_assert(kLdsBytes >= 8 * 34 * 64 * 4, "two key groups hand eight of them over, four or eight meet from eight wavefronts");
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -75,6 +76,16 @@ __device__ __forceinline__ float max_of_halves(float v) {
 }
 // the value lane l+32 (or l-32) holds
 __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 64); }
+
+// Workgroups go to the 8 XCDs round-robin in launch order, and each XCD has its own L2.  Renumber them so that one XCD gets
+// consecutive query blocks -- whole heads, or a contiguous part of one; as many as the others or one more -- and its L2
+// holds the K / V of a few heads instead of a slice of the traffic of all of them.
+__device__ __forceinline__ void place_of_workgroup(uint32_t &x, uint32_t &y) {
+  const uint32_t total = gridDim.x * gridDim.y, launched = blockIdx.y * gridDim.x + blockIdx.x, xcd = launched & 7;
+  const uint32_t logical = xcd * (total >> 3) + min(xcd, total & 7) + (launched >> 3);
+  y = logical / gridDim.x;
+  x = logical - y * gridDim.x;
+}
 
 // ---- any-shape path: one lane per query, the reference loop ----------------------------
 __device__ __forceinline__ void attention_scalar(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
@@ -111,39 +122,33 @@ __device__ __forceinline__ void attention_scalar(const uint16_t *Q, const uint16
 // merges its share of them: 8 / KG of the eight groups of four rows that a query block of 32 has.  (One wavefront per
 // query block merging all of it is as fast for two key groups, 8 x 3000 35.0 against 35.8 us, but not for four, 16 x 768
 // 8.93 against 8.74, or eight.)
-template <int QB, int KG>
-__device__ __forceinline__ void merge_and_store(const f32x16 (&o)[2], float m, float l, uint16_t *__restrict__ Out,
-                                                int64_t firstRow, int64_t endRow, char *lds, int wave, int wq, int wk,
-                                                int lane, bool ragged) {
-  constexpr int kSlot = 34 * 64; // floats per wavefront: 32 accumulator rows, four to a vector, m, l
-  constexpr int kUnits = 8 / KG; // of four rows, per wavefront
-  float *all = reinterpret_cast<float *>(lds);
-  __syncthreads(); // the ring is free
-  {
-    float *mine = all + (wq * KG + wk) * kSlot;
+constexpr int kSlot = 33 * 64; // floats of one partial result: 32 accumulator rows, four to a vector; m, l of every query
+__device__ __forceinline__ void put_partial(const f32x16 (&o)[2], float m, float l, float *slot, int lane) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) // rows of the accumulator's block u / 4
-      *reinterpret_cast<f32x4 *>(mine + (u * 64 + lane) * 4) =
-          f32x4{o[u >> 2][(u & 3) * 4], o[u >> 2][(u & 3) * 4 + 1], o[u >> 2][(u & 3) * 4 + 2], o[u >> 2][(u & 3) * 4 + 3]};
-    mine[32 * 64 + lane] = m;
-    mine[33 * 64 + lane] = l;
-  }
-  __syncthreads();
-  const int qb = wave / KG, first = wave % KG * kUnits; // the query block and the units this wavefront merges
-  const float *of = all + qb * (KG * kSlot);
+  for (int u = 0; u < 8; ++u) // rows of the accumulator's block u / 4
+    *reinterpret_cast<f32x4 *>(slot + (u * 64 + lane) * 4) =
+        f32x4{o[u >> 2][(u & 3) * 4], o[u >> 2][(u & 3) * 4 + 1], o[u >> 2][(u & 3) * 4 + 2], o[u >> 2][(u & 3) * 4 + 3]};
+  if (lane < 32)
+    *reinterpret_cast<float2 *>(slot + 32 * 64 + lane * 2) = float2{m, l};
+}
+// Units first .. first + kUnits - 1 of a query block whose KG partial results begin at `of`.
+template <int KG, int kUnits>
+__device__ __forceinline__ void merge_partials(const float *of, uint16_t *__restrict__ Out, int64_t firstRow, int64_t endRow,
+                                               int first, int lane, bool ragged) {
   float a[KG], mAll = -__builtin_inff(), lAll = 0.0f;
+  float2 ml[KG];
 #pragma unroll
   for (int g = 0; g < KG; ++g) {
-    a[g] = of[g * kSlot + 32 * 64 + lane];
-    mAll = fmaxf(mAll, a[g]);
+    ml[g] = *reinterpret_cast<const float2 *>(of + g * kSlot + 32 * 64 + (lane & 31) * 2);
+    mAll = fmaxf(mAll, ml[g].x);
   }
 #pragma unroll
   for (int g = 0; g < KG; ++g) {
-    a[g] = __builtin_amdgcn_exp2f(a[g] - mAll); // a group without a key: 0
-    lAll += of[g * kSlot + 33 * 64 + lane] * a[g];
+    a[g] = __builtin_amdgcn_exp2f(ml[g].x - mAll); // a group without a key: 0
+    lAll += ml[g].y * a[g];
   }
   const float inv = 1.0f / lAll;
-  const int64_t row = firstRow + qb * 32 + (lane & 31);
+  const int64_t row = firstRow + (lane & 31);
 #pragma unroll
   for (int j = 0; j < kUnits; ++j) {
     const int u = first + j; // lane holds, for its query, d = u*8 + (lane/32)*4 .. +3
@@ -158,6 +163,18 @@ __device__ __forceinline__ void merge_and_store(const f32x16 (&o)[2], float m, f
     if (!ragged || row < endRow)
       *reinterpret_cast<f16x4 *>(Out + row * D + u * 8 + (lane >> 5) * 4) = out4;
   }
+}
+template <int QB, int KG>
+__device__ __forceinline__ void merge_and_store(const f32x16 (&o)[2], float m, float l, uint16_t *__restrict__ Out,
+                                                int64_t firstRow, int64_t endRow, char *lds, int wave, int wq, int wk,
+                                                int lane, bool ragged) {
+  constexpr int kUnits = 8 / KG; // of four rows, per wavefront
+  float *all = reinterpret_cast<float *>(lds);
+  __syncthreads(); // the ring is free
+  put_partial(o, m, l, all + (wq * KG + wk) * kSlot, lane);
+  __syncthreads();
+  const int qb = wave / KG; // the query block of which this wavefront merges a share
+  merge_partials<KG, kUnits>(all + qb * (KG * kSlot), Out, firstRow + qb * 32, endRow, wave % KG * kUnits, lane, ragged);
 }
 
 // ---- MFMA path ---------------------------------------------------------------------------
@@ -182,18 +199,8 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   constexpr int kCopies = BN * KG / (8 * kWaves);  // 1 KiB (8-row) copies per wavefront, stage and operand
   const int wq = wave % QB, wk = wave / QB;
   const int qi = lane & 31, half = lane >> 5;
-  // Workgroups go to the 8 XCDs round-robin in launch order, and each XCD has its own L2.  Renumber
-  // them so that one XCD gets consecutive query blocks -- whole heads, or a contiguous part of one --
-  // and its L2 holds the K / V of a few heads instead of a slice of the traffic of all of them.
-  uint32_t bx = blockIdx.x, by = blockIdx.y;
-  {
-    const uint32_t total = gridDim.x * gridDim.y, launched = by * gridDim.x + bx;
-    if (total % 8 == 0) {
-      const uint32_t logical = (launched & 7) * (total >> 3) + (launched >> 3);
-      by = logical / gridDim.x;
-      bx = logical - by * gridDim.x;
-    }
-  }
+  uint32_t bx, by;
+  place_of_workgroup(bx, by);
   const int64_t head0 = int64_t(by) * N;                 // first row of this (batch, head)
   const int64_t q0 = head0 + int64_t(bx) * (32 * QB) + wq * 32;
   // N_CTX need not divide the tiles.  Queries past the end of the head are computed on a copy of
@@ -442,10 +449,10 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
 
   // -- two key groups: group 1 hands (m, l, O^T) to group 0 through LDS
   __syncthreads(); // the ring is free
-  constexpr int kSlot = 34 * 64; // floats per (query half, key group): 32 accumulator rows, m, l
-  float *xchg = reinterpret_cast<float *>(lds) + wq * (KG - 1) * kSlot;
+  constexpr int kHand = 34 * 64; // floats per query block and key group: 32 accumulator rows, m, l
+  float *xchg = reinterpret_cast<float *>(lds) + wq * (KG - 1) * kHand;
   if (wk != 0) {
-    float *mine = xchg + (wk - 1) * kSlot;
+    float *mine = xchg + (wk - 1) * kHand;
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
@@ -459,14 +466,14 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
     float mAll = m;
 #pragma unroll
     for (int g = 0; g < KG - 1; ++g)
-      mAll = fmaxf(mAll, xchg[g * kSlot + 32 * 64 + lane]);
+      mAll = fmaxf(mAll, xchg[g * kHand + 32 * 64 + lane]);
     float a[KG];
     a[0] = exp2f(m - mAll);
     float lAll = l * a[0];
 #pragma unroll
     for (int g = 0; g < KG - 1; ++g) {
-      a[g + 1] = exp2f(xchg[g * kSlot + 32 * 64 + lane] - mAll);
-      lAll += xchg[g * kSlot + 33 * 64 + lane] * a[g + 1];
+      a[g + 1] = exp2f(xchg[g * kHand + 32 * 64 + lane] - mAll);
+      lAll += xchg[g * kHand + 33 * 64 + lane] * a[g + 1];
     }
     const float inv = 1.0f / lAll;
     // lane holds, for query q = qi, d = db*32 + (r/4)*8 + half*4 + r%4
@@ -481,7 +488,7 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
           float acc = o[db][r] * a[0];
 #pragma unroll
           for (int g = 0; g < KG - 1; ++g)
-            acc += xchg[g * kSlot + (db * 16 + r) * 64 + lane] * a[g + 1];
+            acc += xchg[g * kHand + (db * 16 + r) * 64 + lane] * a[g + 1];
           out4[e] = static_cast<_Float16>(acc * inv);
         }
         if (!kRagged || q0 + qi < head0 + N)
@@ -503,7 +510,7 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
 // cycles of issue per tile, two wavefronts on a SIMD) and, at one wavefront's 8 KiB in flight, by the copies' latency.
 // Sixteen wavefronts, or 64 queries per wavefront, were not faster.
 constexpr int kOwnKeys = 32, kOwnTile = kOwnKeys * D * 2;
-constexpr int kOwnWaves = 8, kOwnLds = kOwnWaves * 34 * 64 * 4; // the partial results; the tiles are 8 KiB per wavefront
+constexpr int kOwnWaves = 8, kOwnLds = kOwnWaves * kSlot * 4; // the partial results; the tiles are 8 KiB per wavefront
 
 template <bool kRagged>
 __device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
@@ -512,15 +519,8 @@ __device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int qi = lane & 31, half = lane >> 5;
-  uint32_t bx = blockIdx.x, by = blockIdx.y; // renumbered as in attention_tiled
-  {
-    const uint32_t total = gridDim.x * gridDim.y, launched = by * gridDim.x + bx;
-    if (total % 8 == 0) {
-      const uint32_t logical = (launched & 7) * (total >> 3) + (launched >> 3);
-      by = logical / gridDim.x;
-      bx = logical - by * gridDim.x;
-    }
-  }
+  uint32_t bx, by;
+  place_of_workgroup(bx, by);
   const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 32;
   const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
   const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
@@ -655,6 +655,236 @@ __device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ 
   merge_and_store<1, kOwnWaves>(o, m, l + other_half(l), Out, q0, head0 + N, lds, wave, 0, wave, lane, kRagged);
 }
 
+template <typename T> __device__ __forceinline__ void pin(T &v) { asm volatile("" : "+v"(v)); }
+
+// ---- every wavefront its own keys, for two blocks of 32 queries -------------------------------
+// 64 queries, eight wavefronts, each of which takes every eighth 32-key tile through both blocks of 32 queries, A and B: a
+// fragment is read from LDS once for two products (half the LDS reads of attention_tiled's two query blocks x four key
+// groups, which this replaced), and no barrier stands between the first and the merge.  The two blocks are half a tile
+// apart: while one's scores go through the softmax, the matrix cores take the other's eight products, one between every two
+// exponentials (a wavefront issues in order: products in a row hold it for 32 cycles each, and a SIMD has two wavefronts
+// here).  The reference that the exponentials are taken against moves only when a score exceeds it by 2^8 (P stays below
+// 256 in f16, relative rounding as before), so the accumulators are rescaled in the first tiles instead of in nearly all.
+// The queries come through LDS, 1 KiB a wavefront: as fragments from memory (32 rows a load) and behind three tiles of
+// copies they held the first product up for 5000 cycles, now 2800.
+//   4 x 4096 28.7 -> 25.0 us, 4 x 4000 29.4 -> 25.8, 8 x 2048 16.7 -> 14.6, 5 x 3001 22.8 -> 20.1, 16 x 1000 11.1 -> 10.7.
+// What bounds it: 1.1 .. 1.3 us per tile of two wavefronts on a SIMD (0.97 on zeros: the clock falls on random operands),
+// issue of 2 x (32 exponentials, 16 products, about 150 others) at 12, 13 and 3.2 cycles, and about 6 us around the loop,
+// 2.5 of them the launch, 1.9 the merge of eight partial results.  Taken back: a barrier per tile or per four (the
+// wavefronts of a SIMD end within 1000 cycles of each other instead of 10000, 4 x 4096 25.5 -> 26.0), s_setprio (none).
+constexpr int kPairWave = 4 * kOwnTile; // two places for K, two for V
+constexpr int kPairLds = kOwnWaves * kPairWave + 64 * D * 2; // the tiles, the queries
+static_assert(kPairLds >= 2 * kOwnWaves * kSlot * 4, "the partial results fit");
+
+template <bool kRagged>
+__device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
+                                                const uint16_t *__restrict__ V, uint16_t *__restrict__ Out, float scale,
+                                                int64_t N, char *lds) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int qi = lane & 31, half = lane >> 5;
+  uint32_t bx, by;
+  place_of_workgroup(bx, by);
+  const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 64;
+  const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
+  const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
+
+  // copies, places and fragment addresses: as in attention_own_keys
+  const __amdgpu_buffer_rsrc_t kRsrc = make_rsrc(K + head0 * D, N * D * 2), vRsrc = make_rsrc(V + head0 * D, N * D * 2);
+  const __amdgpu_buffer_rsrc_t nothing = make_rsrc(K + head0 * D, 0); // past the last tile: nothing moves, but the copies count
+  int kVoff[4], vVoff[4], kVoffT[4], vVoffT[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int r = c * 8 + (lane >> 3), rT = kRagged ? min(r, lastRows - 1) : r;
+    const int kc = (lane & 7) ^ ((r ^ ((r >> 3) & 3)) & 7), vc = (lane & 7) ^ (((r >> 1) & 1) << 2);
+    kVoff[c] = (r * D + kc * 8) * 2;
+    vVoff[c] = (r * D + vc * 8) * 2;
+    kVoffT[c] = (rT * D + kc * 8) * 2;
+    vVoffT[c] = (rT * D + vc * 8) * 2;
+  }
+  char *own = lds + wave * kPairWave; // K, K, V, V
+  auto dma = [&](const __amdgpu_buffer_rsrc_t &rsrc, const int (&off)[4], const int (&offT)[4], int i, int place) {
+    LdsChar *dst = (LdsChar *)own + place * kOwnTile;
+    const int tile = wave + i * kOwnWaves;
+    const bool tail = kRagged && tile == tiles - 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < iters ? rsrc : nothing, dst + c * 1024, 16, tail ? offT[c] : off[c],
+                                               i < iters ? tile * kOwnTile : 0, 0, 0);
+  };
+  auto dma_k = [&](int i) { dma(kRsrc, kVoff, kVoffT, i, i & 1); };
+  auto dma_v = [&](int i) { dma(vRsrc, vVoff, vVoffT, i, 2 + (i & 1)); };
+  int kRd[4], vRd[2];
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds)
+    kRd[ds] = qi * 128 + ((((ds * 2 + half) ^ qi ^ ((qi >> 3) & 3)) & 7) << 4);
+  {
+    const int t = lane & 15, blk = (lane >> 4) & 1, row = half * 4 + (t >> 2);
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+      vRd[db] = 2 * kOwnTile + row * 128 + ((((db ^ ((t >> 3) & 1)) << 2) | (blk << 1) | ((t & 3) >> 1)) * 16) + (t & 1) * 8;
+  }
+  const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  f32x16 oA[2] = {zero, zero}, oB[2] = {zero, zero}, sA, sB;
+  constexpr float kNoKey = -3.40282347e38f; // a reference that every score is above, or -inf
+  float mA = kNoKey, mB = kNoKey, lA = 0.0f, lB = 0.0f;
+  const float c = scale * 1.44269504088896341f;
+  f16x8 qf[2][4], kf[4], vf[2][2], pA[2], pB[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    pA[kk] = pB[kk] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    vf[kk][0] = vf[kk][1] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
+  auto read_k = [&](int i) {
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+      kf[ds] = *reinterpret_cast<const f16x8 *>(own + (i & 1) * kOwnTile + kRd[ds]);
+  };
+  auto read_v = [&](int i) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        const char *p = own + (i & 1) * kOwnTile + vRd[db] + kk * 16 * 128;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsI16x4 *)(p + 8 * 128));
+        vf[kk][db] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+  };
+  auto read_done = [] { // the fragments are in registers: their places may be filled again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // computed here, not where it is used
+  auto stay = [](auto &...v) { (pin(v), ...); };
+  // One block's tile `i` through the softmax, step(0) .. step(7), the other block's products, between its exponentials, and
+  // middle() behind the last of them.
+  auto softmax = [&](f32x16 &s, f16x8 (&p)[2], f32x16 (&o)[2], float &m, float &l, int i, auto &&step, auto &&middle) {
+    if (kRagged && wave + i * kOwnWaves == tiles - 1 && lastRows < kOwnKeys) { // uniform over the wavefront
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[r] = (r >> 2) * 8 + half * 4 + (r & 3) < lastRows ? s[r] : -__builtin_inff();
+    }
+    float part[2] = {s[0], s[1]};
+#pragma unroll
+    for (int r = 2; r < 16; ++r)
+      part[r & 1] = fmaxf(part[r & 1], s[r]);
+    const float mx = max_of_halves(fmaxf(part[0], part[1])) * c;
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
+      const float mNew = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mNew);
+      m = mNew;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          o[db][r] *= alpha;
+    }
+    float x[2], e[2], sum[2] = {0.0f, 0.0f};
+    u32x4 w[2];
+    x[0] = __builtin_fmaf(s[0], c, -m);
+    x[1] = __builtin_fmaf(s[1], c, -m);
+    auto take = [&](int j) { // the exponentials of step j
+      const f16x2 h = {static_cast<_Float16>(e[0]), static_cast<_Float16>(e[1])};
+      uint32_t word = __builtin_bit_cast(uint32_t, h);
+      sum[0] += e[0];
+      sum[1] += e[1];
+      stay(word, sum[0], sum[1]);
+      w[j >> 2][j & 3] = word;
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      step(j);
+      if (j > 0)
+        take(j - 1);
+      e[0] = __builtin_amdgcn_exp2f(x[0]);
+      e[1] = __builtin_amdgcn_exp2f(x[1]);
+      if (j < 7) {
+        x[0] = __builtin_fmaf(s[2 * j + 2], c, -m);
+        x[1] = __builtin_fmaf(s[2 * j + 3], c, -m);
+      }
+      stay(x[0], x[1], e[0], e[1]);
+      if (j == 7)
+        middle();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    take(7);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+      p[kk] = __builtin_bit_cast(f16x8, w[kk]);
+    l += sum[0] + sum[1];
+  };
+
+  // The queries, 8 rows a wavefront, laid out as K's.
+  {
+    const int row = wave * 8 + (lane >> 3), there = kRagged ? int(min(int64_t(row), N - 1 - int64_t(bx) * 64)) : row;
+    const int chunk = (lane & 7) ^ ((row ^ ((row >> 3) & 3)) & 7);
+    const __amdgpu_buffer_rsrc_t qRsrc = make_rsrc(Q + q0 * D, (head0 + N - q0) * D * 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(qRsrc, (LdsChar *)lds + kOwnWaves * kPairWave + wave * 1024, 16,
+                                             (there * D + chunk * 8) * 2, 0, 0, 0);
+  }
+  dma_k(0);
+  dma_k(1);
+  dma_v(0);
+  wait_vmcnt<8>(); // the queries, K(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  if (iters > 0) { // uniform over the wavefront
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds)
+        qf[b][ds] = *reinterpret_cast<const f16x8 *>(lds + kOwnWaves * kPairWave + b * (32 * 128) + kRd[ds]);
+    read_k(0);
+    read_done();
+    dma_v(1);
+    dma_k(2);
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds)
+      sA = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds], qf[0][ds], ds == 0 ? zero : sA, 0, 0, 0);
+    for (int i = 0; i < iters; ++i) {
+      // A's softmax; B's last tile times V(i - 1), B's scores of tile i
+      softmax(sA, pA, oA, mA, lA, i, [&](int j) {
+        if (j < 4)
+          oB[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j >> 1][j & 1], pB[j >> 1], oB[j & 1], 0, 0, 0);
+        else
+          sB = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[j - 4], qf[1][j - 4], j == 4 ? zero : sB, 0, 0, 0);
+      }, [&] {
+        wait_vmcnt<8>(); // K(i + 1), V(i)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read_v(i);
+        read_k(i + 1);
+      });
+      // B's softmax; A's tile i times V(i), A's scores of tile i + 1 (past the end of whatever is there, not used)
+      softmax(sB, pB, oB, mB, lB, i, [&](int j) {
+        if (j == 0) {
+          read_done();
+          dma_k(i + 3);
+          dma_v(i + 2);
+        }
+        if (j < 4)
+          oA[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j >> 1][j & 1], pA[j >> 1], oA[j & 1], 0, 0, 0);
+        else
+          sA = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[j - 4], qf[0][j - 4], j == 4 ? zero : sA, 0, 0, 0);
+      }, [] {});
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      oB[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j >> 1][j & 1], pB[j >> 1], oB[j & 1], 0, 0, 0);
+  }
+  wait_vmcnt<0>();
+  float *all = reinterpret_cast<float *>(lds);
+  __syncthreads(); // everyone's tiles are done with
+  put_partial(oA, mA, lA + other_half(lA), all + wave * kSlot, lane);
+  put_partial(oB, mB, lB + other_half(lB), all + (kOwnWaves + wave) * kSlot, lane);
+  __syncthreads();
+  merge_partials<kOwnWaves, 1>(all, Out, q0, head0 + N, wave, lane, kRagged);
+  merge_partials<kOwnWaves, 1>(all + kOwnWaves * kSlot, Out, q0 + 32, head0 + N, wave, lane, kRagged);
+}
+
 // What the tiled path takes, of the arguments and of the launch.
 __device__ __forceinline__ bool attention_shaped(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                                  const uint16_t *Out, float scale, int64_t ZH, int64_t N) {
@@ -703,8 +933,7 @@ extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_f
 }
 
 // One tiling each, for problems whose tilings by the rule above leave CUs idle or run a nearly empty last round
-// (attentionVariant in KernelCatalog.cpp).  64 and 128 queries are the forms above with the next block's scores formed
-// ahead: 5 x 3001 24.2 -> 21.9, 8 x 2048 17.4 -> 16.4, 4 x 4096 28.9 -> 27.4.
+// (attentionVariant in KernelCatalog.cpp).  128 queries are the form above with the next block's scores formed ahead.
 template <int QB, int KG, bool kScoresAhead>
 __device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                                      uint16_t *Out, float scale, int64_t ZH, int64_t N, char *lds) {
@@ -735,6 +964,15 @@ extern "C" __global__ __launch_bounds__(kOwnWaves *kWave, 4) void imex_flash_att
   else
     attention_own_keys<true>(Q, K, V, Out, sm_scale, N_CTX, lds);
 }
-IMEX_ATTENTION_TILING(64, 2, 4, true)
+extern "C" __global__ __launch_bounds__(kOwnWaves *kWave) void imex_flash_attention_fwd_f16_q64(
+    const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
+  __shared__ __attribute__((aligned(16))) char lds[kPairLds];
+  if (!attention_shaped(Q, K, V, Out, sm_scale, ZH, N_CTX) || blockDim.x != kOwnWaves * kWave || gridDim.x != (N_CTX + 63) / 64)
+    attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
+  else if (N_CTX % 64 == 0)
+    attention_pairs<false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+  else
+    attention_pairs<true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+}
 IMEX_ATTENTION_TILING(128, 4, 2, true)
 IMEX_ATTENTION_TILING(256, 8, 2, false)

@@ -1161,6 +1161,24 @@ def test_flash_attention_tiling_by_size(host, orc, stream, zh, n_ctx, tiling):
     assert np.max(np.abs(got[ok] - ref[ok])) <= 2.0 ** -10 + 2.0 ** -11 * np.max(np.abs(ref[ok]))
 
 
+@pytest.mark.parametrize("order", ["up", "down", "jumps"])
+@pytest.mark.parametrize("zh,n_ctx", [(1, 769), (3, 1000), (2, 2080)])
+def test_flash_attention_moving_maximum(host, orc, stream, zh, n_ctx, order):
+    """Scores that grow by less than a factor of 2^8 from tile to tile, that fall, and that jump from key to key: the
+    reference that the exponentials are taken against lags the maximum; workgroups that 8 does not divide."""
+    n = zh * n_ctx
+    q = orc.fill_uniform(n * 64, "f16", 93, -0.5, 0.5).reshape(n, 64)
+    k = orc.fill_uniform(n * 64, "f16", 94, -0.5, 0.5).reshape(n, 64)
+    v = orc.fill_uniform(n * 64, "f16", 95, -1, 1).reshape(n, 64)
+    q[:, 0] = 0x4000  # 2.0
+    at = np.arange(n) % n_ctx
+    ramp = {"up": at / 64.0, "down": -at / 64.0, "jumps": 40.0 * ((at * 7919) % 13 == 0) - 20.0}[order]
+    k[:, 0] = ramp.astype(np.float16).view(np.uint16)
+    got = host.flash_attention(stream, q, k, v, zh, n_ctx, 0.5)
+    rows = np.unique(np.concatenate([np.arange(0, n, 11), [n_ctx - 1, n - 1]]))
+    assert attention_close(got[rows], orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows), orc)
+
+
 @pytest.mark.parametrize("queries", [32, 64, 128, 256])
 def test_flash_attention_one_tiling_at_any_address(host, orc, stream, queries):
     """A tensor that starts one element behind a 16-byte boundary takes the reference loop of the same kernel."""
