@@ -36,8 +36,9 @@
 //    through LDS and out: a workgroup always has a tile's reads in flight (4096 x 4096 streaming
 //    from HBM: 22.9 us against 24.0 us with one workgroup per tile).  The same walk for the 16-bit
 //    256 x 256 tile (512 lanes, so that two tiles fit the registers) gained 1.5 % and is not used.
-//  * Shapes or bases that break 16-byte alignment: 8 x 8 (4 x 4) blocks at any address, moved back inside at the
-//    edges (tile_unaligned).  Bound by HBM transactions: row segments that are no whole lines cost two partly used
+//  * Shapes or bases that break 16-byte alignment, and by the catalogue's choice results whose rows are no whole 64 bytes
+//    (16-bit 6000 x 6000: 42.0 us with 256 x 256 tiles by diagonals, 34.1 so): 8 x 8 (4 x 4) blocks at any address, moved
+//    back inside at the edges (tile_unaligned).  Bound by HBM transactions: row segments that are no whole lines cost two partly used
 //    ones each (16-bit 5000 x 4097: 22.1 us with buffers that are not in the caches, 3.7 TB/s, where 5000 x 4096 would
 //    take 13.7 at 6 TB/s; 14.4 us over a few buffer sets that the 256 MiB cache holds in part; one element at a time
 //    150 and 119).
@@ -503,7 +504,7 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose3d_b16(cons
   transpose_block<uint16_t>(in, out, View{d0, d2, d1 * d2, d1 * d0}, d1, d2, d0);
 }
 
-// The operators for sizes that are no whole 16-byte vectors, with the LDS of these tiles only: four workgroups on a
+// The operators for sizes that are no whole 16-byte vectors or half lines, with the LDS of these tiles only: four workgroups on a
 // CU where the kernels above leave room for two (16-bit 9999 x 6001: 59.9 us, 79.9 with 64 KiB of LDS and
 // 128 x 128 tiles; 307.8 one element at a time).
 extern "C" __global__ __launch_bounds__(kThreads) void imex_transpose2d_b32_any(const uint32_t *in, uint32_t *out,

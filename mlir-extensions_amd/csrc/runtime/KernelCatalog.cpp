@@ -400,11 +400,18 @@ const char *softmaxVariant(const Entry *e, int64_t rows, int64_t cols) {
 }
 
 // Transposes whose rows are no whole 16-byte vectors on one side or the other go to the kernels with tiles for these,
-// from one vector each way on (16-bit 1203 x 1777: 29.4 -> 4.1 us; 32-bit 333 x 17 x 501: 17.0 -> 5.8).
+// from one vector each way on (16-bit 1203 x 1777: 29.4 -> 4.1 us; 32-bit 333 x 17 x 501: 17.0 -> 5.8).  So do those whose
+// result has rows that are no whole 64 bytes: there neighbouring segments share lines, which those kernels' order of tiles
+// brings together in one L2 (16-bit 6000 x 6000 42.0 -> 34.1 us, 4104 x 4096 18.4 -> 16.1, 11472 x 3312 43.1 -> 37.2, 32-bit
+// 3000 x 2000 14.8 -> 11.7; 98 of 260 timed problems, 0.82 of their time in the mean).  With whole halves of lines it is as
+// often the other way (16-bit 13280 x 2048 22.5, 24.9, 32-bit 6000 x 6000 62.8, 62.4), and so it is with a few columns, which
+// tiles of 64 fit badly (16-bit 63352 x 280 18.3, 22.0).
 const char *transposeVariant(const Entry *e, const int64_t *dims) {
   const int64_t perVec = e->shape == Shape::Transpose2D32 || e->shape == Shape::Transpose3D32 ? 4 : 8;
-  const int64_t rows = dims[0], cols = dims[e->ndims - 1];
-  if (rows < perVec || cols < perVec || (rows % perVec == 0 && cols % perVec == 0))
+  const int64_t rows = dims[0], cols = dims[e->ndims - 1], planes = e->ndims == 3 ? dims[1] : 1;
+  const bool halves = uint64_t(rows) * uint64_t(planes) % uint64_t(4 * perVec) == 0; // of cache lines, in the result
+  if (rows < perVec || cols < perVec ||
+      (rows % perVec == 0 && cols % perVec == 0 && (halves || rows / 128 > cols)))
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s_any", e->name);

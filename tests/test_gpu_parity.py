@@ -625,6 +625,27 @@ def test_transpose_of_any_size_and_address(host, orc, stream, rows, planes, cols
         assert np.array_equal(got[1:-1].reshape(want.shape), want)
 
 
+@pytest.mark.parametrize("rows,planes,cols,bits,form", [
+    (4104, 1, 4120, 16, "_any"), (4128, 1, 4120, 16, ""), (4128, 1, 24, 16, ""), (2184, 1, 16, 16, ""), (2056, 1, 16, 16, "_any"),
+    (4100, 1, 4104, 32, "_any"), (4112, 1, 4120, 32, ""), (40, 7, 104, 16, "_any"), (32, 7, 104, 16, ""),
+    (20, 3, 68, 32, "_any"), (16, 3, 68, 32, "")])
+def test_transpose_by_lines_of_the_result(host, orc, stream, rows, planes, cols, bits, form):
+    """Whole 16-byte vectors: results whose rows are whole 64 bytes, or few and long, by the operator's own kernel; the
+    elements around the result untouched."""
+    dims = [rows, cols] if planes == 1 else [rows, planes, cols]
+    name = "imex_transpose%dd_b%d" % (len(dims), bits)
+    assert host.variant(name, dims) == name + form
+    say("%s %r by its lines" % (name, dims))
+    x = orc.fill_bits(rows * planes * cols, "f32" if bits == 32 else "bf16", rows).view(np.uint32 if bits == 32 else np.uint16)
+    d_in, d_out = stream.to_device(x), stream.to_device(np.full(x.size + 64, 7, x.dtype))
+    stream.launch(name, dims, [d_in, host.Ptr(d_out + 32 * x.itemsize), *dims])
+    stream.wait()
+    got = stream.from_device(d_out, (x.size + 64,), x.dtype)
+    stream.free(d_in), stream.free(d_out)
+    assert np.all(got[:32] == 7) and np.all(got[-32:] == 7)
+    assert np.array_equal(got[32:-32].reshape(dims[::-1]), x.reshape(dims).transpose(*range(len(dims))[::-1]))
+
+
 @pytest.mark.parametrize("rows,cols", [(4096, 4224), (128, 131072), (8192, 4096)])
 def test_transpose_b32_whole_tiles_pipelined(host, orc, stream, rows, cols):
     """32-bit problems made of whole 128 x 128 tiles: at most 512 workgroups, each walking two or more tiles
