@@ -32,7 +32,7 @@ __device__ __forceinline__ int chain_lanes(int64_t segments) { return segments <
 // four where it gets more of them, so that these share it (128 x 32768: 6.5 with eight, 3.9 with four).
 __device__ __forceinline__ int wide_chain_workers(int64_t segments) { return segments <= 4 * 256 ? 8 : 4; }
 
-// What the chains take: a tile's rows -- 64 where a row has more than 1024 segments, 256 at most -- within 32-bit offsets of
+// What the chains take: a tile's rows -- 64 where a row has more than 1024 segments, 512 at most -- within 32-bit offsets of
 // its first one.
 template <io::Dt D> __device__ __forceinline__ bool chains_take(int64_t rows, int64_t cols) {
   return rows > 0 && cols > 0 && cols * io::Elem<D>::kBytes < int64_t(1) << 26 && rows < int64_t(1) << 31;
@@ -77,7 +77,7 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   static constexpr int kTileFloats = kCols * kPitch;
   static constexpr int kLdsFloats = 2 * kTileFloats;
   static_assert(kLanes < 16 || kWorkers > 4 || kTileRows <= 64, "chains_take");
-  static_assert(kCols <= kWave && kTileRows % 64 == 0 && kTileRows <= 256, "a lane per column; the adder takes sixteen rows at a time, four deep");
+  static_assert(kCols <= kWave && kTileRows % 64 == 0 && kTileRows <= 512, "a lane per column; the adder takes sixteen rows at a time, four deep");
 
   typedef uint32_t Raw __attribute__((ext_vector_type(2), aligned(2))); // at any element's address
   struct Tile {

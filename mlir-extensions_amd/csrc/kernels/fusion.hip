@@ -26,7 +26,7 @@
 // block of c = 64 .. 8 columns (the widest that leaves 512 workgroups).  A launch with 256 lanes always gets
 // the last form, one with fewer a lane per column.  The _tall forms, by the 32-byte segments of a row (chain_lanes in
 // column_chain.h): up to 256 block (320,1,1), up to 1024 (576,1,1), beyond that (320,1,1); grid a workgroup per segment
-// of 32, 64 (257 .. 512) or 128 bytes.  With any other block they go as the forms with 256 lanes or fewer.  Workgroups
+// of 32, 64 (257 .. 512) or 128 bytes, of 16 where half_segments() says so.  With any other block they go as the forms with 256 lanes or fewer.  Workgroups
 // stride, so any grid is correct.
 
 #include "column_chain.h"
@@ -530,15 +530,24 @@ __device__ __forceinline__ void input_fusion_chains(const void *__restrict__ a, 
   });
 }
 
-// Four workers for segments of 32 bytes, eight for 64 (wide_chain_workers() for 128).  Other launches, and what the chains
-// do not take, go by blocks of columns, or a lane per column.
+// Segments of 16 bytes where they still fit one round and the rows are many: with 32 a CU's logarithms, not its additions, set
+// the pace (four instructions' cycles for each on four SIMDs, 3.4 .. 4 ns a row against 2.6), and half of the columns are half
+// of them: f16 6750 x 448 27.3 -> 22.2 us, bf16 8192 x 1024 32.5 -> 27.0, f32 8192 x 512 31.1 -> 26.6, and of rows of 4 KiB,
+// which crowd a few channels, f32 8192 x 1024 53.4 -> 42.5.  Fewer rows wait for the first tile instead: f16 2100 x 1100
+// 0.91 of the time, bf16 2100 x 1500 0.96, 1200 x 1500 1.03; f32 5000 x 700 0.92, 2100 x 700 0.98, 900 x 700 1.07.
+template <Dt D> __device__ __forceinline__ bool half_segments(int64_t rows, int64_t row) {
+  return row >= 32 && row <= 128 * 32 && rows >= (D == Dt::F32 ? 4096 : 2048);
+}
+// Four workers for segments of 16 and 32 bytes, eight for 64 (wide_chain_workers() for 128).  Other launches, and what the
+// chains do not take, go by blocks of columns, or a lane per column.
 template <Dt D>
 __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, const void *__restrict__ b,
                                                   void *__restrict__ out, int64_t rows, int64_t cols) {
   __shared__ __attribute__((aligned(16))) float lds[ColumnChain<D, 2, 16, 8>::kLdsFloats];
   __shared__ Logarithms<kMantissaOf<D>> logs;
   const int64_t row = cols * Elem<D>::kBytes, segments = (row + 31) / 32;
-  const int lanes = chain_lanes(segments), workers = lanes == 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
+  const int lanes = half_segments<D>(rows, row) ? 2 : chain_lanes(segments);
+  const int workers = lanes <= 4 ? 4 : lanes == 8 ? 8 : wide_chain_workers(segments);
   if (!chains_take<D>(rows, cols) || (row < 8 && rows * row < 8) || lanes_launched() != (workers + 1) * kWave) {
     if (lanes_launched() < kThreads) {
       input_fusion_by_element<D>(a, b, out, rows, cols, logs);
@@ -547,6 +556,8 @@ __device__ __forceinline__ void input_fusion_tall(const void *__restrict__ a, co
     logs.stage();
     __syncthreads();
     input_fusion_cols<D, 4, kSmallTileElems>(a, b, out, rows, cols, logs, lds);
+  } else if (lanes == 2) {
+    input_fusion_chains<D, 2, 4>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 4 && row < 8) {
     input_fusion_chains<D, 4, 4, true>(a, b, out, rows, cols, logs, lds);
   } else if (lanes == 4) {

@@ -710,14 +710,16 @@ extern "C" int imexHipKernelLaunchShape(const char *kernel, const int64_t *dims,
   case Shape::ReduceTall32:
   case Shape::ReduceTall16:
   case Shape::ColumnChains:
-  case Shape::ColumnChains16: { // a workgroup per segment of 32, 64 or 128 bytes: the kernels' own rule (chain_lanes in column_chain.h)
+  case Shape::ColumnChains16: { // a workgroup per segment of 16 .. 128 bytes: the kernels' own rule (chain_lanes in column_chain.h)
     const bool f32 = e->shape == Shape::ReduceTall32 || e->shape == Shape::ColumnChains;
     const bool reduce = e->shape == Shape::ReduceTall32 || e->shape == Shape::ReduceTall16;
     const int64_t perSegment = f32 ? 8 : 16;
     const size_t segments = ceilDiv(dims[1], perSegment);
     const int64_t times = chainWidth(segments);
     block[0] = (times == 4 && segments <= 4 * 256) || (times == 2 && !reduce) ? 576 : 320; // eight workers or four
-    grid[0] = gridFor(ceilDiv(dims[1], times * perSegment), block[0]);
+    // (the fused chain, half_segments in fusion.hip)
+    const bool half = !reduce && dims[1] >= perSegment && dims[1] <= 128 * perSegment && dims[0] >= (f32 ? 4096 : 2048);
+    grid[0] = gridFor(ceilDiv(dims[1], half ? perSegment / 2 : times * perSegment), block[0]);
     break;
   }
   case Shape::Gemm:

@@ -1019,6 +1019,34 @@ def test_input_fusion_narrow_rows(host, orc, stream, dtype, cols):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+def test_input_fusion_half_segments(host, orc, stream, dtype):
+    """Segments of 16 bytes, on both sides of the lines in rows and columns: tiles of 512 rows, whole, one row more and one
+    fewer; rows that are no whole segments, at any element's address; the elements around the result untouched."""
+    width, line = (4, 4096) if dtype == "f32" else (2, 2048)
+    least, most, name = 32 // width, 4096 // width, "imex_input_fusion_" + dtype
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    for rows in (line - 1, line, line + 1, line + 511):
+        for cols in (least - 1, least, least + 1, 5 * least + 3, most, most + 1):
+            assert host.variant(name, [rows, cols]) == name + "_tall"
+            half = rows >= line and least <= cols <= most
+            assert host.launch_shape(name + "_tall", [rows, cols])[0][0] == -(-cols // (16 // width if half else 32 // width))
+            say("%s %dx%d" % (name, rows, cols))
+            a = orc.fill_uniform(rows * cols, dtype, 97, -5.0, 5.0)
+            b = orc.fill_uniform(rows * cols, dtype, 98, 0.01, 40.0)
+            want = narrow(orc.input_fusion_f32(wide(a).reshape(rows, cols), wide(b).reshape(rows, cols)))
+            beside = narrow(np.full(1, np.nan, np.float32))
+            d_a, d_b = (stream.to_device(np.concatenate([beside, t, beside])) for t in (a, b))
+            d_out = stream.to_device(np.full(cols + 2, 3, a.dtype))
+            stream.launch(name, [rows, cols], [host.Ptr(p + width) for p in (d_a, d_b, d_out)] + [rows, cols])
+            stream.wait()
+            got = stream.from_device(d_out, (cols + 2,), a.dtype)
+            for p in (d_a, d_b, d_out):
+                stream.free(p)
+            assert np.array_equal(got[1:-1], want) and got[0] == 3 and got[-1] == 3
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("rows,segments,extra", [(300, 3, 1), (140, 300, -3), (130, 514, 7), (70, 1030, 5)])
 def test_column_chains_in_place(host, orc, stream, dtype, rows, segments, extra):
     """A result that lies in the first or the last row of its own matrix.  On one workgroup the last block of columns, which
