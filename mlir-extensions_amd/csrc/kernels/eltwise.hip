@@ -18,6 +18,15 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// The last block of a tensor, of fewer vectors than its lanes take: lane's j-th vector, or the last one again for lanes
+// past it, whose results go nowhere; and whether the j-th vectors of this wavefront are any (uniform).  (Element by element
+// the block was up to 32 loads one after the other for a lane, which the whole launch waited for: bf16 SiLU of 4701392
+// 11.6 -> 6.0 us, of 13000000 16.3 -> 11.8, f16 ReLU of 4701392 5.5 -> 5.0.)
+__device__ __forceinline__ int last_vec(int j, int vecs) { return min(j * kThreads + static_cast<int>(threadIdx.x), vecs - 1); }
+__device__ __forceinline__ bool wave_has(int j, int vecs) {
+  return j * kThreads + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) < vecs;
+}
+
 // ---------------------------------------------------------------------------
 // Generic streaming driver: Op works on one 16-byte vector (u32x4) and on one
 // scalar element (for ragged tails and unaligned bases).
@@ -30,16 +39,33 @@ __device__ __forceinline__ void stream_map_impl(const void *__restrict__ in, voi
   const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   // workgroups stride over the blocks, so a grid smaller than ceil(n / kElemsPerBlock) still covers n
   for (int64_t base = int64_t(blockIdx.x) * kElemsPerBlock; base < n; base += int64_t(gridDim.x) * kElemsPerBlock) {
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(in) + base * kElemBytes);
+    u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + base * kElemBytes);
+    u32x4 v[kVecsPerThread];
     if (aligned && base + kElemsPerBlock <= n) {
-      const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(in) + base * kElemBytes);
-      u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + base * kElemBytes);
-      u32x4 v[kVecsPerThread];
 #pragma unroll
       for (int j = 0; j < kVecsPerThread; ++j)
         v[j] = load128<kStream>(src + j * kThreads + threadIdx.x);
 #pragma unroll
       for (int j = 0; j < kVecsPerThread; ++j)
         store128<kStream>(op.vec(v[j]), dst + j * kThreads + threadIdx.x);
+    } else if (aligned) { // the last block
+      const int vecs = static_cast<int>((n - base) / kElemsPerVec);
+      if (vecs > 0) {
+#pragma unroll
+        for (int j = 0; j < kVecsPerThread; ++j)
+          v[j] = load128<kStream>(src + last_vec(j, vecs));
+#pragma unroll
+        for (int j = 0; j < kVecsPerThread; ++j)
+          if (wave_has(j, vecs)) {
+            const u32x4 r = op.vec(v[j]);
+            if (j * kThreads + static_cast<int>(threadIdx.x) < vecs)
+              store128<kStream>(r, dst + j * kThreads + threadIdx.x);
+          }
+      }
+      const int64_t i = base + int64_t(vecs) * kElemsPerVec + threadIdx.x;
+      if (i < n)
+        op.scalar(in, out, i);
     } else {
       for (int64_t i = base + threadIdx.x; i < base + kElemsPerBlock && i < n; i += kThreads)
         op.scalar(in, out, i);
@@ -64,10 +90,13 @@ __device__ __forceinline__ void stream_map2_b32(const uint32_t *__restrict__ a, 
   const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
                          reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   for (int64_t base = int64_t(blockIdx.x) * kElemsPerBlock; base < n; base += int64_t(gridDim.x) * kElemsPerBlock) {
+    const u32x4 *pa = reinterpret_cast<const u32x4 *>(a + base), *pb = reinterpret_cast<const u32x4 *>(b + base);
+    u32x4 *po = reinterpret_cast<u32x4 *>(out + base);
+    u32x4 va[kVecsPerThread], vb[kVecsPerThread];
+    auto result = [&](int j) {
+      return u32x4{op.one(va[j].x, vb[j].x), op.one(va[j].y, vb[j].y), op.one(va[j].z, vb[j].z), op.one(va[j].w, vb[j].w)};
+    };
     if (aligned && base + kElemsPerBlock <= n) {
-      const u32x4 *pa = reinterpret_cast<const u32x4 *>(a + base), *pb = reinterpret_cast<const u32x4 *>(b + base);
-      u32x4 *po = reinterpret_cast<u32x4 *>(out + base);
-      u32x4 va[kVecsPerThread], vb[kVecsPerThread];
 #pragma unroll
       for (int j = 0; j < kVecsPerThread; ++j) {
         va[j] = load128<true>(pa + j * kThreads + threadIdx.x);
@@ -75,9 +104,23 @@ __device__ __forceinline__ void stream_map2_b32(const uint32_t *__restrict__ a, 
       }
 #pragma unroll
       for (int j = 0; j < kVecsPerThread; ++j)
-        store128<true>(u32x4{op.one(va[j].x, vb[j].x), op.one(va[j].y, vb[j].y), op.one(va[j].z, vb[j].z),
-                             op.one(va[j].w, vb[j].w)},
-                       po + j * kThreads + threadIdx.x);
+        store128<true>(result(j), po + j * kThreads + threadIdx.x);
+    } else if (aligned) { // the last block
+      const int vecs = static_cast<int>((n - base) / 4);
+      if (vecs > 0) {
+#pragma unroll
+        for (int j = 0; j < kVecsPerThread; ++j) {
+          va[j] = load128<true>(pa + last_vec(j, vecs));
+          vb[j] = load128<true>(pb + last_vec(j, vecs));
+        }
+#pragma unroll
+        for (int j = 0; j < kVecsPerThread; ++j)
+          if (j * kThreads + static_cast<int>(threadIdx.x) < vecs)
+            store128<true>(result(j), po + j * kThreads + threadIdx.x);
+      }
+      const int64_t i = base + int64_t(vecs) * 4 + threadIdx.x;
+      if (i < n)
+        out[i] = op.one(a[i], b[i]);
     } else {
       for (int64_t i = base + threadIdx.x; i < base + kElemsPerBlock && i < n; i += kThreads)
         out[i] = op.one(a[i], b[i]);

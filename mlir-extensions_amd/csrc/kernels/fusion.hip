@@ -158,36 +158,59 @@ __device__ __forceinline__ void loop_fusion_pass(const void *__restrict__ a, con
                          reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   // workgroups stride over the blocks, so any grid covers n
   for (int64_t base = int64_t(blockIdx.x) * kElemsPerBlock; base < n; base += int64_t(gridDim.x) * kElemsPerBlock) {
+    const u32x4 *pa = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a) + base * E::kBytes);
+    const u32x4 *pb = reinterpret_cast<const u32x4 *>(static_cast<const char *>(b) + base * E::kBytes);
+    u32x4 *po = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + base * E::kBytes);
+    u32x4 va[kVecsPerThread], vb[kVecsPerThread];
+    auto result = [&](int j) {
+      float fa[E::kPerVec], fb[E::kPerVec];
+      E::unpack(va[j], fa);
+      E::unpack(vb[j], fb);
+      bool ordinary = true;
+#pragma unroll
+      for (int i = 0; i < E::kPerVec; ++i)
+        ordinary = ordinary && logf_ordinary(fa[i]);
+      if (__builtin_amdgcn_ballot_w64(!ordinary) == 0) { // uniform over the wavefront
+#pragma unroll
+        for (int i = 0; i < E::kPerVec; ++i)
+          fa[i] = loop_chain<true>(fa[i], fb[i], logs);
+      } else {
+#pragma unroll
+        for (int i = 0; i < E::kPerVec; ++i)
+          fa[i] = loop_chain(fa[i], fb[i], logs);
+      }
+      return E::pack(fa);
+    };
     if (aligned && base + kElemsPerBlock <= n) {
-      const u32x4 *pa = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a) + base * E::kBytes);
-      const u32x4 *pb = reinterpret_cast<const u32x4 *>(static_cast<const char *>(b) + base * E::kBytes);
-      u32x4 *po = reinterpret_cast<u32x4 *>(static_cast<char *>(out) + base * E::kBytes);
-      u32x4 va[kVecsPerThread], vb[kVecsPerThread];
 #pragma unroll
       for (int j = 0; j < kVecsPerThread; ++j) {
         va[j] = load128<true>(pa + j * kThreads + threadIdx.x);
         vb[j] = load128<true>(pb + j * kThreads + threadIdx.x);
       }
 #pragma unroll
-      for (int j = 0; j < kVecsPerThread; ++j) {
-        float fa[E::kPerVec], fb[E::kPerVec];
-        E::unpack(va[j], fa);
-        E::unpack(vb[j], fb);
-        bool ordinary = true;
+      for (int j = 0; j < kVecsPerThread; ++j)
+        store128<true>(result(j), po + j * kThreads + threadIdx.x);
+    } else if (aligned) {
+      // The last block: lanes past its last vector take that one again, and their results go nowhere.  (Element by element
+      // it was up to 32 loads and chains one after the other, which the whole launch waited for: bf16 4701392 11.5 -> 8.2 us.)
+      const int vecs = static_cast<int>((n - base) / E::kPerVec), lane = static_cast<int>(threadIdx.x);
+      if (vecs > 0) {
 #pragma unroll
-        for (int i = 0; i < E::kPerVec; ++i)
-          ordinary = ordinary && logf_ordinary(fa[i]);
-        if (__builtin_amdgcn_ballot_w64(!ordinary) == 0) { // uniform over the wavefront
-#pragma unroll
-          for (int i = 0; i < E::kPerVec; ++i)
-            fa[i] = loop_chain<true>(fa[i], fb[i], logs);
-        } else {
-#pragma unroll
-          for (int i = 0; i < E::kPerVec; ++i)
-            fa[i] = loop_chain(fa[i], fb[i], logs);
+        for (int j = 0; j < kVecsPerThread; ++j) {
+          va[j] = load128<true>(pa + min(j * kThreads + lane, vecs - 1));
+          vb[j] = load128<true>(pb + min(j * kThreads + lane, vecs - 1));
         }
-        store128<true>(E::pack(fa), po + j * kThreads + threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < kVecsPerThread; ++j)
+          if (j * kThreads + __builtin_amdgcn_readfirstlane(lane) < vecs) { // uniform
+            const u32x4 r = result(j);
+            if (j * kThreads + lane < vecs)
+              store128<true>(r, po + j * kThreads + lane);
+          }
       }
+      const int64_t i = base + int64_t(vecs) * E::kPerVec + lane;
+      if (i < n)
+        E::put(out, i, loop_chain(E::get(a, i), E::get(b, i), logs));
     } else {
       for (int64_t i = base + threadIdx.x; i < base + kElemsPerBlock && i < n; i += kThreads)
         E::put(out, i, loop_chain(E::get(a, i), E::get(b, i), logs));

@@ -562,6 +562,39 @@ def test_streaming_kernels_any_grid(host, orc, stream, grid):
     assert np.array_equal(got.view(np.uint32), orc.loop_fusion_f32(x, a).view(np.uint32))
 
 
+@pytest.mark.parametrize("kind,dtype", [("relu", "f32"), ("relu", "bf16"), ("silu", "f32"), ("silu", "f16"), ("silu", "bf16"),
+                                        ("exp", "f32"), ("maximum", "f32"), ("loop_fusion", "f32"), ("loop_fusion", "f16"),
+                                        ("loop_fusion", "bf16")])
+def test_last_block_of_a_tensor(host, orc, stream, kind, dtype):
+    """Tensors that end inside a block of four vectors per lane: fewer elements than a vector, a wavefront's vectors and one
+    more, all but one element, whole blocks; NaN and infinities behind them, nothing written there; against the oracle."""
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    ops = {"relu": lambda a, b: orc.relu_f32(a) if dtype == "f32" else orc.relu_16(a, dtype),
+           "silu": lambda a, b: orc.silu_f32(a) if dtype == "f32" else orc.silu_16(a, dtype),
+           "exp": lambda a, b: orc.expf_n(a), "maximum": lambda a, b: orc.maximum_f32(a, b),
+           "loop_fusion": lambda a, b: narrow(orc.loop_fusion_f32(wide(a), wide(b)))}
+    per, block, whole = (4, 4096, 1 << 22) if dtype == "f32" else (8, 8192, 1 << 22)
+    two, size, tail = kind in ("maximum", "loop_fusion"), whole + 2 * block, 3 * block
+    a = orc.fill_uniform(size, dtype, 33, 0.5, 6.0) if kind == "loop_fusion" else orc.fill_uniform(size, dtype, 33, -6.0, 6.0)
+    b = orc.fill_uniform(size, dtype, 34, -3.0, 3.0)
+    for past in (0, 1, per - 1, per, 64 * per, 65 * per, 256 * per + 3, block - per, block - 1, block):
+        n = whole + past
+        say("%s %s, %d elements" % (kind, dtype, n))
+        beside = narrow(np.resize(np.float32([np.nan, -np.inf, -1.0]), 64))
+        ins = [np.concatenate([t[:n], beside]) for t in ((a, b) if two else (a,))]
+        bufs, d_out = [stream.to_device(t) for t in ins], stream.to_device(np.full(n + 64, 3, a.dtype))
+        stream.launch("imex_%s_%s" % (kind, dtype), [n], bufs + [d_out, n])
+        stream.wait()
+        got = stream.from_device(d_out, (n + 64,), a.dtype)
+        for p in bufs + [d_out]:
+            stream.free(p)
+        bits = np.uint32 if dtype == "f32" else np.uint16
+        want = ops[kind](a[n - tail:n].copy(), b[n - tail:n].copy())
+        assert np.array_equal(got[n - tail:n].view(bits), want.view(bits)), past
+        assert np.all(got[n:] == 3), past
+
+
 # =============================== Transpose =================================
 def test_transpose_golden(host, orc, stream):
     g = GOLD["transpose_f32_10x20"]
