@@ -658,8 +658,7 @@ __device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ 
 template <typename T> __device__ __forceinline__ void pin(T &v) { asm volatile("" : "+v"(v)); }
 
 // ---- every wavefront its own keys, for two blocks of 32 queries -------------------------------
-// 64 QP queries, eight wavefronts: QP pairs of 32-query blocks x 8 / QP key groups.  A wavefront takes its group's 32-key
-// tiles, in LDS of its own, through the two blocks of its pair, A and B: a
+// 64 queries, eight wavefronts, each of which takes every eighth 32-key tile through both blocks of 32 queries, A and B: a
 // fragment is read from LDS once for two products (half the LDS reads of attention_tiled's two query blocks x four key
 // groups, which this replaced), and no barrier stands between the first and the merge.  The two blocks are half a tile
 // apart: while one's scores go through the softmax, the matrix cores take the other's eight products, one between every two
@@ -668,31 +667,27 @@ template <typename T> __device__ __forceinline__ void pin(T &v) { asm volatile("
 // 256 in f16, relative rounding as before), so the accumulators are rescaled in the first tiles instead of in nearly all.
 // The queries come through LDS, 1 KiB a wavefront: as fragments from memory (32 rows a load) and behind three tiles of
 // copies they held the first product up for 5000 cycles, now 2800.
-//   4 x 4096 28.7 -> 25.0 us, 4 x 4000 29.4 -> 25.8, 8 x 2048 16.7 -> 14.6, 5 x 3001 22.8 -> 20.1, 16 x 1000 11.1 -> 10.7;
-//   QP = 2 (against four query blocks x two key groups): 8 x 4096 50.0 -> 46.6, 6 x 4096 45.0 -> 41.0, 12 x 2600 36.5 -> 32.7,
-//   30 x 1000 16.9 -> 16.5; QP = 4 is no faster than sixteen wavefronts (16 x 4096 85.8, 84.2), which stay.
+//   4 x 4096 28.7 -> 25.0 us, 4 x 4000 29.4 -> 25.8, 8 x 2048 16.7 -> 14.6, 5 x 3001 22.8 -> 20.1, 16 x 1000 11.1 -> 10.7.
 // What bounds it: 1.1 .. 1.3 us per tile of two wavefronts on a SIMD (0.97 on zeros: the clock falls on random operands),
 // issue of 2 x (32 exponentials, 16 products, about 150 others) at 12, 13 and 3.2 cycles, and about 6 us around the loop,
 // 2.5 of them the launch, 1.9 the merge of eight partial results.  Taken back: a barrier per tile or per four (the
 // wavefronts of a SIMD end within 1000 cycles of each other instead of 10000, 4 x 4096 25.5 -> 26.0), s_setprio (none).
 constexpr int kPairWave = 4 * kOwnTile; // two places for K, two for V
-template <int QP> constexpr int kPairLds = kOwnWaves * kPairWave + QP * 64 * D * 2; // the tiles, the queries
-static_assert(kPairLds<1> >= 2 * kOwnWaves * kSlot * 4, "the partial results fit");
+constexpr int kPairLds = kOwnWaves * kPairWave + 64 * D * 2; // the tiles, the queries
+static_assert(kPairLds >= 2 * kOwnWaves * kSlot * 4, "the partial results fit");
 
-template <int QP, bool kRagged>
+template <bool kRagged>
 __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
                                                 const uint16_t *__restrict__ V, uint16_t *__restrict__ Out, float scale,
                                                 int64_t N, char *lds) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int qi = lane & 31, half = lane >> 5;
-  constexpr int KG = kOwnWaves / QP;                  // key groups
-  const int pair = wave % QP, group = wave / QP;      // of 64 queries, of keys
   uint32_t bx, by;
   place_of_workgroup(bx, by);
-  const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * (64 * QP);
+  const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 64;
   const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
-  const int iters = tiles > group ? (tiles - group + KG - 1) / KG : 0;
+  const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
 
   // copies, places and fragment addresses: as in attention_own_keys
   const __amdgpu_buffer_rsrc_t kRsrc = make_rsrc(K + head0 * D, N * D * 2), vRsrc = make_rsrc(V + head0 * D, N * D * 2);
@@ -710,7 +705,7 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
   char *own = lds + wave * kPairWave; // K, K, V, V
   auto dma = [&](const __amdgpu_buffer_rsrc_t &rsrc, const int (&off)[4], const int (&offT)[4], int i, int place) {
     LdsChar *dst = (LdsChar *)own + place * kOwnTile;
-    const int tile = group + i * KG;
+    const int tile = wave + i * kOwnWaves;
     const bool tail = kRagged && tile == tiles - 1;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -766,7 +761,7 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
   // One block's tile `i` through the softmax, step(0) .. step(7), the other block's products, between its exponentials, and
   // middle() behind the last of them.
   auto softmax = [&](f32x16 &s, f16x8 (&p)[2], f32x16 (&o)[2], float &m, float &l, int i, auto &&step, auto &&middle) {
-    if (kRagged && group + i * KG == tiles - 1 && lastRows < kOwnKeys) { // uniform over the wavefront
+    if (kRagged && wave + i * kOwnWaves == tiles - 1 && lastRows < kOwnKeys) { // uniform over the wavefront
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         s[r] = (r >> 2) * 8 + half * 4 + (r & 3) < lastRows ? s[r] : -__builtin_inff();
@@ -822,14 +817,12 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
     l += sum[0] + sum[1];
   };
 
-  // The queries, 8 QP rows a wavefront, laid out as K's.
-  const __amdgpu_buffer_rsrc_t qRsrc = make_rsrc(Q + q0 * D, (head0 + N - q0) * D * 2);
-#pragma unroll
-  for (int u = 0; u < QP; ++u) {
-    const int row = (wave * QP + u) * 8 + (lane >> 3);
-    const int there = kRagged ? int(min(int64_t(row), N - 1 - int64_t(bx) * (64 * QP))) : row;
+  // The queries, 8 rows a wavefront, laid out as K's.
+  {
+    const int row = wave * 8 + (lane >> 3), there = kRagged ? int(min(int64_t(row), N - 1 - int64_t(bx) * 64)) : row;
     const int chunk = (lane & 7) ^ ((row ^ ((row >> 3) & 3)) & 7);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(qRsrc, (LdsChar *)lds + kOwnWaves * kPairWave + (wave * QP + u) * 1024, 16,
+    const __amdgpu_buffer_rsrc_t qRsrc = make_rsrc(Q + q0 * D, (head0 + N - q0) * D * 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(qRsrc, (LdsChar *)lds + kOwnWaves * kPairWave + wave * 1024, 16,
                                              (there * D + chunk * 8) * 2, 0, 0, 0);
   }
   dma_k(0);
@@ -843,7 +836,7 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds)
-        qf[b][ds] = *reinterpret_cast<const f16x8 *>(lds + kOwnWaves * kPairWave + (pair * 2 + b) * (32 * 128) + kRd[ds]);
+        qf[b][ds] = *reinterpret_cast<const f16x8 *>(lds + kOwnWaves * kPairWave + b * (32 * 128) + kRd[ds]);
     read_k(0);
     read_done();
     dma_v(1);
@@ -885,13 +878,11 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
   wait_vmcnt<0>();
   float *all = reinterpret_cast<float *>(lds);
   __syncthreads(); // everyone's tiles are done with
-  put_partial(oA, mA, lA + other_half(lA), all + (pair * 2 * KG + group) * kSlot, lane);
-  put_partial(oB, mB, lB + other_half(lB), all + ((pair * 2 + 1) * KG + group) * kSlot, lane);
+  put_partial(oA, mA, lA + other_half(lA), all + wave * kSlot, lane);
+  put_partial(oB, mB, lB + other_half(lB), all + (kOwnWaves + wave) * kSlot, lane);
   __syncthreads();
-  constexpr int kMerging = 4 / QP; // wavefronts that share the merge of a block of 32 queries
-  const int block = wave / kMerging;
-  merge_partials<KG, 8 / kMerging>(all + block * (KG * kSlot), Out, q0 + block * 32, head0 + N, wave % kMerging * (8 / kMerging),
-                                   lane, kRagged);
+  merge_partials<kOwnWaves, 1>(all, Out, q0, head0 + N, wave, lane, kRagged);
+  merge_partials<kOwnWaves, 1>(all + kOwnWaves * kSlot, Out, q0 + 32, head0 + N, wave, lane, kRagged);
 }
 
 // What the tiled path takes, of the arguments and of the launch.
@@ -942,7 +933,7 @@ extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_f
 }
 
 // One tiling each, for problems whose tilings by the rule above leave CUs idle or run a nearly empty last round
-// (attentionVariant in KernelCatalog.cpp).
+// (attentionVariant in KernelCatalog.cpp).  128 queries are the form above with the next block's scores formed ahead.
 template <int QB, int KG, bool kScoresAhead>
 __device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                                      uint16_t *Out, float scale, int64_t ZH, int64_t N, char *lds) {
@@ -956,6 +947,13 @@ __device__ __forceinline__ void attention_one_tiling(const uint16_t *Q, const ui
     attention_tiled<QB, KG, true, kScoresAhead>(Q, K, V, Out, scale, N, lds);
 }
 
+#define IMEX_ATTENTION_TILING(QUERIES, QB, KG, AHEAD)                                                                  \
+  extern "C" __global__ __launch_bounds__(QB *KG *kWave) void imex_flash_attention_fwd_f16_q##QUERIES(                \
+      const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH,             \
+      int64_t N_CTX) {                                                                                                \
+    __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];                                                      \
+    attention_one_tiling<QB, KG, AHEAD>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);                                      \
+  }
 extern "C" __global__ __launch_bounds__(kOwnWaves *kWave, 4) void imex_flash_attention_fwd_f16_q32(
     const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
   __shared__ __attribute__((aligned(16))) char lds[kOwnLds];
@@ -968,32 +966,13 @@ extern "C" __global__ __launch_bounds__(kOwnWaves *kWave, 4) void imex_flash_att
 }
 extern "C" __global__ __launch_bounds__(kOwnWaves *kWave) void imex_flash_attention_fwd_f16_q64(
     const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
-  __shared__ __attribute__((aligned(16))) char lds[kPairLds<1>];
+  __shared__ __attribute__((aligned(16))) char lds[kPairLds];
   if (!attention_shaped(Q, K, V, Out, sm_scale, ZH, N_CTX) || blockDim.x != kOwnWaves * kWave || gridDim.x != (N_CTX + 63) / 64)
     attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
   else if (N_CTX % 64 == 0)
-    attention_pairs<1, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
+    attention_pairs<false>(Q, K, V, Out, sm_scale, N_CTX, lds);
   else
-    attention_pairs<1, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
+    attention_pairs<true>(Q, K, V, Out, sm_scale, N_CTX, lds);
 }
-// Up to 512 keys four query blocks x two key groups have less to merge for their few tiles: 200 x 128 7.2 us, pairs of
-// blocks 7.8, 64 x 512 11.2, 11.5; 40 x 700 14.1, 13.1.
-extern "C" __global__ __launch_bounds__(kOwnWaves *kWave) void imex_flash_attention_fwd_f16_q128(
-    const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
-  __shared__ __attribute__((aligned(16))) char lds[kPairLds<2>];
-  static_assert(kPairLds<2> >= kLdsBytes);
-  if (N_CTX <= 512)
-    attention_one_tiling<4, 2, true>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);
-  else if (!attention_shaped(Q, K, V, Out, sm_scale, ZH, N_CTX) || blockDim.x != kOwnWaves * kWave ||
-           gridDim.x != (N_CTX + 127) / 128)
-    attention_scalar(Q, K, V, Out, sm_scale, ZH, N_CTX);
-  else if (N_CTX % 128 == 0)
-    attention_pairs<2, false>(Q, K, V, Out, sm_scale, N_CTX, lds);
-  else
-    attention_pairs<2, true>(Q, K, V, Out, sm_scale, N_CTX, lds);
-}
-extern "C" __global__ __launch_bounds__(kMaxThreads) void imex_flash_attention_fwd_f16_q256(
-    const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *Out, float sm_scale, int64_t ZH, int64_t N_CTX) {
-  __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
-  attention_one_tiling<8, 2, false>(Q, K, V, Out, sm_scale, ZH, N_CTX, lds);
-}
+IMEX_ATTENTION_TILING(128, 4, 2, true)
+IMEX_ATTENTION_TILING(256, 8, 2, false)

@@ -424,17 +424,14 @@ const char *transposeVariant(const Entry *e, const int64_t *dims) {
 // (1 x 4096 27.6 -> 14.8 us, 8 x 1024 10.0 -> 7.6, 16 x 512 7.1 -> 6.0, 4 x 64 6.0 -> 4.2; at 264 workgroups 24 x 333
 // 7.6, 7.7, at 288 48 x 192 6.2, 7.1), 128 where 64 take two (12 x 1500 27.0 -> 20.1, 6 x 4096 53.1 -> 42.5, 64 x 320 14.2
 // -> 9.2, 200 x 128 11.6 -> 7.0), 256 where 128 take two (12 x 4096 85.1 -> 68.3, 100 x 333 19.1 -> 14.1).  Of the two
-// forms with 64 queries the one whose wavefronts have keys of their own (pairs) from 768 keys on (4 x 4096 30.8 -> 25.0, 16 x
-// 1000 11.6 -> 10.7) and where the last 256 keys are no more than half there (32 x 320 7.7 -> 6.7, 16 x 600 9.1 -> 8.3, 20 x
-// 640 9.3 -> 8.0; it merges more for its few tiles elsewhere: 16 x 700 9.1, 9.1, 24 x 512 7.4, 7.8, 40 x 256 6.0, 6.5); of
-// those with 128 that one from 1025 on (16 x 2000 29.2 -> 27.1, 32 x 1024 16.2, 16.5, 128 x 256 9.3, 9.5).
-// Problems that fill more than one round with 256 queries stay.
+// forms with 64 queries the one whose wavefronts have keys of their own from 768 keys on (4 x 4096 30.8 -> 25.0, 16 x 1000
+// 11.6 -> 10.7, 16 x 768 9.2 -> 8.8; below it merges more for its few tiles, 16 x 700 9.2, 9.3, 40 x 256 6.0, 6.7).  Problems that fill more than one round with 256 queries stay.
 struct Tiling {
   const char *suffix;
   int64_t queries;
   double cost;
 };
-constexpr Tiling kTilings[] = {{"_q32", 32, 15.5}, {"_q64", 64, 23.5}, {"_q128", 128, 40.0}, {"_q256", 256, 68.0}};
+constexpr Tiling kTilings[] = {{"_q32", 32, 15.5}, {"_q64", 64, 23.5}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
 
 const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
   auto workgroups = [&](int64_t queries) { return (N + queries - 1) / queries * ZH; };
@@ -452,8 +449,7 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
       least = cost;
     }
   }
-  const bool pairs = own == 64 ? N >= 768 || (N > 256 && N % 256 >= 1 && N % 256 <= 128) : own == 128 && N > 1024;
-  if (best->queries == own && !pairs)
+  if (best->queries == own && (own != 64 || N < 768))
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s%s", e->name, best->suffix);
