@@ -663,13 +663,16 @@ template <typename T> __device__ __forceinline__ void pin(T &v) { asm volatile("
 // groups, which this replaced), and no barrier stands between the first and the merge.  The two blocks are half a tile
 // apart: while one's scores go through the softmax, the matrix cores take the other's eight products, one between every two
 // exponentials (a wavefront issues in order: products in a row hold it for 32 cycles each, and a SIMD has two wavefronts
-// here).  The reference that the exponentials are taken against moves only when a score exceeds it by 2^8 (P stays below
-// 256 in f16, relative rounding as before), so the accumulators are rescaled in the first tiles instead of in nearly all.
+// here).  The exponentials are taken against the running maximum itself, though a reference that lags it by up to 2^8 would
+// rescale the accumulators in the first tiles only and be 10 % faster (4 x 4096 24.2 us): the largest weights, which are 1 and
+// just below it here, would be rounded anywhere in their binade, and the error against 64 bits grows by as much (2-norm,
+// 4 x 4096: 2.62e-4 before, 2.88e-4 lagging, 2.56e-4 so; a reference half a power of two ahead, 2.69e-4, saves nothing).
 // The queries come through LDS, 1 KiB a wavefront: as fragments from memory (32 rows a load) and behind three tiles of
 // copies they held the first product up for 5000 cycles, now 2800.
-//   4 x 4096 28.7 -> 25.0 us, 4 x 4000 29.4 -> 25.8, 8 x 2048 16.7 -> 14.6, 5 x 3001 22.8 -> 20.1, 16 x 1000 11.1 -> 10.7.
-// What bounds it: 1.1 .. 1.3 us per tile of two wavefronts on a SIMD (0.97 on zeros: the clock falls on random operands),
-// issue of 2 x (32 exponentials, 16 products, about 150 others) at 12, 13 and 3.2 cycles, and about 6 us around the loop,
+//   4 x 4096 28.1 -> 27.6 us, 3 x 3500 25.0 -> 24.3, 5 x 3001 23.5 -> 23.0, 16 x 1000 11.4, 11.4, 16 x 600 9.1 -> 8.6, 20 x
+//   640 9.2 -> 8.1.  (128 queries as two pairs and four key groups 48.9 on 8 x 4096, by the form above 46.8.)
+// What bounds it: about 1.4 us per tile of two wavefronts on a SIMD, issue of 2 x (32 exponentials, 16 products, about 210
+// others) at 12, 13 and 3.2 cycles at the clock that random operands leave, and about 6 us around the loop,
 // 2.5 of them the launch, 1.9 the merge of eight partial results.  Taken back: a barrier per tile or per four (the
 // wavefronts of a SIMD end within 1000 cycles of each other instead of 10000, 4 x 4096 25.5 -> 26.0), s_setprio (none).
 constexpr int kPairWave = 4 * kOwnTile; // two places for K, two for V
@@ -771,7 +774,7 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
     for (int r = 2; r < 16; ++r)
       part[r & 1] = fmaxf(part[r & 1], s[r]);
     const float mx = max_of_halves(fmaxf(part[0], part[1])) * c;
-    if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) { // the running max moved for some query
       const float mNew = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mNew);
       m = mNew;
       l *= alpha;
@@ -881,8 +884,8 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
   put_partial(oA, mA, lA + other_half(lA), all + wave * kSlot, lane);
   put_partial(oB, mB, lB + other_half(lB), all + (kOwnWaves + wave) * kSlot, lane);
   __syncthreads();
-  merge_partials<kOwnWaves, 1>(all, Out, q0, head0 + N, wave, lane, kRagged);
-  merge_partials<kOwnWaves, 1>(all + kOwnWaves * kSlot, Out, q0 + 32, head0 + N, wave, lane, kRagged);
+  const int block = wave / 4; // four wavefronts merge a block of 32 queries
+  merge_partials<kOwnWaves, 2>(all + block * (kOwnWaves * kSlot), Out, q0 + block * 32, head0 + N, wave % 4 * 2, lane, kRagged);
 }
 
 // What the tiled path takes, of the arguments and of the launch.

@@ -424,14 +424,16 @@ const char *transposeVariant(const Entry *e, const int64_t *dims) {
 // (1 x 4096 27.6 -> 14.8 us, 8 x 1024 10.0 -> 7.6, 16 x 512 7.1 -> 6.0, 4 x 64 6.0 -> 4.2; at 264 workgroups 24 x 333
 // 7.6, 7.7, at 288 48 x 192 6.2, 7.1), 128 where 64 take two (12 x 1500 27.0 -> 20.1, 6 x 4096 53.1 -> 42.5, 64 x 320 14.2
 // -> 9.2, 200 x 128 11.6 -> 7.0), 256 where 128 take two (12 x 4096 85.1 -> 68.3, 100 x 333 19.1 -> 14.1).  Of the two
-// forms with 64 queries the one whose wavefronts have keys of their own from 768 keys on (4 x 4096 30.8 -> 25.0, 16 x 1000
-// 11.6 -> 10.7, 16 x 768 9.2 -> 8.8; below it merges more for its few tiles, 16 x 700 9.2, 9.3, 40 x 256 6.0, 6.7).  Problems that fill more than one round with 256 queries stay.
+// forms with 64 queries the one whose wavefronts have keys of their own from 768 keys on (4 x 4096 30.8 -> 27.6, 16 x 1000
+// 11.6 -> 11.4) and where the last 256 keys are no more than half there (16 x 600 9.1 -> 8.6, 32 x 320 7.7 -> 6.8; it merges
+// more for its few tiles elsewhere: 24 x 512 7.5, 7.8, 40 x 256 6.0, 6.5).
+// Problems that fill more than one round with 256 queries stay.
 struct Tiling {
   const char *suffix;
   int64_t queries;
   double cost;
 };
-constexpr Tiling kTilings[] = {{"_q32", 32, 15.5}, {"_q64", 64, 23.5}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
+constexpr Tiling kTilings[] = {{"_q32", 32, 15.5}, {"_q64", 64, 26.0}, {"_q128", 128, 43.0}, {"_q256", 256, 68.0}};
 
 const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
   auto workgroups = [&](int64_t queries) { return (N + queries - 1) / queries * ZH; };
@@ -449,7 +451,8 @@ const char *attentionVariant(const Entry *e, int64_t ZH, int64_t N) {
       least = cost;
     }
   }
-  if (best->queries == own && (own != 64 || N < 768))
+  const bool ownKeys = own == 64 && (N >= 768 || (N > 256 && N % 256 >= 1 && N % 256 <= 128));
+  if (best->queries == own && !ownKeys)
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s%s", e->name, best->suffix);
