@@ -502,8 +502,11 @@ def _check(x, dtype):
 #    (f16 softmax of 1024 x 2000 473 -> 345 us), hence _STAGED_BYTES, the largest of them;
 #  - 3-D transposes likewise (32^3 154 -> 33), but for runs of a few elements (d0 or d2 under 32) with more than a few planes
 #    between them: 2 x 1000 x 60 87 -> 116, where 65536 x 4 x 4 takes 478 -> 350;
-#  - softmax of rows that a workgroup keeps in registers likewise; one of 262144 columns reads its row again and from few
-#    workgroups (1 x 1048576 f32 1081 -> 2145 us), so rows end at _STAGED_SOFTMAX_COLS (1 x 65536: 95 -> 84);
+#  - softmax of rows that a workgroup keeps in registers (_STAGED_SOFTMAX_ROW bytes) likewise, and of longer ones of whole 16-byte
+#    vectors to _STAGED_SOFTMAX_COLS (1 x 65536 f32 97 -> 92, bf16 71 -> 61; one of 262144 columns reads its row again and from
+#    few workgroups, 1 x 1048576 f32 1081 -> 2145).  Longer ones element by element wait for every load of the link twice: 1 x
+#    20001 f32 91 -> 130, 10 x 40001 bf16 206 -> 296, until there are rows enough to wait side by side (_STAGED_SOFTMAX_ROWS: 64 x
+#    20001 633 -> 476, 64 x 65535 1853 -> 1571, one 204 -> 369);
 #  - sums: chains of dependent loads wait for the link (row sums of 65536 x 1 70 -> 79 us, column sums of 8192 x 32
 #    127 -> 138, 32768 x 32 318 -> 464, f16 2000 x 300 120 -> 125) and little is written back (row sums of 2048 x 2048
 #    557 -> 605), so only runs of 32 (rows) or 512 columns, of at most _STAGED_SUMS bytes: 512 x 1024 162 -> 118, columns
@@ -512,6 +515,8 @@ _STAGED_SMALL = 64 << 10
 _STAGED_SUMS = 5 << 19
 _STAGED_BYTES = 32 << 20
 _STAGED_SOFTMAX_COLS = 65536
+_STAGED_SOFTMAX_ROW = 64 << 10
+_STAGED_SOFTMAX_ROWS = 64
 
 
 def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
@@ -655,8 +660,10 @@ def mfma_lds_ceiling(stream, workgroups, iters, mode=0):
 def softmax(stream, x, dtype="f32"):
     """benchmarks/softmax/softmax_gpu.mlir.in:4-44 (last dim of a 2-D tensor)"""
     rows, cols = x.shape
+    row = cols * x.dtype.itemsize
+    fits = row <= _STAGED_SOFTMAX_ROW or row % 16 == 0 or rows >= _STAGED_SOFTMAX_ROWS
     return _unary(stream, "imex_softmax_" + dtype, x, dtype, [rows, cols],
-                  staged=_STAGED_BYTES if cols <= _STAGED_SOFTMAX_COLS else 0)
+                  staged=_STAGED_BYTES if cols <= _STAGED_SOFTMAX_COLS and fits else 0)
 
 
 def rowsum(stream, x, init=0.0):

@@ -384,6 +384,36 @@ def test_staging_block_of_a_queue(host):
     assert not live and s.handle is None
 
 
+class _Way(Exception):
+    """Raised in place of the work by the queue of `way_of`."""
+
+
+def way_of(host, op, shape, dtype="f32"):
+    """"staged" or "device": where the host function `op` puts operands of this shape."""
+    class Queue:
+        def staging(self, nbytes):
+            raise _Way("staged")
+
+        def to_device(self, array):
+            raise _Way("device")
+    x = np.empty(shape, np.float32 if dtype == "f32" else np.uint16)
+    typed = {} if op in ("maximum", "rowsum", "rowmean", "transpose2d", "transpose3d") else {"dtype": dtype}
+    with pytest.raises(_Way) as way:
+        getattr(host, op)(Queue(), *[x] * (1 + (op in ("maximum", "loop_fusion", "input_fusion"))), **typed)
+    return str(way.value)
+
+
+@pytest.mark.parametrize("dtype,kept", [("f32", 16384), ("f16", 32768), ("bf16", 32768)])
+def test_softmax_staging_rule(host, dtype, kept):
+    """Rows that a workgroup cannot keep in registers and that are no whole vectors go through device buffers unless there
+    are many of them: read twice over the link, element by element, one of them took up to 1.8 times as long."""
+    way = lambda rows, cols: way_of(host, "softmax", (rows, cols), dtype)
+    for rows in (1, 10, 63):
+        assert way(rows, kept) == way(rows, kept - 1) == way(rows, kept + 8) == way(rows, 65536) == "staged"
+        assert way(rows, kept + 1) == way(rows, 40001) == way(rows, 65535) == way(rows, 65537) == "device"
+    assert way(64, kept + 1) == way(64, 40001) == "staged" and way(64, 65537) == way(1, 262144) == "device"
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
