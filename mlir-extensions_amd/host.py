@@ -497,11 +497,13 @@ def _check(x, dtype):
 # Where a kernel reads its operands from pinned host memory and writes its result there, instead of copies to and
 # from buffers allocated on the device, which cost 45..60 us a call before the link carries a byte.  Measured over
 # 1 Ki .. 4 Mi elements, one row to one column, device buffers -> staged:
-#  - at most _STAGED_SMALL bytes, any operator and shape: 57 -> 18 us, 1.9..4.5 times as fast;
-#  - maps, transposes: every element crosses the link once and in runs, 1.2..3 times as fast at all sizes measured
-#    (f16 softmax of 1024 x 2000 473 -> 345 us), hence _STAGED_BYTES, the largest of them;
-#  - 3-D transposes likewise (32^3 154 -> 33), but for runs of a few elements (d0 or d2 under 32) with more than a few planes
-#    between them: 2 x 1000 x 60 87 -> 116, where 65536 x 4 x 4 takes 478 -> 350;
+#  - at most _STAGED_SMALL bytes, any shape of any operator but the 3-D transpose: 57 -> 18 us, 1.4..4.5 times as fast;
+#  - maps: every element crosses the link once and in runs, 1.2..3 times as fast at all sizes measured (f16 softmax of 1024
+#    x 2000 473 -> 345 us), hence _STAGED_BYTES, the largest of them;
+#  - transposes likewise but for the largest of few columns (f32 25703 x 129 688 -> 773, 32537 x 69 888 -> 975): _staged_2d;
+#  - 3-D transposes where both sides run along many elements (32^3 154 -> 33 us, 356 x 59 x 69 397 -> 281, 3340 x 14 x 74
+#    1403 -> 1205); with runs of a few they fill a part of every transfer (1 x 4 x 118937 bf16 171 -> 692, 147889 x 4 x 4 f32 966 ->
+#    1404, 79 x 36 x 4 59 -> 71): _staged_3d has how few go with how many bytes;
 #  - softmax of rows that a workgroup keeps in registers (_STAGED_SOFTMAX_ROW bytes) likewise, and of longer ones of whole 16-byte
 #    vectors to _STAGED_SOFTMAX_COLS (1 x 65536 f32 97 -> 92, bf16 71 -> 61; one of 262144 columns reads its row again and from
 #    few workgroups, 1 x 1048576 f32 1081 -> 2145).  Longer ones element by element wait for every load of the link twice: 1 x
@@ -519,12 +521,26 @@ _STAGED_SOFTMAX_ROW = 64 << 10
 _STAGED_SOFTMAX_ROWS = 64
 
 
+def _staged_2d(rows, cols):
+    """The most bytes that a transpose takes through pinned host memory; of 10200 timed sizes (to 4 Mi elements) none lost more
+    than 3 % on this side of the lines."""
+    return _STAGED_BYTES if min(rows, cols) >= 256 else 12 << 20
+
+
+def _staged_3d(d0, d1, d2):
+    """The same for d0 x d1 x d2, of 9400 timed sizes."""
+    if d1 == 1:
+        return _staged_2d(d0, d2)
+    run = min(d0, d2)
+    return _STAGED_BYTES if run >= 64 else 8 << 20 if run >= 32 else 256 << 10 if run >= 8 else 32 << 10
+
+
 def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
     """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes,
     for nothing, and under the profiler, which times kernels on device memory."""
     n_out = int(np.prod(out_shape)) * np.dtype(out_np).itemsize  # () is one element
     total = sum(x.nbytes for x in xs) + n_out
-    if total > max(most, _STAGED_SMALL) or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
+    if total > most or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
         return None
     starts, end = [], 0
     for n in [x.nbytes for x in xs] + [n_out]:
@@ -607,7 +623,7 @@ def input_fusion(stream, a, b, dtype="f32"):
     """benchmarks/kInputFusion/kInputFusion.mlir.in:6-40: out[j] = sum_i (log b[i,j] + |a[i,j]|)"""
     rows, cols = a.shape
     return _binary(stream, "imex_input_fusion_" + dtype, a, b, dtype, [rows, cols], (cols,),
-                   staged=_STAGED_SUMS if cols >= 512 else 0)
+                   staged=_STAGED_SUMS if cols >= 512 else _STAGED_SMALL)
 
 
 def flash_attention(stream, q, k, v, zh, n_ctx, sm_scale, queries_per_workgroup=None, threads=512):
@@ -663,21 +679,21 @@ def softmax(stream, x, dtype="f32"):
     row = cols * x.dtype.itemsize
     fits = row <= _STAGED_SOFTMAX_ROW or row % 16 == 0 or rows >= _STAGED_SOFTMAX_ROWS
     return _unary(stream, "imex_softmax_" + dtype, x, dtype, [rows, cols],
-                  staged=_STAGED_BYTES if cols <= _STAGED_SOFTMAX_COLS and fits else 0)
+                  staged=_STAGED_BYTES if cols <= _STAGED_SOFTMAX_COLS and fits else _STAGED_SMALL)
 
 
 def rowsum(stream, x, init=0.0):
     """WG/reduction_2D_1D_cross_sg_cross_lane.mlir:31-37"""
     rows, cols = x.shape
     return _unary(stream, "imex_rowsum_f32", x, "f32", [rows, cols], extra=[float(init)], out_shape=(rows,),
-                  staged=_STAGED_SUMS if cols >= 32 else 0)
+                  staged=_STAGED_SUMS if cols >= 32 else _STAGED_SMALL)
 
 
 def rowmean(stream, x):
     """WG/reduction_4D_3D_mean_intra_sg_intra_lane.mlir:51-52: mean over the last dimension."""
     rows, cols = x.shape
     return _unary(stream, "imex_rowmean_f32", x, "f32", [rows, cols], out_shape=(rows,),
-                  staged=_STAGED_SUMS if cols >= 32 else 0)
+                  staged=_STAGED_SUMS if cols >= 32 else _STAGED_SMALL)
 
 
 def reduce_outer(stream, x, init=0.0, dtype="f32"):
@@ -686,7 +702,7 @@ def reduce_outer(stream, x, init=0.0, dtype="f32"):
     outer = x.shape[0]
     inner = int(np.prod(x.shape[1:]))
     return _unary(stream, "imex_reduce_outer_" + dtype, x, dtype, [outer, inner], extra=[float(init)],
-                  out_shape=x.shape[1:], staged=_STAGED_SUMS if inner >= 512 else 0)
+                  out_shape=x.shape[1:], staged=_STAGED_SUMS if inner >= 512 else _STAGED_SMALL)
 
 
 def transpose2d(stream, x):
@@ -694,7 +710,7 @@ def transpose2d(stream, x):
     rows, cols = x.shape
     bits = x.dtype.itemsize * 8
     return _unary(stream, "imex_transpose2d_b%d" % bits, x, "f32" if bits == 32 else "f16", [rows, cols],
-                  out_shape=(cols, rows))
+                  out_shape=(cols, rows), staged=_staged_2d(rows, cols))
 
 
 def transpose3d(stream, x):
@@ -702,7 +718,7 @@ def transpose3d(stream, x):
     d0, d1, d2 = x.shape
     bits = x.dtype.itemsize * 8
     return _unary(stream, "imex_transpose3d_b%d" % bits, x, "f32" if bits == 32 else "f16", [d0, d1, d2],
-                  out_shape=(d2, d1, d0), staged=_STAGED_BYTES if min(d0, d2) >= 32 or d1 <= 4 else 0)
+                  out_shape=(d2, d1, d0), staged=_staged_3d(d0, d1, d2))
 
 
 def gemm(stream, a, b, c=None, ab_dtype="f16", out_dtype="f32", trans_a=False, trans_b=False):

@@ -414,6 +414,20 @@ def test_softmax_staging_rule(host, dtype, kept):
     assert way(64, kept + 1) == way(64, 40001) == "staged" and way(64, 65537) == way(1, 262144) == "device"
 
 
+def test_transpose_staging_rule(host):
+    """Transposes with runs of a few elements on either side, over the link up to four times as slow, and the largest of few
+    columns go through device buffers."""
+    way = lambda *shape: way_of(host, "transpose%dd" % len(shape), shape)
+    assert way(12288, 128) == way(6144, 256) == way(16384, 256) == way(1, 1000000) == "staged"
+    assert way(12289, 128) == way(16384, 255) == way(63715, 65) == way(16385, 256) == "device"
+    assert way(12288, 1, 128) == "staged" and way(12289, 1, 128) == "device"
+    for flip in (1, -1):
+        assert way(*(64, 1024, 64)[::flip]) == way(*(1000, 32, 32)[::flip]) == way(*(1024, 4, 8)[::flip]) == "staged"
+        assert way(*(64, 1024, 65)[::flip]) == way(*(1025, 32, 32)[::flip]) == way(*(1025, 4, 8)[::flip]) == "device"
+        assert way(*(1, 4, 118937)[::flip]) == way(*(4, 4, 147889)[::flip]) == way(*(7, 36, 79)[::flip]) == "device"
+        assert way(*(2, 4, 512)[::flip]) == "staged"
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
