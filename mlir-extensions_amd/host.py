@@ -511,8 +511,9 @@ def _check(x, dtype):
 #    20001 633 -> 476, 64 x 65535 1853 -> 1571, one 204 -> 369);
 #  - sums: chains of dependent loads wait for the link (row sums of 65536 x 1 70 -> 79 us, column sums of 8192 x 32
 #    127 -> 138, 32768 x 32 318 -> 464, f16 2000 x 300 120 -> 125) and little is written back (row sums of 2048 x 2048
-#    557 -> 605), so only runs of 32 (rows) or 512 columns, of at most _STAGED_SUMS bytes: 512 x 1024 162 -> 118, columns
-#    168 -> 124, past that 0.9..1.3 times as fast.
+#    557 -> 605): row sums of 32 columns and more up to _STAGED_SUMS bytes, column sums by the lines of _staged_columns.  Most
+#    so the fused chain with column sums, whose forms for few rows read a row in pieces (127 x 1784 139 -> 387, 12 x 31117 bf16
+#    121 -> 141, 96 x 968 f16 84 -> 100): _staged_chain.
 _STAGED_SMALL = 64 << 10
 _STAGED_SUMS = 5 << 19
 _STAGED_BYTES = 32 << 20
@@ -533,6 +534,17 @@ def _staged_3d(d0, d1, d2):
         return _staged_2d(d0, d2)
     run = min(d0, d2)
     return _STAGED_BYTES if run >= 64 else 8 << 20 if run >= 32 else 256 << 10 if run >= 8 else 32 << 10
+
+
+def _staged_columns(rows, cols):
+    """The most bytes that column sums take through pinned host memory; of 8800 timed sizes none lost more than 3 % on this
+    side of the lines (512 x 1024 168 -> 124 us, past the first line 1548 x 599 bf16 136 -> 154)."""
+    return _STAGED_SUMS if cols >= 128 and rows <= 512 else 1 << 20 if cols >= 256 else _STAGED_SMALL
+
+
+def _staged_chain(rows, cols):
+    """The same for the fused chain with column sums, of 5200 timed sizes (480 x 624 bf16 115 -> 90 us, 342 x 807 232 -> 147)."""
+    return _STAGED_SUMS if cols >= 512 and (rows >= 128 or rows <= 4) else 256 << 10
 
 
 def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
@@ -623,7 +635,7 @@ def input_fusion(stream, a, b, dtype="f32"):
     """benchmarks/kInputFusion/kInputFusion.mlir.in:6-40: out[j] = sum_i (log b[i,j] + |a[i,j]|)"""
     rows, cols = a.shape
     return _binary(stream, "imex_input_fusion_" + dtype, a, b, dtype, [rows, cols], (cols,),
-                   staged=_STAGED_SUMS if cols >= 512 else _STAGED_SMALL)
+                   staged=_staged_chain(rows, cols))
 
 
 def flash_attention(stream, q, k, v, zh, n_ctx, sm_scale, queries_per_workgroup=None, threads=512):
@@ -702,7 +714,7 @@ def reduce_outer(stream, x, init=0.0, dtype="f32"):
     outer = x.shape[0]
     inner = int(np.prod(x.shape[1:]))
     return _unary(stream, "imex_reduce_outer_" + dtype, x, dtype, [outer, inner], extra=[float(init)],
-                  out_shape=x.shape[1:], staged=_STAGED_SUMS if inner >= 512 else _STAGED_SMALL)
+                  out_shape=x.shape[1:], staged=_staged_columns(outer, inner))
 
 
 def transpose2d(stream, x):

@@ -428,6 +428,20 @@ def test_transpose_staging_rule(host):
         assert way(*(2, 4, 512)[::flip]) == "staged"
 
 
+def test_sums_staging_rule(host):
+    """Column sums and the fused chain with them: through pinned host memory on one side of measured lines, through device
+    buffers on the other, where the link made them up to 2.8 times as slow."""
+    way = lambda op, *shape: way_of(host, op, shape)
+    assert way("reduce_outer", 512, 1024) == way("reduce_outer", 511, 1280) == way("reduce_outer", 512, 128) == "staged"
+    assert way("reduce_outer", 512, 1280) == way("reduce_outer", 513, 1024) == way("reduce_outer", 1600, 600) == "device"
+    assert way("reduce_outer", 1023, 256) == way("reduce_outer", 8191, 1) == "staged"
+    assert way("reduce_outer", 1024, 256) == way("reduce_outer", 200, 127) == "device"
+    assert way("input_fusion", 128, 2000) == way("input_fusion", 4, 70000) == way("input_fusion", 5000, 6) == "staged"
+    assert way("input_fusion", 15, 2000) == way("input_fusion", 60, 540) == "staged"
+    for shape in ((127, 1784), (125, 1557), (12, 31117), (5, 15846), (63, 1494), (64, 540), (128, 511), (128, 2600)):
+        assert way("input_fusion", *shape) == "device", shape
+
+
 def test_profiler_stats_vs_oracle(host, orc):
     rng = np.random.default_rng(3)
     for n in (1, 2, 3, 4, 7, 100, 1000):
