@@ -18,6 +18,7 @@ import operator
 import os
 import re
 import struct
+import threading
 
 import numpy as np
 
@@ -296,6 +297,7 @@ class Stream:
         self.handle = self.rt.gpuCreateStream(None, hip_stream)
         self._plans = {}  # (operator, dims) -> _Plan
         self._staging = []  # the block that `staging` keeps: [(address, bytes as a numpy array)]
+        self._staging_lock = threading.Lock()  # held by the operator that works on the block
 
     def close(self):
         if self.handle:
@@ -344,7 +346,7 @@ class Stream:
         """A block of at least `nbytes` of pinned host memory that kernels read and write: (address, numpy
         bytes), the caller's alone for the `with` block, at whose end no launch that uses it is pending.
         Allocating and freeing one takes 30 us, so the queue keeps the last one, whose size is a power of two
-        (at most _STAGED_BYTES for the operators below), until it is closed."""
+        (at most _STAGED_BYTES for the operators below, which use one block at a time), until it is closed."""
         try:
             ptr, block = self._staging.pop()  # atomic: two threads never hold the same block
         except IndexError:
@@ -548,8 +550,9 @@ def _staged_chain(rows, cols):
 
 
 def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
-    """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes,
-    for nothing, and under the profiler, which times kernels on device memory."""
+    """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes
+    (or _STAGED_BYTES with each array on 256), for nothing, while another thread's call has the queue's block, and under
+    the profiler, which times kernels on device memory."""
     n_out = int(np.prod(out_shape)) * np.dtype(out_np).itemsize  # () is one element
     total = sum(x.nbytes for x in xs) + n_out
     if total > most or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
@@ -558,12 +561,17 @@ def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
     for n in [x.nbytes for x in xs] + [n_out]:
         starts.append(end)
         end += -(-n // 256) * 256
-    with stream.staging(end) as (ptr, block):
-        for x, at in zip(xs, starts):
-            block[at:at + x.nbytes].view(x.dtype).reshape(x.shape)[...] = x
-        stream.launch(kernel, dims, [Ptr(ptr + at) for at in starts] + list(dims) + list(extra))
-        stream.wait()
-        return block[starts[-1]:starts[-1] + n_out].view(out_np).reshape(out_shape).copy()
+    if end > _STAGED_BYTES or not stream._staging_lock.acquire(blocking=False):  # another thread has the block
+        return None
+    try:
+        with stream.staging(end) as (ptr, block):
+            for x, at in zip(xs, starts):
+                block[at:at + x.nbytes].view(x.dtype).reshape(x.shape)[...] = x
+            stream.launch(kernel, dims, [Ptr(ptr + at) for at in starts] + list(dims) + list(extra))
+            stream.wait()
+            return block[starts[-1]:starts[-1] + n_out].view(out_np).reshape(out_shape).copy()
+    finally:
+        stream._staging_lock.release()
 
 
 def _unary(stream, kernel, x, dtype, dims, extra=(), out_shape=None, out_np=None, staged=_STAGED_BYTES):

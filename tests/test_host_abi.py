@@ -7,6 +7,7 @@ import os
 import re
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -384,6 +385,78 @@ def test_staging_block_of_a_queue(host):
     assert not live and s.handle is None
 
 
+class FakeMemory:
+    """The runtime's side of a queue whose memory is the host's: what is allocated now, and how large its blocks were."""
+
+    def __init__(self):
+        self.live, self.sizes = {}, []
+
+    def gpuMemAlloc(self, handle, nbytes, alignment, shared):
+        buf = C.create_string_buffer(nbytes)
+        self.live[C.addressof(buf)] = buf
+        self.sizes.append((nbytes, shared))
+        return C.addressof(buf)
+
+    def gpuMemFree(self, handle, ptr):
+        del self.live[ptr]
+
+    def gpuMemCopy(self, handle, dst, src, nbytes):
+        C.memmove(dst, src, nbytes)
+
+    def gpuCreateStream(self, device, context):
+        return 1
+
+    def gpuStreamDestroy(self, handle):
+        assert not self.live
+
+    def gpuWait(self, handle):
+        pass
+
+
+@pytest.fixture
+def fake_stream(host, monkeypatch):
+    """A queue on fake memory, whose launches call `on_launch` in place of a kernel."""
+    monkeypatch.setattr(host, "runtime", lambda rt=FakeMemory(): rt)
+    stream = host.Stream()
+    stream.on_launch = lambda: None
+    stream.launch = lambda *args: stream.on_launch()
+    yield stream
+    stream.close()
+
+
+def pinned(stream):
+    """Bytes of pinned blocks that the queue has asked for, one entry each."""
+    return [n for n, shared in stream.rt.sizes if shared]
+
+
+def test_staged_operators_pin_no_more_than_they_say(host, fake_stream):
+    """Operands that are within _STAGED_BYTES only without the space between them would get a block of twice that."""
+    for n in (2796201, 2796202):
+        x = np.zeros(n, np.float32)
+        for _ in range(2):
+            host.maximum(fake_stream, x, x)
+        assert max(pinned(fake_stream), default=0) <= host._STAGED_BYTES, n
+    assert 12 * 2796202 <= host._STAGED_BYTES
+
+
+def test_staged_operators_share_one_block(host, fake_stream):
+    """A second thread's call goes through device buffers while the first one's has the queue's block."""
+    x, calls = np.zeros(1000, np.float32), []
+
+    def second():
+        fake_stream.on_launch = lambda: None
+        before = len(pinned(fake_stream))
+        thread = threading.Thread(target=lambda: calls.append(host.relu(fake_stream, x)))
+        thread.start()
+        thread.join()
+        assert len(pinned(fake_stream)) == before
+    for _ in range(8):
+        host.relu(fake_stream, x)
+    fake_stream.on_launch = second
+    host.relu(fake_stream, x)
+    assert len(calls) == 1 and len(fake_stream._staging) == 1 and len(pinned(fake_stream)) == 1
+
+
 class _Way(Exception):
     """Raised in place of the work by the queue of `way_of`."""
 
@@ -391,6 +464,8 @@ class _Way(Exception):
 def way_of(host, op, shape, dtype="f32"):
     """"staged" or "device": where the host function `op` puts operands of this shape."""
     class Queue:
+        _staging_lock = threading.Lock()
+
         def staging(self, nbytes):
             raise _Way("staged")
 
