@@ -298,6 +298,7 @@ class Stream:
         self._plans = {}  # (operator, dims) -> _Plan
         self._staging = []  # the block that `staging` keeps: [(address, bytes as a numpy array)]
         self._staging_lock = threading.Lock()  # held by the operator that works on the block
+        self._unstaged = 0  # operators that have gone without a block of their size since the last one was made
 
     def close(self):
         if self.handle:
@@ -345,8 +346,8 @@ class Stream:
     def staging(self, nbytes):
         """A block of at least `nbytes` of pinned host memory that kernels read and write: (address, numpy
         bytes), the caller's alone for the `with` block, at whose end no launch that uses it is pending.
-        Allocating and freeing one takes 30 us, so the queue keeps the last one, whose size is a power of two
-        (at most _STAGED_BYTES for the operators below, which use one block at a time), until it is closed."""
+        The queue keeps the last one, whose size is a power of two (at most _STAGED_BYTES for the operators below,
+        which use one block at a time), until it is closed: staging_pays says what making one costs."""
         try:
             ptr, block = self._staging.pop()  # atomic: two threads never hold the same block
         except IndexError:
@@ -354,7 +355,7 @@ class Stream:
         if len(block) < nbytes:
             if ptr is not None:
                 self.free(ptr)
-            size = max(1 << 18, 1 << (nbytes - 1).bit_length())
+            size = _staging_size(nbytes)
             ptr = self.alloc(size, shared=True)
             block = np.frombuffer((C.c_uint8 * size).from_address(ptr), np.uint8)
         keep = False
@@ -366,6 +367,20 @@ class Stream:
                 self._staging.append((ptr, block))
             else:
                 self.free(ptr)  # waits for the queue
+
+    def staging_pays(self, nbytes):
+        """Whether an operator that needs `nbytes` should take `staging`: if the kept block is large enough, or if as many
+        as the new block has MiB (one at least) have gone without.  A new block's pages are mapped one by one as they are
+        first touched, 0.36 ms per MiB beyond the first few: a queue's first relu over 8 MiB took 3.8 ms instead of 2.3, over
+        32 MiB 13.6 instead of 2.2.  A later call gains 0.02 (to 2 MiB) .. 0.45 ms, so the calls that waited and those that
+        are still to come lose less by either choice than by the other at its worst."""
+        if self._staging and len(self._staging[0][1]) >= nbytes:
+            return True
+        self._unstaged += 1
+        if self._unstaged <= max(1, _staging_size(nbytes) >> 20):
+            return False
+        self._unstaged = 0
+        return True
 
     # -- kernels --------------------------------------------------------------
     def kernel(self, name):
@@ -474,6 +489,11 @@ class Stream:
                 "global_bytes": mem.value}
 
 
+def _staging_size(nbytes):
+    """Bytes of the pinned block that serves `nbytes`."""
+    return max(1 << 18, 1 << (nbytes - 1).bit_length())
+
+
 def compute_stats(times_ms):
     v = (C.c_float * len(times_ms))(*times_ms)
     out = (C.c_float * 9)()
@@ -551,8 +571,8 @@ def _staged_chain(rows, cols):
 
 def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
     """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes
-    (or _STAGED_BYTES with each array on 256), for nothing, while another thread's call has the queue's block, and under
-    the profiler, which times kernels on device memory."""
+    (or _STAGED_BYTES with each array on 256), for nothing, before the queue's block pays, while another thread's call has
+    it, and under the profiler, which times kernels on device memory."""
     n_out = int(np.prod(out_shape)) * np.dtype(out_np).itemsize  # () is one element
     total = sum(x.nbytes for x in xs) + n_out
     if total > most or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
@@ -564,6 +584,8 @@ def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
     if end > _STAGED_BYTES or not stream._staging_lock.acquire(blocking=False):  # another thread has the block
         return None
     try:
+        if not stream.staging_pays(end):
+            return None
         with stream.staging(end) as (ptr, block):
             for x, at in zip(xs, starts):
                 block[at:at + x.nbytes].view(x.dtype).reshape(x.shape)[...] = x

@@ -384,3 +384,14 @@ def test_operators_on_host_memory(host, op, shapes, monkeypatch):
                 got = getattr(host, op)(s, *ins)
                 assert got.shape == want.shape and np.array_equal(got.view(np.uint32), want.view(np.uint32)), shape
     assert any(t is not None for t in taken)
+
+
+@pytest.mark.parametrize("op,shapes", [
+    ("relu", [(1,), (4194304,), (1023, 17)]), ("softmax", [(3, 65536), (2, 32769), (64, 20001)]),
+    ("reduce_outer", [(512, 1024), (513, 1024), (33, 8, 64)]), ("maximum", [(2796160,), (2796202,), (5, 1001)]),
+    ("input_fusion", [(128, 2000), (127, 1784)]), ("transpose2d", [(12288, 128), (257, 1031)]),
+    ("transpose3d", [(1000, 32, 32), (4, 4, 5000)])])
+def test_operators_on_host_memory_from_the_first_call(host, op, shapes, monkeypatch):
+    """The same on both sides of the lines of 32 MiB and of shapes, with every call that may taking the block."""
+    monkeypatch.setattr(host.Stream, "staging_pays", lambda self, nbytes: True)
+    test_operators_on_host_memory(host, op, shapes, monkeypatch)

@@ -431,6 +431,7 @@ def pinned(stream):
 
 def test_staged_operators_pin_no_more_than_they_say(host, fake_stream):
     """Operands that are within _STAGED_BYTES only without the space between them would get a block of twice that."""
+    fake_stream.staging_pays = lambda nbytes: True
     for n in (2796201, 2796202):
         x = np.zeros(n, np.float32)
         for _ in range(2):
@@ -457,6 +458,33 @@ def test_staged_operators_share_one_block(host, fake_stream):
     assert len(calls) == 1 and len(fake_stream._staging) == 1 and len(pinned(fake_stream)) == 1
 
 
+@pytest.mark.parametrize("n,waits", [(1, 1), (1 << 17, 1), ((1 << 17) + 1, 2), (1 << 20, 8), (1 << 22, 32)])
+def test_staged_operators_wait_for_a_block(host, fake_stream, n, waits):
+    """A queue's first calls go through device buffers, as many as the pinned block that they would get has MiB: one call
+    on 32 MiB paid 11 ms for it, 60 times what it gained."""
+    x = np.zeros(n, np.float32)
+    for call in range(waits):
+        host.relu(fake_stream, x)
+        assert not pinned(fake_stream), call
+    for _ in range(3):
+        host.relu(fake_stream, x)
+    assert len(pinned(fake_stream)) == 1 and pinned(fake_stream)[0] >= 8 * n
+
+
+def test_staged_operators_grow_their_block_by_the_same_rule(host, fake_stream):
+    """Smaller calls take the block that is kept and do not bring a larger one any nearer."""
+    small, large = np.zeros(100, np.float32), np.zeros(1 << 19, np.float32)  # 4 MiB for the larger
+    for _ in range(40):
+        host.relu(fake_stream, small)
+    assert pinned(fake_stream) == [1 << 18]
+    for _ in range(4):
+        host.relu(fake_stream, large)
+        host.relu(fake_stream, small)
+    assert pinned(fake_stream) == [1 << 18]
+    host.relu(fake_stream, large)
+    assert pinned(fake_stream) == [1 << 18, 1 << 22] and len(fake_stream._staging) == 1
+
+
 class _Way(Exception):
     """Raised in place of the work by the queue of `way_of`."""
 
@@ -466,7 +494,7 @@ def way_of(host, op, shape, dtype="f32"):
     class Queue:
         _staging_lock = threading.Lock()
 
-        def staging(self, nbytes):
+        def staging_pays(self, nbytes):
             raise _Way("staged")
 
         def to_device(self, array):
