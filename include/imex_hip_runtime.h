@@ -180,6 +180,10 @@ void imexHipComputeStats(const float *values, size_t n, float *out);
 int imexHipDeviceInfo(void *queue, int *cuCount, int *clockKHz, size_t *l2Bytes, size_t *globalBytes,
                       char *name, size_t nameLen);
 
+/* `size` bytes as gpuMemAlloc(queue, size, 64, isShared = 1) gives them, or NULL where there is no such memory: the only
+ * allocation that does not end the process then, for callers that can do without.  gpuMemFree frees them. */
+void *imexHipTrySharedAlloc(void *queue, size_t size);
+
 /* The device ordinal a queue of gpuCreateStream runs on; -1 for NULL. */
 int imexHipQueueDevice(void *queue);
 

@@ -813,6 +813,15 @@ extern "C" void imexHipComputeStats(const float *values, size_t n, float *out) {
   out[8] = s.middleThirdAvg;
 }
 
+extern "C" void *imexHipTrySharedAlloc(void *queue, size_t size) {
+  try {
+    return allocMemory(asQueue(queue), size, 64, true);
+  } catch (...) {
+    (void)hipGetLastError(); // the next call must not report it
+    return nullptr;
+  }
+}
+
 extern "C" int imexHipQueueDevice(void *queue) { return queue ? asQueue(queue)->device : -1; }
 
 extern "C" int imexHipDeviceInfo(void *queue, int *cuCount, int *clockKHz, size_t *l2Bytes,

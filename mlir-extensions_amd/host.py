@@ -83,6 +83,7 @@ _RUNTIME_SYMBOLS = {
     "imexHipComputeStats": (None, [C.POINTER(C.c_float), C.c_size_t, C.POINTER(C.c_float)]),
     "imexHipDeviceInfo": (C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_size_t),
                                     C.POINTER(C.c_size_t), C.c_char_p, C.c_size_t]),
+    "imexHipTrySharedAlloc": (C.c_void_p, [C.c_void_p, C.c_size_t]),
     "imexHipQueueDevice": (C.c_int, [C.c_void_p]),
 }
 
@@ -357,7 +358,7 @@ class Stream:
                 self.free(ptr)
             size = _staging_size(nbytes)
             ptr = self.alloc(size, shared=True)
-            block = np.frombuffer((C.c_uint8 * size).from_address(ptr), np.uint8)
+            block = _bytes_at(ptr, size)
         keep = False
         try:
             yield ptr, block
@@ -370,16 +371,24 @@ class Stream:
 
     def staging_pays(self, nbytes):
         """Whether an operator that needs `nbytes` should take `staging`: if the kept block is large enough, or if as many
-        as the new block has MiB (one at least) have gone without.  A new block's pages are mapped one by one as they are
-        first touched, 0.36 ms per MiB beyond the first few: a queue's first relu over 8 MiB took 3.8 ms instead of 2.3, over
-        32 MiB 13.6 instead of 2.2.  A later call gains 0.02 (to 2 MiB) .. 0.45 ms, so the calls that waited and those that
-        are still to come lose less by either choice than by the other at its worst."""
+        as the new block has MiB (one at least) have gone without and there is memory to pin, which is kept then.  A new
+        block's pages are mapped one by one as they are first touched, 0.36 ms per MiB beyond the first few: a queue's
+        first relu over 8 MiB took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 (to
+        2 MiB) .. 0.45 ms, so the calls that waited and those that are still to come lose less by either choice than by
+        the other at its worst."""
         if self._staging and len(self._staging[0][1]) >= nbytes:
             return True
+        size = _staging_size(nbytes)
         self._unstaged += 1
-        if self._unstaged <= max(1, _staging_size(nbytes) >> 20):
+        if self._unstaged <= max(1, size >> 20):
             return False
         self._unstaged = 0
+        ptr = self.rt.imexHipTrySharedAlloc(self.handle, size)
+        if not ptr:
+            return False
+        while self._staging:
+            self.free(self._staging.pop()[0])
+        self._staging.append((Ptr(ptr), _bytes_at(ptr, size)))
         return True
 
     # -- kernels --------------------------------------------------------------
@@ -492,6 +501,11 @@ class Stream:
 def _staging_size(nbytes):
     """Bytes of the pinned block that serves `nbytes`."""
     return max(1 << 18, 1 << (nbytes - 1).bit_length())
+
+
+def _bytes_at(ptr, size):
+    """Host memory as a numpy array that does not own it."""
+    return np.frombuffer((C.c_uint8 * size).from_address(ptr), np.uint8)
 
 
 def compute_stats(times_ms):

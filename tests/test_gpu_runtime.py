@@ -395,3 +395,17 @@ def test_operators_on_host_memory_from_the_first_call(host, op, shapes, monkeypa
     """The same on both sides of the lines of 32 MiB and of shapes, with every call that may taking the block."""
     monkeypatch.setattr(host.Stream, "staging_pays", lambda self, nbytes: True)
     test_operators_on_host_memory(host, op, shapes, monkeypatch)
+
+
+def test_shared_memory_or_none(host):
+    """Pinned memory that a caller can do without: usable and freed as gpuMemAlloc's, NULL for a queue that is none."""
+    assert not host.runtime().imexHipTrySharedAlloc(None, 4096)
+    with host.Stream() as s:
+        p = s.rt.imexHipTrySharedAlloc(s.handle, 1 << 20)
+        assert p
+        x = np.frombuffer((C.c_uint8 * (1 << 20)).from_address(p), np.float32)
+        x[:] = -1.0
+        s.launch("imex_relu_f32", [x.size], [host.Ptr(p), host.Ptr(p), x.size])
+        s.wait()
+        assert np.all(x == 0.0)
+        s.free(p)

@@ -389,13 +389,16 @@ class FakeMemory:
     """The runtime's side of a queue whose memory is the host's: what is allocated now, and how large its blocks were."""
 
     def __init__(self):
-        self.live, self.sizes = {}, []
+        self.live, self.sizes, self.can_pin = {}, [], True
 
     def gpuMemAlloc(self, handle, nbytes, alignment, shared):
         buf = C.create_string_buffer(nbytes)
         self.live[C.addressof(buf)] = buf
         self.sizes.append((nbytes, shared))
         return C.addressof(buf)
+
+    def imexHipTrySharedAlloc(self, handle, nbytes):
+        return self.gpuMemAlloc(handle, nbytes, 64, 1) if self.can_pin else None
 
     def gpuMemFree(self, handle, ptr):
         del self.live[ptr]
@@ -483,6 +486,24 @@ def test_staged_operators_grow_their_block_by_the_same_rule(host, fake_stream):
     assert pinned(fake_stream) == [1 << 18]
     host.relu(fake_stream, large)
     assert pinned(fake_stream) == [1 << 18, 1 << 22] and len(fake_stream._staging) == 1
+
+
+def test_staged_operators_do_without_pinned_memory(host, fake_stream):
+    """Where none is to be had every call goes through device buffers, as it did before there was a block, and a smaller
+    block that is kept stays."""
+    small, large = np.zeros(100, np.float32), np.zeros(1 << 19, np.float32)
+    fake_stream.rt.can_pin = False
+    for _ in range(9):
+        host.relu(fake_stream, small)
+    assert not pinned(fake_stream) and not fake_stream._staging
+    fake_stream.rt.can_pin = True
+    for _ in range(2):
+        host.relu(fake_stream, small)
+    fake_stream.rt.can_pin = False
+    for _ in range(9):
+        host.relu(fake_stream, large)
+    assert pinned(fake_stream) == [len(fake_stream._staging[0][1])] == [1 << 18]
+    host.relu(fake_stream, small)
 
 
 class _Way(Exception):
