@@ -181,8 +181,10 @@ int imexHipDeviceInfo(void *queue, int *cuCount, int *clockKHz, size_t *l2Bytes,
                       char *name, size_t nameLen);
 
 /* `size` bytes as gpuMemAlloc(queue, size, 64, isShared = 1) gives them, or NULL where there is no such memory: the only
- * allocation that does not end the process then, for callers that can do without.  gpuMemFree frees them. */
+ * allocation that does not end the process then, for callers that can do without.  gpuMemFree frees them, or
+ * imexHipSharedFree without a queue, for memory that no pending work uses. */
 void *imexHipTrySharedAlloc(void *queue, size_t size);
+void imexHipSharedFree(void *ptr);
 
 /* The device ordinal a queue of gpuCreateStream runs on; -1 for NULL. */
 int imexHipQueueDevice(void *queue);

@@ -207,18 +207,20 @@ void *allocMemory(GpuHipQueue *queue, size_t size, size_t alignment, bool isShar
   return user;
 }
 
+AllocInfo takeAllocation(void *ptr, const char *who) {
+  std::lock_guard<std::mutex> lock(allocMutex);
+  auto it = allocRegistry.find(ptr);
+  if (it == allocRegistry.end())
+    throw std::runtime_error(std::string(who) + ": pointer was not returned by gpuMemAlloc");
+  AllocInfo info = it->second;
+  allocRegistry.erase(it);
+  return info;
+}
+
 void freeMemory(GpuHipQueue *queue, void *ptr) {
   if (!queue || !ptr)
     return;
-  AllocInfo info;
-  {
-    std::lock_guard<std::mutex> lock(allocMutex);
-    auto it = allocRegistry.find(ptr);
-    if (it == allocRegistry.end())
-      throw std::runtime_error("gpuMemFree: pointer was not returned by gpuMemAlloc");
-    info = it->second;
-    allocRegistry.erase(it);
-  }
+  AllocInfo info = takeAllocation(ptr, "gpuMemFree");
   CHECK_HIP(hipSetDevice(queue->device));
   // Work that still uses the buffer may be in flight on the stream.
   CHECK_HIP(hipStreamSynchronize(queue->stream));
@@ -820,6 +822,18 @@ extern "C" void *imexHipTrySharedAlloc(void *queue, size_t size) {
     (void)hipGetLastError(); // the next call must not report it
     return nullptr;
   }
+}
+
+extern "C" void imexHipSharedFree(void *ptr) {
+  catchAll([&]() {
+    if (!ptr)
+      return;
+    AllocInfo info = takeAllocation(ptr, "imexHipSharedFree");
+    if (info.kind != AllocKind::HostShared)
+      throw std::runtime_error("imexHipSharedFree: not a shared allocation");
+    if (hipHostFree(info.base) != hipSuccess) // a finaliser's call: nobody is there to be told
+      (void)hipGetLastError();
+  });
 }
 
 extern "C" int imexHipQueueDevice(void *queue) { return queue ? asQueue(queue)->device : -1; }

@@ -19,6 +19,7 @@ import os
 import re
 import struct
 import threading
+import weakref
 
 import numpy as np
 
@@ -84,6 +85,7 @@ _RUNTIME_SYMBOLS = {
     "imexHipDeviceInfo": (C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_size_t),
                                     C.POINTER(C.c_size_t), C.c_char_p, C.c_size_t]),
     "imexHipTrySharedAlloc": (C.c_void_p, [C.c_void_p, C.c_size_t]),
+    "imexHipSharedFree": (None, [C.c_void_p]),
     "imexHipQueueDevice": (C.c_int, [C.c_void_p]),
 }
 
@@ -299,6 +301,7 @@ class Stream:
         self._plans = {}  # (operator, dims) -> _Plan
         self._staging = []  # the block that `staging` keeps: [(address, bytes as a numpy array)]
         self._staging_lock = threading.Lock()  # held by the operator that works on the block
+        weakref.finalize(self, _free_staging, self.rt, self._staging).atexit = False  # a queue that nobody closes
         self._unstaged = 0  # operators that have gone without a block of their size since the last one was made
 
     def close(self):
@@ -501,6 +504,12 @@ class Stream:
 def _staging_size(nbytes):
     """Bytes of the pinned block that serves `nbytes`."""
     return max(1 << 18, 1 << (nbytes - 1).bit_length())
+
+
+def _free_staging(rt, staging):
+    """What is left of a queue's pinned memory when the object goes, through no queue: one that it adopted may be gone."""
+    while staging:
+        rt.imexHipSharedFree(staging.pop()[0])
 
 
 def _bytes_at(ptr, size):

@@ -409,3 +409,7 @@ def test_shared_memory_or_none(host):
         s.wait()
         assert np.all(x == 0.0)
         s.free(p)
+        q = s.rt.imexHipTrySharedAlloc(s.handle, 4096)
+        assert q
+        s.rt.imexHipSharedFree(q)
+        s.rt.imexHipSharedFree(None)

@@ -403,6 +403,9 @@ class FakeMemory:
     def gpuMemFree(self, handle, ptr):
         del self.live[ptr]
 
+    def imexHipSharedFree(self, ptr):
+        del self.live[ptr]
+
     def gpuMemCopy(self, handle, dst, src, nbytes):
         C.memmove(dst, src, nbytes)
 
@@ -504,6 +507,26 @@ def test_staged_operators_do_without_pinned_memory(host, fake_stream):
         host.relu(fake_stream, large)
     assert pinned(fake_stream) == [len(fake_stream._staging[0][1])] == [1 << 18]
     host.relu(fake_stream, small)
+
+
+def test_queues_that_nobody_closes_give_their_block_back(host, monkeypatch):
+    """The pinned block goes with the object, without its queue; a queue that was closed has freed it already."""
+    rt = FakeMemory()
+    monkeypatch.setattr(host, "runtime", lambda: rt)
+    monkeypatch.setattr(host.Stream, "launch", lambda *args: None)
+    x = np.zeros(1000, np.float32)
+    for closed in (False, True):
+        s = host.Stream()
+        for _ in range(3):
+            host.relu(s, x)
+        assert len(rt.live) == 1
+        if closed:
+            s.close()
+        else:
+            rt.gpuMemFree = None
+        del s
+        assert not rt.live
+        vars(rt).pop("gpuMemFree", None)
 
 
 class _Way(Exception):
