@@ -373,17 +373,17 @@ class Stream:
                 self.free(ptr)  # waits for the queue
 
     def staging_pays(self, nbytes):
-        """Whether an operator that needs `nbytes` should take `staging`: if the kept block is large enough, or if as many
-        as the new block has MiB (one at least) have gone without and there is memory to pin, which is kept then.  A new
-        block's pages are mapped one by one as they are first touched, 0.36 ms per MiB beyond the first few: a queue's
-        first relu over 8 MiB took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 (to
-        2 MiB) .. 0.45 ms, so the calls that waited and those that are still to come lose less by either choice than by
-        the other at its worst."""
+        """Whether an operator that needs `nbytes` should take `staging`: if the kept block is large enough, or if five
+        for every two MiB of the new block (one at least) have gone without and there is memory to pin, which is kept then.  A
+        new block's pages are mapped one by one as they are first touched, 0.36 ms per MiB: a queue's first relu over 8 MiB
+        took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 ms (to 2 MiB), 0.09 (4 MiB) ..
+        0.15, so a block pays after about that many: a queue that ends just then has lost a quarter by it (ten calls on 8
+        MiB that got it after eight 5.2 -> 8.1 ms), and one of a hundred calls gains 0.43 .. 0.8 of the time."""
         if self._staging and len(self._staging[0][1]) >= nbytes:
             return True
         size = _staging_size(nbytes)
         self._unstaged += 1
-        if self._unstaged <= max(1, size >> 20):
+        if self._unstaged <= max(1, 5 * size >> 21):
             return False
         self._unstaged = 0
         ptr = self.rt.imexHipTrySharedAlloc(self.handle, size)

@@ -464,10 +464,10 @@ def test_staged_operators_share_one_block(host, fake_stream):
     assert len(calls) == 1 and len(fake_stream._staging) == 1 and len(pinned(fake_stream)) == 1
 
 
-@pytest.mark.parametrize("n,waits", [(1, 1), (1 << 17, 1), ((1 << 17) + 1, 2), (1 << 20, 8), (1 << 22, 32)])
+@pytest.mark.parametrize("n,waits", [(1, 1), (1 << 16, 1), (1 << 17, 2), ((1 << 17) + 1, 5), (1 << 20, 20), (1 << 22, 80)])
 def test_staged_operators_wait_for_a_block(host, fake_stream, n, waits):
-    """A queue's first calls go through device buffers, as many as the pinned block that they would get has MiB: one call
-    on 32 MiB paid 11 ms for it, 60 times what it gained."""
+    """A queue's first calls go through device buffers, five for every two MiB of the pinned block that they would get:
+    one call on 32 MiB paid 11 ms for it, 60 times what it gained."""
     x = np.zeros(n, np.float32)
     for call in range(waits):
         host.relu(fake_stream, x)
@@ -483,7 +483,7 @@ def test_staged_operators_grow_their_block_by_the_same_rule(host, fake_stream):
     for _ in range(40):
         host.relu(fake_stream, small)
     assert pinned(fake_stream) == [1 << 18]
-    for _ in range(4):
+    for _ in range(10):
         host.relu(fake_stream, large)
         host.relu(fake_stream, small)
     assert pinned(fake_stream) == [1 << 18]
@@ -503,7 +503,7 @@ def test_staged_operators_do_without_pinned_memory(host, fake_stream):
     for _ in range(2):
         host.relu(fake_stream, small)
     fake_stream.rt.can_pin = False
-    for _ in range(9):
+    for _ in range(30):
         host.relu(fake_stream, large)
     assert pinned(fake_stream) == [len(fake_stream._staging[0][1])] == [1 << 18]
     host.relu(fake_stream, small)
