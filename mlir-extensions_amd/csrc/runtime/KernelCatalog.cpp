@@ -257,18 +257,21 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
 // 9.8 (16 x 16), 2414 x 2104 x 2208 49.1 / 36.4 (256 x 128); 4096 x 4096 x 1024 36.6, against 53.3 with 128 x 128 tiles.
 //
 // Workgroups that fetch for others (fetch_ahead in gemm_small.h) change what a step costs: stepAhead per step, aheadMib per
-// MiB of operands and `ahead` once, where it is worth more than the launch of 256 workgroups.  From 2100 other problems,
-// operands from beyond the L2s (us without / with, from HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x
-// 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from the 256 MiB cache 11.3 / 7.1 for the second): the launches that
-// get them took 0.90 of their time, and with the tiles chosen by these numbers products of bias and SiLU 0.95, others 0.99.
-// Not below 768 k or 2 MiB, which are there before a helper could fetch them (K = 512 .. 767: 1.00), nor above 32 MiB, which
-// HBM's rate bounds (32 .. 48 MiB: 1.01), with fewer than 96 helpers (176 .. 192 tiles: up to 1.4) or for 128 x 128 tiles and
-// larger, which their own steps bound (above 16 MiB 1.03 .. 1.04).
+// MiB of operands and `ahead` once, where it is worth more than the launch of 256 workgroups (fitted to 2100 other problems,
+// operands from beyond the L2s).  Timed on 1100 further ones, each with and without them on every tile (us without / with, from
+// HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from
+// the 256 MiB cache 11.3 / 7.1 for the second): the launches that get them take 0.71 of their time from HBM, 0.86 from that
+// cache and 0.89 where the L2s have the operands, there more than 1.02 on 7 of 290, 1.06 at most.  Not below 3.75 MiB and 1024
+// k, or 2 MiB and 2560 k, which the L2s may have (there 2 x 1560 x 1080 1.21, 391 x 176 x 1928 1.17), nor above 32 MiB, which
+// HBM's rate bounds (32 .. 48 MiB: 1.01), with fewer than 96 helpers (176 .. 192 tiles: up to 1.5) or for 128 x 128 tiles and
+// larger, which their own steps bound (above 16 MiB 1.03 .. 1.04).  They draw a problem to other tiles only where that holds from the
+// L2s too: not to 16 x 64 (from 16 x 32 1.03 of the time in the mean, 151 x 576 x 3456 1.21) and not to 16 x 32 with B^T (48 x
+// 1000 x 2064 1.12).
 struct GemmTile {
   const char *suffix;
   int tileM, tileN, stepK, constant, setup, store, step, stepMore;
   bool shared;
-  int stepAhead, aheadMib, ahead; // (0: as without)
+  int stepAhead, aheadMib, ahead; // (0: chosen as without)
 };
 constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810, false, 0, 0, 0},
                                    {"_t256x128", 256, 128, 64, 1238, 5315, 773, 717, 956, false, 0, 0, 0},
@@ -277,14 +280,14 @@ constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810,
                                    {"_t128x64s", 128, 64, 64, 1616, 1283, 100, 399, 311, false, 0, 0, 0},
                                    {"_t64", 64, 64, 64, 1621, 1410, 100, 259, 332, true, 181, 23, -171},
                                    {"_t32", 32, 64, 128, 814, 1512, 50, 375, 339, false, 225, 52, 966},
-                                   {"_t16", 16, 64, 256, 837, 2121, 25, 574, 722, false, 370, 69, 309},
+                                   {"_t16", 16, 64, 256, 837, 2121, 25, 574, 722, false, 0, 0, 0},
                                    {"_t16x32", 16, 32, 256, 1799, 466, 37, 489, 397, false, 196, 70, 889},
                                    {"_t16x16", 16, 16, 256, 2031, 385, 25, 379, 282, false, 146, 94, 761}};
 
 // Whether workgroups without a tile are launched to fetch what the others read.
 bool fetchesAhead(const GemmTile &t, int64_t M, int64_t N, int64_t K) {
   const double mib = 2.0 * double(K) * (double(M) + double(N)) / (1 << 20);
-  return K >= 768 && mib >= 2.0 && mib <= 32.0 && t.tileM * t.tileN <= 128 * 64 &&
+  return ((K >= 1024 && mib >= 3.75) || (K >= 2560 && mib >= 2.0)) && mib <= 32.0 && t.tileM * t.tileN <= 128 * 64 &&
          ceilDiv(M, t.tileM) * ceilDiv(N, t.tileN) <= 160;
 }
 
@@ -338,7 +341,7 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
     const double load = t.shared ? std::max(1.0, tiles / 256.0) : std::ceil(tiles / 256.0);
     const double once = t.constant + load * (t.setup + t.store * storeBytes(e));
     double ns = once + steps * (t.step + (load - 1.0) * t.stepMore);
-    if (t.stepAhead && fetchesAhead(t, M, N, K))
+    if (t.stepAhead && fetchesAhead(t, M, N, K) && !(transB && t.tileM * t.tileN == 16 * 32))
       ns = std::min(ns, once + steps * t.stepAhead + 2.0 * double(K) * (double(M) + double(N)) / (1 << 20) * t.aheadMib + t.ahead);
     if (!best || ns < least) {
       best = &t;

@@ -378,7 +378,7 @@ class Stream:
         new block's pages are mapped one by one as they are first touched, 0.36 ms per MiB: a queue's first relu over 8 MiB
         took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 ms (to 2 MiB), 0.09 (4 MiB) ..
         0.15, so a block pays after about that many: a queue that ends just then has lost a quarter by it (ten calls on 8
-        MiB that got it after eight 5.2 -> 8.1 ms), and one of a hundred calls gains 0.43 .. 0.8 of the time."""
+        MiB that got it after eight 5.2 -> 8.1 ms), and one of a hundred takes 0.43 .. 0.8 of the time."""
         if self._staging and len(self._staging[0][1]) >= nbytes:
             return True
         size = _staging_size(nbytes)

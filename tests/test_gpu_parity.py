@@ -1666,31 +1666,40 @@ def test_gemm_unaligned_narrow_tiles(host, orc, stream, tile, M, N, K):
 
 
 @pytest.mark.parametrize("tile", ["_t128x64", "_t128x64s", "_t64", "_t32", "_t16", "_t16x32", "_t16x16"])
-@pytest.mark.parametrize("M,N,K", [(40, 232, 4104), (8, 1096, 1032), (1000, 24, 1032), (264, 72, 3592), (336, 112, 2504)])
+@pytest.mark.parametrize("M,N,K", [(40, 232, 4104), (8, 2120, 1032), (1000, 24, 2568), (264, 72, 3592), (336, 112, 2568)])
 def test_gemm_workgroups_that_fetch(host, orc, stream, tile, M, N, K):
     """Launches with workgroups that have no tile and fetch what the others read: one and several bands of tile rows for an
-    XCD, bands that it shares with the next, tiles that eight does not divide, ragged edges.  Integer operands, exact sums."""
-    launched = 0
-    for which in ("plain", "acc", "ta", "tb", "f16"):
-        kind = {"plain": "bf16_bf16_f32", "acc": "f16_f16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb", "f16": "f16_f16_f16"}[which]
-        name, dtype = "imex_gemm_" + kind + tile, "bf16" if which == "plain" else "f16"
+    XCD, bands that it shares with the next, tiles that eight does not divide, ragged edges.  Integer operands, exact sums;
+    bias and SiLU of such a sum within the rounding of the 16-bit result."""
+    for which in ("plain", "acc", "ta", "tb", "f16", "silu"):
+        kind = {"plain": "bf16_bf16_f32", "acc": "f16_f16_f32_acc", "ta": "f16_f16_f32_ta", "tb": "f16_f16_f32_tb",
+                "f16": "f16_f16_f16", "silu": "bf16_bias_silu_bf16"}[which]
+        name, dtype = "imex_gemm_" + kind + tile, "bf16" if which in ("plain", "silu") else "f16"
         n = N - 3 if which == "tb" else N
-        launched += host.launch_shape(name, [M, n, K])[0][0] == 256
+        assert host.launch_shape(name, [M, n, K])[0][0] == 256
         a, b = orc.fill_int(M * K, dtype, 95, -1, 1).reshape(M, K), orc.fill_int(K * n, dtype, 96, -1, 1).reshape(K, n)
         want = (orc.to_float(a, dtype) @ orc.to_float(b, dtype)).astype(np.int64) + (7 if which == "acc" else 0)
-        fill = np.full((M + 4, n), 7, np.uint16 if which == "f16" else np.float32)
+        fill = np.full((M + 4, n), 7, np.uint16 if which in ("f16", "silu") else np.float32)
         bufs = [stream.to_device(np.ascontiguousarray(a.T) if which == "ta" else a),
                 stream.to_device(np.ascontiguousarray(b.T) if which == "tb" else b), stream.to_device(fill)]
+        if which == "silu":
+            bias = np.arange(n, dtype=np.float32) % 9 - 4
+            bufs.insert(2, stream.to_device(bias))
+            x = want + bias.astype(np.float64)
+            want = x / (1 + np.exp(-x))
         for grid in (None, (256, 1, 1), (331, 1, 1)):
-            stream.copy(bufs[2], fill.ctypes.data, fill.nbytes)
+            stream.copy(bufs[-1], fill.ctypes.data, fill.nbytes)
             stream.launch(name, [M, n, K], bufs + [M, n, K], grid=grid or host.launch_shape(name, [M, n, K])[0])
             stream.wait()
-            got = stream.from_device(bufs[2], fill.shape, fill.dtype)
-            assert np.array_equal((orc.half_to_float(got[:M]) if which == "f16" else got[:M]).astype(np.int64), want), (name, grid)
+            got = stream.from_device(bufs[-1], fill.shape, fill.dtype)
+            if which == "silu":  # half an ulp of the result, and what the f32 exponential and quotient lose
+                assert np.all(np.abs(orc.to_float(got[:M], dtype) - want) <= 2.0 ** -8 * np.abs(want) + 1e-30), (name, grid)
+            else:
+                sums = orc.half_to_float(got[:M]) if which == "f16" else got[:M]
+                assert np.array_equal(sums.astype(np.int64), want), (name, grid)
             assert np.array_equal(got[M:], fill[M:]), (name, grid)
         for p in bufs:
             stream.free(p)
-    assert launched or tile == "_t16x16" and M == 1000 or -(-M // 16) * -(-N // 16) > 160
 
 
 @pytest.mark.parametrize("which", ["", "_ta", "_tb"])

@@ -275,6 +275,20 @@ def test_gemm_workgroups_that_fetch_rule(host):
     assert grid("_t16x16", 16, 1680, 3992) == grid("_t32", 128, 2048, 4096) == grid("_t128x64", 1000, 1000, 1024) == 256
     assert grid("_t16x16", 16, 1680, 760) == 105 and grid("_t16x16", 16, 640, 1024) == 40 and grid("_t64", 16, 8192, 4096) == 128
     assert grid("_t16x16", 16, 2816, 1024) == 176 and grid("_t128", 1000, 1000, 1024) == 64
+    # operands that the L2s may hold: from 1024 k and 3.75 MiB, or 2560 k and 2 MiB
+    assert [grid("_t16x16", 2, n, 1024) for n in (1912, 1920)] == [120, 256] and grid("_t16x16", 2, 2000, 1016) == 125
+    assert [grid("_t16x16", 2, n, 2560) for n in (400, 424)] == [25, 256] and grid("_t16x16", 2, 424, 2552) == 27
+    assert grid("_t16x16", 2, 1560, 1080) == 98 and grid("_t16x32", 391, 176, 1928) == 150
+
+
+def test_gemm_workgroups_that_fetch_do_not_draw_problems_to_slower_tiles(host):
+    """Problems that lost up to a fifth of their speed to tiles of 16 x 64 (or 16 x 32 with B^T) and workgroups that fetch."""
+    tile = lambda kind, *dims: host.variant("imex_gemm_" + kind, list(dims))[len("imex_gemm_" + kind):]
+    for m, n, k in ((151, 576, 3456), (257, 416, 2656), (219, 479, 3256), (682, 143, 2680)):
+        assert tile("f16_f16_f32_tb", m, n, k) == "_t16x32", (m, n, k)
+    assert tile("bf16_bf16_f32_acc", 329, 288, 2432) == tile("f16_f16_f32_acc", 551, 224, 3056) == "_t16x32"
+    assert tile("f16_f16_f32_tb", 48, 1000, 2064) == "_t16x16" and tile("f16_f16_f16", 156, 400, 2152) == "_t16x16"
+    assert tile("f16_f16_f32_ta", 104, 1648, 3288) == "_t32" and tile("bf16_bias_silu_bf16", 15, 2624, 2904) == "_t16x32"
 
 
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
