@@ -306,12 +306,10 @@ constexpr GemmTile kUnalignedTiles[] = {{"_u128", 128, 128, 64, -568, 4171, 645,
                                         {"_u32", 32, 64, 128, 2564, 464, 141, 492, 456, false, 0, 0, 0},
                                         {"_u16x32", 16, 32, 256, 2842, 0, 105, 591, 611, false, 0, 0, 0},
                                         {"_u16x16", 16, 16, 256, 2485, 50, 96, 467, 471, false, 0, 0, 0}};
-// Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit.
+// Products that are small and whose sums are short stay with that loop, which adds in the sequential order bit for bit; small
+// ones of longer sums take 0.70 of the time of 64 x 64 tiles in the mean (1350 of fewer than 2^21 products, at most 0.97).
 constexpr double kUnalignedFrom = double(1 << 23);
 constexpr int64_t kUnalignedFromK = 192;
-// The few that are smaller still but have longer sums keep the bits that 64 x 64 tiles give them (101 x 101 x 193 4.9 us, 3.6
-// with 16 x 16).
-constexpr double kUnalignedNarrowFrom = double(1 << 21);
 // From 129 k to there the second step of 128 or the first of 256 k is part empty: narrow tiles where they should gain 6 %.  Of
 // 260 such problems 31 were more than 2 % slower with less (A^T 798 x 549 x 185 1.09 of the time with 64 x 64, B^T 1233 x 137
 // x 189 1.07), none is so (0.92 in the mean); not those of bias and SiLU, whose results weigh more in the wide ones.
@@ -334,8 +332,6 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
         (K < kUnalignedFromK && double(M) * double(N) * double(K) < kUnalignedFrom))
       return e->name;
     first = std::begin(kUnalignedTiles), last = std::end(kUnalignedTiles);
-    if (double(M) * double(N) * double(K) < kUnalignedNarrowFrom)
-      last = first + 2;
   }
   const bool partEmpty = first == std::begin(kUnalignedTiles) && K > 128 && K < kUnalignedFromK && !strstr(e->name, "silu");
   const GemmTile *best = nullptr;

@@ -181,7 +181,7 @@ def test_kernel_variants_for_unaligned_rows(host):
     for base in ("imex_gemm_f16_f16_f32", "imex_gemm_f16_f16_f32_ta", "imex_gemm_f16_f16_f32_tb",
                  "imex_gemm_bf16_bias_silu_bf16"):
         assert v(base, [129, 129, 17]) == base and v(base, [101, 101, 191]) == base
-        assert v(base, [101, 101, 193]) == base + "_u64" and v(base, [1001, 1003, 99]) == base + "_u64"
+        assert v(base, [101, 101, 193]) == base + "_u16x16" and v(base, [1001, 1003, 99]) == base + "_u64"
         assert v(base, [4097, 4097, 4097]) == base + "_u128"
         assert shape(base + "_u64", [130, 65, 9])[0][0] == 6 and shape(base + "_u128", [130, 65, 9])[0][0] == 2
         assert v(base, [4097, 4097, 7]) == base and v(base, [4097, 4097, (1 << 22) + 1]) == base
