@@ -12,10 +12,10 @@
 // it touches: the change of layout costs no instruction.  One barrier per tile of rows hands a tile over and the other
 // one back; loads run one tile ahead or three (kAhead).
 // Workgroups of neighbouring segments run on one XCD, whose L2 then fetches a 128-byte line once for all of them (in launch
-// order / so: f32 sums of 8192 x 4096 42.7 / 37.0 us, 8192 x 2048 44.1 / 25.3, bf16 8192 x 4096 44.5 / 26.3; ordinary loads:
+// order / so: f32 sums of 8192 x 4096, one tile ahead, 42.7 / 37.0 us, 8192 x 2048 44.1 / 25.3, bf16 8192 x 4096 44.5 / 26.3; ordinary loads:
 // non-temporal ones lose the line, fused chain of f32 8192 x 512 50 us against 32).
 // What is left: f32 8192 x 8, one workgroup, takes 23.7 us, 2.6 ns a row behind the launch.  8192 x 2048 hides its loads
-// behind that (24.7); 8192 x 4096 does not, 33.3 us, 4.3 TB/s in 64-byte pieces of rows 16 KiB apart (rows of 16000 bytes 29.3).
+// behind that (24.7); 8192 x 4096 does not, 33.6 us, 4.0 TB/s in 64-byte pieces of rows 16 KiB apart (rows of 16000 bytes 29.1).
 #ifndef IMEX_HIP_COLUMN_CHAIN_H
 #define IMEX_HIP_COLUMN_CHAIN_H
 
@@ -32,6 +32,11 @@ __device__ __forceinline__ int chain_lanes(int64_t segments) { return segments <
 // four where it gets more of them, so that these share it (128 x 32768: 6.5 with eight, 3.9 with four).
 __device__ __forceinline__ int wide_chain_workers(int64_t segments) { return segments <= 4 * 256 ? 8 : 4; }
 
+// Whether a matrix of 64-byte segments is taken three tiles ahead: from 84 MiB on, a third of the 256 MiB cache, where
+// matrices in use together come from HBM (three in turn: from 92 MB on 0.91 .. 1.00 of the time with one tile, to 82 MB 1.00 ..
+// 1.15).
+__device__ __forceinline__ bool ahead_of(int64_t rows, int64_t pitch) { return rows * pitch >= int64_t(84) << 20; }
+
 // What the chains take: a tile's rows -- 64 where a row has more than 1024 segments, 512 at most -- within 32-bit offsets of
 // its first one.
 template <io::Dt D> __device__ __forceinline__ bool chains_take(int64_t rows, int64_t cols) {
@@ -46,7 +51,7 @@ __device__ __forceinline__ int lanes_launched() {
 }
 
 // kInputs matrices; kLanes lanes of a worker cover a row's segment with 8 bytes each; kWorkers wavefronts of workers.
-template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain {
+template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_, int kAhead_ = 1> struct ColumnChain {
   using E = io::Elem<D>;
   static constexpr int kInputs = kInputs_, kLanes = kLanes_, kWorkers = kWorkers_;
   static constexpr int kPer = 8 / E::kBytes;                    // columns per lane
@@ -54,13 +59,14 @@ template <io::Dt D, int kInputs_, int kLanes_, int kWorkers_> struct ColumnChain
   static constexpr int kRowsPerWave = 4 * (kWave / kLanes);     // rows of a tile that one worker wavefront takes
   static constexpr int kTileRows = kWorkers * kRowsPerWave;
   static constexpr int kThreads = (kWorkers + 1) * kWave;
-  // Tiles whose loads are in flight while one is evaluated.  Three for 64-byte segments of one input, of which a CU has one
-  // workgroup: one 8 KiB tile at a time left it waiting for memory, f32 8192 x 4096 37.2 us, 33.3 so, bf16 8192 x 8000 35.1 /
-  // 29.3 (five: 34.8, 30.2).  One elsewhere: 32-byte segments wait for their additions (4041 x 1792 13.3, with three 14.2),
-  // 128-byte ones of whole 4 KiB rows ask too much of the same channels (8192 x 8192 45.7 / 50.9, of other pitches 5 %
-  // faster), several workgroups on a CU have tiles of each other's in flight (8192 x 12000 65.0 / 75.1) and two inputs
-  // take the registers (fused chain of f32 1500 x 2048 9.1 / 10.0).
-  static constexpr int kAhead = kInputs == 1 && kLanes == 8 ? 3 : 1;
+  // Tiles whose loads are in flight while one is evaluated.  Three for 64-byte segments of one input from HBM, of which a CU
+  // has one workgroup: one 8 KiB tile at a time left it waiting for memory, f32 7449 x 3680 27.4 us, 25.2 so, bf16 8192 x 8000
+  // 31.6 / 29.1 (five: 30.2).  One where the caches have the matrix (ahead_of): f32 3745 x 4096 13.8, with three 14.5, f16 1261
+  // x 8192 6.4 / 7.0, 126 problems under 50 MB 1.06 times as long with three in the mean.  One elsewhere: 32-byte segments wait
+  // for their additions (4041 x 1792 13.3, with three 14.2), 128-byte ones of whole 4 KiB rows ask too much of the same channels
+  // (8192 x 8192 45.7 / 50.9, of other pitches 5 % faster), several workgroups on a CU have tiles of each other's in flight
+  // (8192 x 12000 65.0 / 75.1) and two inputs take the registers (fused chain of f32 1500 x 2048 9.1 / 10.0).
+  static constexpr int kAhead = kAhead_;
   static constexpr bool kNarrow = kLanes == 4; // takes rows of less than a segment too
   // Floats from one column of a tile to the next, and where a column keeps its rows: four rows (a "quad") are 16 bytes,
   // and quad q of a column that lane group j wrote is at place q ^ swizzle(j) within its four.  128-bit LDS accesses

@@ -457,11 +457,11 @@ extern "C" __global__ __launch_bounds__(kThreads) void imex_reduce_outer_bf16_de
 // form above) leaves the chip idle and waits for one slice's latency per four slices.  Column chains instead
 // (column_chain.h), whose workers have nothing to do but widen: the additions of one output are ordered, so a column costs
 // `outer` dependent additions whatever is done, 2.7 ns each here.  f32 8192 x 4096: 980 us in the plain form, 45.2 with a
-// 32-bit LDS read for every addition, 37.0 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 13.9;
+// 32-bit LDS read for every addition, 33.6 so (floor 21.3 for its bytes, 22 for the chain); 4041 x 1792 24.1 -> 13.9;
 // bf16 8192 x 4096 58.0 -> 26.3, where the adder widened as well; f16 2000 x 1001 16.6 -> 8.1, 500 x 20000 9.5 -> 5.8.
-template <io::Dt D, int kLanes, int kWorkers, bool kShort = false>
+template <io::Dt D, int kLanes, int kWorkers, bool kShort = false, int kAhead = 1>
 __device__ __forceinline__ void reduce_outer_chains(const void *in, void *out, int64_t outer, int64_t inner, float init, float *lds) {
-  using C = ColumnChain<D, 1, kLanes, kWorkers>;
+  using C = ColumnChain<D, 1, kLanes, kWorkers, kAhead>;
   using E = io::Elem<D>;
   C::template run<kShort>(in, nullptr, out, outer, inner, init, lds, [] {}, [](const typename C::Raw(&v)[1][4], float(&f)[4][C::kPer]) {
 #pragma unroll
@@ -492,6 +492,8 @@ __device__ __forceinline__ void reduce_outer_tall(const void *in, void *out, int
     reduce_outer_chains<D, 4, 4, true>(in, out, outer, inner, init, lds);
   else if (lanes == 4)
     reduce_outer_chains<D, 4, 4>(in, out, outer, inner, init, lds);
+  else if (lanes == 8 && ahead_of(outer, slice))
+    reduce_outer_chains<D, 8, 4, false, 3>(in, out, outer, inner, init, lds);
   else if (lanes == 8)
     reduce_outer_chains<D, 8, 4>(in, out, outer, inner, init, lds);
   else if (workers == 8)

@@ -929,9 +929,8 @@ def test_column_chains_bit_exact(host, orc, stream, dtype, rows, segments, extra
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("segments,extra", [(288, 1), (384, 0), (512, 0)])
 def test_column_chains_tiles_ahead(host, orc, stream, dtype, segments, extra):
-    """Sums of 64-byte segments, whose workers have three tiles of 128 rows in flight, over 1 .. 9 tiles and last tiles that
-    end on and beside the sixteen rows that are added at a time; rows of whole 4 KiB too, which pairs of XCDs share line by
-    line.  The oracle's bits, also with a sum of -0 behind which the padding of the last sixteen rows must leave no trace."""
+    """Sums of 64-byte segments over 1 .. 9 tiles of 128 rows and last tiles that end on and beside the sixteen rows that are
+    added at a time; rows of whole 4 KiB too.  The oracle's bits, also with a sum of -0 behind which the padding of the last sixteen rows must leave no trace."""
     cols = segments * (32 // (4 if dtype == "f32" else 2)) + extra
     wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
     narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
@@ -945,6 +944,30 @@ def test_column_chains_tiles_ahead(host, orc, stream, dtype, segments, extra):
             stream.wait()
             got = stream.from_device(d_out, (cols,), a.dtype)
             want = narrow(orc.reduce_outer_f32(wide(a[:rows]), -0.0))
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (rows, grid)
+    stream.free(d_in), stream.free(d_out)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("segments,extra", [(399, 3), (512, 0)])
+def test_column_chains_from_memory(host, orc, stream, dtype, segments, extra):
+    """The same from 84 MiB on, where three tiles are in flight: on both sides of the line, every number of tiles modulo the
+    four of the ring, last tiles that end on and beside sixteen rows.  The oracle's bits."""
+    cols = segments * (32 // (4 if dtype == "f32" else 2)) + extra
+    wide = lambda t: t if dtype == "f32" else orc.to_float(t, dtype)
+    narrow = lambda t: t if dtype == "f32" else orc.from_float(t, dtype)
+    first = -(-(84 << 20) // (cols * (4 if dtype == "f32" else 2)))
+    tiles = -(-first // 128)
+    most = (tiles + 4) * 128
+    a = orc.fill_uniform(most * cols, dtype, 64, -5.0, 5.0).reshape(most, cols)
+    d_in, d_out = stream.to_device(a), stream.alloc(cols * a.itemsize)
+    for rows in (first - 1, first, tiles * 128, tiles * 128 + 1, tiles * 128 + 144, tiles * 128 + 257, most - 1, most):
+        say("%d x %d" % (rows, cols))
+        for grid in (None, (7, 1, 1)):
+            stream.launch("imex_reduce_outer_%s_tall" % dtype, [rows, cols], [d_in, d_out, rows, cols, 0.25], grid=grid)
+            stream.wait()
+            got = stream.from_device(d_out, (cols,), a.dtype)
+            want = narrow(orc.reduce_outer_f32(wide(a[:rows]), 0.25))
             assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (rows, grid)
     stream.free(d_in), stream.free(d_out)
 
