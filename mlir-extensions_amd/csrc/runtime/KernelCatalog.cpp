@@ -260,13 +260,14 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
 // MiB of operands and `ahead` once, where it is worth more than the launch of 256 workgroups (fitted to 2100 other problems,
 // operands from beyond the L2s).  Timed on 1100 further ones, each with and without them on every tile (us without / with, from
 // HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from
-// the 256 MiB cache 11.3 / 7.1 for the second): the launches that get them take 0.71 of their time from HBM, 0.86 from that
-// cache and 0.89 where the L2s have the operands, there more than 1.02 on 7 of 290, 1.06 at most.  Not below 3.75 MiB and 1024
-// k, or 2 MiB and 2560 k, which the L2s may have (there 2 x 1560 x 1080 1.21, 391 x 176 x 1928 1.17), nor above 32 MiB, which
-// HBM's rate bounds (32 .. 48 MiB: 1.01), with fewer than 96 helpers (176 .. 192 tiles: up to 1.5) or for 128 x 128 tiles and
-// larger, which their own steps bound (above 16 MiB 1.03 .. 1.04).  They draw a problem to other tiles only where that holds from the
-// L2s too: not to 16 x 64 (from 16 x 32 1.03 of the time in the mean, 151 x 576 x 3456 1.21) and not to 16 x 32 with B^T (48 x
-// 1000 x 2064 1.12).
+// the 256 MiB cache 11.3 / 7.1 for the second): the launches that get them take 0.70 of their time from HBM, 0.86 from that
+// cache and 0.89 where the L2s have the operands, there more than 1.02 on 7 of 270, 1.06 at most.  Not below 3.75 MiB and 1024
+// k, or 2 MiB and 2560 k with half of the CUs free, which the L2s may have (there 2 x 1560 x 1080 1.21, 391 x 176 x 1928 1.17, 141
+// x 544 x 2800 1.08), nor above 32 MiB, which HBM's rate bounds (32 .. 48 MiB: 1.01; 128 x 64 tiles 16 MiB: B^T 3409 x 296 x 3776
+// 1.21), with fewer than 96 helpers (176 .. 192 tiles: up to 1.5) or for 128 x 128 tiles and larger, which their own steps
+// bound (above 16 MiB 1.03 .. 1.04).  They draw a problem to other tiles only where that holds from the L2s too: from 3.75 MiB
+// on (405 x 144 x 2920 1.09), not to 16 x 64 (from 16 x 32 1.03 of the time in the mean, 151 x 576 x 3456 1.21) and not to 16 x
+// 32 with B^T (48 x 1000 x 2064 1.12).
 struct GemmTile {
   const char *suffix;
   int tileM, tileN, stepK, constant, setup, store, step, stepMore;
@@ -284,11 +285,17 @@ constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810,
                                    {"_t16x32", 16, 32, 256, 1799, 466, 37, 489, 397, false, 196, 70, 889},
                                    {"_t16x16", 16, 16, 256, 2031, 385, 25, 379, 282, false, 146, 94, 761}};
 
+double operandMib(int64_t M, int64_t N, int64_t K) { return 2.0 * double(K) * (double(M) + double(N)) / (1 << 20); }
+
 // Whether workgroups without a tile are launched to fetch what the others read.
 bool fetchesAhead(const GemmTile &t, int64_t M, int64_t N, int64_t K) {
-  const double mib = 2.0 * double(K) * (double(M) + double(N)) / (1 << 20);
-  return ((K >= 1024 && mib >= 3.75) || (K >= 2560 && mib >= 2.0)) && mib <= 32.0 && t.tileM * t.tileN <= 128 * 64 &&
-         ceilDiv(M, t.tileM) * ceilDiv(N, t.tileN) <= 160;
+  const double mib = operandMib(M, N, K), tiles = double(ceilDiv(M, t.tileM)) * double(ceilDiv(N, t.tileN));
+  return ((K >= 1024 && mib >= 3.75 && tiles <= 160) || (K >= 2560 && mib >= 2.0 && tiles <= 128)) &&
+         t.tileM * t.tileN <= 128 * 64 && mib <= (t.tileM == 128 ? 16.0 : 32.0);
+}
+// Whether they count in the choice of a tile.
+bool drawnByFetching(const GemmTile &t, bool transB, int64_t M, int64_t N, int64_t K) {
+  return t.stepAhead && fetchesAhead(t, M, N, K) && operandMib(M, N, K) >= 3.75 && !(transB && t.tileM * t.tileN == 16 * 32);
 }
 
 // Bytes moved for an element of the result: read and written again, or written; the 16-bit result of bias and SiLU counts
@@ -342,8 +349,8 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
     const double load = t.shared ? std::max(1.0, tiles / 256.0) : std::ceil(tiles / 256.0);
     const double once = t.constant + load * (t.setup + t.store * storeBytes(e));
     double ns = once + steps * (t.step + (load - 1.0) * t.stepMore);
-    if (t.stepAhead && fetchesAhead(t, M, N, K) && !(transB && t.tileM * t.tileN == 16 * 32))
-      ns = std::min(ns, once + steps * t.stepAhead + 2.0 * double(K) * (double(M) + double(N)) / (1 << 20) * t.aheadMib + t.ahead);
+    if (drawnByFetching(t, transB, M, N, K))
+      ns = std::min(ns, once + steps * t.stepAhead + operandMib(M, N, K) * t.aheadMib + t.ahead);
     if (partEmpty && t.tileM * t.tileN < 64 * 64)
       ns /= kUnalignedNarrowGain;
     if (!best || ns < least) {

@@ -289,6 +289,9 @@ def test_gemm_workgroups_that_fetch_rule(host):
     assert [grid("_t16x16", 2, n, 1024) for n in (1912, 1920)] == [120, 256] and grid("_t16x16", 2, 2000, 1016) == 125
     assert [grid("_t16x16", 2, n, 2560) for n in (400, 424)] == [25, 256] and grid("_t16x16", 2, 424, 2552) == 27
     assert grid("_t16x16", 2, 1560, 1080) == 98 and grid("_t16x32", 391, 176, 1928) == 150
+    assert grid("_t16x32", 141, 544, 2800) == 153 and grid("_t16x32", 141, 448, 2800) == 256  # 2 MiB: 128 tiles at most
+    assert grid("_t128x64", 3409, 296, 3776) == 135 and grid("_t64", 1500, 296, 4096) == grid("_t128x64", 1500, 296, 4096) == 256
+    assert grid("_t64", 1500, 384, 4096) == 256 and grid("_t128x64", 1700, 392, 4096) == 98
 
 
 def test_gemm_workgroups_that_fetch_do_not_draw_problems_to_slower_tiles(host):
@@ -298,6 +301,8 @@ def test_gemm_workgroups_that_fetch_do_not_draw_problems_to_slower_tiles(host):
         assert tile("f16_f16_f32_tb", m, n, k) == "_t16x32", (m, n, k)
     assert tile("bf16_bf16_f32_acc", 329, 288, 2432) == tile("f16_f16_f32_acc", 551, 224, 3056) == "_t16x32"
     assert tile("f16_f16_f32_tb", 48, 1000, 2064) == "_t16x16" and tile("f16_f16_f16", 156, 400, 2152) == "_t16x16"
+    for m, n, k in ((405, 144, 2920), (414, 136, 3456), (286, 144, 2784), (178, 224, 2656)):
+        assert tile("f16_f16_f32", m, n, k) == "_t16x16", (m, n, k)
     assert tile("f16_f16_f32_ta", 104, 1648, 3288) == "_t32" and tile("bf16_bias_silu_bf16", 15, 2624, 2904) == "_t16x32"
 
 
