@@ -418,13 +418,16 @@ const char *softmaxVariant(const Entry *e, int64_t rows, int64_t cols) {
 // brings together in one L2 (16-bit 6000 x 6000 42.0 -> 34.1 us, 4104 x 4096 18.4 -> 16.1, 11472 x 3312 43.1 -> 37.2, 32-bit
 // 3000 x 2000 14.8 -> 11.7; 98 of 260 timed problems, 0.82 of their time in the mean).  With whole halves of lines it is as
 // often the other way (16-bit 13280 x 2048 22.5, 24.9, 32-bit 6000 x 6000 62.8, 62.4), and so it is with a few columns, which
-// tiles of 64 fit badly (16-bit 63352 x 280 18.3, 22.0).
+// tiles of 64 fit badly (16-bit 63352 x 280 18.3, 22.0): tall 16-bit ones of 5.5 .. 15 MB, of 500 timed problems the only ones
+// that were more than 4 % slower (16336 x 200 1.14 of the time, 20568 x 264 6.9, 7.3, 20360 x 232 6.0, 6.4; 16336 x 256 0.74).
 const char *transposeVariant(const Entry *e, const int64_t *dims) {
   const int64_t perVec = e->shape == Shape::Transpose2D32 || e->shape == Shape::Transpose3D32 ? 4 : 8;
   const int64_t rows = dims[0], cols = dims[e->ndims - 1], planes = e->ndims == 3 ? dims[1] : 1;
   const bool halves = uint64_t(rows) * uint64_t(planes) % uint64_t(4 * perVec) == 0; // of cache lines, in the result
-  if (rows < perVec || cols < perVec ||
-      (rows % perVec == 0 && cols % perVec == 0 && (halves || rows / 128 > cols)))
+  const double bytes = 16.0 / double(perVec) * double(rows) * double(cols);
+  const bool tall = rows / 128 > cols ||
+                    (perVec == 8 && planes == 1 && rows / 12 > cols && cols % 64 != 0 && bytes >= 5.5e6 && bytes <= 15e6);
+  if (rows < perVec || cols < perVec || (rows % perVec == 0 && cols % perVec == 0 && (halves || tall)))
     return e->name;
   char name[96];
   snprintf(name, sizeof name, "%s_any", e->name);
