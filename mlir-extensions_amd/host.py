@@ -304,10 +304,15 @@ class Stream:
         weakref.finalize(self, _free_staging, self.rt, self._staging).atexit = False  # a queue that nobody closes
         self._unstaged = 0  # operators that have gone without a block of their size since the last one was made
 
+    def _free_kept(self):
+        """What `staging` keeps goes, but for what another thread takes first."""
+        with contextlib.suppress(IndexError):
+            while True:
+                self.free(self._staging.pop()[0])
+
     def close(self):
         if self.handle:
-            while self._staging:
-                self.free(self._staging.pop()[0])
+            self._free_kept()
             self.rt.gpuStreamDestroy(self.handle)
             self.handle = None
 
@@ -379,7 +384,7 @@ class Stream:
         took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 ms (to 2 MiB), 0.09 (4 MiB) ..
         0.15, so a block pays after about that many: a queue that ends just then has lost a quarter by it (ten calls on 8
         MiB that got it after eight 5.2 -> 8.1 ms), and one of a hundred takes 0.43 .. 0.8 of the time."""
-        if self._staging and len(self._staging[0][1]) >= nbytes:
+        if any(len(block) >= nbytes for _, block in self._staging[:1]):  # another thread's `staging` may take it meanwhile
             return True
         size = _staging_size(nbytes)
         self._unstaged += 1
@@ -389,8 +394,7 @@ class Stream:
         ptr = self.rt.imexHipTrySharedAlloc(self.handle, size)
         if not ptr:
             return False
-        while self._staging:
-            self.free(self._staging.pop()[0])
+        self._free_kept()
         self._staging.append((Ptr(ptr), _bytes_at(ptr, size)))
         return True
 

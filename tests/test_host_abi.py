@@ -503,6 +503,24 @@ def test_staged_operators_share_one_block(host, fake_stream):
     assert len(calls) == 1 and len(fake_stream._staging) == 1 and len(pinned(fake_stream)) == 1
 
 
+def test_staged_operators_beside_a_thread_that_takes_the_block(host, fake_stream):
+    """`staging` of another thread may take the kept block at any moment: between a look whether there is one and a look
+    at it, or before it is given back for a larger one."""
+    class Taken(list):  # as a list from which the one block goes right after the look
+        def __bool__(self):
+            return True
+
+        def __len__(self):
+            return 1
+    small, large = np.zeros(100, np.float32), np.zeros(1 << 19, np.float32)
+    for x in [small] * 3 + [large] * 11:
+        fake_stream._staging = Taken()
+        assert np.array_equal(host.relu(fake_stream, x), x)
+        while list.__len__(fake_stream._staging):
+            fake_stream.free(fake_stream._staging.pop()[0])
+    fake_stream._staging = []
+
+
 @pytest.mark.parametrize("n,waits", [(1, 1), (1 << 16, 1), (1 << 17, 2), ((1 << 17) + 1, 5), (1 << 20, 20), (1 << 22, 80)])
 def test_staged_operators_wait_for_a_block(host, fake_stream, n, waits):
     """A queue's first calls go through device buffers, five for every two MiB of the pinned block that they would get:
