@@ -51,7 +51,9 @@ template <typename T, bool kStrided, int TR, int BK> struct UnalignedOperand : S
   int shift[kCopies];      // places by which the piece has to move down in the last step
   int put;                 // per-lane LDS address of copy 0 inside the image
 
-  // K >= 8, and ld >= 8 where kStrided; ld < 2^22 keeps the offsets below 2^30
+  // K >= 8, and ld >= 8 where kStrided.  ld < 2^22 keeps a strided operand's offsets, (BK - 1) rows and one row's columns, below
+  // 2^31 with BK = 256, and a k-contiguous one's, TR - 1 rows and the last step's end, below 2^30.
+  static_assert((uint64_t(kStrided ? BK : TR) << 22) * 2 <= uint64_t(1) << 31, "rows of up to 2^22 elements within 32-bit offsets");
   __device__ __forceinline__ void setup(const uint16_t *ptr, int64_t ld, int64_t first, int64_t rows, int w0, int wave,
                                         int lane, int steps, int kRem) {
     this->setup_read(w0, lane);
