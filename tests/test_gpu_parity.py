@@ -1266,11 +1266,13 @@ def test_flash_attention_tiling_by_size(host, orc, stream, zh, n_ctx, tiling):
     assert np.max(np.abs(got[ok] - ref[ok])) <= 2.0 ** -10 + 2.0 ** -11 * np.max(np.abs(ref[ok]))
 
 
+@pytest.mark.parametrize("queries", [32, 64, 128, 256])
 @pytest.mark.parametrize("order", ["up", "down", "jumps"])
 @pytest.mark.parametrize("zh,n_ctx", [(1, 769), (3, 1000), (2, 2080)])
-def test_flash_attention_moving_maximum(host, orc, stream, zh, n_ctx, order):
-    """Scores that grow by less than a factor of 2^8 from tile to tile, that fall, and that jump from key to key: the
-    reference that the exponentials are taken against lags the maximum; workgroups that 8 does not divide."""
+def test_flash_attention_moving_maximum(host, orc, stream, zh, n_ctx, order, queries):
+    """Scores that grow by less than a factor of 2^8 from tile to tile, so that every tile rescales what the ones before it
+    left, that fall, so that none but the first does, and that jump from key to key, in the kernels with one tiling each;
+    workgroups that 8 does not divide."""
     n = zh * n_ctx
     q = orc.fill_uniform(n * 64, "f16", 93, -0.5, 0.5).reshape(n, 64)
     k = orc.fill_uniform(n * 64, "f16", 94, -0.5, 0.5).reshape(n, 64)
@@ -1279,7 +1281,13 @@ def test_flash_attention_moving_maximum(host, orc, stream, zh, n_ctx, order):
     at = np.arange(n) % n_ctx
     ramp = {"up": at / 64.0, "down": -at / 64.0, "jumps": 40.0 * ((at * 7919) % 13 == 0) - 20.0}[order]
     k[:, 0] = ramp.astype(np.float16).view(np.uint16)
-    got = host.flash_attention(stream, q, k, v, zh, n_ctx, 0.5)
+    say("attention %dx%d %s, %d queries per workgroup" % (zh, n_ctx, order, queries))
+    d_q, d_k, d_v, d_o = (stream.to_device(t) for t in (q, k, v, np.zeros_like(q)))
+    stream.launch("imex_flash_attention_fwd_f16_q%d" % queries, [zh, n_ctx], [d_q, d_k, d_v, d_o, 0.5, zh, n_ctx])
+    stream.wait()
+    got = stream.from_device(d_o, q.shape, np.uint16)
+    for p in (d_q, d_k, d_v, d_o):
+        stream.free(p)
     rows = np.unique(np.concatenate([np.arange(0, n, 11), [n_ctx - 1, n - 1]]))
     assert attention_close(got[rows], orc.flash_attention_rows(q, k, v, n_ctx, 0.5, rows), orc)
 
