@@ -351,9 +351,10 @@ __device__ __forceinline__ void fetch_ahead(const uint16_t *A, const uint16_t *B
   };
   const Block blocks[2] = {block(from, turnover), block(turnover, to)};
   uint32_t turn;
-  // Rows (k-contiguous) or columns (strided) first .. last - 1 of an operand, ks of its k from k0 on: a row, or a k row, for
-  // each wavefront in turn.  (Few instructions per copy: with addresses in 64 bits the copies of 200 bytes and less, 0.15 us
-  // each, took longer than the tiles.)
+  // Rows (k-contiguous) or columns (strided) first .. last - 1 of an operand, ks of its k from k0 on: a row for each wavefront
+  // in turn, or as many k rows as 64 pieces of 16 bytes hold.  (Few instructions per copy, and few copies, 0.15 us each: with
+  // addresses in 64 bits, or one k row of 200 bytes and less in each, they took longer than the tiles.  One k row each, operands
+  // in the L2s: A^T 112 x 72 x 6760 8.7 us without workgroups that fetch, 13.7 with them.)
   auto fetch = [&](const uint16_t *ptr, bool strided, uint32_t ld, uint32_t first, uint32_t last, uint32_t k0, uint32_t ks) {
     const uint32_t count = strided ? ks : last - first, bytes = (strided ? last - first : ks) * 2, pitch = ld * 2;
     if (first >= last || uint64_t(count) * pitch >= kOutOfRange)
@@ -361,6 +362,15 @@ __device__ __forceinline__ void fetch_ahead(const uint16_t *A, const uint16_t *B
     const uint16_t *base = ptr + (strided ? uint64_t(k0) * ld + first : uint64_t(first) * ld + k0);
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(base), 0, int((count - 1) * pitch + bytes), 0x00020000);
+    if (strided && bytes <= 512) {
+      const uint32_t pieces = bytes / 16, rows = 64 / pieces, row = lane / pieces, off = row * pitch + (lane - row * pieces) * 16;
+      const uint32_t copies = (count + rows - 1) / rows;
+      for (; turn < copies; turn += turns)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, sink, 16, row < min(rows, count - turn * rows) ? turn * rows * pitch + off : kOutOfRange,
+                                                 0, 0, 0);
+      turn -= copies;
+      return;
+    }
     for (; turn < count; turn += turns)
       for (uint32_t b = 0; b < bytes; b += 1024)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, sink, 16, b + lane * 16 < bytes ? b + lane * 16 : kOutOfRange,
