@@ -258,16 +258,19 @@ extern "C" const void *imexHipKernelModule(const char *kernel, size_t *size) {
 //
 // Workgroups that fetch for others (fetch_ahead in gemm_small.h) change what a step costs: stepAhead per step, aheadMib per
 // MiB of operands and `ahead` once, where it is worth more than the launch of 256 workgroups (fitted to 2100 other problems,
-// operands from beyond the L2s).  Timed on 1100 further ones, each with and without them on every tile (us without / with, from
-// HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from
-// the 256 MiB cache 11.3 / 7.1 for the second): the launches that get them take 0.70 of their time from HBM, 0.86 from that
-// cache and 0.89 where the L2s have the operands, there more than 1.02 on 7 of 270, 1.06 at most.  Not below 3.75 MiB and 1024
-// k, or 2 MiB and 2560 k with half of the CUs free, which the L2s may have (there 2 x 1560 x 1080 1.21, 391 x 176 x 1928 1.17, 141
-// x 544 x 2800 1.08), nor above 32 MiB, which HBM's rate bounds (32 .. 48 MiB: 1.01; 128 x 64 tiles 16 MiB: B^T 3409 x 296 x 3776
-// 1.21), with fewer than 96 helpers (176 .. 192 tiles: up to 1.5) or for 128 x 128 tiles and larger, which their own steps
-// bound (above 16 MiB 1.03 .. 1.04).  They draw a problem to other tiles only where that holds from the L2s too: from 3.75 MiB
-// on (405 x 144 x 2920 1.09), not to 16 x 64 (from 16 x 32 1.03 of the time in the mean, 151 x 576 x 3456 1.21) and not to 16 x
-// 32 with B^T (48 x 1000 x 2064 1.12).
+// operands from beyond the L2s; us without / with, from HBM: 16 x 1024 x 4096 10.9 / 6.2, 16 x 2048 x 4096 14.0 / 7.2, 16 x
+// 1680 x 3992 11.8 / 7.3, 128 x 2048 x 4096 15.3 / 10.8; from the 256 MiB cache 11.3 / 7.1 for the second).  On 900 further ones
+// the launches that get them, with the tiles chosen by these numbers, take 0.84 of the time without from that cache (more than
+// 1.04 on 15, 1.12 at most) and 0.94 where the L2s have the operands (more than 1.1 on 29).  Not below 3.75 MiB and 1024 k, 16 x
+// 16 tiles 1400, or 2 MiB and 2560 k with half of the CUs free, which the L2s may have (there 2 x 1560 x 1080 1.21, 391 x 176 x
+// 1928 1.17, 141 x 544 x 2800 1.08; 5 x 1720 x 1184 1.18, from the cache 1.11), nor above 32 MiB, which HBM's rate bounds (32 ..
+// 48 MiB: 1.01; 128 x 64 tiles 16 MiB: B^T 3409 x 296 x 3776 1.21), with fewer than 96 helpers (176 .. 192 tiles: up to 1.5) or for
+// 128 x 128 tiles and larger, which their own steps bound (above 16 MiB 1.03 .. 1.04).  An XCD's share of the operands beyond
+// its 4 MiB L2 is gone before it is read: from 6 MiB on there are none (1560 x 168 x 9680 1.06), and they draw a problem to
+// other tiles below 4 MiB only (above, 12 of 12 that went from 16 x 64 to 32 x 64 1.03 .. 1.18, 640 x 600 x 12064 to 64 x 64
+// 1.32; below 0.87 in the mean), and only where that holds from the L2s too: from 3.75 MiB of all operands on (405 x 144 x 2920
+// 1.09), not to 16 x 64 (from 16 x 32 1.03 of the time in the mean, 151 x 576 x 3456 1.21) and not to 16 x 32 with B^T (48 x 1000
+// x 2064 1.12).
 struct GemmTile {
   const char *suffix;
   int tileM, tileN, stepK, constant, setup, store, step, stepMore;
@@ -287,15 +290,25 @@ constexpr GemmTile kGemmTiles[] = {{"", 256, 256, 32, 3705, 5101, 691, 581, 810,
 
 double operandMib(int64_t M, int64_t N, int64_t K) { return 2.0 * double(K) * (double(M) + double(N)) / (1 << 20); }
 
+// MiB that the tiles of one XCD, an eighth of them in bands of four tile rows (small_tile_origin), read.
+double operandMibOfXcd(const GemmTile &t, int64_t M, int64_t N, int64_t K) {
+  const double tilesM = double(ceilDiv(M, t.tileM)), tilesN = double(ceilDiv(N, t.tileN)), tiles = std::ceil(tilesM * tilesN / 8.0);
+  const double rows = std::min(4.0, tilesM), cols = std::min(tilesN, std::ceil(tiles / rows));
+  const double bands = std::ceil(tiles / (rows * tilesN));
+  return operandMib(std::min(M, int64_t(bands * rows) * t.tileM), std::min(N, int64_t(cols) * t.tileN), K);
+}
+
 // Whether workgroups without a tile are launched to fetch what the others read.
 bool fetchesAhead(const GemmTile &t, int64_t M, int64_t N, int64_t K) {
   const double mib = operandMib(M, N, K), tiles = double(ceilDiv(M, t.tileM)) * double(ceilDiv(N, t.tileN));
-  return ((K >= 1024 && mib >= 3.75 && tiles <= 160) || (K >= 2560 && mib >= 2.0 && tiles <= 128)) &&
-         t.tileM * t.tileN <= 128 * 64 && mib <= (t.tileM == 128 ? 16.0 : 32.0);
+  const int64_t from = t.tileM * t.tileN <= 16 * 16 ? 1400 : 1024;
+  return ((K >= from && mib >= 3.75 && tiles <= 160) || (K >= 2560 && mib >= 2.0 && tiles <= 128)) &&
+         t.tileM * t.tileN <= 128 * 64 && mib <= (t.tileM == 128 ? 16.0 : 32.0) && operandMibOfXcd(t, M, N, K) < 6.0;
 }
 // Whether they count in the choice of a tile.
 bool drawnByFetching(const GemmTile &t, bool transB, int64_t M, int64_t N, int64_t K) {
-  return t.stepAhead && fetchesAhead(t, M, N, K) && operandMib(M, N, K) >= 3.75 && !(transB && t.tileM * t.tileN == 16 * 32);
+  return t.stepAhead && fetchesAhead(t, M, N, K) && operandMib(M, N, K) >= 3.75 && operandMibOfXcd(t, M, N, K) < 4.0 &&
+         !(transB && t.tileM * t.tileN == 16 * 32);
 }
 
 // Bytes moved for an element of the result: read and written again, or written; the 16-bit result of bias and SiLU counts

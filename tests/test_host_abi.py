@@ -295,8 +295,11 @@ def test_gemm_workgroups_that_fetch_rule(host):
     assert grid("_t16x16", 16, 1680, 3992) == grid("_t32", 128, 2048, 4096) == grid("_t128x64", 1000, 1000, 1024) == 256
     assert grid("_t16x16", 16, 1680, 760) == 105 and grid("_t16x16", 16, 640, 1024) == 40 and grid("_t64", 16, 8192, 4096) == 128
     assert grid("_t16x16", 16, 2816, 1024) == 176 and grid("_t128", 1000, 1000, 1024) == 64
-    # operands that the L2s may hold: from 1024 k and 3.75 MiB, or 2560 k and 2 MiB
-    assert [grid("_t16x16", 2, n, 1024) for n in (1912, 1920)] == [120, 256] and grid("_t16x16", 2, 2000, 1016) == 125
+    # operands that the L2s may hold: from 1024 k (16 x 16 1400) and 3.75 MiB, or 2560 k and 2 MiB
+    assert [grid("_t16x32", 2, n, 1024) for n in (1912, 1920)] == [60, 256] and grid("_t16x32", 2, 2000, 1016) == 63
+    assert [grid("_t16x16", 5, 1720, k) for k in (1184, 1392, 1400)] == [108, 108, 256]
+    # an XCD's share of the operands: below 6 MiB, of a 4 MiB L2
+    assert [grid("_t32", 1560, 168, k) for k in (7416, 7424, 9680)] == [256, 147, 147]
     assert [grid("_t16x16", 2, n, 2560) for n in (400, 424)] == [25, 256] and grid("_t16x16", 2, 424, 2552) == 27
     assert grid("_t16x16", 2, 1560, 1080) == 98 and grid("_t16x32", 391, 176, 1928) == 150
     assert grid("_t16x32", 141, 544, 2800) == 153 and grid("_t16x32", 141, 448, 2800) == 256  # 2 MiB: 128 tiles at most
@@ -314,6 +317,17 @@ def test_gemm_workgroups_that_fetch_do_not_draw_problems_to_slower_tiles(host):
     for m, n, k in ((405, 144, 2920), (414, 136, 3456), (286, 144, 2784), (178, 224, 2656)):
         assert tile("f16_f16_f32", m, n, k) == "_t16x16", (m, n, k)
     assert tile("f16_f16_f32_ta", 104, 1648, 3288) == "_t32" and tile("bf16_bias_silu_bf16", 15, 2624, 2904) == "_t16x32"
+
+
+def test_gemm_workgroups_that_fetch_do_not_draw_problems_beyond_an_l2(host):
+    """Problems whose tiles of one XCD read more than its 4 MiB L2, where the fetched lines were gone before their use: up to
+    1.3 times as long with the tiles that they were drawn to."""
+    tile = lambda kind, *dims: host.variant("imex_gemm_" + kind, list(dims))[len("imex_gemm_" + kind):]
+    for kind, *dims in (("f16_f16_f16", 200, 800, 12944), ("bf16_bf16_f32", 416, 320, 8480), ("f16_f16_f32_tb", 496, 360, 11656),
+                        ("bf16_bf16_f32_acc", 64, 2272, 6520), ("bf16_bias_silu_bf16", 27, 4184, 3936)):
+        assert tile(kind, *dims) == "_t16", (kind, dims)
+    assert tile("f16_f16_f32", 640, 600, 12064) == "_t32"
+    assert tile("bf16_bias_silu_bf16", 155, 912, 6552) == "_t32" and tile("bf16_bias_silu_bf16", 155, 912, 6560) == "_t16"
 
 
 def test_plan_packs_arguments_as_the_kernel_declares_them(host):
