@@ -79,12 +79,20 @@ __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 
 
 // Workgroups go to the 8 XCDs round-robin in launch order, and each XCD has its own L2.  Renumber them so that one XCD gets
 // consecutive query blocks -- whole heads, or a contiguous part of one; as many as the others or one more -- and its L2
-// holds the K / V of a few heads instead of a slice of the traffic of all of them.
-__device__ __forceinline__ void place_of_workgroup(uint32_t &x, uint32_t &y) {
-  const uint32_t total = gridDim.x * gridDim.y, launched = blockIdx.y * gridDim.x + blockIdx.x, xcd = launched & 7;
-  const uint32_t logical = xcd * (total >> 3) + min(xcd, total & 7) + (launched >> 3);
-  y = logical / gridDim.x;
-  x = logical - y * gridDim.x;
+// holds the K / V of a few heads instead of a slice of the traffic of all of them.  A launch that 8 does not divide only
+// where `uneven` says so: the way there takes 0.1 .. 0.3 us longer than launch order, which 32 queries, whose one round has
+// little to share, and few keys do not get back (1 x 52 with it 4.50 us, 3.89 so; 28 such problems of 32 queries of 1024 keys
+// and more 1.00 .. 1.02 of the time with it; others from 256 keys on 0.85 .. 1.00: 165 x 513 38.4 in launch order, 35.3).
+__device__ __forceinline__ void place_of_workgroup(uint32_t &x, uint32_t &y, bool uneven) {
+  const uint32_t total = gridDim.x * gridDim.y;
+  x = blockIdx.x;
+  y = blockIdx.y;
+  if (total % 8 == 0 || uneven) {
+    const uint32_t launched = y * gridDim.x + x, xcd = launched & 7;
+    const uint32_t logical = xcd * (total >> 3) + min(xcd, total & 7) + (launched >> 3);
+    y = logical / gridDim.x;
+    x = logical - y * gridDim.x;
+  }
 }
 
 // ---- any-shape path: one lane per query, the reference loop ----------------------------
@@ -200,7 +208,7 @@ __device__ __forceinline__ void attention_tiled(const uint16_t *__restrict__ Q, 
   const int wq = wave % QB, wk = wave / QB;
   const int qi = lane & 31, half = lane >> 5;
   uint32_t bx, by;
-  place_of_workgroup(bx, by);
+  place_of_workgroup(bx, by, N >= 256);
   const int64_t head0 = int64_t(by) * N;                 // first row of this (batch, head)
   const int64_t q0 = head0 + int64_t(bx) * (32 * QB) + wq * 32;
   // N_CTX need not divide the tiles.  Queries past the end of the head are computed on a copy of
@@ -520,7 +528,7 @@ __device__ __forceinline__ void attention_own_keys(const uint16_t *__restrict__ 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int qi = lane & 31, half = lane >> 5;
   uint32_t bx, by;
-  place_of_workgroup(bx, by);
+  place_of_workgroup(bx, by, false);
   const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 32;
   const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
   const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
@@ -687,7 +695,7 @@ __device__ __forceinline__ void attention_pairs(const uint16_t *__restrict__ Q, 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int qi = lane & 31, half = lane >> 5;
   uint32_t bx, by;
-  place_of_workgroup(bx, by);
+  place_of_workgroup(bx, by, N >= 256);
   const int64_t head0 = int64_t(by) * N, q0 = head0 + int64_t(bx) * 64;
   const int tiles = int((N + kOwnKeys - 1) / kOwnKeys), lastRows = int(N - int64_t(tiles - 1) * kOwnKeys);
   const int iters = tiles > wave ? (tiles - wave + kOwnWaves - 1) / kOwnWaves : 0;
