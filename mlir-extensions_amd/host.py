@@ -14,6 +14,7 @@ from __future__ import annotations
 import contextlib
 import ctypes as C
 import functools
+import math
 import operator
 import os
 import re
@@ -384,7 +385,8 @@ class Stream:
         took 3.8 ms instead of 2.3, over 32 MiB 13.6 instead of 2.2.  A later call gains 0.02 ms (to 2 MiB), 0.09 (4 MiB) ..
         0.15, so a block pays after about that many: a queue that ends just then has lost a quarter by it (ten calls on 8
         MiB that got it after eight 5.2 -> 8.1 ms), and one of a hundred takes 0.43 .. 0.8 of the time."""
-        if any(len(block) >= nbytes for _, block in self._staging[:1]):  # another thread's `staging` may take it meanwhile
+        kept = self._staging[:1]  # another thread's `staging` may take it meanwhile
+        if kept and len(kept[0][1]) >= nbytes:
             return True
         size = _staging_size(nbytes)
         self._unstaged += 1
@@ -600,7 +602,7 @@ def _staged(stream, kernel, xs, dims, extra, out_shape, out_np, most):
     """The operator through pinned host memory, or None where that is not the faster way: for more than `most` bytes
     (or _STAGED_BYTES with each array on 256), for nothing, before the queue's block pays, while another thread's call has
     it, and under the profiler, which times kernels on device memory."""
-    n_out = int(np.prod(out_shape)) * np.dtype(out_np).itemsize  # () is one element
+    n_out = math.prod(out_shape) * np.dtype(out_np).itemsize  # () is one element
     total = sum(x.nbytes for x in xs) + n_out
     if total > most or not n_out or not xs[0].nbytes or "IMEX_ENABLE_PROFILING" in os.environ:
         return None
@@ -628,7 +630,7 @@ def _unary(stream, kernel, x, dtype, dims, extra=(), out_shape=None, out_np=None
     _check(x, dtype)
     out_shape = x.shape if out_shape is None else out_shape
     out_np = x.dtype if out_np is None else out_np
-    n_out = int(np.prod(out_shape)) if len(out_shape) else 1
+    n_out = math.prod(out_shape)
     out = _staged(stream, kernel, [x], dims, extra, out_shape, out_np, staged)
     if out is not None:
         return out
@@ -658,7 +660,7 @@ def _binary(stream, kernel, a, b, dtype, dims, out_shape, staged=_STAGED_BYTES):
     _check(b, dtype)
     if a.shape != b.shape:
         raise ValueError("operand shapes differ: %s vs %s" % (a.shape, b.shape))
-    n_out = int(np.prod(out_shape))
+    n_out = math.prod(out_shape)
     out = _staged(stream, kernel, [a, b], dims, (), out_shape, a.dtype, staged)
     if out is not None:
         return out
@@ -769,7 +771,7 @@ def reduce_outer(stream, x, init=0.0, dtype="f32"):
     """benchmarks/reduce/reduce_gpu.mlir.in:4-21: the outermost dim is summed away (f16 / bf16: bit
     patterns in and out, f32 accumulation)."""
     outer = x.shape[0]
-    inner = int(np.prod(x.shape[1:]))
+    inner = math.prod(x.shape[1:])
     return _unary(stream, "imex_reduce_outer_" + dtype, x, dtype, [outer, inner], extra=[float(init)],
                   out_shape=x.shape[1:], staged=_staged_columns(outer, inner))
 
