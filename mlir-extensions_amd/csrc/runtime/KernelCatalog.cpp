@@ -387,7 +387,9 @@ const char *gemmVariant(const Entry *e, int64_t M, int64_t N, int64_t K) {
 //          f16 15 x 2283888 18.3, 12.6);
 //   tall   a launch, a slice's share of the chain, and what a CU pays for further workgroups; 4.9 TB/s at most;
 //   deep   a slice costs its share of sixteen slices' latency, which its bytes hide little of; 8.0 (5.1) TB/s at most.
-// 8192 x 4096 f32: plain 980, tall 37, deep 540 us; 62 x 32296: tall 4.1, deep 7.0; 568 x 197848: 102, 66.  Below 64
+// 8192 x 4096 f32: plain 980, tall 34, deep 540 us; 62 x 32296: tall 3.7, deep 7.0; 568 x 197848: 102, 66.  With three tiles
+// in flight tall is up to 0.87 of its estimate, where deep is far off: of 150 problems of 200 .. 3000 segments the choice is the
+// faster one of the two on all, but for what two runs differ (0.4 % in the mean).  Below 64
 // outputs (1 .. 15, 8 .. 10^5 slices) tall is never slower than deep by more than 0.1 us: 64 x 4 both 3.3, 256 x 4 3.3 / 8.5.
 const char *reduceVariant(const Entry *e, int64_t outer, int64_t inner) {
   const bool f32 = e->shape == Shape::ReduceOuter;
