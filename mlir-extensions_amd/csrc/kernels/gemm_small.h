@@ -297,7 +297,8 @@ __device__ __forceinline__ void gemm_small_tile(const uint16_t *__restrict__ A, 
 }
 
 // Tile number -> tile, as tile_origin of gemm_tile.h: the workgroups of an XCD (ids congruent mod 8) take a compact
-// band of tiles, four tile rows high; as many tiles for each XCD, or one more.
+// band of tiles, four tile rows high; as many tiles for each XCD, or one more.  (With the last tiles % 8 in launch order behind
+// eight equal shares instead, 411 products that 8 does not divide take 1.006 of the time in the mean, 0.93 .. 1.11.)
 constexpr uint32_t kXcds = 8;
 __device__ __forceinline__ uint32_t first_tile_of_xcd(uint32_t xcd, uint32_t tiles) {
   return xcd * (tiles / kXcds) + min(xcd, tiles % kXcds);
